@@ -116,6 +116,9 @@ __global__ void __launch_bounds__(256) bias_prepass_kernel(const void* __restric
 	}
 }
 
+// one slot of a bias ring: 32 rows x 64 keys, and behind them one dword per row where rows start at any element
+constexpr int bias_slot_bytes(int bmode) { return bmode == 3 ? 4096 + 128 : 4096; }
+
 // DP: head_dim padded to a multiple of 32 (32 or 64).  NW: wavefronts per workgroup.  L2DOM: log2
 // variant (bias from the workspace, or no bias at all).  BIAS_F32: bias stored as fp32 (natural
 // variant only).  SPLIT: for launches too small to fill the chip -- the NW wavefronts of a workgroup
@@ -151,13 +154,15 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 	constexpr int QT         = SPLIT ? 32 : KS2 ? NW * 16 : NW * 32;
 	constexpr int  LDS_SETS   = SPLIT ? NW : 1;  // private K/V buffer sets
 	constexpr bool BIAS_F32   = BMODE == 1;      // natural variant, bias stored as fp32, read in place
-	constexpr bool BRING      = BMODE == 2;      // natural variant, bf16 bias streamed through a per-wavefront LDS ring
+	constexpr bool BRING      = BMODE >= 2;      // natural variant, bf16 bias streamed through a per-wavefront LDS ring
+	constexpr bool RAGGED     = BMODE == 3;      // ... whose rows start at any element: fetched from the dword below, shifted when read
+	constexpr int  SLOT_BYTES = bias_slot_bytes(BMODE);
 	// tile buffers of the K/V ring and slots of a bias ring.  With loading wavefronts the loads run two tiles ahead; KS2 in
 	// addition has every tile in LDS one barrier before its first use, so that a stage's LDS operands are fetched at the end of
 	// the stage before it (AHEAD: the tile that has landed when iteration j passes its barrier is j + AHEAD).
 	constexpr int  AHEAD      = KS2 ? 2 : 1;
 	constexpr int  NBUF       = LOADERS ? AHEAD + 3 : 3;
-	constexpr int  RING_BYTES = BRING ? (KS2 ? NW / 2 : NW) * NBUF * 4096 : 0;  // (KS2: one ring per pair of wavefronts)
+	constexpr int  RING_BYTES = BRING ? (KS2 ? NW / 2 : NW) * NBUF * SLOT_BYTES : 0;  // (KS2: one ring per pair of wavefronts)
 	constexpr int  MASK_BASE  = LDS_SETS * 2 * NBUF * TILE_BYTES + RING_BYTES;
 	static_assert(!(L2DOM && BMODE != 0), "the log2 variant reads its bias from the workspace");
 	static_assert(FUSED || (LOADERS ? NI % 4 == 0 : NW <= NI), "every wavefront that loads fetches a whole number of 1 KB pieces of each tile");
@@ -275,16 +280,51 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 	// chunk per lane, 32 rows at once) spread over the banks.  Rows past L fetch row L - 1 and chunks of
 	// keys past L (last tile) the row's last valid chunk, so padding behind a row's L valid entries is
 	// never read and every byte of a slot is written with finite data by every load.
-	const u32x4    b_rsrc    = raw_rsrc(BRING ? static_cast<const uint16_t*>(p.bias) + h * p.bias_stride[0] : nullptr,
-										BRING ? (uint32_t)(((L - 1) * p.bias_stride[1] + L) * 2) : 0u);
-	unsigned char* const bring = smem + LDS_SETS * 2 * NBUF * TILE_BYTES + (BRING ? (KS2 ? wblk : wave) * NBUF * 4096 : 0);  // (compute wavefronts)
+	//
+	// RAGGED: a row starts at any element, so on a multiple of 2 bytes; the loads take the row from the dword that holds its
+	// first key (loads of dwords want dword addresses), i.e. one key early where that dword's upper half is the row's
+	// start.  The reader shifts such rows by 16 bits, for which the last chunk needs one more dword per row: a fifth load of
+	// 32 dwords, behind the 4 KB of the slot.  Nothing is redirected at the end of a row here: what lies behind key
+	// L - 1 (the next row, padding, or past the range) is replaced by zeros in the fragments of the row's last tile.
+	const uintptr_t b_base   = BRING ? reinterpret_cast<uintptr_t>(static_cast<const uint16_t*>(p.bias) + h * p.bias_stride[0]) : 0;
+	const int       b_odd    = RAGGED ? (int)(b_base & 2) : 0;  // bytes between the range's start and the matrix'
+	const u32x4    b_rsrc    = raw_rsrc(reinterpret_cast<const void*>(b_base - b_odd), BRING ? (uint32_t)((((L - 1) * p.bias_stride[1] + L) * 2 + b_odd + 3) & ~3ll) : 0u);
+	unsigned char* const bring = smem + LDS_SETS * 2 * NBUF * TILE_BYTES + (BRING ? (KS2 ? wblk : wave) * NBUF * SLOT_BYTES : 0);  // (compute wavefronts)
 	const uint32_t bring_addr = lds_addr_of(bring);
-	const int      b_voff     = (int)((lane >> 3) * p.bias_stride[1] * 2) + (((lane & 7) ^ (lane >> 3)) << 4);
-	const int      b_row0     = (int)((qtile * QT + wblk * 32) * p.bias_stride[1] * 2);
-	const int      b_row8     = (int)(8 * p.bias_stride[1] * 2);
+	const int      b_row_bytes = (int)(p.bias_stride[1] * 2);
+	const int      b_voff     = (lane >> 3) * b_row_bytes + (((lane & 7) ^ (lane >> 3)) << 4);
+	const int      b_row0     = (qtile * QT + wblk * 32) * b_row_bytes;
+	const int      b_row8     = 8 * b_row_bytes;
 	const int      b_key      = ((lane & 7) ^ (lane >> 3)) * 8;  // first key of this lane's chunk within a tile
+	// the tile's rows [row0 + 8 j, + 8) of one query block (RAGGED)
+	auto load_bias_ragged_piece = [&](int kt, int row0, int j, uint32_t slot_addr) {
+		int row = row0 + 8 * j + (lane >> 3);
+		row     = row < (int)L ? row : (int)L - 1;
+		lds_dma_b128(b_rsrc, slot_addr + j * 1024, ((b_odd + row * b_row_bytes) & ~3) + kt * (KT * 2) + (((lane & 7) ^ (lane >> 3)) << 4));
+	};
+	// ... and the dword behind the tile of each of its 32 rows
+	auto load_bias_ragged_tail = [&](int kt, int row0, uint32_t slot_addr) {
+		int row = row0 + n;
+		row     = row < (int)L ? row : (int)L - 1;
+		if(half == 0) lds_dma_b32(b_rsrc, slot_addr + 4096, ((b_odd + row * b_row_bytes) & ~3) + (kt + 1) * (KT * 2));
+	};
 	auto load_bias_tile = [&](int kt, int slot_i) {
 		if(!BRING) return;
+		if constexpr(RAGGED) {
+			if constexpr(LOADERS) {  // rows 8 ld .. of every query block's tile and the tail dwords of block ld (loaders past the last block repeat one)
+				if(!is_loader) return;
+				constexpr int  NBLK  = KS2 ? NW / 2 : NW;
+				const uint32_t rings = lds_addr_of(smem + LDS_SETS * 2 * NBUF * TILE_BYTES);
+#pragma unroll
+				for(int wb = 0; wb < NBLK; wb++) load_bias_ragged_piece(kt, qtile * QT + wb * 32, ld, rings + (wb * NBUF + slot_i) * SLOT_BYTES);
+				load_bias_ragged_tail(kt, qtile * QT + (ld % NBLK) * 32, rings + ((ld % NBLK) * NBUF + slot_i) * SLOT_BYTES);
+			} else {
+#pragma unroll
+				for(int j = 0; j < 4; j++) load_bias_ragged_piece(kt, qtile * QT + wblk * 32, j, bring_addr + slot_i * SLOT_BYTES);
+				load_bias_ragged_tail(kt, qtile * QT + wblk * 32, bring_addr + slot_i * SLOT_BYTES);
+			}
+			return;
+		}
 		const int in_row   = kt * KT + b_key < (int)L ? b_voff + kt * (KT * 2) : b_voff - b_key * 2 + ((int)L - 8) * 2;
 		if constexpr(LOADERS) {  // eight rows (piece ld) of the tiles of all the workgroup's query blocks, by loader wavefront ld
 			if(!is_loader) return;
@@ -297,7 +337,7 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 					const int over = blk_row0 + 8 * ld + (lane >> 3) - ((int)L - 1);
 					if(over > 0) off -= over * (int)(p.bias_stride[1] * 2);
 				}
-				lds_dma_b128(b_rsrc, rings + (wb * NBUF + slot_i) * 4096 + ld * 1024, off);
+				lds_dma_b128(b_rsrc, rings + (wb * NBUF + slot_i) * SLOT_BYTES + ld * 1024, off);
 			}
 			return;
 		}
@@ -309,7 +349,7 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 				const int over = blk_row0 + 8 * j + (lane >> 3) - ((int)L - 1);
 				if(over > 0) off -= over * (int)(p.bias_stride[1] * 2);
 			}
-			lds_dma_b128(b_rsrc, bring_addr + slot_i * 4096 + j * 1024, off);
+			lds_dma_b128(b_rsrc, bring_addr + slot_i * SLOT_BYTES + j * 1024, off);
 		}
 	};
 	// ---- key-mask bytes: requested first.  With 4-byte aligned mask rows
@@ -440,7 +480,7 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 			// ---- a loader wavefront: tile j of the walk goes to buffer j % NBUF and is requested AHEAD + 1 tiles before the compute
 			// wavefronts fetch K fragments from it.  Its barriers mirror theirs one for one: one in front of the first S^T, one
 			// per live tile, and (pairs) three in the merge. ----
-			constexpr int PER_TILE = 2 * (NI / 4) + (BRING ? (KS2 ? NW / 2 : NW) : 0);  // this wavefront's loads per tile
+			constexpr int PER_TILE = 2 * (NI / 4) + (BRING ? (KS2 ? NW / 2 : NW) : 0) + (RAGGED ? 1 : 0);  // this wavefront's loads per tile
 			static_assert(PER_TILE <= 63, "the wait counter has six bits");
 			auto walk = [&](int j) -> int { return __builtin_amdgcn_readfirstlane((int)live_list[j < nlive ? j : nlive - 1]); };
 			const int kt0 = walk(0);
@@ -639,11 +679,9 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 		const bool has_bias = p.bias != nullptr && !all_dropped;
 		// natural variant: direct bias access through per-lane row pointers
 		const unsigned char* bias_row = nullptr;
-		bool                 bias_vec = false;
-		if(!L2DOM && has_bias) {
+		if(!L2DOM && !BRING && has_bias) {
 			const int64_t esz = BIAS_F32 ? 4 : 2;
 			bias_row = static_cast<const unsigned char*>(p.bias) + (h * p.bias_stride[0] + (row_ok ? qrow : 0) * p.bias_stride[1]) * esz;
-			bias_vec = !BIAS_F32 && ((reinterpret_cast<uintptr_t>(p.bias) & 15) == 0) && (p.bias_stride[0] % 8 == 0) && (p.bias_stride[1] % 8 == 0);
 		}
 		// log2 variant: fragment-ordered workspace; the tile base is wave-uniform
 		const u32x4* ws_wave = nullptr;
@@ -694,24 +732,13 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 				return;
 			}
 			const int64_t key0 = (int64_t)kt * KT + 8 * half + 32 * sub;
-			if(bias_vec && (int64_t)(kt + 1) * KT <= L) {  // wave-uniform: whole tile in range, aligned rows
-				const uint16_t* bp = reinterpret_cast<const uint16_t*>(bias_row) + key0;
-				if(row_ok) {
 #pragma unroll
-					for(int f = 2 * SUB; f < 2 * SUB + 2; f++) bfrag[f] = bias_frag_finite(*reinterpret_cast<const u32x4*>(bp + 16 * f));
-				} else {
+			for(int f = 2 * SUB; f < 2 * SUB + 2; f++) {
+				float v8[8];
+				load_bias8_guarded<BIAS_F32>(bias_row, key0 + 16 * f, L, row_ok, v8);
 #pragma unroll
-					for(int f = 2 * SUB; f < 2 * SUB + 2; f++) bfrag[f] = u32x4{0u, 0u, 0u, 0u};
-				}
-			} else {
-#pragma unroll
-				for(int f = 2 * SUB; f < 2 * SUB + 2; f++) {
-					float v8[8];
-					load_bias8_guarded<BIAS_F32>(bias_row, key0 + 16 * f, L, row_ok, v8);
-#pragma unroll
-					for(int j = 0; j < 4; j++) bfrag[f][j] = pack_bf16x2(v8[2 * j], v8[2 * j + 1]);
-					bfrag[f] = bias_frag_finite(bfrag[f]);
-				}
+				for(int j = 0; j < 4; j++) bfrag[f][j] = pack_bf16x2(v8[2 * j], v8[2 * j + 1]);
+				bfrag[f] = bias_frag_finite(bfrag[f]);
 			}
 		};
 
@@ -862,9 +889,55 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 						vprev[cp][db][2 * t + 1] = rr[1];
 					}
 		};
+		// RAGGED: a lane reads chunk c of its row and the dword that follows it -- the first of the next chunk, or, for the last
+		// chunk, of the dwords behind the slot's rows -- and shifts the five down by one key (in bias_mfma, so that the shift
+		// does not wait for the reads right behind them) where the row's start is the upper half of its first dword.
+		const int b_shift = RAGGED ? 8 * ((b_odd + (int)(row_ok ? qrow : L - 1) * b_row_bytes) & 2) : 0;
+		[[maybe_unused]] int      b_follow[2][2];  // [SUB][c2]: address of the dword that follows
+		[[maybe_unused]] uint32_t bfollow[4];
+		if constexpr(RAGGED) {
+#pragma unroll
+			for(int s2 = 0; s2 < 2; s2++)
+#pragma unroll
+				for(int c2 = 0; c2 < 2; c2++) {
+					const int c      = 4 * (s2 ^ sub) + 2 * c2 + half + 1;  // (sub is only ever 1 where s2 stays 0)
+					b_follow[s2][c2] = c < 8 ? n * 128 + ((c ^ (n & 7)) << 4) : 4096 + n * 4;
+				}
+		}
+		// kt: the tile in the slot
+		auto read_bias_ring = [&](int slot_off, auto sub_c, int kt) {
+			constexpr int SUB = decltype(sub_c)::value;
+			if constexpr(RAGGED) {
+#pragma unroll
+				for(int c2 = 0; c2 < 2; c2++) {
+					bfrag[2 * SUB + c2]   = *reinterpret_cast<const u32x4*>(bring + slot_off + (b_rd ^ ((4 * SUB + 2 * c2) << 4)));
+					bfollow[2 * SUB + c2] = *reinterpret_cast<const uint32_t*>(bring + slot_off + b_follow[SUB][c2]);
+				}
+				if(kt == n_ktiles - 1) {  // (wave-uniform) what stands for keys from L on: zero
+#pragma unroll
+					for(int c2 = 0; c2 < 2; c2++) {
+						const int left = (int)L - (kt * KT + 32 * (SUB ^ sub) + 16 * c2 + 8 * half) + (b_shift >> 4);  // halves of the five dwords that stand for keys below L
+#pragma unroll
+						for(int j = 0; j < 5; j++) {
+							const uint32_t x = j < 4 ? bfrag[2 * SUB + c2][j & 3] : bfollow[2 * SUB + c2];
+							const uint32_t y = left >= 2 * j + 2 ? x : (left == 2 * j + 1 ? x & 0xffffu : 0u);
+							if(j < 4) bfrag[2 * SUB + c2][j & 3] = y;
+							else bfollow[2 * SUB + c2] = y;
+						}
+					}
+				}
+				return;
+			}
+#pragma unroll
+			for(int c2 = 0; c2 < 2; c2++) bfrag[2 * SUB + c2] = bias_frag_finite(*reinterpret_cast<const u32x4*>(bring + slot_off + (b_rd ^ ((4 * SUB + 2 * c2) << 4))));
+		};
 		auto bias_mfma = [&](f32x16 s, int f) -> f32x16 {
 			if(L2DOM) return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, idf[f & 1]), __builtin_bit_cast(f16x8, bfrag[f & 1]), s, 0, 0, 0);
-			return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, idf[f & 1]), __builtin_bit_cast(bf16x8, bfrag[f]), s, 0, 0, 0);
+			u32x4 w = bfrag[f];
+			if constexpr(RAGGED)
+				w = bias_frag_finite(u32x4{__builtin_amdgcn_alignbit(w[1], w[0], b_shift), __builtin_amdgcn_alignbit(w[2], w[1], b_shift), __builtin_amdgcn_alignbit(w[3], w[2], b_shift),
+										   __builtin_amdgcn_alignbit(bfollow[f], w[3], b_shift)});
+			return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, idf[f & 1]), __builtin_bit_cast(bf16x8, w), s, 0, 0, 0);
 		};
 		// plain (not interleaved) S^T of one sub-tile; used once, for the very first sub-tile
 		auto compute_s_plain = [&](int k_off, int sub, int mask_addr, int fb) -> f32x16 {
@@ -879,11 +952,6 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 			return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, maskA), __builtin_bit_cast(bf16x8, maskB), s, 0, 0, 0);
 		};
 
-		auto read_bias_ring = [&](int slot_off, auto sub_c) {
-			constexpr int SUB = decltype(sub_c)::value;
-#pragma unroll
-			for(int c2 = 0; c2 < 2; c2++) bfrag[2 * SUB + c2] = bias_frag_finite(*reinterpret_cast<const u32x4*>(bring + slot_off + (b_rd ^ ((4 * SUB + 2 * c2) << 4))));
-		};
 		// ring_off (BRING): byte offset of the ring slot that holds the bias tile of sub-tile j+1
 		// The LDS operands of S^T(j+1): K fragments, bias fragments (ring variants), mask entries.  KS2 fetches them at the end of
 		// the stage before (every tile is in LDS one barrier early there), so that their latency hides behind that stage's
@@ -891,17 +959,17 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 		// else to run in that time.
 		u32x4    kf[NC];
 		uint32_t mask_next = 0;
-		auto fetch_operands = [&](auto subn_c, int k_off, int mask_addr_next, int ring_off) {
+		auto fetch_operands = [&](auto subn_c, int k_off, int mask_addr_next, int ring_off, int ring_kt) {
 			constexpr int SUBN = decltype(subn_c)::value;
-			if(BRING) read_bias_ring(ring_off, subn_c);
+			if(BRING) read_bias_ring(ring_off, subn_c, ring_kt);
 #pragma unroll
 			for(int c = 0; c < NC; c++) kf[c] = read_kfrag(k_off, SUBN, c);
 			mask_next = *reinterpret_cast<const uint32_t*>(smem + mask_addr_next + SUBN * 32 * 4);
 		};
-		// k_next / mask_next_addr / ring_next (KS2): where the operands of the stage after this one are
-		auto stage = [&](auto subn_c, int k_off, int mask_addr_next, int v_off, auto subc_c, int bias_kt, auto bias_sub_c, int ring_off, int k_next, int mask_next_addr, int ring_next) {
+		// k_next / mask_next_addr / ring_next (KS2): where the operands of the stage after this one are; ring_kt: the tile whose bias the ring slot read here holds
+		auto stage = [&](auto subn_c, int k_off, int mask_addr_next, int v_off, auto subc_c, int bias_kt, auto bias_sub_c, int ring_off, int k_next, int mask_next_addr, int ring_next, int ring_kt) {
 			constexpr int SUBN = decltype(subn_c)::value, SUBC = decltype(subc_c)::value, FB = 2 * SUBN;
-			if constexpr(!KS2) fetch_operands(subn_c, k_off, mask_addr_next, ring_off);
+			if constexpr(!KS2) fetch_operands(subn_c, k_off, mask_addr_next, ring_off, ring_kt);
 			maskA[0] = mask_next;
 			u32x4  pcur[2];
 			f32x16 sn;
@@ -951,7 +1019,7 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 			AF3_CHUNK_END();
 #undef AF3_CHUNK_END
 			rowsum_mfma(pcur[1]);
-			if constexpr(KS2) fetch_operands(subn_c, k_next, mask_next_addr, ring_next);  // (this stage's have been consumed)
+			if constexpr(KS2) fetch_operands(subn_c, k_next, mask_next_addr, ring_next, ring_kt);  // (this stage's have been consumed)
 			// The running sum stays below L * 2^REF_SLACK <= 2^25 while every probability respects the
 			// reference, so this also catches a single probability near or beyond the limit (inf, NaN).  A sum that is still
 			// zero (log2 variant: leading sub-tiles of dropped keys, or live logits so far below the initial reference that
@@ -993,13 +1061,13 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 			if(!BIAS_LATE) load_bias_frags(kt0, ic<1>{});
 			asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 			if(!SPLIT && !FUSED) __syncthreads();
-			if(BRING) read_bias_ring(0, ic<0>{});
+			if(BRING) read_bias_ring(0, ic<0>{}, kt0);
 			sc = compute_s_plain(FUSED ? kt0 * TILE_BYTES : 0, 0, mask_rd + kt0 * mask_stride, 0);
 			rereference(sc, nullptr, true);
 			if constexpr(KS2) {
 				const int kt1_first = __builtin_amdgcn_readfirstlane(live_at(1));
 				load_bias_frags(kt1_first, ic<0>{});                                                // this wavefront's next sub-tile is in the next tile
-				fetch_operands(ic<0>{}, TILE_BYTES, mask_rd + kt1_first * mask_stride, 4096);  // operands of the first stage: second tile of the walk, buffer 1
+				fetch_operands(ic<0>{}, TILE_BYTES, mask_rd + kt1_first * mask_stride, SLOT_BYTES, kt1_first);  // operands of the first stage: second tile of the walk, buffer 1
 			} else if(BIAS_LATE) load_bias_frags(kt0, ic<1>{});
 			else if(my_n > 1) load_bias_frags(__builtin_amdgcn_readfirstlane(live_at(1)), ic<0>{});
 
@@ -1018,11 +1086,11 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 					// reads issued, from the buffer of tile it+1) may stay in flight.  LDS reads return in issue order.  (The counter
 					// also counts scalar memory loads, which do not: this relies on the loop holding none -- every kernel argument
 					// is in registers before the loop, and the compiler has no reason to fetch one again while none is spilled.)
-					constexpr int OPERAND_READS = NC + 1 + (BRING ? 2 : 0);
+					constexpr int OPERAND_READS = NC + 1 + (BRING ? RAGGED ? 4 : 2 : 0);
 					asm volatile("s_waitcnt lgkmcnt(%0)\n\ts_barrier" ::"n"(OPERAND_READS) : "memory");
 					const int kt3_v = live_at(it + 3);  // (behind the barrier, which would wait for this read)
-					stage(ic<0>{}, bufn * TILE_BYTES, mask_rd + kt1 * mask_stride, buf * TILE_BYTES, ic<0>{}, kt2, ic<0>{}, bufn * 4096, bufnn * TILE_BYTES, mask_rd + kt2 * mask_stride,
-						  bufnn * 4096);
+					stage(ic<0>{}, bufn * TILE_BYTES, mask_rd + kt1 * mask_stride, buf * TILE_BYTES, ic<0>{}, kt2, ic<0>{}, bufn * SLOT_BYTES, bufnn * TILE_BYTES, mask_rd + kt2 * mask_stride,
+						  bufnn * SLOT_BYTES, kt2);
 					buf = bufn;
 					kt  = kt1;
 					kt1 = kt2;
@@ -1042,7 +1110,7 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 				// LDS offsets of tile it and of tile it+1: ring buffers, or the tiles' own places when all of K and V is resident
 				const int off_cur = (FUSED ? kt : buf) * TILE_BYTES, off_next = (FUSED ? kt1 : bufn) * TILE_BYTES;
 				// sub-tile (it, 0): next is (it, 1) in the same buffer
-				stage(ic<1>{}, off_cur, mask_rd + kt * mask_stride, off_cur, ic<0>{}, kt1, ic<0>{}, buf * 4096, 0, 0, 0);
+				stage(ic<1>{}, off_cur, mask_rd + kt * mask_stride, off_cur, ic<0>{}, kt1, ic<0>{}, buf * SLOT_BYTES, 0, 0, 0, kt);
 				if(!BIAS_LATE) load_bias_frags(kt1, ic<1>{});
 				// Tile it+1 (issued one iteration ago) must have landed, and every wavefront must be done
 				// with tile it-1, whose buffer tile it+2 is about to overwrite.  Loads complete in issue
@@ -1058,7 +1126,7 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 					load_bias_tile(kt2, bufnn);  // (its slot held tile it-1, last read in the stage above)
 				}
 				// sub-tile (it, 1): next is (it+1, 0) in the next buffer (harmless stale data after the last tile)
-				stage(ic<0>{}, off_next, mask_rd + kt1 * mask_stride, off_cur, ic<1>{}, kt1, ic<1>{}, bufn * 4096, 0, 0, 0);
+				stage(ic<0>{}, off_next, mask_rd + kt1 * mask_stride, off_cur, ic<1>{}, kt1, ic<1>{}, bufn * SLOT_BYTES, 0, 0, 0, kt1);
 				if(!BIAS_LATE) load_bias_frags(kt2, ic<0>{});
 				buf = bufn;
 				kt  = kt1;
@@ -1265,7 +1333,7 @@ static size_t lds_bytes(const af3_dpa_params& p) {
 	constexpr bool   KS2  = KSL == 1;
 	const size_t writers  = SPLIT ? 1 : KS2 ? NW / 2 : NW;  // wavefronts that own a block of query rows
 	constexpr size_t NBUF = KSL == 1 ? 5 : KSL ? 4 : 3;  // (as in the kernel)
-	return (size_t)(SPLIT ? NW : 1) * 2 * NBUF * KT * DP * 2 + (BMODE == 2 ? (KS2 ? NW / 2 : NW) * NBUF * 4096 : 0) + (n_ktiles * KT + 64) * 4 + n_ktiles * 2 + 16 +
+	return (size_t)(SPLIT ? NW : 1) * 2 * NBUF * KT * DP * 2 + (BMODE >= 2 ? (KS2 ? NW / 2 : NW) * NBUF * bias_slot_bytes(BMODE) : 0) + (n_ktiles * KT + 64) * 4 + n_ktiles * 2 + 16 +
 		   (p.gate ? writers * 32 * DP * 2 : 0);
 }
 
@@ -1356,6 +1424,7 @@ int launch_grid_fused(const af3_grid_attention_params& g, hipStream_t s) {
 
 template <int DP, bool L2DOM, int BMODE>
 static int launch_nw(const af3_dpa_params& p, hipStream_t s) {
+	if constexpr(!L2DOM && BMODE == 0) return launch_one<DP, 4, L2DOM, BMODE>(p, s);  // (a bias beyond 32-bit offsets: one form serves it)
 	// the largest workgroup that still gives the 256 CUs a few workgroups each
 	const int64_t groups = p.B * p.H;
 	if(groups * ((p.L + 127) / 128) >= 768) return launch_one<DP, 4, L2DOM, BMODE>(p, s);
@@ -1407,16 +1476,16 @@ int launch_dpa_mfma_bf16(const af3_dpa_params& p, hipStream_t s) {
 		if(rc != AF3_OK) return rc;
 	}
 	const bool l2dom = use_ws || !p.bias;
-	// in-place bf16 bias: through the LDS ring when its rows can be fetched in aligned 16-byte chunks that
-	// never straddle the end of a row's L valid entries, element-wise otherwise
-	const bool ring = !l2dom && !bf32 && ((reinterpret_cast<uintptr_t>(p.bias) & 15) == 0) && (p.bias_stride[0] % 8 == 0) && (p.bias_stride[1] % 8 == 0) && (p.L % 8 == 0) &&
-					  ((p.L - 1) * p.bias_stride[1] + p.L) * 2 < (int64_t)1 << 31;
-	if(p.D <= 32) {
-		if(l2dom) return launch_nw<32, true, 0>(p, s);
-		return bf32 ? launch_nw<32, false, 1>(p, s) : ring ? launch_nw<32, false, 2>(p, s) : launch_nw<32, false, 0>(p, s);
-	}
-	if(l2dom) return launch_nw<64, true, 0>(p, s);
-	return bf32 ? launch_nw<64, false, 1>(p, s) : ring ? launch_nw<64, false, 2>(p, s) : launch_nw<64, false, 0>(p, s);
+	// In-place bf16 bias: through the LDS ring.  Where rows are whole aligned 16-byte chunks that never straddle the end of a
+	// row's L valid entries a fragment is one LDS read (2); anywhere else (3) it is two and four shifts.
+	// Element by element (0) only where a head's slab exceeds the loads' 32-bit offsets.
+	const int mode = l2dom ? 0 : bf32 ? 1 : ((p.L - 1) * p.bias_stride[1] + p.L) * 2 >= ((int64_t)1 << 31) - 64 * 1024 ? 0 :
+					 (reinterpret_cast<uintptr_t>(p.bias) & 15) == 0 && p.bias_stride[0] % 8 == 0 && p.bias_stride[1] % 8 == 0 && p.L % 8 == 0 ? 2 : 3;
+	auto go = [&](auto dp_c) {
+		constexpr int DP = decltype(dp_c)::value;
+		return l2dom ? launch_nw<DP, true, 0>(p, s) : mode == 1 ? launch_nw<DP, false, 1>(p, s) : mode == 2 ? launch_nw<DP, false, 2>(p, s) : mode == 3 ? launch_nw<DP, false, 3>(p, s) : launch_nw<DP, false, 0>(p, s);
+	};
+	return p.D <= 32 ? go(ic<32>{}) : go(ic<64>{});
 }
 
 }  // namespace af3

@@ -53,6 +53,10 @@ __device__ __forceinline__ float half_swap_max(float x) {
 __device__ __forceinline__ void lds_dma_b128(const u32x4& rsrc, uint32_t lds_addr, int voff) {
 	asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds_addr), "v"(voff), "s"(rsrc) : "memory");
 }
+// ... 4 bytes per lane (lane i lands at lds_addr + 4*i)
+__device__ __forceinline__ void lds_dma_b32(const u32x4& rsrc, uint32_t lds_addr, int voff) {
+	asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds" ::"s"(lds_addr), "v"(voff), "s"(rsrc) : "memory");
+}
 __device__ __forceinline__ u32x4 raw_rsrc(const void* base, uint32_t bytes) {
 	const uint64_t a = reinterpret_cast<uint64_t>(base);
 	return u32x4{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a), (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)(a >> 32) & 0xFFFFu)),
