@@ -1429,38 +1429,37 @@ static int launch_nw(const af3_dpa_params& p, hipStream_t s) {
 	const int64_t groups = p.B * p.H;
 	if(groups * ((p.L + 127) / 128) >= 768) return launch_one<DP, 4, L2DOM, BMODE>(p, s);
 	if(L2DOM && groups * ((p.L + 63) / 64) >= 768) return launch_one<DP, 2, L2DOM, BMODE>(p, s);
-	// Small launches: one 32-row block per workgroup, its key tiles split over 2 or 4 wavefronts so that
+	const int64_t blocks1 = groups * ((p.L + 31) / 32), ktiles = (p.L + KT - 1) / KT;
+	if(!L2DOM) {
+		// In-place bias (one batch row): every form below puts at most one workgroup on a compute unit, and each is taken up to
+		// the point where its workgroups no longer fit the 256 compute units in one round -- a second, nearly empty round
+		// doubles the time -- with the most wavefronts per query block first.  Measured, us (B=1 H=16, GPU time per call):
+		//   head_dim 24                  L=256    512    768   1024   1280   1536
+		//   tiles split over four          5.5    6.6   13.6   16.0   26.4   29.3
+		//   a pair per workgroup           6.0    7.3   15.5   18.7   31.1   35.1
+		//   two pairs on shared tiles      6.5    7.9    9.4   11.0   23.3   26.2
+		//   four pairs on shared tiles     8.1   10.1   12.2   14.5   16.7   18.9
+		//   head_dim 48                  L=256    512    768   1024   1280   1536
+		//   a pair per workgroup           7.0    8.5   18.6   22.1   36.9   41.7
+		//   two pairs on shared tiles      7.5    9.2   11.0   13.4   27.7   31.3
+		//   one wavefront per block, x 4   8.3   11.6   14.9   18.1   21.3   24.6
+		// (Pairs and the last form have four loading wavefronts.  Four pairs at head_dim 48 do not fit in LDS.)
+		const int64_t wg64 = groups * ((p.L + 63) / 64), wg128 = groups * ((p.L + 127) / 128);
+		if constexpr(DP == 32) {
+			if(blocks1 <= 256 && ktiles >= 4 && lds_bytes<DP, 4, BMODE, true>(p) <= LDS_LIMIT) return launch_one<DP, 4, L2DOM, BMODE, true>(p, s);
+		}
+		if(blocks1 <= 256) return launch_one<DP, 2, L2DOM, BMODE, false, 1>(p, s);
+		if(wg64 <= 256 && lds_bytes<DP, 4, BMODE, false, 1>(p) <= LDS_LIMIT) return launch_one<DP, 4, L2DOM, BMODE, false, 1>(p, s);
+		if constexpr(DP == 32) {
+			if(wg128 <= 256 && lds_bytes<DP, 8, BMODE, false, 1>(p) <= LDS_LIMIT) return launch_one<DP, 8, L2DOM, BMODE, false, 1>(p, s);
+		}
+		if(wg128 <= 256 && lds_bytes<DP, 4, BMODE, false, 2>(p) <= LDS_LIMIT) return launch_one<DP, 4, L2DOM, BMODE, false, 2>(p, s);
+		return launch_one<DP, 4, L2DOM, BMODE>(p, s);
+	}
+	// Small launches through the workspace: one 32-row block per workgroup, its key tiles split over 2 or 4 wavefronts so that
 	// more of the 1024 SIMDs have work.  The private LDS buffers limit a compute unit to one 4-wave or
 	// three 2-wave workgroups, so each split is only taken while the whole grid is resident at once
 	// (measured: beyond that the second round of workgroups costs more than the split gains).
-	const int64_t blocks1 = groups * ((p.L + 31) / 32), ktiles = (p.L + KT - 1) / KT;
-	if(!L2DOM) {
-		// In-place bias (one batch row): every single-wave workgroup would re-read the whole K and V of
-		// its head from L2, which then outweighs the bias stream; from 512 query blocks on, four blocks
-		// share each K/V tile instead (measured, B=1 H=16 D=24: L=1536 25.6 us against 32.7 us with
-		// single-wave workgroups; L=768 14.0 us split in two against 14.3 / 17.8; L=384 8.5 us split in four).
-		// Long rows with too few 128-row workgroups to fill the 256 compute units: pairs of wavefronts share a query block and
-		// the workgroup's K/V tiles.  The work per SIMD is unchanged -- two wavefronts of half the length instead of one -- but
-		// the two overlap their matrix and vector phases, and four more wavefronts issue the workgroup's loads (measured,
-		// B=1 H=16 L=1536: 22.0 against 31.1 us at head_dim 24; at head_dim 48, padded to 64, the pairing gained nothing, so
-		// that size keeps one wavefront per query block).  With 256..511 query blocks the same pairing in workgroups of
-		// four compute wavefronts gives every compute unit at most one workgroup of uniform length, where 2-wave
-		// workgroups with private tiles put two on half of the compute units and fetch every tile twice as often
-		// (measured, B=1 H=16 L=768 D=24: 11.2 against 12.8 us; with 192 blocks, L=384, the four-way split of private
-		// tiles stays ahead: 7.5 against 8.4 us, and with 768 blocks eight compute wavefronts per workgroup: 22.0 against 29.9).
-		if constexpr(DP == 32) {
-			if(blocks1 >= 512 && blocks1 <= 1024 && ktiles >= 8) return launch_one<DP, 8, L2DOM, BMODE, false, true>(p, s);
-			if(blocks1 >= 256 && blocks1 < 512 && ktiles >= 8) return launch_one<DP, 4, L2DOM, BMODE, false, true>(p, s);
-		}
-		// One wavefront per query block, too few 128-row workgroups to give a compute unit more than one: the four loading
-		// wavefronts again (measured, B=1 H=16 L=1536 D=48: 27.0 against 31.0 us).
-		if(blocks1 >= 512 && blocks1 <= 1024 && lds_bytes<DP, 4, BMODE, false, 2>(p) <= LDS_LIMIT) return launch_one<DP, 4, L2DOM, BMODE, false, 2>(p, s);
-		if(blocks1 >= 512) return launch_one<DP, 4, L2DOM, BMODE>(p, s);
-		// (the split variants' private buffers plus a long row's mask table can exceed the LDS of a compute unit: then the next one)
-		if(DP == 32 && ktiles >= 4 && blocks1 <= 256 && lds_bytes<DP, 4, BMODE, true>(p) <= LDS_LIMIT) return launch_one<DP, 4, L2DOM, BMODE, true>(p, s);
-		if(ktiles >= 2 && lds_bytes<DP, 2, BMODE, true>(p) <= LDS_LIMIT) return launch_one<DP, 2, L2DOM, BMODE, true>(p, s);
-		return launch_one<DP, 1, L2DOM, BMODE>(p, s);
-	}
 	if(DP == 32 && ktiles >= 4 && blocks1 <= 256 && lds_bytes<DP, 4, BMODE, true>(p) <= LDS_LIMIT) return launch_one<DP, 4, L2DOM, BMODE, true>(p, s);
 	if(ktiles >= 2 && blocks1 <= 768 && lds_bytes<DP, 2, BMODE, true>(p) <= LDS_LIMIT) return launch_one<DP, 2, L2DOM, BMODE, true>(p, s);
 	return launch_one<DP, 1, L2DOM, BMODE>(p, s);

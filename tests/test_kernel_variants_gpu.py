@@ -20,7 +20,8 @@ def f32np(t):
 @pytest.mark.parametrize("H,L,D,pad,first", [
     (1, 1, 24, 0, 0), (2, 2, 24, 1, 1), (3, 31, 32, 0, 1), (2, 33, 8, 3, 0), (1, 63, 24, 0, 0), (1, 65, 48, 0, 1),   # one wavefront, last tile nearly empty
     (2, 129, 24, 0, 0), (2, 190, 32, 5, 1), (3, 257, 24, 0, 0),   # key tiles split over four wavefronts
-    (2, 129, 48, 0, 1), (2, 322, 64, 0, 0),                       # ... over two
+    (2, 129, 48, 0, 1), (2, 322, 64, 0, 0),                       # a pair of wavefronts per workgroup
+    (16, 513, 48, 1, 0),                                          # two pairs, head_dim padded to 64
     (16, 515, 24, 1, 1),                                          # pairs on shared tiles, four computing wavefronts
     (16, 1027, 24, 0, 0), (16, 1024, 24, 7, 1),                   # ... eight
     (16, 1027, 48, 0, 1),                                         # loading wavefronts, one query block each
