@@ -90,6 +90,22 @@ def load():
     return _lib
 
 
+class _MissingHost:
+    def __getattr__(self, name):
+        raise ImportError(f"{os.path.join(_HERE, '_host.so')} is missing: build it with `python -m af3_kernels_amd.build`.")
+
+
+def load_host():
+    """The native host side of the entry points (csrc/host.cpp).  A package that has not been built yet can still be imported
+    (to build it); the first call then says what is missing."""
+    if not os.path.exists(os.path.join(_HERE, "_host.so")):
+        return _MissingHost()
+    load()
+    import torch  # noqa: F401 -- its libraries must be loaded first
+    from . import _host
+    return _host
+
+
 def check(status: int, what: str):
     if status != 0:
         msg = load().af3_status_string(status).decode()

@@ -1,4 +1,4 @@
-"""Builds libaf3_dpa.so (hand-written HIP for gfx950) in-tree with hipcc.
+"""Builds libaf3_dpa.so (hand-written HIP for gfx950) in-tree with hipcc, and the Python entry points' native host side (_host.so).
 
     python -m af3_kernels_amd.build [--force]
 
@@ -12,6 +12,8 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJDIR = os.path.join(CSRC, "_obj")
+HOST_SRC = os.path.join(CSRC, "host.cpp")
+HOST = os.path.join(HERE, "_host.so")
 LIB = os.path.join(HERE, "libaf3_dpa.so")
 SOURCES = ["api.hip", "dpa_generic.hip", "dpa_mfma.hip", "dpa_mfma_rows.hip", "dpa_mfma_f32.hip", "dpa_mfma_fp8.hip", "elementwise.hip", "pair_bias.hip", "glu.hip"]
 HEADERS = [os.path.join(CSRC, "common.hpp"), os.path.join(CSRC, "mfma_helpers.hpp"), os.path.join(HERE, "..", "include", "af3_dpa.h")]
@@ -42,6 +44,26 @@ def _compile(src, force):
     return obj
 
 
+def _build_host():
+    """The native host side of the Python entry points: a CPython extension on torch's C++ interface, no device code."""
+    import importlib.util
+    import sysconfig
+    torch_dir = os.path.dirname(importlib.util.find_spec("torch").origin)
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(HIPCC)))
+    includes = [os.path.join(torch_dir, "include"), os.path.join(torch_dir, "include", "torch", "csrc", "api", "include"), os.path.join(rocm, "include"), sysconfig.get_paths()["include"]]
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1"]
+    for i in includes:
+        cmd += ["-isystem", i]
+    # (torch's libraries are loaded by the time the module is imported; the kernels' library stands beside it)
+    cmd += [HOST_SRC, "-o", HOST, "-L", HERE, "-l:" + os.path.basename(LIB), "-Wl,-rpath,$ORIGIN", "-L", os.path.join(torch_dir, "lib"),
+            "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-ltorch_python"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("compiling the host module failed:\n" + r.stdout + r.stderr)
+    if r.stderr.strip():
+        print(r.stderr, file=sys.stderr)
+
+
 def build(force=False, verbose=False):
     os.makedirs(OBJDIR, exist_ok=True)
     with ThreadPoolExecutor(max_workers=min(8, len(SOURCES) + 1)) as ex:
@@ -50,8 +72,11 @@ def build(force=False, verbose=False):
         r = subprocess.run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB] + objs, capture_output=True, text=True)
         if r.returncode != 0:
             raise RuntimeError("link failed:\n" + r.stdout + r.stderr)
+    if force or _stale(HOST, [HOST_SRC, LIB, HEADERS[-1]]):
+        _build_host()
     if verbose:
         print("built", LIB)
+        print("built", HOST)
     return LIB
 
 

@@ -27,6 +27,7 @@ from typing import Optional
 import torch
 
 from . import _lib, ops
+from .ops import _host
 
 # One workgroup of the fused kernel serves one (batch row, head) and holds a compute unit's LDS: launches with
 # fewer workgroups than this leave most of the 256 compute units idle and take the three-launch path instead.
@@ -83,6 +84,13 @@ def clear_weight_cache() -> None:
     updates (`copy_`, `load_state_dict`, optimiser steps) are noticed without it."""
     with _CACHE_LOCK:
         _W_CACHE.clear()
+        _host.forget()
+
+
+def _remember(what: int, head: int, dtype: torch.dtype, value: torch.Tensor, *sources) -> torch.Tensor:
+    """Leaves a matrix derived from weights where the native path of the next call finds it."""
+    _host.remember(what | head << 8 | ops._DTYPE_CODE[dtype] << 40, value, *sources)
+    return value
 
 
 def _fused_weight(ws, head: int, dtype: torch.dtype) -> torch.Tensor:
@@ -95,7 +103,7 @@ def _fused_weight(ws, head: int, dtype: torch.dtype) -> torch.Tensor:
         K = C // head
         q, k, v, g = (_unpack_panels(w, head).to(dtype).view(C, head, K) for w in ws)
         return torch.stack((k, v, q, g), dim=2).reshape(C, 4 * C).t().contiguous()
-    return _cached(tuple(ws), (head, dtype), make)
+    return _remember(_host.FUSED_WEIGHT, head, dtype, _cached(tuple(ws), (head, dtype), make), *ws)
 
 
 def _q_bias_row(q_bias: torch.Tensor, head: int, dtype: torch.dtype) -> torch.Tensor:
@@ -106,7 +114,7 @@ def _q_bias_row(q_bias: torch.Tensor, head: int, dtype: torch.dtype) -> torch.Te
         row = torch.zeros(head, 4, K, dtype=dtype, device=q_bias.device)
         row[:, 2] = q_bias.reshape(head, K).to(dtype)
         return row.view(4 * C)
-    return _cached((q_bias,), (head, dtype, "q_bias"), make)
+    return _remember(_host.Q_BIAS_ROW, head, dtype, _cached((q_bias,), (head, dtype, "q_bias"), make), q_bias)
 
 
 def _check_weights(C: int, head: int, ws):
@@ -186,7 +194,12 @@ def _attend(y: torch.Tensor, B: int, N: int, head: int, mask, bias) -> torch.Ten
 def _fused_grid_kernel(pair: torch.Tensor, mask, bias, ws, head: int) -> Optional[torch.Tensor]:
     """Projections, attention and gate in ONE kernel (af3_grid_attention_forward) when the library supports the
     shape (bfloat16, 128 channels, 4 heads, K and V of a head fit in LDS); None otherwise.  Returns [B, N, C]."""
-    if ops._exact_bias or any(w.dtype != pair.dtype for w in ws):
+    if ops._exact_bias:
+        return None
+    out = _host.grid_kernel(pair, mask, bias, *ws, head)
+    if out is not None:
+        return out if out.__class__ is not int else _lib.check(out, "af3_grid_attention_forward")
+    if any(w.dtype != pair.dtype for w in ws):
         return None
     B, N, C = pair.shape
     if pair.stride(-1) != 1:
@@ -252,9 +265,13 @@ def _attention_cpp(
     gated = _fused_grid_kernel(pair, mask, bias, ws, head) if B * head >= _FUSED_MIN_GROUPS else None
     if gated is None:
         gated = _attend(_project(pair.reshape(B * N, C), ws, None, head), B, N, head, mask, bias)
+    out = _host.out_projection(gated, out_proj)
+    if out is not None:
+        return out if out.__class__ is not int else _lib.check(out, "af3_linear")
     rows = gated.view(B * N, C)
     if out_proj.dtype == dtype and _narrow_linear_ok(rows, C):
         w = _cached((out_proj,), ("out_proj",), lambda: out_proj.t().contiguous())      # nn.Linear layout [out, in]
+        _host.remember(_host.OUT_PROJ_T, w, out_proj)
         return _linear_rows(rows, w).view(B, N, C)
     return torch.matmul(rows, out_proj.to(dtype)).view(B, N, C)
 
@@ -282,6 +299,9 @@ def self_attention_cpp(
     [S, N, C] -- S diffusion samples of the same tokens, mask [N] or [S, N] -- and the S samples then go through ONE
     projection GEMM and ONE attention launch in which they share every bias tile (the pair bias, the largest operand,
     is streamed once instead of S times).  Returns [S, N, C]."""
+    out = _host.self_attention(pair, mask, bias, q_proj, k_proj, v_proj, gating_query, q_bias, head, ops._rows_kernel_hint, ops._exact_bias)
+    if out is not None:
+        return out if out.__class__ is not int else _lib.check(out, "af3_dpa_forward")
     ops._require_device(pair, mask, bias, q_proj, q_bias, k_proj, v_proj, gating_query)
     if pair.dim() == 3:
         S, N, C = pair.shape
@@ -307,6 +327,9 @@ def layernorm_pair_bias(pair: torch.Tensor, ln_weight: torch.Tensor, ln_bias: to
     one pass over the pair tensor: returns (normed [N1, N2, C], bias [head, N1, N2]).  One HIP kernel: a specialised one
     for bfloat16 pairs with 128 channels and 4 heads (the pair tensor's own shape), one wavefront per token for any other
     channel and head count (C <= 2048) in bfloat16 or float32.  Parameters in another dtype are cast to the pair's."""
+    out = _host.layernorm_pair_bias(pair, ln_weight, ln_bias, eps, proj_weight)
+    if out is not None:
+        return out if out.__class__ is not int else _lib.check(out, "af3_layernorm_pair_bias")
     ops._require_device(pair, ln_weight, ln_bias, proj_weight)
     if pair.dim() != 3 or proj_weight.dim() != 2 or proj_weight.shape[1] != pair.shape[-1] or ln_weight.numel() != pair.shape[-1] or ln_bias.numel() != pair.shape[-1]:
         raise ValueError(f"pair must be [N1, N2, C] with ln_weight, ln_bias [C] and proj_weight [head, C], got {tuple(pair.shape)}, {tuple(ln_weight.shape)}, "
@@ -369,6 +392,14 @@ class GridSelfAttentionCpp(torch.nn.Module):
         return self.q_proj, self.k_proj, self.v_proj, self.gq, self.out_proj
 
     def forward(self, pair: torch.Tensor, mask: torch.Tensor) -> torch.Tensor:
+        if not self.first_run:
+            # (straight from the module's dictionaries: an attribute lookup that falls through to them costs a microsecond each)
+            parts = self.__dict__["_modules"]
+            norm, proj = parts["act_norm"], parts["pair_bias_projection"]
+            out = _host.grid_block(pair, norm._parameters.get("weight"), norm._parameters.get("bias"), norm.eps, proj._parameters.get("weight"), mask, self.q_proj, self.k_proj,
+                                   self.v_proj, self.gq, self.out_proj, self.num_head, self.transpose, _FUSED_MIN_GROUPS, ops._rows_kernel_hint, ops._exact_bias)
+            if out is not None:
+                return out if out.__class__ is not int else _lib.check(out, "grid attention block")
         normed, bias = layernorm_pair_bias(pair, self.act_norm.weight, self.act_norm.bias, self.act_norm.eps, self.pair_bias_projection.weight)  # bias [head, N, N]
         rows = normed.transpose(0, 1) if self.transpose else normed         # attend along columns when transposed
         out = _attention_cpp(rows, mask, bias, *self._packed_weights(), self.num_head, False, 128 if pair.shape[1] > 256 else 64, 0)
@@ -409,6 +440,10 @@ def gated_linear_unit_cpp(x: torch.Tensor, weight: torch.Tensor, vnni_repacked: 
     stored); other shapes (bfloat16 or float32) are a library GEMM for x @ W followed by the silu-and-multiply kernel
     (af3_silu_mul).  M_BLK and N_BLK are CPU blocking sizes (N_BLK also names the panel width of a repacked weight) and
     change nothing else."""
+    tag = _host.GLU_T | bool(vnni_repacked) << 8 | N_BLK << 16
+    out = _host.gated_linear_unit(x, weight, tag)
+    if out is not None:
+        return out if out.__class__ is not int else _lib.check(out, "af3_gated_linear_unit")
     ops._require_device(x, weight)
     if weight.dim() != 2 or weight.shape[0] != x.shape[-1] or weight.shape[1] % 2 != 0:
         raise ValueError(f"weight must be [K, 2N] with K = x.shape[-1] = {x.shape[-1]}, got {tuple(weight.shape)}")
@@ -426,6 +461,7 @@ def gated_linear_unit_cpp(x: torch.Tensor, weight: torch.Tensor, vnni_repacked: 
             _lib.check(_lib.load().af3_silu_mul(y.data_ptr(), out.data_ptr(), y.shape[0], N, ops._DTYPE_CODE[x.dtype], ops._stream_ptr(x.device)), "af3_silu_mul")
         return out.view(*lead, N)
     wt = _cached((weight,), (bool(vnni_repacked), N_BLK, "glu"), lambda: _plain_weight(weight, vnni_repacked, N_BLK).t().contiguous())
+    _host.remember(tag, wt, weight)
     x2 = x.reshape(-1, K)
     if not x2.is_contiguous() or x2.data_ptr() % 16:
         x2 = x2.contiguous()
@@ -450,6 +486,9 @@ class Linear(torch.nn.Module):
         self.M_BLK, self.N_BLK = M_BLK, N_BLK
 
     def forward(self, input: torch.Tensor) -> torch.Tensor:
+        out = _host.linear(input, self.weight)
+        if out is not None:
+            return out if out.__class__ is not int else _lib.check(out, "af3_linear")
         ops._require_device(input, self.weight)
         x2 = input.reshape(-1, self.in_features)
         if self.weight.dtype == input.dtype and self.weight.is_contiguous() and _narrow_linear_ok(x2, self.out_features):

@@ -19,6 +19,7 @@ if hasattr(torch, "float8_e4m3fn"):
     _DTYPE_CODE[torch.float8_e4m3fn] = AF3_FP8_E4M3
 if hasattr(torch, "float8_e5m2"):
     _DTYPE_CODE[torch.float8_e5m2] = AF3_FP8_E5M2
+_host = _lib.load_host()   # plain calls run in native code from here on; None comes back for anything it leaves to the code below
 KERNEL_NAMES = {0: "fp32_fma", 1: "bf16_mfma", 2: "fp8_mfma", 3: "fp32_mfma"}
 
 
@@ -314,6 +315,10 @@ def dot_product_attention_cpp(
     mask is broadcast over the batch (the harness semantics, examples/dot_product_attention.py:
     34-37).  use_flash_attention / BLK_SZ / FLASH_SZ are accepted and ignored: they tune CPU
     cache blocking and never change results (the kernel is always an online-softmax kernel)."""
+    if not _timers.enabled:
+        out = _host.attention(q, k, v, mask, bias, _rows_kernel_hint, _exact_bias)
+        if out is not None:
+            return out if out.__class__ is not int else _lib.check(out, "af3_dpa_forward")
     code = _DTYPE_CODE.get(q.dtype)
     if code not in (AF3_F32, AF3_BF16):
         raise ValueError(f"unsupported dtype {q.dtype}: float32 or bfloat16 (use dot_product_attention_fp8 for the fp8 path)")
@@ -406,6 +411,9 @@ def dot_product_attention_fp8(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     residuals and the logits are q8.k8 + q8.k_lo + q_lo.k8 (three e4m3 MFMAs per chunk), which is
     what keeps the result within 6e-2 of the fp32 formula; without it only q8.k8 is computed.
     No reference counterpart (the reference has no fp8 path)."""
+    out = _host.attention_fp8(q, k, v, mask, bias, bool(compensated))
+    if out is not None:
+        return out if out.__class__ is not int else _lib.check(out, "af3_dpa_forward(fp8)")
     _require_device(q, k, v, mask, bias)
     B, H, L, D = q.shape
     if q.dtype not in (torch.float32, torch.bfloat16):

@@ -43,3 +43,45 @@ def test_single_row_bias_at_any_address(af3, oracle, H, L, D, pad, first):
     torch.cuda.synchronize()
     want = oracle.dpa_formula(f32np(q), f32np(k), f32np(v), keep.numpy(), f32np(bias[:, :L, :L]))
     assert np.abs(f32np(out) - want).max() <= 2e-2
+
+
+@pytest.mark.parametrize("rank", [None, 1, 2, 4, "float"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+def test_native_host_path_equals_the_python_path(af3, dtype, rank):
+    """Plain calls are prepared in native code, the rest (here: the implementation called directly, a mask that is not bool) in
+    Python: same bits, whatever the mask's shape; strided q, k, v and a padded bias included."""
+    from af3_kernels_amd import ops
+    B, H, L, D = 3, 4, 72, 32
+    g = torch.Generator().manual_seed(3)
+    q, k, v = (torch.randn(B, L, H, D, generator=g).to(dtype).cuda().transpose(1, 2) for _ in range(3))
+    bias = torch.randn(H, L + 8, L + 8, generator=g).to(dtype).cuda()
+    keep = (torch.rand(B, L, generator=g) < 0.8).cuda()
+    mask = {None: None, 1: keep[0], 2: keep, 4: keep[:, None, None, :], "float": keep.float()}[rank]
+    got = af3.dot_product_attention_cpp(q, k, v, mask, bias)
+    want = ops._dpa_forward_impl(q, k, v, ops._lift_mask(mask, L), bias, ops._DTYPE_CODE[dtype], False)
+    assert got.shape == q.shape and torch.equal(got, want)
+
+
+def test_native_host_path_follows_updated_weights(af3):
+    """Matrices derived from weights are recomputed when a weight changes in place or is replaced."""
+    from af3_kernels_amd import fused
+    g = torch.Generator().manual_seed(4)
+    n, C, head = 48, 128, 4
+    x, mask, bias = torch.randn(n, C, generator=g).to(torch.bfloat16).cuda(), torch.ones(n, dtype=torch.bool).cuda(), torch.randn(head, n, n, generator=g).to(torch.bfloat16).cuda()
+    ws = [af3.vnni_repack_tensor((torch.randn(C, C, generator=g) / C ** 0.5).to(torch.bfloat16).cuda(), 2, C // head) for _ in range(4)]
+    qb = torch.randn(C, generator=g).to(torch.bfloat16).cuda()
+    glu_w = (torch.randn(C, 2 * C, generator=g) / C ** 0.5).to(torch.bfloat16).cuda()
+
+    def both():
+        return af3.self_attention_cpp(x, mask, bias, ws[0], qb, ws[1], ws[2], ws[3], head), af3.gated_linear_unit_cpp(x, glu_w)
+
+    first = both()
+    assert all(torch.equal(a, b) for a, b in zip(first, both()))
+    for change in (lambda: (ws[1].mul_(2), glu_w.mul_(2)), lambda: (ws.__setitem__(2, ws[2] * 2), qb.add_(1)), lambda: (qb.data.mul_(3), fused.clear_weight_cache())):
+        before = both()
+        change()
+        after = both()
+        assert not torch.equal(before[0], after[0])
+        fused.clear_weight_cache()
+        assert all(torch.equal(a, b) for a, b in zip(after, both()))
+    assert not torch.equal(first[1], both()[1])
