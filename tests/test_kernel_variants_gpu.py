@@ -85,3 +85,40 @@ def test_native_host_path_follows_updated_weights(af3):
         fused.clear_weight_cache()
         assert all(torch.equal(a, b) for a, b in zip(after, both()))
     assert not torch.equal(first[1], both()[1])
+
+
+@pytest.mark.parametrize("B,H,L,D", [
+    (1, 2, 97, 32), (2, 3, 130, 24), (1, 1, 1023, 32),       # four wavefronts per block of 32 query rows
+    (5, 4, 385, 32), (16, 4, 255, 8),                        # ... two blocks per workgroup
+    (16, 4, 385, 32), (64, 4, 97, 24),                       # two wavefronts per block, four blocks
+    (3, 4, 161, 64), (9, 8, 250, 40),                        # head_dim padded to 64, two wavefronts per block
+    (33, 8, 131, 32), (40, 8, 97, 64), (3, 2, 95, 20),       # one wavefront per block
+])
+@pytest.mark.parametrize("kind", ["random", "lopsided", "ramp", "far"])
+def test_fp32_forms(af3, oracle, B, H, L, D, kind):
+    """The fp32 kernel's launch forms; masks that leave wavefronts of a key split without a tile, logits that run away from the
+    first tile's reference, references of extreme magnitude."""
+    g = torch.Generator().manual_seed(B + L + D)
+    q, k, v = (torch.randn(B, H, L, D, generator=g) for _ in range(3))
+    bias = torch.randn(H, L, L, generator=g)
+    keep = torch.rand(B, L, generator=g) < 0.8
+    if kind == "lopsided":
+        keep[:] = False
+        keep[::2, : min(L, 40)] = True
+        keep[1::2, L // 2] = True
+        keep[B // 2] = False
+    elif kind == "ramp":
+        bias += torch.linspace(-60.0, 80.0, L)
+    elif kind == "far":
+        bias[:, ::3] -= 3.0e6
+        bias[:, 1::3, : L // 2] = float("-inf")
+    if kind != "lopsided":
+        keep[:, L - 1] = True
+    out = af3.dot_product_attention_cpp(q.cuda(), k.cuda(), v.cuda(), keep.cuda(), bias.cuda())
+    torch.cuda.synchronize()
+    want = oracle.dpa_formula(f32np(q), f32np(k), f32np(v), keep.numpy(), f32np(bias))
+    rows = slice(None) if kind != "far" else slice(1, None, 3)      # (an offset of 3e6 leaves a logit two bits behind the point)
+    assert np.isfinite(f32np(out)).all()
+    assert np.abs(f32np(out) - want)[:, :, rows].max() <= 2e-5
+    if kind == "far":
+        assert np.abs(f32np(out) - want).max() <= 0.5
