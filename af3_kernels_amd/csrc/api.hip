@@ -89,6 +89,13 @@ extern "C" int64_t af3_dpa_workspace_bytes(const af3_dpa_params* params) {
 	return select_kernel(*params) == 1 ? mfma_bf16_workspace_bytes(*params) : 0;
 }
 
+// For the Python entry points' native host side (host.cpp), which allocates what this call will use, not what such a call may.
+extern "C" int64_t af3_dpa_workspace_used(const af3_dpa_params* params) {
+	const int rc = validate(params);
+	if(rc != AF3_OK) return rc;
+	return select_kernel(*params) == 1 ? mfma_bf16_workspace_used(*params) : 0;
+}
+
 extern "C" int af3_dpa_select_kernel(const af3_dpa_params* params) {
 	const int rc = validate(params);
 	if(rc != AF3_OK) return rc;

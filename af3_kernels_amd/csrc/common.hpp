@@ -74,6 +74,7 @@ bool mfma_rows_suits_a_small_batch(const af3_dpa_params& p);  // fewer than 128 
 int launch_dpa_mfma_rows(const af3_dpa_params& p, hipStream_t s);
 bool mfma_bf16_eligible(const af3_dpa_params& p);
 int64_t mfma_bf16_workspace_bytes(const af3_dpa_params& p);
+int64_t mfma_bf16_workspace_used(const af3_dpa_params& p);
 bool mfma_fp8_eligible(const af3_dpa_params& p);
 int launch_dpa_mfma_f32(const af3_dpa_params& p, hipStream_t s);
 bool mfma_f32_eligible(const af3_dpa_params& p);

@@ -64,13 +64,15 @@ __device__ __forceinline__ void load_bias8_guarded(const void* bias_row, int64_t
 // -2^126 rather than the most negative finite value so that the product with log2 e stays finite when a row's first
 // keys all carry it and it becomes the softmax reference for a while.  +inf and +NaN pass through and yield NaN, as
 // they do in the reference.  One packed unsigned minimum per dword.
+// (lim: that limit, twice.  Batches that have this kernel or the shared-bias kernel read the bias in place for speed take the
+// latter's limit of -2^16: a query row whose biases all lie beyond it is the softmax of q.k alone, whichever kernel serves it.)
+constexpr uint32_t BIAS_LIMIT_SINGLE = 0xFE80FE80u, BIAS_LIMIT_BATCH = 0xC780C780u;
 typedef __attribute__((ext_vector_type(2))) unsigned short u16x2;
-__device__ __forceinline__ u32x4 bias_frag_finite(u32x4 w) {
-	const u16x2 lim = {(unsigned short)0xFE80, (unsigned short)0xFE80};
+__device__ __forceinline__ u32x4 bias_frag_finite(u32x4 w, uint32_t lim) {
 #pragma unroll
 	for(int j = 0; j < 4; j++) {
 		const uint32_t x = w[j];  // (a copy: __builtin_bit_cast applied to the vector element itself reads element 0 with this compiler)
-		w[j] = __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2, x), lim));
+		w[j] = __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2, x), __builtin_bit_cast(u16x2, lim)));
 	}
 	return w;
 }
@@ -81,7 +83,7 @@ __device__ __forceinline__ u32x4 bias_frag_finite(u32x4 w) {
 // fp16(bias[q][64*kt + 16*f + 8*g + 0..7] * log2 e), zero outside the L x L corner.
 template <bool BIAS_F32>
 __global__ void __launch_bounds__(256) bias_prepass_kernel(const void* __restrict__ bias, u32x4* __restrict__ ws, int64_t H, int64_t L, int64_t stride_h,
-															 int64_t stride_q, int n_qblocks, int n_ktiles, bool vec_ok) {
+															 int64_t stride_q, int n_qblocks, int n_ktiles) {
 	// one workgroup per (head, query block, key tile) and trip: the index arithmetic (divisions) is per workgroup, on the
 	// scalar unit, not per thread; the launcher keeps the number of units below 2^31
 	const uint32_t units = (uint32_t)(H * n_qblocks * (int64_t)n_ktiles);
@@ -97,8 +99,8 @@ __global__ void __launch_bounds__(256) bias_prepass_kernel(const void* __restric
 		const int64_t esz  = BIAS_F32 ? 4 : 2;
 		const unsigned char* rowp = static_cast<const unsigned char*>(bias) + (h * stride_h + (row < L ? row : 0) * stride_q) * esz;
 		float f[8];
-		if(!BIAS_F32 && vec_ok && row < L && key + 8 <= L) {
-			const u32x4 raw = *reinterpret_cast<const u32x4*>(rowp + key * 2);
+		if(!BIAS_F32 && row < L && key + 8 <= L) {
+			const u32x4 raw = *reinterpret_cast<const u32x4_any*>(rowp + key * 2);
 #pragma unroll
 			for(int j = 0; j < 4; j++) f[2 * j] = bf16_bits_to_f32(raw[j] & 0xffffu), f[2 * j + 1] = bf16_bits_to_f32(raw[j] >> 16);
 		} else {
@@ -194,7 +196,7 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 	// two launch counts, waits, tests the early exit below, and only then requests the fields of p -- two memory latencies
 	// in a row, which every wavefront of a launch too small to hide them stands through.
 	asm volatile("" ::"s"(n_qtiles), "s"(n_groups), "s"(p.q), "s"(p.k), "s"(p.v), "s"(p.bias), "s"(p.key_mask), "s"(p.H), "s"(p.L), "s"(p.D), "s"(p.key_mask_stride_b),
-				 "s"(p.bias_stride[0]), "s"(p.bias_stride[1]));
+				 "s"(p.bias_stride[0]), "s"(p.bias_stride[1]), "s"(p.reserved));
 	asm volatile("" ::"s"(p.q_stride[0]), "s"(p.q_stride[1]), "s"(p.q_stride[2]), "s"(p.k_stride[0]), "s"(p.k_stride[1]), "s"(p.k_stride[2]), "s"(p.v_stride[0]), "s"(p.v_stride[1]),
 				 "s"(p.v_stride[2]));
 	const int64_t wg    = blockIdx.x;
@@ -212,6 +214,7 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 	const int     wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 	const int     n = lane & 31, half = lane >> 5;
 	const int64_t L = p.L;
+	[[maybe_unused]] const uint32_t bias_lim = (uint32_t)p.reserved;  // (the launcher's: BIAS_LIMIT_*)
 	// KS2: the workgroup has four wavefronts more than the NW that compute (one per SIMD).  They issue the tile loads of the
 	// workgroup, two or three tiles ahead, a quarter of every tile each, and otherwise only keep the barriers' count.  A wavefront that
 	// issues a tile's loads itself stands still while the compute unit's load path (64 bytes per clock) takes them in -- with
@@ -738,7 +741,7 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 				load_bias8_guarded<BIAS_F32>(bias_row, key0 + 16 * f, L, row_ok, v8);
 #pragma unroll
 				for(int j = 0; j < 4; j++) bfrag[f][j] = pack_bf16x2(v8[2 * j], v8[2 * j + 1]);
-				bfrag[f] = bias_frag_finite(bfrag[f]);
+				bfrag[f] = bias_frag_finite(bfrag[f], bias_lim);
 			}
 		};
 
@@ -929,14 +932,14 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 				return;
 			}
 #pragma unroll
-			for(int c2 = 0; c2 < 2; c2++) bfrag[2 * SUB + c2] = bias_frag_finite(*reinterpret_cast<const u32x4*>(bring + slot_off + (b_rd ^ ((4 * SUB + 2 * c2) << 4))));
+			for(int c2 = 0; c2 < 2; c2++) bfrag[2 * SUB + c2] = bias_frag_finite(*reinterpret_cast<const u32x4*>(bring + slot_off + (b_rd ^ ((4 * SUB + 2 * c2) << 4))), bias_lim);
 		};
 		auto bias_mfma = [&](f32x16 s, int f) -> f32x16 {
 			if(L2DOM) return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, idf[f & 1]), __builtin_bit_cast(f16x8, bfrag[f & 1]), s, 0, 0, 0);
 			u32x4 w = bfrag[f];
 			if constexpr(RAGGED)
 				w = bias_frag_finite(u32x4{__builtin_amdgcn_alignbit(w[1], w[0], b_shift), __builtin_amdgcn_alignbit(w[2], w[1], b_shift), __builtin_amdgcn_alignbit(w[3], w[2], b_shift),
-										   __builtin_amdgcn_alignbit(bfollow[f], w[3], b_shift)});
+										   __builtin_amdgcn_alignbit(bfollow[f], w[3], b_shift)}, bias_lim);
 			return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, idf[f & 1]), __builtin_bit_cast(bf16x8, w), s, 0, 0, 0);
 		};
 		// plain (not interleaved) S^T of one sub-tile; used once, for the very first sub-tile
@@ -1289,22 +1292,44 @@ static int64_t ws_bytes_needed(const af3_dpa_params& p) {
 	return p.H * n_qblocks * n_ktiles * 256 * 16;
 }
 
-// Whether the call goes to the kernel of dpa_mfma_rows.hip (four batch rows per wavefront sharing each bias tile): its
-// shape limits, enough workgroups of four-row groups to give every compute unit one (smaller launches through its workspace
-// do better with this file's variants: 16 x 4 x 768 x 32 26 us here against 32 us there) or fewer than 128 batch rows whose
+// Byte offsets inside a head's bf16 bias, and the loads' overhang at its end, fit 32 bits.
+static bool ring_bias_ok(const af3_dpa_params& p) {
+	return p.bias && p.bias_dtype == AF3_BF16 && ((p.L - 1) * p.bias_stride[1] + p.L) * 2 < ((int64_t)1 << 31) - 64 * 1024;
+}
+
+// Two or more batch rows in so small a launch that the one-row kernel, reading the bias in place once per batch row, beats
+// both a rewrite of the whole bias (3 us and up) and the shared-bias kernel (whose four chains per wavefront leave the chip
+// empty).  Measured, us, shared-bias kernel with the bias staged / one-row kernel with a rewritten bias / one-row kernel in place:
+//   128-row workgroups                      64               192               384               480              512              768              1024
+//   head_dim 24, 16 heads   2x512 16.4/15.0/8.1  2x768 21.4/22.7/12.3  3x1024 26.7/36.5/22.5  5x768 27.6/29.3/18.1  8x512 16.8/20.0/14.3  8x768 28.2/31.7/27.9  16x512 22.1/28.2/25.7
+//   head_dim 48, 16 heads   2x255  - /11.0/7.4   2x768  - /40.5/15.4   2x1536  - /83.4/56.1   5x768  - /44.0/32.8   2x2048 - /142/74      -                 5x1536 (960) - /100/112
+// (2x2048 at head_dim 24, 512 workgroups: 46.8/95.7/57.7 -- long rows make up for the shared-bias kernel's start.)
+static bool one_row_in_place(const af3_dpa_params& p) {
+	if(p.B < 2 || !ring_bias_ok(p)) return false;
+	const int64_t wg128 = p.B * p.H * ((p.L + 127) / 128);
+	return p.D > 32 ? wg128 <= 768 : wg128 <= 256 || (wg128 <= 512 && p.L <= 1536);
+}
+
+// Whether the shape suits the kernel of dpa_mfma_rows.hip (four batch rows per wavefront sharing each bias tile): its
+// shape limits, enough workgroups of four-row groups to give every compute unit one or fewer than 128 batch rows whose
 // bias it can stage in place, and the caller's hint (af3_dpa_params.reserved: 1 = take it whenever the shape allows, 2 = never).
-static bool rows_kernel_wanted(const af3_dpa_params& p) {
-	if(p.reserved == 2 || !mfma_rows_eligible(p)) return false;
-	if(p.reserved == 1) return true;
+static bool rows_kernel_suits(const af3_dpa_params& p) {
+	if((p.reserved & 3) == 2 || !mfma_rows_eligible(p)) return false;
+	if((p.reserved & 3) == 1) return true;
 	if((p.B / 4) * p.H * ((p.L + 127) / 128) >= 256) return true;  // (workgroups of the launch that takes the groups of four rows)
 	return mfma_rows_suits_a_small_batch(p);
 }
+static bool rows_kernel_wanted(const af3_dpa_params& p) { return rows_kernel_suits(p) && ((p.reserved & 3) == 1 || !one_row_in_place(p)); }
 
-// The rewrite costs one extra pass over the bias; it pays off as soon as two batch rows share it.
+// What a call may use at most: the rewritten bias of the kernel that suits its shape.
 int64_t mfma_bf16_workspace_bytes(const af3_dpa_params& p) {
 	if(!mfma_bf16_eligible(p) || !p.bias || p.B < 2) return 0;
-	if(rows_kernel_wanted(p)) return mfma_rows_workspace_bytes(p);
-	return ws_bytes_needed(p);
+	return rows_kernel_suits(p) ? mfma_rows_workspace_bytes(p) : ws_bytes_needed(p);
+}
+// ... and what this call will use.
+int64_t mfma_bf16_workspace_used(const af3_dpa_params& p) {
+	if(!mfma_bf16_eligible(p) || !p.bias || p.B < 2) return 0;
+	return rows_kernel_wanted(p) ? mfma_rows_workspace_bytes(p) : one_row_in_place(p) ? 0 : ws_bytes_needed(p);
 }
 
 // bias -> fp16(bias * log2 e) in fragment order, into p.workspace
@@ -1314,13 +1339,12 @@ static int launch_bias_prepass(const af3_dpa_params& p, hipStream_t s) {
 	const int64_t  total     = p.H * n_qblocks * (int64_t)n_ktiles * 256;
 	if(total / 256 >= ((int64_t)1 << 31)) return AF3_ERR_BAD_SHAPE;  // (the prepass counts its units in 32 bits)
 	const unsigned g         = (unsigned)((total + 255) / 256 > 65536 ? 65536 : (total + 255) / 256);
-	const bool     vec_ok    = ((reinterpret_cast<uintptr_t>(p.bias) & 15) == 0) && (p.bias_stride[0] % 8 == 0) && (p.bias_stride[1] % 8 == 0);
 	if(bf32)
 		hipLaunchKernelGGL(bias_prepass_kernel<true>, dim3(g), dim3(256), 0, s, p.bias, static_cast<u32x4*>(p.workspace), p.H, p.L, p.bias_stride[0], p.bias_stride[1], n_qblocks,
-						   n_ktiles, vec_ok);
+						   n_ktiles);
 	else
 		hipLaunchKernelGGL(bias_prepass_kernel<false>, dim3(g), dim3(256), 0, s, p.bias, static_cast<u32x4*>(p.workspace), p.H, p.L, p.bias_stride[0], p.bias_stride[1], n_qblocks,
-						   n_ktiles, vec_ok);
+						   n_ktiles);
 	return launch_status();
 }
 
@@ -1468,7 +1492,7 @@ static int launch_nw(const af3_dpa_params& p, hipStream_t s) {
 int launch_dpa_mfma_bf16(const af3_dpa_params& p, hipStream_t s) {
 	if(rows_kernel_wanted(p) && mfma_rows_can_serve(p)) return launch_dpa_mfma_rows(p, s);
 	const bool bf32   = p.bias && p.bias_dtype == AF3_F32;
-	const bool use_ws = p.bias && p.workspace && mfma_bf16_workspace_bytes(p) > 0 && p.workspace_bytes >= ws_bytes_needed(p) &&
+	const bool use_ws = p.bias && p.workspace && p.B >= 2 && !one_row_in_place(p) && p.workspace_bytes >= ws_bytes_needed(p) &&
 						(reinterpret_cast<uintptr_t>(p.workspace) & 15) == 0;
 	if(use_ws) {
 		const int rc = launch_bias_prepass(p, s);
@@ -1478,11 +1502,14 @@ int launch_dpa_mfma_bf16(const af3_dpa_params& p, hipStream_t s) {
 	// In-place bf16 bias: through the LDS ring.  Where rows are whole aligned 16-byte chunks that never straddle the end of a
 	// row's L valid entries a fragment is one LDS read (2); anywhere else (3) it is two and four shifts.
 	// Element by element (0) only where a head's slab exceeds the loads' 32-bit offsets.
-	const int mode = l2dom ? 0 : bf32 ? 1 : ((p.L - 1) * p.bias_stride[1] + p.L) * 2 >= ((int64_t)1 << 31) - 64 * 1024 ? 0 :
+	const int mode = l2dom ? 0 : bf32 ? 1 : !ring_bias_ok(p) ? 0 :
 					 (reinterpret_cast<uintptr_t>(p.bias) & 15) == 0 && p.bias_stride[0] % 8 == 0 && p.bias_stride[1] % 8 == 0 && p.L % 8 == 0 ? 2 : 3;
+	const bool batch_limit = p.B >= 2 && (p.workspace || (p.reserved & 4) || (rows_kernel_suits(p) && mfma_rows_workspace_bytes(p) == 0));
+	af3_dpa_params pl = p;
+	pl.reserved       = (int32_t)(batch_limit ? BIAS_LIMIT_BATCH : BIAS_LIMIT_SINGLE);
 	auto go = [&](auto dp_c) {
 		constexpr int DP = decltype(dp_c)::value;
-		return l2dom ? launch_nw<DP, true, 0>(p, s) : mode == 1 ? launch_nw<DP, false, 1>(p, s) : mode == 2 ? launch_nw<DP, false, 2>(p, s) : mode == 3 ? launch_nw<DP, false, 3>(p, s) : launch_nw<DP, false, 0>(p, s);
+		return l2dom ? launch_nw<DP, true, 0>(pl, s) : mode == 1 ? launch_nw<DP, false, 1>(pl, s) : mode == 2 ? launch_nw<DP, false, 2>(pl, s) : mode == 3 ? launch_nw<DP, false, 3>(pl, s) : launch_nw<DP, false, 0>(pl, s);
 	};
 	return p.D <= 32 ? go(ic<32>{}) : go(ic<64>{});
 }

@@ -38,7 +38,7 @@ constexpr float BIAS_FLOOR = -0x1p17f;     // lowest value the rewritten bias ho
 // follow their fp32 precision to within 2^-6.
 template <bool BIAS_F32>
 __global__ void __launch_bounds__(256) bias_rows_prepass_kernel(const void* __restrict__ bias, f32x4* __restrict__ ws, int64_t H, int64_t L, int64_t stride_h, int64_t stride_q,
-																  int n_qblocks, int n_tiles, bool vec_ok) {
+																  int n_qblocks, int n_tiles) {
 	// one workgroup per (head, query block, key tile) and trip: the index arithmetic (divisions) is per workgroup, on the
 	// scalar unit, not per thread; the launcher keeps the number of units below 2^31
 	const uint32_t units = (uint32_t)(H * n_qblocks * (int64_t)n_tiles);
@@ -56,8 +56,8 @@ __global__ void __launch_bounds__(256) bias_rows_prepass_kernel(const void* __re
 			const int64_t off = h * stride_h + row * stride_q + key;
 			if(BIAS_F32) {
 				const float* bp = static_cast<const float*>(bias) + off;
-				if(vec_ok && key + 4 <= L) {
-					const f32x4 raw = *reinterpret_cast<const f32x4*>(bp);
+				if(key + 4 <= L) {
+					const f32x4 raw = *reinterpret_cast<const f32x4_any*>(bp);
 					f[0] = raw[0], f[1] = raw[1], f[2] = raw[2], f[3] = raw[3];
 				} else {
 #pragma unroll
@@ -66,8 +66,8 @@ __global__ void __launch_bounds__(256) bias_rows_prepass_kernel(const void* __re
 				}
 			} else {
 				const uint16_t* bp = static_cast<const uint16_t*>(bias) + off;
-				if(vec_ok && key + 4 <= L) {
-					const u32x2 raw = *reinterpret_cast<const u32x2*>(bp);
+				if(key + 4 <= L) {
+					const u32x2 raw = *reinterpret_cast<const u32x2_any*>(bp);
 					f[0] = bf16_bits_to_f32(raw[0] & 0xffffu), f[1] = bf16_bits_to_f32(raw[0] >> 16);
 					f[2] = bf16_bits_to_f32(raw[1] & 0xffffu), f[3] = bf16_bits_to_f32(raw[1] >> 16);
 				} else {
@@ -815,14 +815,12 @@ int launch_dpa_mfma_rows(const af3_dpa_params& p, hipStream_t s) {
 		const int64_t  total     = p.H * n_qblocks * (int64_t)n_t_all * 256;
 		if(total / 256 >= ((int64_t)1 << 31)) return AF3_ERR_BAD_SHAPE;  // (the prepass counts its units in 32 bits)
 		const unsigned g         = (unsigned)((total + 255) / 256 > 65536 ? 65536 : (total + 255) / 256);
-		const int64_t  esz       = bf32 ? 4 : 2;
-		const bool     vec_ok    = ((reinterpret_cast<uintptr_t>(p.bias) & (4 * esz - 1)) == 0) && (p.bias_stride[0] % 4 == 0) && (p.bias_stride[1] % 4 == 0);
 		if(bf32)
 			hipLaunchKernelGGL(bias_rows_prepass_kernel<true>, dim3(g), dim3(256), 0, s, p.bias, static_cast<f32x4*>(p.workspace), p.H, p.L, p.bias_stride[0], p.bias_stride[1],
-							   n_qblocks, n_t_all, vec_ok);
+							   n_qblocks, n_t_all);
 		else
 			hipLaunchKernelGGL(bias_rows_prepass_kernel<false>, dim3(g), dim3(256), 0, s, p.bias, static_cast<f32x4*>(p.workspace), p.H, p.L, p.bias_stride[0], p.bias_stride[1],
-							   n_qblocks, n_t_all, vec_ok);
+							   n_qblocks, n_t_all);
 		const int rc = launch_status();
 		if(rc != AF3_OK) return rc;
 	}

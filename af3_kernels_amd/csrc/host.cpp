@@ -24,6 +24,8 @@
 
 #include "../../include/af3_dpa.h"
 
+extern "C" int64_t af3_dpa_workspace_used(const af3_dpa_params*);   // (api.hip; not part of the ABI)
+
 namespace {
 
 using at::Tensor;
@@ -94,7 +96,8 @@ af3_dpa_params block(int64_t B, int64_t H, int64_t L, int64_t D, int code, int64
 }
 int forward(af3_dpa_params& p, bool exact_bias, int dev) {
 	at::DataPtr   ws;
-	const int64_t bytes = exact_bias ? 0 : af3_dpa_workspace_bytes(&p);
+	if(!exact_bias) p.reserved |= 4;
+	const int64_t bytes = exact_bias ? 0 : af3_dpa_workspace_used(&p);
 	if(bytes > 0) ws = new_scratch(bytes), p.workspace = ws.get(), p.workspace_bytes = bytes;
 	return af3_dpa_forward(&p, current_stream(dev));
 }

@@ -14,6 +14,10 @@ constexpr float PSUM_LIMIT = 0x1p30f;  // per-lane row-sum bound that triggers t
 typedef __attribute__((ext_vector_type(2))) __bf16   bf16x2;
 typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
 typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
+// vectors at any element's address (global memory takes them; the compiler must be told not to split the access)
+typedef __attribute__((ext_vector_type(4), aligned(2))) uint32_t u32x4_any;
+typedef __attribute__((ext_vector_type(2), aligned(2))) uint32_t u32x2_any;
+typedef __attribute__((ext_vector_type(4), aligned(4))) float    f32x4_any;
 template <int V>
 using ic = std::integral_constant<int, V>;
 

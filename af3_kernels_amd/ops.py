@@ -125,7 +125,7 @@ def _fill_params(q, k, v, keep, bias, out, mma_dtype, force_generic, descales=No
     """The argument block of one call.  Everything that depends on the layout alone is filled once per layout and copied
     from a byte template afterwards (building the ctypes arrays anew costs more host time than a small call's kernel runs);
     only the addresses are set per call."""
-    key = (q.shape, q.stride(), k.stride(), v.stride(), out.stride(), q.dtype, out.dtype, mma_dtype, bool(force_generic), _rows_kernel_hint, softmax_scale,
+    key = (q.shape, q.stride(), k.stride(), v.stride(), out.stride(), q.dtype, out.dtype, mma_dtype, bool(force_generic), _rows_kernel_hint, _exact_bias, softmax_scale,
            None if bias is None else (bias.stride(0), bias.stride(1), bias.dtype),
            None if keep is None else (keep.shape[0], keep.stride(0)),
            None if gate is None else gate.stride())
@@ -149,7 +149,7 @@ def _fill_params(q, k, v, keep, bias, out, mma_dtype, force_generic, descales=No
         t.softmax_scale = float(D) ** -0.5 if softmax_scale is None else softmax_scale
         t.q_descale = t.k_descale = t.v_descale = 1.0
         t.force_generic = int(bool(force_generic))
-        t.reserved = _rows_kernel_hint
+        t.reserved = _rows_kernel_hint | (0 if _exact_bias else 4)
         if gate is not None:
             t.gate_stride = (ctypes.c_int64 * 3)(*gate.stride()[:3])
         template = bytes(t)

@@ -100,7 +100,8 @@ typedef struct af3_dpa_params {
 	int32_t        force_generic; /* non-zero: always take the fp32-FMA kernel (testing aid) */
 	int32_t        reserved;      /* kernel hint for batched bf16 calls that the shared-bias kernel (two to four batch rows per
 	                                 wavefront) can take (head_dim <= 32, B >= 2, L <= 4096): 0 = chosen by launch size, 1 = always,
-	                                 2 = never (testing aids) */
+	                                 2 = never (testing aids).  Plus 4: entries of a bias read in place by a batch are clamped from
+	                                 below at -2^16, as when a workspace is given, though this call needs none */
 	/* Optional: 3 device floats {q_descale, k_descale, v_descale} as written by
 	 * af3_quantize_fp8_e4m3; when non-NULL they override the three host values above, so a
 	 * quantise -> attend sequence needs no device-to-host copy. */
@@ -159,10 +160,11 @@ typedef struct af3_dpa_params {
  */
 int af3_dpa_forward(const af3_dpa_params* params, void* hip_stream);
 
-/* Bytes of workspace the call would use (0 when a workspace would not help, e.g. B == 1,
+/* Bytes of workspace the call may use at most: 0 when a workspace would not help, e.g. B == 1,
  * no bias, a bf16 bias with 16-byte aligned rows under too few batch rows for a rewrite to pay
  * off -- fewer than about 224 + 2.4e8 / (H L^2); it is then read in place, exactly -- or a kernel
- * that does not take one); negative = af3_status error.  Host only. */
+ * that does not take one; negative = af3_status error.  (A launch that fills little of the GPU reads
+ * its bias in place whatever workspace it is given.)  Host only. */
 int64_t af3_dpa_workspace_bytes(const af3_dpa_params* params);
 
 /*

@@ -122,3 +122,26 @@ def test_fp32_forms(af3, oracle, B, H, L, D, kind):
     assert np.abs(f32np(out) - want)[:, :, rows].max() <= 2e-5
     if kind == "far":
         assert np.abs(f32np(out) - want).max() <= 0.5
+
+
+@pytest.mark.parametrize("B,H,L,D,pad", [
+    (37, 4, 37, 32, 0), (2, 1, 1, 8, 3), (3, 2, 129, 24, 1), (16, 4, 128, 32, 0),      # one round of workgroups
+    (128, 4, 128, 32, 0), (125, 4, 127, 32, 1),                                        # 512 and 500 workgroups of 128 rows: the most that read in place
+    (129, 4, 128, 32, 0), (129, 4, 127, 24, 0),                                        # 516: shared-bias kernel
+    (5, 16, 191, 48, 0), (2, 16, 255, 64, 1), (48, 16, 70, 48, 0), (49, 16, 70, 48, 3),   # head_dim padded to 64; up to 768 workgroups, past it a workspace
+    (40, 4, 200, 24, 5), (64, 4, 203, 32, 0),                                          # workspace written from rows at any address
+])
+def test_batched_bias_at_any_address(af3, oracle, B, H, L, D, pad):
+    """Batches on both sides of the line up to which the one-row kernel reads the bias in place, and rewrites of ragged rows."""
+    g = torch.Generator().manual_seed(B + L)
+    q, k, v = (torch.randn(B, H, L, D, generator=g).to(torch.bfloat16) for _ in range(3))
+    M = L + pad
+    bias = torch.full((H, M, M), float("nan")).to(torch.bfloat16)
+    bias[:, :L, :L] = torch.randn(H, L, L, generator=g).to(torch.bfloat16)
+    keep = torch.rand(B, L, generator=g) < 0.8
+    keep[:, L // 2] = True
+    keep[B // 2] = False
+    out = af3.dot_product_attention_cpp(q.cuda(), k.cuda(), v.cuda(), keep.cuda(), bias.cuda())
+    torch.cuda.synchronize()
+    want = oracle.dpa_formula(f32np(q), f32np(k), f32np(v), keep.numpy(), f32np(bias[:, :L, :L]))
+    assert np.abs(f32np(out) - want).max() <= 2e-2
