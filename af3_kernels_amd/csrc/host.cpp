@@ -25,6 +25,8 @@
 #include "../../include/af3_dpa.h"
 
 extern "C" int64_t af3_dpa_workspace_used(const af3_dpa_params*);   // (api.hip; not part of the ABI)
+extern "C" int af3_project_suits(int64_t, int64_t, int64_t);              // (projection.hip, likewise)
+extern "C" int af3_project(const void*, const void*, const void*, void*, int64_t, int64_t, int64_t, int32_t, void*);
 
 namespace {
 
@@ -267,6 +269,18 @@ int attend(const Tensor& y, int64_t B, int64_t N, int64_t head, const key_mask& 
 	return forward(p, exact, dev);
 }
 
+// rows of x [.., C] times the fused projection weight [4C, C], plus the row: this library's kernel where it suits, a library GEMM otherwise
+Tensor project(const Tensor& x, int64_t M, const Tensor& weight, const Tensor* row, int dev, int& rc) {
+	const int64_t K = weight.size(1), N = weight.size(0);
+	rc = AF3_OK;
+	if(x.scalar_type() == at::kBFloat16 && weight.is_contiguous() && af3_project_suits(M, N, K) && reinterpret_cast<uintptr_t>(x.const_data_ptr()) % 16 == 0) {
+		Tensor y = new_tensor({M, N}, at::kBFloat16, dev);
+		rc = af3_project(x.const_data_ptr(), weight.const_data_ptr(), row ? row->const_data_ptr() : nullptr, y.data_ptr(), M, N, K, 0, current_stream(dev));
+		return y;
+	}
+	return at::linear(x.dim() == 2 ? x : x.reshape({M, K}), weight, row ? *row : Tensor());
+}
+
 // self_attention(x [N, C] or [S, N, C], mask, bias, wq, wk, wv, wg, q_bias, head, kernel hint, exact bias)
 PyObject* py_self_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
 	HANDLE_TH_ERRORS
@@ -290,8 +304,9 @@ PyObject* py_self_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
 	int    rc;
 	{
 		without_gil g;
-		const Tensor y = at::linear(x->dim() == 3 ? x->view({S * N, C}) : *x, weight, row);
-		if(y.scalar_type() != x->scalar_type() || !y.is_contiguous()) rc = 1;  // (autocast)
+		const Tensor y = project(*x, S * N, weight, &row, dev, rc);
+		if(rc != AF3_OK) {
+		} else if(y.scalar_type() != x->scalar_type() || !y.is_contiguous()) rc = 1;  // (autocast)
 		else {
 			out = new_tensor(x->sizes(), x->scalar_type(), dev);
 			rc  = attend(y, S, N, head, m, bias, out, hint, exact, dev);

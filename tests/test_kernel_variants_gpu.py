@@ -145,3 +145,25 @@ def test_batched_bias_at_any_address(af3, oracle, B, H, L, D, pad):
     torch.cuda.synchronize()
     want = oracle.dpa_formula(f32np(q), f32np(k), f32np(v), keep.numpy(), f32np(bias[:, :L, :L]))
     assert np.abs(f32np(out) - want).max() <= 2e-2
+
+
+@pytest.mark.parametrize("with_row", [True, False])
+@pytest.mark.parametrize("M,N,K,form", [
+    (1, 64, 64, 0), (65, 128, 64, 11), (63, 320, 192, 11), (129, 64, 128, 21), (200, 256, 320, 13), (64, 192, 64, 13), (257, 192, 256, 22),
+    (127, 448, 64, 23), (129, 384, 448, 23), (1000, 1536, 384, 0), (2049, 3072, 768, 0),
+])
+def test_projection_forms(af3, M, N, K, form, with_row):
+    """The projection product against the same product in float32, per tile form; rows behind M and columns behind N are not touched."""
+    import ctypes
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x, w, row = (torch.randn(*s, generator=g, device="cuda", dtype=torch.bfloat16) for s in ((M, K), (N, K), (N,)))
+    out = torch.full((M + 1, N), 7.0, device="cuda", dtype=torch.bfloat16)
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())
+    print("case", M, N, K, form, with_row, flush=True)
+    rc = af3._lib.load().af3_project(ptr(x), ptr(w), ptr(row) if with_row else None, ptr(out), ctypes.c_int64(M), ctypes.c_int64(N), ctypes.c_int64(K), form,
+                                     ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert rc == 0
+    want = x.float() @ w.float().t() + (row.float() if with_row else 0.0)
+    assert (out[:M].float() - want).abs().max() <= 2 ** -8 * want.abs().max()
+    assert bool((out[M] == 7.0).all())
