@@ -8,15 +8,32 @@
 //     q8 = e4m3(q * softmax_scale * sq),  k8 = e4m3(k * sk),  v8t = e4m3(v * sv) transposed to [B,H,D,L]
 // with power-of-two scales, so that with alpha = 1/(sq*sk)
 //     logits = alpha * (q8 . k8^T) + bias            (natural units)
-// Layout is the "transposed" one of the bf16 kernel (dpa_mfma.hip): S^T = K8 . Q8^T with lane
-// (q = lane%32, half = lane/32) holding 16 keys of one query row; the bias rides an identity MFMA
-// whose diagonal is 1/alpha (a power of two, exact in bf16), the key mask a third MFMA;
+// Layout is the "transposed" one of the bf16 kernel (dpa_mfma.hip): S^T = K8 . Q8^T with a lane
+// holding 16 keys of one query row; the bias rides an identity MFMA
+// whose diagonal is 1/alpha (a power of two, exact in bf16), the key mask a third MFMA, in tiles that drop a key;
 // P^T = exp(logit - m) * 2^8 is quantised to e4m3 in registers (values in (0, 256], e4m3 tops out at
 // 448) and is the B operand of O^T += V8^T . P^T.  The row maximum m is the true running maximum
 // (no slack: P must stay below the e4m3 range), the row sum is taken over the quantised P, on the matrix pipe.
-// V arrives transposed, so V^T fragments are plain 4-byte LDS reads (no transposing loads exist for
-// 8-bit data paired with this accumulator layout).
-#include "common.hpp"
+//
+// What bounds it: the vector port (16 fma, 16 exponentials, 8 packs, a dozen maxima and, while maxima still move, 17 products
+// per 32 x 32 logits), then the matrix pipe (256 to 288 clocks), shared by up to four wavefronts per SIMD; everything else must
+// stay out of their way:
+//   * Key order.  Row r = 8 a + 4 g + e of S^T holds key 16 g + 4 a + e of its 32 keys (K rows, mask entries and the identity are
+//     read in that order), so that a lane's 16 keys are consecutive and its V^T operand is ONE 16-byte LDS read.  Chunks are
+//     XOR-swizzled: no bank conflicts.  (In natural order V^T took four 4-byte reads of eight-fold conflicts and K 8-byte ones.)
+//   * K.Q^T on the 64-deep instruction.  Head_dim up to 32, compensated: a lane's 32 bytes are the K row (lower half-wave) or its
+//     residual (upper), so that (k8 | k_lo) meets (q8 | q8) and then (q_lo | 0): 128 clocks instead of the 192 of six 16-deep ones.
+//   * Row sums through P.V: where head columns are padded, rows D and D + 4 of the V^T tile are ones, and the sum is a row of O^T.
+//   * A stage overlaps the logits of the next 32 keys with the exponentials of these, and leaves P.V to run under the next maxima.
+//   * The bias tile of each wavefront travels through LDS as whole 64-byte row segments, by loads that write LDS directly, a tile
+//     ahead (16-byte loads from 32 rows per instruction before); rows that start at any element are fetched from the dword
+//     below and shifted when read (element by element before).
+//   * 39 KB of LDS and 128 registers: four workgroups of four wavefronts per compute unit.
+// us per call with its two quantising launches (12 to 14 us), 16 heads of 24, before / now: 5x1536 89.0/71.3, 8x1536 133.6/104.9, 8x1301 (ragged
+// rows) -/101.7, 8x1000 66.7/54.2, 5x300 37.9/20.3, 1x1536 42.1/34.2.  Measured on the way: the bias loads are 13 us of the
+// 57 that the kernel takes at 5x1536, the exponentials 4; four workgroups per compute unit instead of three changed nothing, nor did
+// pinning the matrix instructions between the exponentials: the vector port is busy three quarters of the time.
+#include "mfma_helpers.hpp"
 
 namespace af3 {
 
@@ -26,33 +43,39 @@ constexpr int KT8   = 64;    // keys per tile
 constexpr int NW8   = 4;     // wavefronts per workgroup (32 query rows each)
 constexpr int MAX_L8 = 8192;
 constexpr float P_SHIFT = 8.f;  // P is stored as p * 2^8
+constexpr int BIAS_HALF8 = 2048 + 128;   // 32 rows x 32 keys of bf16, and one dword per row behind them (rows that start at any element)
+constexpr int16_t TILE_FULL = 0x4000;    // flag in a tile list entry: no key of the tile is dropped
+typedef __attribute__((ext_vector_type(8))) int i32x8;
 
-typedef __attribute__((ext_vector_type(2))) uint32_t u32v2;
-
-__device__ __forceinline__ float hswap_max(float x) {
-	auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-	return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+__device__ __forceinline__ float max3(float a, float b, float c) {   // (written out: fmaxf quiets its operands first)
+	float r;
+	asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+	return r;
 }
 
 // DP: head_dim padded to 32 or 64 (bytes per K row in LDS, rows of the V^T tile).
 // COMP: compensated logits q8.k8 + q8.k_lo + q_lo.k8 (the residual tensors recover the e4m3 rounding of q and k).
-template <int DP, bool COMP>
-__global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(2))) dpa_mfma_fp8_kernel(af3_dpa_params p, int n_qtiles, int64_t n_groups) {
-	constexpr int NC       = DP / 16;       // contraction chunks of QK^T
+// ONES: head_dim < DP, row sums through P.V; otherwise two 16x16x32 instructions per 32 keys.
+// BMODE: 0 = no bias, 1 = element by element (a head's slab beyond 32-bit offsets), 2 = through LDS, rows of whole aligned
+// 16-byte chunks, 3 = through LDS, rows that start at any element.
+template <int DP, bool COMP, bool ONES, int BMODE>
+__global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(DP == 32 ? 4 : 3))) dpa_mfma_fp8_kernel(af3_dpa_params p, int n_qtiles, int64_t n_groups) {
 	constexpr int NDB      = DP / 32;       // 32-row blocks of O^T
 	constexpr int K_TILE1  = KT8 * DP;      // bytes of one K tile
 	constexpr int K_TILE   = K_TILE1 * (COMP ? 2 : 1);  // hi tile followed by the residual tile
 	constexpr int V_TILE   = DP * KT8;      // bytes: [DP rows d][64 keys]
-	constexpr int K_LOADS  = K_TILE1 / 1024; // 1 KB wave loads per K tile (2 or 4)
-	constexpr int V_LOADS  = V_TILE / 1024;
+	constexpr int TILE     = K_TILE + V_TILE;
+	constexpr int K_LOADS  = K_TILE / 1024, V_LOADS = V_TILE / 1024; // 1 KB wave loads per tile
+	constexpr bool RING    = BMODE >= 2, RAGGED = BMODE == 3;
 
 	extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-	unsigned char* const k_lds     = smem;                  // [2][K_TILE]
-	unsigned char* const v_lds     = smem + 2 * K_TILE;     // [2][V_TILE]
-	uint32_t* const      mask_tab  = reinterpret_cast<uint32_t*>(smem + 2 * K_TILE + 2 * V_TILE);
+	// [3][K tile, V^T tile] [two half slots of bias per wavefront] [mask table: bf16 bits per key] [tile list]
+	constexpr int        SLOT_BASE = 3 * TILE;
+	constexpr int        MASK_BASE = SLOT_BASE + (RING ? NW8 * 2 * BIAS_HALF8 : 0);
+	uint16_t* const      mask_tab  = reinterpret_cast<uint16_t*>(smem + MASK_BASE);
 	const int            n_ktiles  = (int)((p.L + KT8 - 1) / KT8);
-	int16_t* const       live_list = reinterpret_cast<int16_t*>(mask_tab + n_ktiles * KT8 + 64);
-	__shared__ int       s_nvalid, s_nlive;
+	int16_t* const       live_list = reinterpret_cast<int16_t*>(mask_tab + n_ktiles * KT8) + 4;
+	int32_t* const       counts    = reinterpret_cast<int32_t*>(mask_tab + n_ktiles * KT8);   // [0] any live key, [1] tiles to walk (a static array would cost 1 KB)
 
 	// workgroup -> (batch, head, query tile), all query tiles of one (batch, head) on one XCD
 	// the kernel arguments that the start of a workgroup needs, requested in one batch (otherwise: the launch counts, a wait,
@@ -75,41 +98,186 @@ __global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(2
 	const int64_t L = p.L;
 	const int     D = (int)p.D;
 
-	// zero both tile buffers (padded head columns and rows past L are never written; e4m3 zero is 0x00)
-	for(int i = tid; i < (2 * K_TILE + 2 * V_TILE) / 16; i += NW8 * 64) reinterpret_cast<u32x4*>(smem)[i] = u32x4{0u, 0u, 0u, 0u};
-	if(tid == 0) s_nvalid = 0;
-	if(tid < 64) mask_tab[n_ktiles * KT8 + tid] = 0u;
+	const int64_t qrow   = (int64_t)qtile * (NW8 * 32) + wave * 32 + n;
+	const bool    row_ok = qrow < L;
+	const int     key_of_row = 16 * ((n >> 2) & 1) + 4 * (n >> 3) + (n & 3);   // the key that row n of S^T holds, of its 32
+
+	// ---- tile loaders (1 KB per wave instruction, straight into LDS) ----
+	// K: lane i of a load -> tile row i / (DP/16), chunk position i % (DP/16); V^T: lane i -> row d = i / 4, position i % 4 of
+	// its 64 keys.  Positions hold the chunks under the swizzles k_sw, v_sw.  K rows past L repeat row L - 1 (their keys carry the
+	// out-of-range mask value); head columns past D are not fetched (the buffers are cleared first: a stale byte there must not be a NaN
+	// pattern), nor rows past D of V^T.
+	auto k_sw = [](int row) -> int { return DP == 32 ? (row >> 4) & 1 : ((row >> 4) & 1) | (((row >> 2) & 1) << 1); };
+	auto v_sw = [](int row) -> int { return (row >> 2) & 3; };
+	const uint32_t k_bytes  = (uint32_t)((L - 1) * p.k_stride[2] + D);
+	const u32x4    k_rsrc   = raw_rsrc(static_cast<const uint8_t*>(p.k) + b * p.k_stride[0] + h * p.k_stride[1], k_bytes);
+	const u32x4    klo_rsrc = raw_rsrc(static_cast<const uint8_t*>(COMP ? p.k_lo : p.k) + b * p.k_stride[0] + h * p.k_stride[1], k_bytes);
+	const u32x4    v_rsrc   = raw_rsrc(static_cast<const uint8_t*>(p.v) + b * p.v_stride[0] + h * p.v_stride[1], (uint32_t)(D * p.v_stride[2]));
+	constexpr int KCPR = DP / 16;       // 16-byte chunks per K row
+	constexpr int KRPI = 1024 / DP;     // K rows per wave load
+	constexpr int KPW  = (K_LOADS + NW8 - 1) / NW8, VPW = (V_LOADS + NW8 - 1) / NW8;   // loads per wavefront at most
+	constexpr int KV_MIN = K_LOADS / NW8;   // ... and at least (V loads of padded rows only are not issued)
+	const uint32_t lds0 = lds_addr_of(smem);
+	const int      k_row_bytes = (int)p.k_stride[2];
+	int  k_voff[KPW], v_voff[VPW];
+	bool k_on[KPW], v_on[VPW];
+#pragma unroll
+	for(int t = 0; t < KPW; t++) {
+		const int j = wave + NW8 * t, r = (COMP ? j % (K_LOADS / 2) : j) * KRPI + lane / KCPR, ch = (lane % KCPR) ^ k_sw(r);
+		k_voff[t] = r * k_row_bytes + ch * 16, k_on[t] = j < K_LOADS && ch * 16 < D;
+	}
+#pragma unroll
+	for(int t = 0; t < VPW; t++) {
+		const int j = NW8 - 1 - wave + NW8 * t, d = j * 16 + (lane >> 2);   // (from the last wavefront on: the first ones may have one K load more)
+		v_voff[t] = d * (int)p.v_stride[2] + (((lane & 3) ^ v_sw(d)) << 4), v_on[t] = j < V_LOADS && d < D;
+	}
+	auto load_tile = [&](int kt, int buf_off) {
+#pragma unroll
+		for(int t = 0; t < KPW; t++) {
+			const int  j  = wave + NW8 * t;
+			const bool lo = COMP && j >= K_LOADS / 2;
+			int        o  = k_voff[t] + kt * (KT8 * k_row_bytes);
+			if((kt + 1) * KT8 > (int)L) {   // (wave-uniform: the last tile)
+				const int over = kt * KT8 + (COMP ? j % (K_LOADS / 2) : j) * KRPI + lane / KCPR - ((int)L - 1);
+				if(over > 0) o -= over * k_row_bytes;
+			}
+			if(k_on[t]) lds_dma_b128(lo ? klo_rsrc : k_rsrc, lds0 + buf_off + j * 1024, o);
+		}
+#pragma unroll
+		for(int t = 0; t < VPW; t++) {
+			const int j = NW8 - 1 - wave + NW8 * t;
+			if(v_on[t]) lds_dma_b128(v_rsrc, lds0 + buf_off + K_TILE + j * 1024, v_voff[t] + kt * KT8);
+		}
+	};
+	// ---- bias half slots (32 keys each): two loads of sixteen 64-byte row segments, chunk c of row r at position c ^ ((r >> 2) & 3);
+	// RAGGED: from the dword that holds a row's first key, plus the dword behind the half of each row (see dpa_mfma.hip) ----
+	const uintptr_t b_base = RING ? reinterpret_cast<uintptr_t>(static_cast<const uint16_t*>(p.bias) + h * p.bias_stride[0]) : 0;
+	const int       b_odd  = RAGGED ? (int)(b_base & 2) : 0;
+	const u32x4     b_rsrc = raw_rsrc(reinterpret_cast<const void*>(b_base - b_odd), RING ? (uint32_t)((((L - 1) * p.bias_stride[1] + L) * 2 + b_odd + 3) & ~3ll) : 0u);
+	const int       b_row_bytes = (int)(p.bias_stride[1] * 2), q0 = qtile * (NW8 * 32) + wave * 32;
+	const uint32_t  slot_addr   = lds0 + SLOT_BASE + wave * (2 * BIAS_HALF8);
+	constexpr int   BIAS_LOADS  = RAGGED ? 3 : RING ? 2 : 0;
+	int b_voff[2] = {0, 0}, b_tail = 0;
+	const int b_chunk = (lane & 3) ^ ((lane >> 4) & 3);   // (row 16 j + lane / 4)
+	if constexpr(RING) {
+#pragma unroll
+		for(int j = 0; j < 2; j++) {
+			const int row = q0 + 16 * j + (lane >> 2) < (int)L ? q0 + 16 * j + (lane >> 2) : (int)L - 1;
+			b_voff[j]     = ((b_odd + row * b_row_bytes) & (RAGGED ? ~3 : ~0)) + b_chunk * 16;
+		}
+		const int row = q0 + n < (int)L ? q0 + n : (int)L - 1;
+		b_tail        = ((b_odd + row * b_row_bytes) & ~3) + 64;
+	}
+	auto load_bias = [&](int kt, int sub) {
+		if constexpr(!RING) return;
+		int off = kt * (KT8 * 2) + sub * 64;
+		if(!RAGGED && (kt + 1) * KT8 > (int)L) {   // (wave-uniform: the last tile) chunks past L: the row's last one again
+			asm volatile("");   // (kept a branch: as selects it costs every tile six instructions)
+			const int over = kt * KT8 + sub * 32 + b_chunk * 8 - ((int)L - 8);
+			if(over > 0) off -= over * 2;
+		}
+#pragma unroll
+		for(int j = 0; j < 2; j++) lds_dma_b128(b_rsrc, slot_addr + sub * BIAS_HALF8 + j * 1024, b_voff[j] + off);
+		if constexpr(RAGGED)
+			if(half == 0) lds_dma_b32(b_rsrc, slot_addr + sub * BIAS_HALF8 + 2048, b_tail + off);
+	};
+
+	// ---- requested first: the key-mask bytes (four keys per lane and load where rows allow), q, and -- once the buffers are cleared -- the
+	// first tile and its bias, on the guess that it holds a live key ----
+	const uint8_t* keep     = p.key_mask ? p.key_mask + b * p.key_mask_stride_b : nullptr;
+	const bool     mask_vec = !keep || (((reinterpret_cast<uintptr_t>(p.key_mask) | (uintptr_t)p.key_mask_stride_b | (uintptr_t)L) & 3) == 0);
+	const int      n_chunks = (n_ktiles * KT8 + 255) / 256;
+	uint32_t       mraw[2];
+	auto request_mask = [&](int c0) {
+#pragma unroll
+		for(int i = 0; i < 2; i++) {
+			const int64_t key0 = (int64_t)(c0 + i * NW8) * 256 + 4 * lane;
+			mraw[i]            = 0u;
+			if(c0 + i * NW8 < n_chunks) mraw[i] = !keep ? 0x01010101u : (key0 < L ? *reinterpret_cast<const uint32_t*>(keep + key0) : 0u);
+		}
+	};
+	if(mask_vec) request_mask(wave);
+	// q operands of the 64-deep instruction: lane (q, g = half) holds columns [32 g, ..) of q8 and q_lo (DP = 64), or all 32 columns
+	// of q8 in both half-waves (not compensated: in the lower) and of q_lo in the lower (DP = 32); zeros elsewhere
+	i32x8 qa, qb;
+	{
+		const int64_t qoff = b * p.q_stride[0] + h * p.q_stride[1] + qrow * p.q_stride[2];
+#pragma unroll
+		for(int c = 0; c < 4; c++) {
+			const int d0 = (DP == 64 ? 32 * half : 0) + 8 * c;
+			u32x2     x = {0u, 0u}, y = {0u, 0u};
+			if(row_ok && d0 < D && (DP == 64 || COMP || half == 0)) x = *reinterpret_cast<const u32x2*>(static_cast<const uint8_t*>(p.q) + qoff + d0);
+			if(COMP && row_ok && d0 < D && (DP == 64 || half == 0)) y = *reinterpret_cast<const u32x2*>(static_cast<const uint8_t*>(p.q_lo) + qoff + d0);
+			qa[2 * c] = (int)x[0], qa[2 * c + 1] = (int)x[1], qb[2 * c] = (int)y[0], qb[2 * c + 1] = (int)y[1];
+		}
+	}
+	for(int i = tid; i < SLOT_BASE / 16; i += NW8 * 64) reinterpret_cast<u32x4*>(smem)[i] = u32x4{0u, 0u, 0u, 0u};
 	__syncthreads();
-	const uint8_t* keep = p.key_mask ? p.key_mask + b * p.key_mask_stride_b : nullptr;
-	for(int kt = wave; kt < n_ktiles; kt += NW8) {
-		const int64_t key  = (int64_t)kt * KT8 + lane;
-		const bool    in   = key < L;
-		const bool    live = in && (keep ? keep[key] != 0 : true);
-		mask_tab[kt * KT8 + lane] = live ? 0u : (in ? (uint32_t)MASK_DROPPED_BF16 : (uint32_t)MASK_OUT_OF_RANGE_BF16);
-		const unsigned long long bal = __ballot(live);
-		if(lane == 0) {
-			live_list[kt] = bal ? 1 : 0;
-			if(bal) atomicAdd(&s_nvalid, 1);
+	load_tile(0, 0);
+	load_bias(0, 0);
+	load_bias(0, 1);
+	if constexpr(ONES) {   // (e4m3 1.0; no load writes these rows)
+		if(tid < 96) {
+			const int buf = tid >> 5, r = (tid >> 4) & 1, w = tid & 15;
+			reinterpret_cast<uint32_t*>(smem + buf * TILE + K_TILE + (D + 4 * r) * KT8)[w] = 0x38383838u;
+		}
+	}
+
+	// ---- key-mask table, flags of the tiles with a live key, list of those tiles ----
+	auto flag_of = [&](bool any_live, bool any_not) -> int16_t { return (int16_t)((any_live ? 1 : 0) | (any_not ? 0 : TILE_FULL)); };
+	if(mask_vec) {
+		for(int c0 = wave; c0 < n_chunks; c0 += 2 * NW8) {
+			if(c0 != wave) request_mask(c0);
+#pragma unroll
+			for(int i = 0; i < 2; i++) {
+				const int c = c0 + i * NW8;
+				if(c >= n_chunks) break;
+				const int key0 = c * 256 + 4 * lane;
+				uint32_t  e[4];
+				bool      any = false, all = true;
+#pragma unroll
+				for(int j = 0; j < 4; j++) {
+					const bool in   = key0 + j < (int)L;
+					const bool live = in && ((mraw[i] >> (8 * j)) & 0xffu) != 0;
+					any             = any || live, all = all && live;
+					e[j]            = live ? 0u : (in ? (uint32_t)MASK_DROPPED_BF16 : (uint32_t)MASK_OUT_OF_RANGE_BF16);
+				}
+				if(key0 < n_ktiles * KT8) *reinterpret_cast<u32x2*>(mask_tab + key0) = u32x2{e[0] | (e[1] << 16), e[2] | (e[3] << 16)};
+				const unsigned long long bal = __ballot(any), baln = __ballot(!all);   // 16 lanes per tile
+				if(lane < 4 && 4 * c + lane < n_ktiles) live_list[4 * c + lane] = flag_of(((bal >> (16 * lane)) & 0xffffull) != 0, ((baln >> (16 * lane)) & 0xffffull) != 0);
+			}
+		}
+	} else {
+		for(int kt = wave; kt < n_ktiles; kt += NW8) {
+			const int64_t key  = (int64_t)kt * KT8 + lane;
+			const bool    in   = key < L;
+			const bool    live = in && keep[in ? key : 0] != 0;
+			mask_tab[kt * KT8 + lane] = live ? (uint16_t)0 : (in ? MASK_DROPPED_BF16 : MASK_OUT_OF_RANGE_BF16);
+			const unsigned long long bal = __ballot(live);
+			if(lane == 0) live_list[kt] = flag_of(bal != 0, bal != ~0ull);
 		}
 	}
 	__syncthreads();
 	if(wave == 0) {
-		const bool all = (s_nvalid == 0);
+		bool any_live = false;
+		for(int base = 0; base < n_ktiles; base += 64) any_live = any_live || __ballot(base + lane < n_ktiles && (live_list[base + lane] & 1) != 0) != 0;
+		const bool all = !any_live;   // no key is live: every tile is kept, the result is the mean over all L keys
 		int        cnt = 0;
 		for(int base = 0; base < n_ktiles; base += 64) {
-			const int  kt     = base + lane;
-			const bool keepit = kt < n_ktiles && (all || live_list[kt] != 0);
+			const int     kt     = base + lane;
+			const int16_t f      = kt < n_ktiles ? live_list[kt] : (int16_t)0;
+			const bool    keepit = kt < n_ktiles && (all || (f & 1) != 0);
 			const unsigned long long bal = __ballot(keepit);
 			const int rank = __builtin_amdgcn_mbcnt_hi((unsigned)(bal >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)bal, 0));
 			__builtin_amdgcn_wave_barrier();
-			if(keepit) live_list[cnt + rank] = (int16_t)kt;
+			if(keepit) live_list[cnt + rank] = (int16_t)(kt | (f & TILE_FULL));
 			cnt += __builtin_popcountll(bal);
 		}
-		if(lane == 0) s_nlive = cnt;
+		if(lane == 0) counts[0] = any_live ? 1 : 0, counts[1] = cnt;
 	}
 	__syncthreads();
-	const int  nlive       = __builtin_amdgcn_readfirstlane(s_nlive);
-	const bool all_dropped = __builtin_amdgcn_readfirstlane(s_nvalid) == 0;
+	const int  nlive       = __builtin_amdgcn_readfirstlane(counts[1]);
+	const bool all_dropped = __builtin_amdgcn_readfirstlane(counts[0]) == 0;
 
 	// scales: real = stored * descale
 	float dq = p.q_descale, dk = p.k_descale, dv = p.v_descale;
@@ -117,141 +285,85 @@ __global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(2
 	const float alpha = dq * dk * p.softmax_scale;  // logits = alpha * (q8 . k8) + bias
 	const float c_exp = alpha * LOG2E;              // exp(logit - m) = exp2(acc*c_exp - m_acc*c_exp), m_acc in accumulator units
 
-	const int64_t qrow   = (int64_t)qtile * (NW8 * 32) + wave * 32 + n;
-	const bool    row_ok = qrow < L;
-
-	// Q fragments: lane (q, g = half) holds q8[q][16c + 8g .. +7] (8 bytes)
-	long qf[NC];
-	{
-		const uint8_t* qp = static_cast<const uint8_t*>(p.q) + b * p.q_stride[0] + h * p.q_stride[1] + qrow * p.q_stride[2];
+	if(all_dropped) {
 #pragma unroll
-		for(int c = 0; c < NC; c++) {
-			const int d0 = 16 * c + 8 * half;
-			u32v2     w  = {0u, 0u};
-			if(row_ok && d0 < D && !all_dropped) w = *reinterpret_cast<const u32v2*>(qp + d0);
-			qf[c] = __builtin_bit_cast(long, w);
-		}
-	}
-	long qlo[NC];
-	if(COMP) {
-		const uint8_t* qp = static_cast<const uint8_t*>(p.q_lo) + b * p.q_stride[0] + h * p.q_stride[1] + qrow * p.q_stride[2];
-#pragma unroll
-		for(int c = 0; c < NC; c++) {
-			const int d0 = 16 * c + 8 * half;
-			u32v2     w  = {0u, 0u};
-			if(row_ok && d0 < D && !all_dropped) w = *reinterpret_cast<const u32v2*>(qp + d0);
-			qlo[c] = __builtin_bit_cast(long, w);
-		}
+		for(int i = 0; i < 8; i++) qa[i] = 0, qb[i] = 0;
 	}
 	// identity fragments scaled by 1/alpha (power of two times 1/softmax_scale folded by the caller: exact in bf16
-	// when alpha is a power of two)
+	// when alpha is a power of two): row n of S^T takes the bias of its key.  Lane (q, g) supplies keys 16 c2 + 8 g + j.
 	bf16x8 idf[2];
 	{
 		const uint32_t one_over_alpha = f32_to_bf16_bits(1.f / alpha);
 #pragma unroll
 		for(int c2 = 0; c2 < 2; c2++) {
 			u32x4     v = {0u, 0u, 0u, 0u};
-			const int j = n - 16 * c2 - 8 * half;
+			const int j = key_of_row - 16 * c2 - 8 * half;
 			if(j >= 0 && j < 8) v[j >> 1] = one_over_alpha << ((j & 1) * 16);
 			idf[c2] = __builtin_bit_cast(bf16x8, v);
 		}
 	}
-	u32x4 maskB = {0u, 0u, 0u, 0u};
-	if(half == 0) maskB[0] = 0x3F80u;
-	u32x4 maskA = {0u, 0u, 0u, 0u};
+	// mask: a 32x32x8 product, contraction slot 0 = (mask value) x 1.0
+	u32x2       maskA = {0u, 0u};
+	const u32x2 maskB = {half == 0 ? 0x3F80u : 0u, 0u};
 
-	const bool           has_bias = p.bias != nullptr && !all_dropped;
-	const unsigned char* bias_row = nullptr;
-	bool                 bias_vec = false;
-	if(has_bias) {
-		bias_row = static_cast<const unsigned char*>(p.bias) + (h * p.bias_stride[0] + (row_ok ? qrow : 0) * p.bias_stride[1]) * 2;
-		bias_vec = ((reinterpret_cast<uintptr_t>(p.bias) & 15) == 0) && (p.bias_stride[0] % 8 == 0) && (p.bias_stride[1] % 8 == 0);
-	}
-
-	// ---- tile loaders (LDS-direct buffer loads, 1 KB per wave instruction) ----
-	// K: lane i of load j -> tile row j*(1024/DP) + i/(DP/16), 16-byte chunk i%(DP/16)
-	// V^T: lane i of load j -> row d = j*16 + i/4, 16-byte chunk i%4 of the 64-key row
-	const __amdgpu_buffer_rsrc_t k_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-		const_cast<uint8_t*>(static_cast<const uint8_t*>(p.k) + b * p.k_stride[0] + h * p.k_stride[1]), 0, (int)((L - 1) * p.k_stride[2] + D), 0x00020000);  // exact end of the slab: rows are fetched in 16-byte chunks, range-checked per dword, so the tail of the last chunk reads as zero
-	const __amdgpu_buffer_rsrc_t klo_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-		const_cast<uint8_t*>(static_cast<const uint8_t*>(COMP ? p.k_lo : p.k) + b * p.k_stride[0] + h * p.k_stride[1]), 0, (int)((L - 1) * p.k_stride[2] + D), 0x00020000);
-	const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-		const_cast<uint8_t*>(static_cast<const uint8_t*>(p.v) + b * p.v_stride[0] + h * p.v_stride[1]), 0, (int)((D - 1) * p.v_stride[2] + p.v_stride[2]), 0x00020000);
-	constexpr int KCPR = DP / 16;       // 16-byte chunks per K row
-	constexpr int KRPI = 1024 / DP;     // K rows per wave load
-	const int  k_row = lane / KCPR, k_ch = lane % KCPR;
-	const int  k_voff = (int)(k_row * p.k_stride[2]) + k_ch * 16;
-	const bool k_act  = k_ch * 16 < D;
-	const int  v_row = lane >> 2, v_ch = lane & 3;
-	const int  v_voff = (int)(v_row * p.v_stride[2]) + v_ch * 16;
-	auto load_tile = [&](int kt, int buf) {
+	const bool           has_bias = BMODE != 0 && !all_dropped;
+	const unsigned char* bias_row = BMODE == 1 ? static_cast<const unsigned char*>(p.bias) + (h * p.bias_stride[0] + (row_ok ? qrow : 0) * p.bias_stride[1]) * 2 : nullptr;
+	// half slot -> the two fragments of 32 keys: lane (n, half), fragment c2: keys 16 c2 + 8 half .. + 7 of query row n
+	const int b_rd    = SLOT_BASE + wave * (2 * BIAS_HALF8) + n * 64, b_sw = (n >> 2) & 3;
+	const int b_shift = RAGGED ? 8 * ((b_odd + (int)(row_ok ? qrow : L - 1) * b_row_bytes) & 2) : 0;
+	u32x4     bfrag[2] = {u32x4{0u, 0u, 0u, 0u}, u32x4{0u, 0u, 0u, 0u}};
+	auto read_bias = [&](int kt, int sub) {
+		if constexpr(BMODE == 0) return;
+		if(!has_bias) return;
 #pragma unroll
-		for(int t = 0; t < (K_LOADS + NW8 - 1) / NW8; t++) {
-			const int j = wave + NW8 * t;
-			if(j < K_LOADS && k_act) {
-				__builtin_amdgcn_raw_ptr_buffer_load_lds(k_rsrc, (__attribute__((address_space(3))) void*)(k_lds + buf * K_TILE + j * 1024), 16, k_voff,
-														 (int)((kt * KT8 + j * KRPI) * p.k_stride[2]), 0, 0);
-				if(COMP)
-					__builtin_amdgcn_raw_ptr_buffer_load_lds(klo_rsrc, (__attribute__((address_space(3))) void*)(k_lds + buf * K_TILE + K_TILE1 + j * 1024), 16, k_voff,
-															 (int)((kt * KT8 + j * KRPI) * p.k_stride[2]), 0, 0);
-			}
-		}
+		for(int c2 = 0; c2 < 2; c2++) {
+			const int c = 2 * c2 + half;
+			if constexpr(RING) bfrag[c2] = *reinterpret_cast<const u32x4*>(smem + b_rd + sub * BIAS_HALF8 + ((c ^ b_sw) << 4));
+			if constexpr(RAGGED) {
+				const int follow = c + 1 < 4 ? b_rd + (((c + 1) ^ b_sw) << 4) : b_rd - n * 64 + 2048 + n * 4;
+				uint32_t  w[5]   = {bfrag[c2][0], bfrag[c2][1], bfrag[c2][2], bfrag[c2][3], *reinterpret_cast<const uint32_t*>(smem + follow + sub * BIAS_HALF8)};
+				if(kt == n_ktiles - 1) {  // (wave-uniform) what stands for keys from L on: zero
+					const int left = (int)L - (kt * KT8 + 32 * sub + 16 * c2 + 8 * half) + (b_shift >> 4);
 #pragma unroll
-		for(int t = 0; t < (V_LOADS + NW8 - 1) / NW8; t++) {
-			const int j = wave + NW8 * t;
-			if(j < V_LOADS && j * 16 + v_row < D)
-				__builtin_amdgcn_raw_ptr_buffer_load_lds(v_rsrc, (__attribute__((address_space(3))) void*)(v_lds + buf * V_TILE + j * 1024), 16, v_voff,
-														 (int)(j * 16 * p.v_stride[2]) + kt * KT8, 0, 0);
-		}
-	};
-	u32x4 bfrag[4];
-	auto  load_bias_tile = [&](int kt) {
-		if(!has_bias) {
-#pragma unroll
-			for(int f = 0; f < 4; f++) bfrag[f] = u32x4{0u, 0u, 0u, 0u};
-			return;
-		}
-		const int64_t   key0 = (int64_t)kt * KT8 + 8 * half;
-		const uint16_t* bp   = reinterpret_cast<const uint16_t*>(bias_row);
-		if(bias_vec && (int64_t)(kt + 1) * KT8 <= L) {
-#pragma unroll
-			for(int f = 0; f < 4; f++) bfrag[f] = row_ok ? *reinterpret_cast<const u32x4*>(bp + key0 + 16 * f) : u32x4{0u, 0u, 0u, 0u};
-		} else {
-#pragma unroll
-			for(int f = 0; f < 4; f++) {
-				u32x4 r = {0u, 0u, 0u, 0u};
-#pragma unroll
-				for(int j = 0; j < 8; j++) {
-					const int64_t  key = key0 + 16 * f + j;
-					const uint32_t e   = (row_ok && key < L) ? (uint32_t)bp[key] : 0u;
-					r[j >> 1] |= e << ((j & 1) * 16);
+					for(int j = 0; j < 5; j++) w[j] = left >= 2 * j + 2 ? w[j] : (left == 2 * j + 1 ? w[j] & 0xffffu : 0u);
 				}
-				bfrag[f] = r;
+#pragma unroll
+				for(int j = 0; j < 4; j++) bfrag[c2][j] = __builtin_amdgcn_alignbit(w[j + 1], w[j], b_shift);
+			}
+			if constexpr(BMODE == 1) {
+				const uint16_t* bp = reinterpret_cast<const uint16_t*>(bias_row);
+#pragma unroll
+				for(int j = 0; j < 8; j += 2) {
+					const int64_t  key = (int64_t)kt * KT8 + 32 * sub + 16 * c2 + 8 * half + j;
+					const uint32_t e0  = row_ok && key < L ? (uint32_t)bp[key] : 0u, e1 = row_ok && key + 1 < L ? (uint32_t)bp[key + 1] : 0u;
+					bfrag[c2][j >> 1]  = e0 | (e1 << 16);
+				}
 			}
 		}
 	};
 
-	// per-lane LDS read offsets
-	const int k_rd   = n * DP + 8 * half;                 // + 16*c, + sub*32*DP, + buf*K_TILE
-	const int v_rd   = n * KT8 + 4 * half;                // row d = n (+32*db), + 32*sub + 16*cp (+8)
-	const int mask_rd     = 2 * K_TILE + 2 * V_TILE + (half == 0 ? n * 4 : (n_ktiles * KT8 + n) * 4);
-	const int mask_stride = half == 0 ? KT8 * 4 : 0;
+	// per-lane LDS read addresses (buffer 0, sub-tile 0).  K: two 16-byte chunks of row key_of_row; DP = 32: of the K row (lower
+	// half-wave) or of its residual (upper), DP = 64: columns 32 half .. (the swizzle repeats every 32 rows)
+	int k_rd[2], v_rd[2];
+#pragma unroll
+	for(int i = 0; i < 2; i++) k_rd[i] = key_of_row * DP + (((DP == 64 ? 2 * half + i : i) ^ k_sw(key_of_row)) << 4) + (DP == 32 && COMP && half ? K_TILE1 : 0);
+#pragma unroll
+	for(int sub = 0; sub < 2; sub++) v_rd[sub] = K_TILE + n * KT8 + (((2 * sub + half) ^ v_sw(n)) << 4);   // (+ 32 KT8 per block of O^T)
+	const int mask_rd = MASK_BASE + key_of_row * 2;
 
-	float  m_run = 0.f, mc = 0.f;  // m_run in accumulator units; mc = m_run*c_exp - P_SHIFT
-	bool   first = true;
-	// Row sums on the matrix pipe (as in dpa_mfma.hip): a 16x16x32 MFMA whose A operand is a 0/1 pattern adds the 16 quantised
-	// probabilities that a query's two lanes hold of a fragment; register 0 of the result is, in every lane, the running sum of
+	float m_run = -INFINITY, mc = 0.f;  // m_run in accumulator units; mc = m_run*c_exp - P_SHIFT
+	// Row sums.  ONES: rows D and D + 4 of V^T are ones, i.e. the sum of exactly the e4m3 weights that enter P.V is in register 4 (D % 32) / 8
+	// of both half-waves.  Otherwise on the matrix pipe (as in dpa_mfma.hip): a 16x16x32 MFMA whose A operand is a 0/1 pattern adds
+	// the 16 quantised probabilities that a query's two lanes hold of a fragment; register 0 of the result is, in every lane, the running sum of
 	// that lane's own query row.  As a B operand of the 16x16x32 shape the P fragment's lane l is column l%16, contraction
 	// group l/16, and holds query l%32: groups 0,2 belong to queries 0..15, groups 1,3 to queries 16..31; output register 0
-	// of lane l is row 4*(l/16): rows 0 and 8 select the even groups, rows 4 and 12 the odd ones.  The normaliser is thus the
-	// sum of exactly the e4m3 weights that enter P.V (the result is a convex combination of V rows), and 16 vector adds per
-	// 32 x 32 block become two half-size matrix instructions.
+	// of lane l is row 4*(l/16): rows 0 and 8 select the even groups, rows 4 and 12 the odd ones.
 	f32x4 lacc = {0.f, 0.f, 0.f, 0.f};
-	long  ones_a;
-	{
+	long  ones_a = 0;
+	if constexpr(!ONES) {
 		const int  i16 = lane & 15, kg = lane >> 4;
 		const bool on  = ((i16 == 0 || i16 == 8) && (kg & 1) == 0) || ((i16 == 4 || i16 == 12) && (kg & 1) == 1);
-		const u32v2 w  = {on ? 0x38383838u : 0u, on ? 0x38383838u : 0u};  // e4m3 1.0
+		const u32x2 w  = {on ? 0x38383838u : 0u, on ? 0x38383838u : 0u};  // e4m3 1.0
 		ones_a = __builtin_bit_cast(long, w);
 	}
 	f32x16 oacc[NDB];
@@ -260,90 +372,172 @@ __global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(2
 #pragma unroll
 		for(int i = 0; i < 16; i++) oacc[db][i] = 0.f;
 
-	__syncthreads();
-	const int kt0 = __builtin_amdgcn_readfirstlane((int)live_list[0]);
-	load_tile(kt0, 0);
-	load_bias_tile(kt0);
-	asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-	__syncthreads();
+	auto read_k = [&](int off, int res) -> i32x8 {   // (res: DP = 64, the residual tile)
+		const u32x4 lo = *reinterpret_cast<const u32x4*>(smem + off + k_rd[0] + res * K_TILE1), hi = *reinterpret_cast<const u32x4*>(smem + off + k_rd[1] + res * K_TILE1);
+		return i32x8{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
+	};
+	auto kq = [&](const i32x8& k, const i32x8& q, const f32x16& c) -> f32x16 { return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(k, q, c, 0, 0, 0, 0, 0, 0); };
+	auto bias_mfma = [&](const f32x16& c, int c2) -> f32x16 { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(idf[c2], __builtin_bit_cast(bf16x8, bfrag[c2]), c, 0, 0, 0); };
+	auto mask_mfma = [&](const f32x16& c) -> f32x16 {
+		return __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(__builtin_bit_cast(s16x4, maskA), __builtin_bit_cast(s16x4, maskB), c, 0, 0, 0);
+	};
+	auto exp_part = [&](const f32x16& s, u32x2 (&pf)[2], auto i_c) {   // logits 4 I .. 4 I + 3
+		constexpr int I = decltype(i_c)::value;
+		const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[4 * I], c_exp, -mc)), p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[4 * I + 1], c_exp, -mc));
+		const float p2 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[4 * I + 2], c_exp, -mc)), p3 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[4 * I + 3], c_exp, -mc));
+		int w;
+		asm("" : "=v"(w));   // (both halves are written)
+		w = __builtin_amdgcn_cvt_pk_fp8_f32(p0, p1, w, false);
+		w = __builtin_amdgcn_cvt_pk_fp8_f32(p2, p3, w, true);
+		pf[I >> 1][I & 1] = (uint32_t)w;
+	};
 
-	for(int it = 0; it < nlive; it++) {
-		const int  kt       = __builtin_amdgcn_readfirstlane((int)live_list[it]);
-		const int  buf      = it & 1;
-		const bool has_next = it + 1 < nlive;
-		const int  ktn      = has_next ? __builtin_amdgcn_readfirstlane((int)live_list[it + 1]) : kt;
-		if(has_next) load_tile(ktn, buf ^ 1);
-		u32x4 bcur[4];
+	f32x16 sc;
+	// One stage: on entry `sc` holds the finished logits of 32 keys (half SUB of the tile whose V^T tile is at v_off); it leaves those of
+	// the next 32 (half 1 - SUB of tile kt_n, K tile at k_off) in `sc` and adds these keys' P.V.  after_bias runs once the bias fragments have been read.
+	auto stage = [&](auto sub_c, int kt_n, bool full_n, int k_off, int v_off, auto&& after_bias) {
+		constexpr int SUB = decltype(sub_c)::value, SUBN = 1 - SUB;
+		const i32x8 ka = read_k(k_off + SUBN * 32 * DP, 0);
+		i32x8       kb = ka;
+		if constexpr(DP == 64 && COMP) kb = read_k(k_off + SUBN * 32 * DP, 1);
+		read_bias(kt_n, SUBN);
+		if(!full_n) maskA[0] = *reinterpret_cast<const uint16_t*>(smem + mask_rd + kt_n * (KT8 * 2) + SUBN * 64);
+		// online softmax with the true running maximum (in accumulator units)
+		// (two chains of three-operand maxima)
+		float mx0 = max3(sc[0], sc[1], sc[2]), mx1 = max3(sc[3], sc[4], sc[5]);
+		mx0 = max3(mx0, sc[6], sc[7]), mx1 = max3(mx1, sc[8], sc[9]);
+		mx0 = max3(mx0, sc[10], sc[11]), mx1 = max3(mx1, sc[12], sc[13]);
+		mx0 = max3(mx0, sc[14], sc[15]);
+		mx0 = fmaxf(mx0, mx1);
+		const auto  sw    = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx0), __float_as_uint(mx0), false, false);
+		const float m_new = max3(m_run, __uint_as_float(sw[0]), __uint_as_float(sw[1]));
+		if(__ballot(m_new > m_run)) {   // (the first time from -inf: the factor is 0, and nothing has been accumulated)
+			const float a = __builtin_amdgcn_exp2f((m_run - m_new) * c_exp);
+			if constexpr(!ONES) lacc[0] *= a;
 #pragma unroll
-		for(int f = 0; f < 4; f++) bcur[f] = bfrag[f];
-		if(has_next) load_bias_tile(ktn);
-		const int mask_addr = mask_rd + kt * mask_stride;
+			for(int db = 0; db < NDB; db++)
 #pragma unroll
-		for(int sub = 0; sub < 2; sub++) {
-			f32x16 s;
+				for(int i = 0; i < 16; i++) oacc[db][i] *= a;
+			m_run = m_new;
+			mc    = m_new * c_exp - P_SHIFT;
+		}
+		// (the accumulators keep their registers whether or not they were rescaled: the compiler would copy them otherwise)
 #pragma unroll
-			for(int i = 0; i < 16; i++) s[i] = 0.f;
+		for(int db = 0; db < NDB; db++) asm volatile("" : "+v"(oacc[db]));
+		after_bias();
+		u32x2  pf[2];
+		f32x16 sn;
 #pragma unroll
-			for(int c = 0; c < NC; c++) {
-				const long kf = *reinterpret_cast<const long*>(k_lds + buf * K_TILE + k_rd + sub * 32 * DP + 16 * c);
-				s = __builtin_amdgcn_mfma_f32_32x32x16_fp8_fp8(kf, qf[c], s, 0, 0, 0);
-				if(COMP) {
-					const long kl = *reinterpret_cast<const long*>(k_lds + buf * K_TILE + K_TILE1 + k_rd + sub * 32 * DP + 16 * c);
-					s = __builtin_amdgcn_mfma_f32_32x32x16_fp8_fp8(kl, qf[c], s, 0, 0, 0);
-					s = __builtin_amdgcn_mfma_f32_32x32x16_fp8_fp8(kf, qlo[c], s, 0, 0, 0);
-				}
-			}
+		for(int i = 0; i < 16; i++) sn[i] = 0.f;
+		// One matrix instruction, then a quarter of the exponentials, and so on; the empty asm statements pin that order (matrix
+		// intrinsics are values to the compiler and would all be issued in front, each waiting for the one before)
+		auto pin = [&](auto i_c) {
+			constexpr int I = decltype(i_c)::value;
+			float    a_ = sn[0];
+			uint32_t b_ = pf[I >> 1][I & 1];
+			asm volatile("" : "+v"(a_), "+v"(b_));
+			sn[0] = a_, pf[I >> 1][I & 1] = b_;
+			__builtin_amdgcn_sched_barrier(0);
+		};
+		__builtin_amdgcn_sched_barrier(0);
+		sn = kq(ka, qa, sn);
+		exp_part(sc, pf, ic<0>{});
+		pin(ic<0>{});
+		if constexpr(COMP && DP == 64) sn = kq(kb, qa, sn);
+		if constexpr(COMP) sn = kq(ka, qb, sn);
+		exp_part(sc, pf, ic<1>{});
+		pin(ic<1>{});
+		u32x4 vf[NDB];
 #pragma unroll
-			for(int c2 = 0; c2 < 2; c2++) s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(idf[c2], __builtin_bit_cast(bf16x8, bcur[2 * sub + c2]), s, 0, 0, 0);
-			maskA[0] = *reinterpret_cast<const uint32_t*>(smem + mask_addr + sub * 32 * 4);
-			s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, maskA), __builtin_bit_cast(bf16x8, maskB), s, 0, 0, 0);
-
-			// online softmax with the true running maximum (in accumulator units)
-			float mx = fmaxf(fmaxf(s[0], s[1]), s[2]);
-#pragma unroll
-			for(int i = 3; i < 15; i += 2) mx = fmaxf(fmaxf(mx, s[i]), s[i + 1]);
-			mx = hswap_max(fmaxf(mx, s[15]));
-			const float m_new = first ? mx : fmaxf(m_run, mx);
-			if(__ballot(first || m_new > m_run)) {
-				const float a = first ? 1.f : __builtin_amdgcn_exp2f((m_run - m_new) * c_exp);
-#pragma unroll
-				for(int i = 0; i < 4; i++) lacc[i] *= a;
-#pragma unroll
-				for(int db = 0; db < NDB; db++)
-#pragma unroll
-					for(int i = 0; i < 16; i++) oacc[db][i] *= a;
-				m_run = m_new;
-				mc    = m_new * c_exp - P_SHIFT;
-				first = false;
-			}
-			u32v2 pf[2];
-#pragma unroll
-			for(int i = 0; i < 16; i += 4) {
-				const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], c_exp, -mc)), p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i + 1], c_exp, -mc));
-				const float p2 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i + 2], c_exp, -mc)), p3 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i + 3], c_exp, -mc));
-				uint32_t w = 0;
-				w = __builtin_amdgcn_cvt_pk_fp8_f32(p0, p1, w, false);
-				w = __builtin_amdgcn_cvt_pk_fp8_f32(p2, p3, w, true);
-				pf[i >> 3][(i & 7) >> 2] = w;
-			}
+		for(int db = 0; db < NDB; db++) vf[db] = *reinterpret_cast<const u32x4*>(smem + v_off + v_rd[SUB] + db * 32 * KT8);
+		if constexpr(BMODE != 0) sn = bias_mfma(sn, 0);
+		exp_part(sc, pf, ic<2>{});
+		pin(ic<2>{});
+		if constexpr(BMODE != 0) sn = bias_mfma(sn, 1);
+		exp_part(sc, pf, ic<3>{});
+		pin(ic<3>{});
+		if(!full_n) sn = mask_mfma(sn);
+		if constexpr(!ONES) {
 #pragma unroll
 			for(int cp = 0; cp < 2; cp++) lacc = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(ones_a, __builtin_bit_cast(long, pf[cp]), lacc, 0, 0, 0);
-			// O^T += V8^T . P^T: contraction slot j of chunk cp is key 16cp + 8(j/4) + 4half + j%4
-#pragma unroll
-			for(int cp = 0; cp < 2; cp++)
-#pragma unroll
-				for(int db = 0; db < NDB; db++) {
-					const unsigned char* vp = v_lds + buf * V_TILE + v_rd + db * 32 * KT8 + 32 * sub + 16 * cp;
-					u32v2 vf = {*reinterpret_cast<const uint32_t*>(vp), *reinterpret_cast<const uint32_t*>(vp + 8)};
-					oacc[db] = __builtin_amdgcn_mfma_f32_32x32x16_fp8_fp8(__builtin_bit_cast(long, vf), __builtin_bit_cast(long, pf[cp]), oacc[db], 0, 0, 0);
-				}
 		}
-		asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-		__syncthreads();
+		// O^T += V8^T . P^T: contraction slot 8 half + j of chunk cp is key 16 half + 8 cp + j
+#pragma unroll
+		for(int cp = 0; cp < 2; cp++)
+#pragma unroll
+			for(int db = 0; db < NDB; db++)
+				oacc[db] = __builtin_amdgcn_mfma_f32_32x32x16_fp8_fp8(__builtin_bit_cast(long, u32x2{vf[db][2 * cp], vf[db][2 * cp + 1]}), __builtin_bit_cast(long, pf[cp]), oacc[db], 0, 0, 0);
+		sc = sn;
+	};
+
+	// ---- prologue: first tile, its first logits; second tile under way ----
+	auto entry_at = [&](int j) -> int { return __builtin_amdgcn_readfirstlane((int)live_list[j < nlive ? j : nlive - 1]); };
+	int entry = entry_at(0), entry1 = entry_at(1);
+	if((entry & ~TILE_FULL) != 0) {   // (the guess was wrong; loads land in issue order)
+		load_tile(entry & ~TILE_FULL, 0);
+		load_bias(entry & ~TILE_FULL, 0);
+		load_bias(entry & ~TILE_FULL, 1);
+	}
+	asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+	{
+		const int kt0 = entry & ~TILE_FULL;
+		read_bias(kt0, 0);
+		asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+		if(nlive > 1) {
+			load_tile(entry1 & ~TILE_FULL, TILE);
+			load_bias(entry1 & ~TILE_FULL, 0);
+		}
+#pragma unroll
+		for(int i = 0; i < 16; i++) sc[i] = 0.f;
+		const i32x8 ka = read_k(0, 0);
+		sc = kq(ka, qa, sc);
+		if constexpr(COMP) {
+			if constexpr(DP == 64) sc = kq(read_k(0, 1), qa, sc);
+			sc = kq(ka, qb, sc);
+		}
+		if constexpr(BMODE != 0) sc = bias_mfma(bias_mfma(sc, 0), 1);
+		maskA[0] = *reinterpret_cast<const uint16_t*>(smem + mask_rd + kt0 * (KT8 * 2));
+		sc = mask_mfma(sc);
+	}
+	// Tile `it` is in buffer it % 3.  Order of this wavefront's loads: tile it + 1 (behind the barrier of iteration it - 1), its
+	// first half of bias (in the second stage of it - 1), its second half (in the first stage of it), tile it + 2, ...
+	int cur = 0;
+	for(int it = 0; it < nlive; it++) {
+		const int  kt = entry & ~TILE_FULL, kt1 = entry1 & ~TILE_FULL;
+		const int  nxt = cur == 2 * TILE ? 0 : cur + TILE, nxt2 = nxt == 2 * TILE ? 0 : nxt + TILE;
+		const bool has1 = it + 1 < nlive, has2 = it + 2 < nlive;
+		const int  entry2 = entry_at(it + 2);
+		// the second half of this tile's bias has landed (younger: tile it + 1 and the first half of its bias)
+		if(has1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(KV_MIN + BIAS_LOADS) : "memory");
+		else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+		stage(ic<0>{}, kt, (entry & TILE_FULL) != 0, cur, cur, [&]() {
+			if constexpr(RING)
+				if(has1) {
+					asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (the half slot has been read)
+					load_bias(kt1, 1);
+				}
+		});
+		// tile it + 1 and the first half of its bias have landed (younger: the second half); behind the barrier everyone is done with tile it - 1
+		if(has1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(BIAS_LOADS) : "memory");
+		else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+		if(has2) load_tile(entry2 & ~TILE_FULL, nxt2);
+		stage(ic<1>{}, kt1, (entry1 & TILE_FULL) != 0, nxt, cur, [&]() {
+			if constexpr(RING)
+				if(has2) {
+					asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+					load_bias(entry2 & ~TILE_FULL, 0);
+				}
+		});
+		entry = entry1, entry1 = entry2, cur = nxt;
 	}
 
 	// epilogue: out = O * dv / l   (l was summed over p * 2^8, the same factor O carries; both half-waves are in it)
-	const float inv = dv / lacc[0];
+	float l_tot = lacc[0];
+	if constexpr(ONES) {
+		const int i = (D & 31) >> 3;   // 1, 2 or 3: register 4 i of the last block
+		l_tot = i == 1 ? oacc[NDB - 1][4] : i == 2 ? oacc[NDB - 1][8] : oacc[NDB - 1][12];
+	}
+	const float inv = dv / l_tot;
 	if(row_ok) {
 		const int64_t ooff = b * p.out_stride[0] + h * p.out_stride[1] + qrow * p.out_stride[2];
 #pragma unroll
@@ -354,8 +548,8 @@ __global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(2
 				if(d0 >= D) continue;
 				const float o0 = oacc[db][4 * g4] * inv, o1 = oacc[db][4 * g4 + 1] * inv, o2 = oacc[db][4 * g4 + 2] * inv, o3 = oacc[db][4 * g4 + 3] * inv;
 				if(p.out_dtype == AF3_BF16) {
-					u32v2 w = {pack_bf16x2(o0, o1), pack_bf16x2(o2, o3)};
-					*reinterpret_cast<u32v2*>(static_cast<uint16_t*>(p.out) + ooff + d0) = w;
+					u32x2 w = {pack_bf16x2(o0, o1), pack_bf16x2(o2, o3)};
+					*reinterpret_cast<u32x2*>(static_cast<uint16_t*>(p.out) + ooff + d0) = w;
 				} else {
 					float4 w = {o0, o1, o2, o3};
 					*reinterpret_cast<float4*>(static_cast<float*>(p.out) + ooff + d0) = w;
@@ -364,16 +558,32 @@ __global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(2
 	}
 }
 
-template <int DP, bool COMP>
+template <int DP, bool COMP, bool ONES, int BMODE>
 int launch8(const af3_dpa_params& p, hipStream_t s) {
 	const int     n_qtiles = (int)((p.L + NW8 * 32 - 1) / (NW8 * 32));
 	const int     n_ktiles = (int)((p.L + KT8 - 1) / KT8);
 	const int64_t n_groups = p.B * p.H;
 	const int64_t blocks   = ((n_groups + 7) / 8) * 8 * n_qtiles;
 	if(blocks <= 0 || blocks > 0x7fffffffLL) return AF3_ERR_BAD_SHAPE;
-	const size_t smem = (size_t)(COMP ? 6 : 4) * KT8 * DP + ((size_t)n_ktiles * KT8 + 64) * 4 + (size_t)n_ktiles * 2 + 16;
-	hipLaunchKernelGGL((dpa_mfma_fp8_kernel<DP, COMP>), dim3((unsigned)blocks), dim3(NW8 * 64), smem, s, p, n_qtiles, n_groups);
+	const size_t smem = (size_t)3 * (COMP ? 3 : 2) * KT8 * DP + (BMODE >= 2 ? NW8 * 2 * BIAS_HALF8 : 0) + (size_t)n_ktiles * KT8 * 2 + (size_t)n_ktiles * 2 + 16;
+	auto         kern = dpa_mfma_fp8_kernel<DP, COMP, ONES, BMODE>;
+	if(smem > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) return AF3_ERR_LAUNCH;
+	hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW8 * 64), smem, s, p, n_qtiles, n_groups);
 	return launch_status();
+}
+template <int DP, bool COMP, bool ONES>
+int launch8_bias(const af3_dpa_params& p, hipStream_t s) {
+	if(!p.bias) return launch8<DP, COMP, ONES, 0>(p, s);
+	// offsets of a head's bias (and the loads' overhang at its end) fit 32 bits; whole aligned chunks that never straddle the end of a row, or the ragged form
+	if(((p.L - 1) * p.bias_stride[1] + p.L) * 2 >= ((int64_t)1 << 31) - 64 * 1024) return launch8<DP, COMP, ONES, 1>(p, s);
+	const bool aligned = (reinterpret_cast<uintptr_t>(p.bias) & 15) == 0 && p.bias_stride[0] % 8 == 0 && p.bias_stride[1] % 8 == 0 && p.L % 8 == 0;
+	return aligned ? launch8<DP, COMP, ONES, 2>(p, s) : launch8<DP, COMP, ONES, 3>(p, s);
+}
+template <int DP>
+int launch8_form(const af3_dpa_params& p, hipStream_t s) {
+	const bool comp = p.q_lo != nullptr && p.k_lo != nullptr;
+	if(p.D < DP) return comp ? launch8_bias<DP, true, true>(p, s) : launch8_bias<DP, false, true>(p, s);
+	return comp ? launch8_bias<DP, true, false>(p, s) : launch8_bias<DP, false, false>(p, s);
 }
 
 }  // namespace
@@ -398,9 +608,7 @@ bool mfma_fp8_eligible(const af3_dpa_params& p) {
 }
 
 int launch_dpa_mfma_fp8(const af3_dpa_params& p, hipStream_t s) {
-	const bool comp = p.q_lo != nullptr && p.k_lo != nullptr;
-	if(p.D <= 32) return comp ? launch8<32, true>(p, s) : launch8<32, false>(p, s);
-	return comp ? launch8<64, true>(p, s) : launch8<64, false>(p, s);
+	return p.D <= 32 ? launch8_form<32>(p, s) : launch8_form<64>(p, s);
 }
 
 }  // namespace af3

@@ -167,3 +167,32 @@ def test_projection_forms(af3, M, N, K, form, with_row):
     want = x.float() @ w.float().t() + (row.float() if with_row else 0.0)
     assert (out[:M].float() - want).abs().max() <= 2 ** -8 * want.abs().max()
     assert bool((out[M] == 7.0).all())
+
+
+@pytest.mark.parametrize("compensated", [True, False])
+@pytest.mark.parametrize("B,H,L,D,mask_kind", [
+    (1, 1, 1, 24, "none"), (2, 3, 33, 24, "random"), (1, 2, 64, 32, "none"), (2, 2, 65, 16, "tail"), (3, 2, 127, 48, "random"), (1, 3, 128, 64, "tail"),
+    (5, 2, 200, 24, "late"), (2, 4, 259, 24, "random"), (1, 2, 321, 56, "late"), (2, 16, 512, 24, "tail"), (1, 16, 1027, 24, "random"),
+])
+def test_fp8_bias_forms_and_tile_flags(af3, B, H, L, D, mask_kind, compensated):
+    """Bias rows at any address, tiles with and without dropped keys, leading tiles without a live key: the kernel against the formula on the
+    dequantised operands (for the compensated product: on q and k themselves)."""
+    g = torch.Generator().manual_seed(L + D + B)
+    q, k, v = (torch.randn(B, H, L, D, generator=g).to(torch.bfloat16).cuda() for _ in range(3))
+    bias = torch.randn(H, L, L, generator=g).to(torch.bfloat16).cuda()
+    keep = {"none": torch.ones(L), "random": (torch.rand(L, generator=g) < 0.8).float(), "tail": (torch.arange(L) < L - L // 10).float(), "late": (torch.arange(L) >= L * 5 // 8).float()}[mask_kind].bool()
+    keep[L - 1] = True
+    print("case", B, H, L, D, mask_kind, compensated, flush=True)
+    out = af3.dot_product_attention_fp8(q, k, v, keep.cuda(), bias, compensated=compensated)
+    torch.cuda.synchronize()
+    vd, vs = af3.quantize_fp8_e4m3(v)
+    qq, kk = q.float() * D ** -0.5, k.float()
+    if not compensated:
+        (q8, qs), (k8, ks) = af3.quantize_fp8_e4m3(q, D ** -0.5), af3.quantize_fp8_e4m3(k)
+        qq, kk = q8.float() * qs, k8.float() * ks
+    s = qq.matmul(kk.transpose(-1, -2)) + bias.float()
+    p = s.masked_fill(~keep.cuda(), float("-inf")).softmax(-1)
+    want = p.matmul(vd.float() * vs)
+    # e4m3 weights: each within 2^-4 of itself
+    bound = 2 ** -4 * p.matmul((vd.float() * vs).abs()) + 2e-2
+    assert bool(((out.float() - want).abs() <= bound).all())
