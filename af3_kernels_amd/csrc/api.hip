@@ -96,6 +96,9 @@ extern "C" int64_t af3_dpa_workspace_used(const af3_dpa_params* params) {
 	return select_kernel(*params) == 1 ? mfma_bf16_workspace_used(*params) : 0;
 }
 
+// ... and which must know, before it lays out q, whether the kernel that will serve this call takes its logits in units of log2 e.
+extern "C" int af3_dpa_log2_domain(const af3_dpa_params* params) { return validate(params) == AF3_OK && select_kernel(*params) == 1 && mfma_bf16_log2_domain(*params) ? 1 : 0; }
+
 extern "C" int af3_dpa_select_kernel(const af3_dpa_params* params) {
 	const int rc = validate(params);
 	if(rc != AF3_OK) return rc;

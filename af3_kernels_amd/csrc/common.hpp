@@ -41,7 +41,7 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
 }
 
 // sigmoid for the optional output gate (reference: tpp::SigmoidFwdTPP, src/csrc/xsmm_functors.h:2694-2731)
-__device__ __forceinline__ float sigmoidf_fast(float x) { return 1.f / (1.f + __builtin_amdgcn_exp2f(-x * LOG2E)); }
+__device__ __forceinline__ float sigmoidf_fast(float x) { return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-x * LOG2E)); }
 
 // Extra kernel arguments of the fused grid-attention variant of the bf16 kernel: the input rows and the four
 // per-head projection matrices (weight^T in the reference's panel layout [head][C/2][32][2]).
@@ -75,6 +75,7 @@ int launch_dpa_mfma_rows(const af3_dpa_params& p, hipStream_t s);
 bool mfma_bf16_eligible(const af3_dpa_params& p);
 int64_t mfma_bf16_workspace_bytes(const af3_dpa_params& p);
 int64_t mfma_bf16_workspace_used(const af3_dpa_params& p);
+bool mfma_bf16_log2_domain(const af3_dpa_params& p);   // the call's kernel scales q by log2 e
 bool mfma_fp8_eligible(const af3_dpa_params& p);
 int launch_dpa_mfma_f32(const af3_dpa_params& p, hipStream_t s);
 bool mfma_f32_eligible(const af3_dpa_params& p);

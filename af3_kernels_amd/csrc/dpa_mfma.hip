@@ -1489,11 +1489,15 @@ static int launch_nw(const af3_dpa_params& p, hipStream_t s) {
 	return launch_one<DP, 1, L2DOM, BMODE>(p, s);
 }
 
+static bool uses_workspace(const af3_dpa_params& p) {   // (the one-row kernel)
+	return p.bias && p.workspace && p.B >= 2 && !one_row_in_place(p) && p.workspace_bytes >= ws_bytes_needed(p) && (reinterpret_cast<uintptr_t>(p.workspace) & 15) == 0;
+}
+bool mfma_bf16_log2_domain(const af3_dpa_params& p) { return (rows_kernel_wanted(p) && mfma_rows_can_serve(p)) || uses_workspace(p) || !p.bias; }
+
 int launch_dpa_mfma_bf16(const af3_dpa_params& p, hipStream_t s) {
 	if(rows_kernel_wanted(p) && mfma_rows_can_serve(p)) return launch_dpa_mfma_rows(p, s);
 	const bool bf32   = p.bias && p.bias_dtype == AF3_F32;
-	const bool use_ws = p.bias && p.workspace && p.B >= 2 && !one_row_in_place(p) && p.workspace_bytes >= ws_bytes_needed(p) &&
-						(reinterpret_cast<uintptr_t>(p.workspace) & 15) == 0;
+	const bool use_ws = uses_workspace(p);
 	if(use_ws) {
 		const int rc = launch_bias_prepass(p, s);
 		if(rc != AF3_OK) return rc;

@@ -93,7 +93,8 @@ __global__ void __launch_bounds__(256) bias_rows_prepass_kernel(const void* __re
 // two 2 KB halves of the wavefront's slot, a tile ahead of its conversion (needs 16-byte aligned rows; a quarter of mode
 // 2's cache-line requests, whose lanes each fetch from a row of their own).
 // The launch covers batch rows [b_first, b_first + b_count) in groups of ROWS.
-template <int ROWS, int BMODE>
+// GATE: out *= sigmoid(gate) in the epilogue.
+template <int ROWS, int BMODE, bool GATE>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) dpa_rows_bf16_kernel(af3_dpa_params p, int n_qtiles, int64_t n_groups, int64_t b_first, int64_t b_count) {
 	static_assert(ROWS >= 2 && ROWS <= 4, "two to four row chains per wavefront");
 	constexpr int  NW       = 4;
@@ -176,6 +177,23 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 	};
 	auto load_tile = [&](int t, int buf_off) {
 		load_tile_piece(t, buf_off, ic<0>{}), load_tile_piece(t, buf_off, ic<1>{}), load_tile_piece(t, buf_off, ic<2>{}), load_tile_piece(t, buf_off, ic<3>{});
+	};
+	// Output gate: the 2 ROWS pieces of this wavefront's gate rows (16 query rows of a batch row, 1 KB each) go into the tile buffers
+	// that the last two tiles leave free -- the places of tiles n_t and n_t + 1, requested where those tiles would be -- and are
+	// read in the epilogue.  (Loaded there, they exposed a memory latency per workgroup: 36 of 448 us at 768 x 4 x 768 x 32, 9 of 81 at 384.)
+	auto load_gate = [&](int part, int buf_off) {
+		if constexpr(!GATE) return;
+#pragma unroll
+		for(int i = 0; i < ROWS; i++) {
+			const int     k = part * ROWS + i, r = k >> 1;
+			const int64_t br = b0 + r < b_end ? b0 + r : b_end - 1, row = (int64_t)qtile * (NW * 32) + wave * 32 + 16 * (k & 1) + (lane >> 2);
+			const u32x4   g_rsrc = raw_rsrc(static_cast<const uint16_t*>(p.gate) + br * p.gate_stride[0] + h * p.gate_stride[1], (uint32_t)(((L - 1) * p.gate_stride[2] + D) * 2));
+			lds_dma_b128(g_rsrc, lds_addr_of(smem) + buf_off + (wave * ROWS + i) * 1024, (lane & 3) * 8 < D && row < L ? (int)(row * p.gate_stride[2] * 2) + (lane & 3) * 16 : 0x7FFF0000);
+		}
+	};
+	auto load_tile_or_gate = [&](int t, int buf_off) {
+		if(t < n_t) load_tile(t, buf_off);
+		else load_gate(t - n_t, buf_off);
 	};
 	// bias fragment of key tile t: 4 KB of this (head, query block)'s slab of the workspace -> this wavefront's slot
 	const int     n_qblocks = (int)((L + 31) / 32);
@@ -613,7 +631,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 					step(r_c, first_c, anydrop_c, fr, k2, m1, vc, [&](auto s_c) {
 						constexpr int S = decltype(s_c)::value;
 						if constexpr(S == 1) {
-							load_tile(t + 2, bufnn);
+							load_tile_or_gate(t + 2, bufnn);
 							next_bias_fragment(t + 1);
 							load_bias_direct(t + 2);
 							load_bias_staged(t + 2);   // (into the half that held fragment t, read a tile ago)
@@ -637,7 +655,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 		// (tile 0 and bias fragment 0 were requested at the top of the kernel and are complete)
 		next_bias_fragment(0);  // fragment 0 -> registers
 		asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-		load_tile(1, BUF_R);
+		load_tile_or_gate(1, BUF_R);
 		load_bias(1);
 		load_bias_direct(1);
 		load_bias_staged(1);
@@ -664,6 +682,18 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 			buf = bufn;
 		}
 	};
+	if((int64_t)qtile * (NW * 32) + wave * 32 >= L) {
+		// ---- no query row of this wavefront exists (L % 128 != 0, the last query tile): it fetches its batch row's tiles, keeps the
+		// barriers' count -- one per tile -- and leaves the vector and matrix pipes to others ----
+		load_tile(1, BUF_R);
+		int bufnn = 2 * BUF_R;
+		for(int t = 0; t < n_t; t++) {
+			asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+			load_tile(t + 2, bufnn);
+			bufnn = bufnn == (NBUF_R - 1) * BUF_R ? 0 : bufnn + BUF_R;
+		}
+		return;
+	}
 	if(n_t > 0) {
 		bool any_dropped = false;
 #pragma unroll
@@ -678,26 +708,23 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 
 	// ---- epilogue: O^T register i is head column 8*(i/4) + 4*half + i%4; optional output gate (out *= sigmoid(gate), the
 	// reference's "weighted_avg *= sigmoid(gating_query(pair))", src/csrc/dot_product_attention.cpp:335-349) ----
+	const int gate_buf[2] = {(n_t % NBUF_R) * BUF_R, ((n_t + 1) % NBUF_R) * BUF_R};
 	if(row_ok) {
 #pragma unroll
 		for(int r = 0; r < ROWS; r++) {
 			if(b0 + r >= b_end) break;
+			[[maybe_unused]] const int gk = 2 * r + (n >> 4);   // this query row's piece of the gate
+			[[maybe_unused]] const unsigned char* const gate_row = smem + (gk < ROWS ? gate_buf[0] : gate_buf[1]) + (wave * ROWS + (gk < ROWS ? gk : gk - ROWS)) * 1024 + (n & 15) * 64;
 			const float   inv  = 1.f / lsum[r];
 			const int64_t ooff = (b0 + r) * p.out_stride[0] + h * p.out_stride[1] + qrow * p.out_stride[2];
-			u32x2         gw[4] = {u32x2{0u, 0u}, u32x2{0u, 0u}, u32x2{0u, 0u}, u32x2{0u, 0u}};
-			if(p.gate) {
-				const uint16_t* gp = static_cast<const uint16_t*>(p.gate) + (b0 + r) * p.gate_stride[0] + h * p.gate_stride[1] + qrow * p.gate_stride[2];
-#pragma unroll
-				for(int g4 = 0; g4 < 4; g4++)
-					if(8 * g4 + 4 * half < D) gw[g4] = *reinterpret_cast<const u32x2*>(gp + 8 * g4 + 4 * half);
-			}
 #pragma unroll
 			for(int g4 = 0; g4 < 4; g4++) {
 				const int d0 = 8 * g4 + 4 * half;
 				if(d0 >= D) continue;
 				float o0 = oacc[r][4 * g4] * inv, o1 = oacc[r][4 * g4 + 1] * inv, o2 = oacc[r][4 * g4 + 2] * inv, o3 = oacc[r][4 * g4 + 3] * inv;
-				if(p.gate) {
-					const uint32_t g0 = gw[g4][0], g1 = gw[g4][1];
+				if constexpr(GATE) {
+					const u32x2    gw = *reinterpret_cast<const u32x2*>(gate_row + d0 * 2);
+					const uint32_t g0 = gw[0], g1 = gw[1];
 					o0 *= sigmoidf_fast(bf16_bits_to_f32(g0 & 0xffffu)), o1 *= sigmoidf_fast(bf16_bits_to_f32(g0 >> 16));
 					o2 *= sigmoidf_fast(bf16_bits_to_f32(g1 & 0xffffu)), o3 *= sigmoidf_fast(bf16_bits_to_f32(g1 >> 16));
 				}
@@ -761,7 +788,7 @@ int launch_rows(const af3_dpa_params& p, int64_t b_first, int64_t b_count, hipSt
 	if(blocks <= 0 || blocks > 0x7fffffffLL) return AF3_ERR_BAD_SHAPE;
 	const size_t n_t_all = (size_t)((p.L + KT_R - 1) / KT_R);
 	const size_t smem    = (size_t)NBUF_R * ROWS * 2 * TILE_R + (BMODE == 1 || BMODE == 3 ? 4 * 4096 : 0) + (n_t_all + 1) * ROWS * 32 * 2;
-	auto         kern    = dpa_rows_bf16_kernel<ROWS, BMODE>;
+	auto         kern    = p.gate ? dpa_rows_bf16_kernel<ROWS, BMODE, true> : dpa_rows_bf16_kernel<ROWS, BMODE, false>;
 	if(smem > 64 * 1024) {
 		if(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) return AF3_ERR_LAUNCH;
 	}
@@ -777,10 +804,10 @@ int launch_rows_n(int rows, const af3_dpa_params& p, int64_t b_first, int64_t b_
 }  // namespace
 
 // Shapes the kernel takes: what dpa_mfma.hip's kernel takes (mfma_bf16_eligible, checked by the caller), and in addition
-// head_dim <= 32, at least two batch rows, a length whose mask table fits beside the tile buffers, 8-byte aligned gate rows.
+// head_dim <= 32, at least two batch rows, a length whose mask table fits beside the tile buffers, 16-byte aligned gate rows.
 bool mfma_rows_eligible(const af3_dpa_params& p) {
 	if(p.D > 32 || p.B < 2 || p.L > MAX_L_ROWS) return false;
-	if(p.gate && ((reinterpret_cast<uintptr_t>(p.gate) & 7) || p.gate_stride[0] % 4 || p.gate_stride[1] % 4 || p.gate_stride[2] % 4)) return false;
+	if(p.gate && ((reinterpret_cast<uintptr_t>(p.gate) & 15) || p.gate_stride[0] % 8 || p.gate_stride[1] % 8 || p.gate_stride[2] % 8)) return false;
 	return true;
 }
 

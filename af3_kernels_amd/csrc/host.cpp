@@ -25,7 +25,10 @@
 #include "../../include/af3_dpa.h"
 
 extern "C" int64_t af3_dpa_workspace_used(const af3_dpa_params*);   // (api.hip; not part of the ABI)
+extern "C" int     af3_dpa_log2_domain(const af3_dpa_params*);            // (likewise)
 extern "C" int af3_project_suits(int64_t, int64_t, int64_t);              // (projection.hip, likewise)
+extern "C" int af3_grid_project(const void*, const int64_t*, const void*, const void*, float, const void*, const void*, const void*, const void*, const void*, int64_t, int64_t, int32_t, float, void*,
+								void*, void*, void*, void*, void*);        // (grid_project.hip, likewise)
 extern "C" int af3_project(const void*, const void*, const void*, void*, int64_t, int64_t, int64_t, int32_t, void*);
 
 namespace {
@@ -96,11 +99,15 @@ af3_dpa_params block(int64_t B, int64_t H, int64_t L, int64_t D, int code, int64
 	p.reserved = (int32_t)hint;
 	return p;
 }
-int forward(af3_dpa_params& p, bool exact_bias, int dev) {
+at::DataPtr workspace_for(af3_dpa_params& p, bool exact_bias) {
 	at::DataPtr   ws;
 	if(!exact_bias) p.reserved |= 4;
 	const int64_t bytes = exact_bias ? 0 : af3_dpa_workspace_used(&p);
 	if(bytes > 0) ws = new_scratch(bytes), p.workspace = ws.get(), p.workspace_bytes = bytes;
+	return ws;
+}
+int forward(af3_dpa_params& p, bool exact_bias, int dev) {
+	const at::DataPtr ws = workspace_for(p, exact_bias);
 	return af3_dpa_forward(&p, current_stream(dev));
 }
 PyObject* answer(int rc, Tensor&& out) { return rc == AF3_OK ? wrap(std::move(out)) : PyLong_FromLong(rc); }
@@ -467,6 +474,36 @@ PyObject* py_layernorm_pair_bias(PyObject*, PyObject* const* a, Py_ssize_t n) {
 	END_HANDLE_TH_ERRORS
 }
 
+// LayerNorm, pair bias and projections in one kernel (128 channels in 4 heads, bfloat16), then the attention launch on q, k, v and the
+// gate [B, 4, N, 32]: into `gated` [B, N, C]; 1 where this form does not take the tensors.
+bool grid_projected_ok(const ln_args& r, const Tensor* const (&ws)[4]) {
+	const auto odd = [](const Tensor* t, int to) { return reinterpret_cast<uintptr_t>(t->const_data_ptr()) % to != 0; };
+	return r.pair->size(2) == 128 && r.proj->size(0) == 4 && r.pair->scalar_type() == at::kBFloat16 && r.pair->stride(0) % 8 == 0 && r.pair->stride(1) % 8 == 0 && !odd(r.pair, 16) &&
+		   !odd(r.gamma, 16) && !odd(r.beta, 16) && !odd(r.proj, 16) && !odd(ws[0], 4) && !odd(ws[1], 4) && !odd(ws[2], 4) && !odd(ws[3], 4);
+}
+int grid_projected(const ln_args& r, const key_mask& m, const Tensor* const (&ws)[4], bool turned, int64_t hint, bool exact, Tensor& gated, int dev) {
+	const int64_t n_i = r.pair->size(0), n_j = r.pair->size(1), B = turned ? n_j : n_i, N = turned ? n_i : n_j, each = n_i * n_j * 128;
+	const at::DataPtr mem = new_scratch((4 * each + 4 * n_i * n_j) * 2);
+	auto* const       q = static_cast<uint16_t*>(mem.get());
+	uint16_t *const   k = q + each, *const v = k + each, *const gate = v + each, *const bias = gate + each;
+	gated = new_tensor({B, N, 128}, at::kBFloat16, dev);
+	af3_dpa_params p = block(B, 4, N, 32, AF3_BF16, hint);
+	p.q = q, p.k = k, p.v = v, p.gate = gate, p.out = gated.data_ptr(), p.bias = bias;
+	const int64_t st[3] = {4 * N * 32, N * 32, 32}, so[3] = {N * 128, 32, 128};
+	for(int i = 0; i < 3; i++) p.q_stride[i] = p.k_stride[i] = p.v_stride[i] = p.gate_stride[i] = st[i], p.out_stride[i] = so[i];
+	p.bias_stride[0] = n_i * n_j, p.bias_stride[1] = n_j, p.bias_dtype = AF3_BF16;
+	p.key_mask = m.ptr, p.key_mask_stride_b = m.stride;
+	const at::DataPtr work = workspace_for(p, exact);
+	// The whole scale of the logits goes into q where it is projected, in fp32: one rounding.  What is left for the attention
+	// kernel is 1 in its own units (a product with it gives the same bits back).
+	const float log2e = 1.4426950408889634f, q_scale = af3_dpa_log2_domain(&p) ? p.softmax_scale * log2e : p.softmax_scale;
+	p.softmax_scale = q_scale == p.softmax_scale ? 1.f : 1.f / log2e;
+	const int64_t ps[2] = {r.pair->stride(0), r.pair->stride(1)};
+	const int     rc = af3_grid_project(r.pair->const_data_ptr(), ps, r.gamma->const_data_ptr(), r.beta->const_data_ptr(), r.eps, r.proj->const_data_ptr(), ws[0]->const_data_ptr(),
+										ws[1]->const_data_ptr(), ws[2]->const_data_ptr(), ws[3]->const_data_ptr(), n_i, n_j, turned, q_scale, q, k, v, gate, bias, current_stream(dev));
+	return rc != AF3_OK ? rc : af3_dpa_forward(&p, current_stream(dev));
+}
+
 // grid_block(pair, ln_weight, ln_bias, eps, proj_weight, mask, wq, wk, wv, wg, out_proj, head, transpose, least (batch row, head) pairs of
 // the one-kernel form, kernel hint, exact bias): the whole block of GridSelfAttentionCpp.forward
 PyObject* py_grid_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -490,8 +527,9 @@ PyObject* py_grid_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
 	{
 		without_gil g;
 		Tensor normed, bias, gated;
-		rc = ln_pair_bias(r, normed, bias, dev);
-		if(rc == AF3_OK) {
+		const bool projected = grid_projected_ok(r, ws);
+		rc = projected ? grid_projected(r, m, ws, turned, hint, exact, gated, dev) : ln_pair_bias(r, normed, bias, dev);
+		if(rc == AF3_OK && !projected) {
 			const Tensor rows = turned ? normed.transpose(0, 1) : normed;
 			rc = B * head >= least && !exact ? grid_kernel(rows, m, &bias, ws, head, gated, dev) : 1;
 			if(rc == 1 && fused.defined()) {

@@ -117,6 +117,13 @@ def _q_bias_row(q_bias: torch.Tensor, head: int, dtype: torch.dtype) -> torch.Te
     return _remember(_host.Q_BIAS_ROW, head, dtype, _cached((q_bias,), (head, dtype, "q_bias"), make), q_bias)
 
 
+def _out_proj_t(out_proj: torch.Tensor) -> torch.Tensor:
+    """The output projection in nn.Linear layout [out, in], left where the native path finds it."""
+    w = _cached((out_proj,), ("out_proj",), lambda: out_proj.t().contiguous())
+    _host.remember(_host.OUT_PROJ_T, w, out_proj)
+    return w
+
+
 def _check_weights(C: int, head: int, ws):
     if C % head != 0:
         raise ValueError(f"channel count {C} is not divisible by head={head}")
@@ -270,9 +277,7 @@ def _attention_cpp(
         return out if out.__class__ is not int else _lib.check(out, "af3_linear")
     rows = gated.view(B * N, C)
     if out_proj.dtype == dtype and _narrow_linear_ok(rows, C):
-        w = _cached((out_proj,), ("out_proj",), lambda: out_proj.t().contiguous())      # nn.Linear layout [out, in]
-        _host.remember(_host.OUT_PROJ_T, w, out_proj)
-        return _linear_rows(rows, w).view(B, N, C)
+        return _linear_rows(rows, _out_proj_t(out_proj)).view(B, N, C)
     return torch.matmul(rows, out_proj.to(dtype)).view(B, N, C)
 
 
@@ -391,15 +396,22 @@ class GridSelfAttentionCpp(torch.nn.Module):
             self.first_run = False
         return self.q_proj, self.k_proj, self.v_proj, self.gq, self.out_proj
 
+    def _native_block(self, pair: torch.Tensor, mask: torch.Tensor):
+        # (straight from the module's dictionaries: an attribute lookup that falls through to them costs a microsecond each)
+        parts = self.__dict__["_modules"]
+        norm, proj = parts["act_norm"], parts["pair_bias_projection"]
+        return _host.grid_block(pair, norm._parameters.get("weight"), norm._parameters.get("bias"), norm.eps, proj._parameters.get("weight"), mask, self.q_proj, self.k_proj,
+                                self.v_proj, self.gq, self.out_proj, self.num_head, self.transpose, _FUSED_MIN_GROUPS, ops._rows_kernel_hint, ops._exact_bias)
+
     def forward(self, pair: torch.Tensor, mask: torch.Tensor) -> torch.Tensor:
-        if not self.first_run:
-            # (straight from the module's dictionaries: an attribute lookup that falls through to them costs a microsecond each)
-            parts = self.__dict__["_modules"]
-            norm, proj = parts["act_norm"], parts["pair_bias_projection"]
-            out = _host.grid_block(pair, norm._parameters.get("weight"), norm._parameters.get("bias"), norm.eps, proj._parameters.get("weight"), mask, self.q_proj, self.k_proj,
-                                   self.v_proj, self.gq, self.out_proj, self.num_head, self.transpose, _FUSED_MIN_GROUPS, ops._rows_kernel_hint, ops._exact_bias)
-            if out is not None:
-                return out if out.__class__ is not int else _lib.check(out, "grid attention block")
+        if self.first_run:
+            self._packed_weights()
+        out = self._native_block(pair, mask)
+        if out is None and self.out_proj.is_cuda:   # (the first call: the closing projection's matrix is not where the native path looks for it)
+            _out_proj_t(self.out_proj)
+            out = self._native_block(pair, mask)
+        if out is not None:
+            return out if out.__class__ is not int else _lib.check(out, "grid attention block")
         normed, bias = layernorm_pair_bias(pair, self.act_norm.weight, self.act_norm.bias, self.act_norm.eps, self.pair_bias_projection.weight)  # bias [head, N, N]
         rows = normed.transpose(0, 1) if self.transpose else normed         # attend along columns when transposed
         out = _attention_cpp(rows, mask, bias, *self._packed_weights(), self.num_head, False, 128 if pair.shape[1] > 256 else 64, 0)

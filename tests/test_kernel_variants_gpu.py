@@ -196,3 +196,40 @@ def test_fp8_bias_forms_and_tile_flags(af3, B, H, L, D, mask_kind, compensated):
     # e4m3 weights: each within 2^-4 of itself
     bound = 2 ** -4 * p.matmul((vd.float() * vs).abs()) + 2e-2
     assert bool(((out.float() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("transpose", [False, True])
+@pytest.mark.parametrize("N", [1, 2, 31, 33, 64, 97, 150, 161, 200, 229, 330])
+def test_grid_block_projected_form(af3, N, transpose):
+    """The grid block (projections in one pass, attention, output projection) against the same steps in float32, with bf16 roundings where
+    the block stores bf16: partial token blocks, heads in separate workgroups and together, query tiles with idle wavefronts, gate rows of one to
+    four batch rows, both orientations."""
+    g = torch.Generator(device="cuda").manual_seed(N)
+    mod = af3.GridSelfAttentionCpp(128, 4, transpose).to("cuda", torch.bfloat16).eval().requires_grad_(False)
+    for name, p in mod.named_parameters():
+        p.copy_(torch.randn(p.shape, generator=g, device="cuda") * (128 ** -0.5 if p.dim() == 2 else 0.1) + (1.0 if name == "act_norm.weight" else 0.0))
+    pair = torch.randn(N, N, 128, generator=g, device="cuda").mul_(2.0).add_(0.5).to(torch.bfloat16)
+    keep = torch.rand(N, N, generator=g, device="cuda") < 0.8
+    keep[:, 0] = True
+    if N > 2:
+        keep[1] = False   # a row without any live key
+    print("case", N, transpose, flush=True)
+    out = mod(pair, keep)
+    again = mod(pair, keep)
+    torch.cuda.synchronize()
+    assert torch.equal(out, again)
+    bf = lambda t: t.to(torch.bfloat16).float()
+    f = lambda m: m.weight.float()
+    x = bf(torch.nn.functional.layer_norm(pair.float(), (128,), f(mod.act_norm), mod.act_norm.bias.float(), mod.act_norm.eps))
+    bias = bf(torch.nn.functional.linear(x, f(mod.pair_bias_projection))).permute(2, 0, 1)
+    rows = x.transpose(0, 1) if transpose else x
+    q, k, v, gate = (torch.nn.functional.linear(rows, f(m)).view(N, N, 4, 32).transpose(1, 2).contiguous()
+                     for m in (mod.q_projection, mod.k_projection, mod.v_projection, mod.gating_query))
+    s = bf(q * 32 ** -0.5).matmul(bf(k).transpose(-1, -2).contiguous()) + bias
+    s = s.masked_fill(~keep[:, None, None, :], -1e9)
+    o = s.softmax(-1).matmul(bf(v)) * torch.sigmoid(bf(gate))
+    want = torch.nn.functional.linear(bf(o.transpose(1, 2).reshape(N, N, 128)), f(mod.output_projection))
+    if transpose:
+        want = want.transpose(0, 1)
+    err = (out.float() - want).abs()
+    assert err.max() <= 3e-2 * max(1.0, float(want.abs().max())) and err.norm() <= 1e-2 * want.norm()
