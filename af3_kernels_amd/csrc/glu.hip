@@ -13,16 +13,17 @@
 //     rows, sixteen wavefronts per block -- was tried: twice as slow);
 //   * out^T[col][row] = W^T . x^T on v_mfma_f32_32x32x16_bf16: lane = row, registers = 4 x 4 consecutive columns, so
 //     silu * value is in-lane;
-//   * the 32 x 32 result tile is turned through a private LDS patch so that it leaves as 16-byte stores, four lanes per
-//     64-byte row segment (8-byte stores straight from the accumulator layout made the memory system handle four times
-//     as many write requests).
-// Two details keep a wavefront from waiting for its own stores to be acknowledged in every block:
-//   * loads and stores go through buffer descriptors of one block each (wave-uniform base, hardware range check), so rows
-//     past M read zeros / store nothing without a branch around the instruction -- after a branch the compiler waits for
-//     ALL outstanding memory operations where only the next block's rows are needed;
-//   * the registers that feed the stores are kept out of circulation until the next block's stores (the compiler waits for
-//     a store before it lets anything overwrite the store's data registers, and would otherwise hand them to the next
-//     block's first matrix instruction).
+//   * the results of all wavefronts meet in an LDS tile (32 rows x up to 512 columns, double-buffered) and leave during the next
+//     block as whole rows, 1 KB per wavefront and store: for 512 columns the block's output is one contiguous 32 KB (8-byte stores straight from
+//     the accumulator layout made the memory system handle four times as many write requests; 64-byte row segments per wavefront took
+//     201 against 192 us at n = 768 and K = 128, 129 against 113 at K = 64, with stores that bypass the caches in the faster figures).
+//     Weight rows are permuted so that a lane's sixteen results are consecutive columns: two 16-byte LDS writes, swizzled, no conflicts.
+// Loads and stores go through buffer descriptors of one block each (wave-uniform base, hardware range check), so rows
+// past M read zeros / store nothing without a branch around the instruction -- after a branch the compiler waits for
+// ALL outstanding memory operations where only the next block's rows are needed.  The stores of a block are younger than the
+// fetch of the next one, which is all that a wavefront waits for.
+// What bounds it: power.  The chip holds 1.8 GHz at n = 768, K = 128; matrix instructions, the two transcendentals per element and
+// the memory traffic each add their share (without the stores 158 us, without the sigmoid 169, without both 131).
 // Also measured and not kept: four 16 x 16 sub-tiles on v_mfma_f32_16x16x32_bf16 with the silu of one sub-tile placed
 // behind the next one's products (same instruction count, meant to overlap the two pipes inside a wavefront): 13-18 % slower.
 #include <type_traits>
@@ -37,7 +38,8 @@ constexpr int GLU_MAX_WAVES = 16;
 
 // KS: contraction steps of 16 channels (K = 16 * KS).  WAVES: wavefronts per workgroup = 32-column tiles it owns.
 // GATED: out = silu(x . Wa) * (x . Wb) with wt = [Wa | Wb]^T; otherwise the plain product out = x . W with wt = W^T.
-template <int KS, int WAVES, bool GATED>
+// NT: stores that do not stay in the caches (outputs larger than those).
+template <int KS, int WAVES, bool GATED, bool NT>
 // (four wavefronts per SIMD whatever the workgroup size: 128 registers each)
 __global__ void __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(4))) glu_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ wt, uint16_t* __restrict__ out, int64_t M, int64_t N) {
 	constexpr int K          = 16 * KS;
@@ -46,25 +48,27 @@ __global__ void __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu
 	constexpr int TPB        = TILE_BYTES / (WAVES * 64);  // bytes of a block per thread: 4 .. 32
 	constexpr int PIECE      = TPB < 16 ? TPB : 16;         // moved in pieces of at most 16 bytes
 	constexpr int PPT        = TPB / PIECE;
-	constexpr int OUT_STRIDE = 80;  // bytes per row of the output patch: 64 of data, padded so that rows start in different banks
+	constexpr int OUT_STRIDE = WAVES * 64;  // bytes per row of the output tile, its 16-byte chunks XOR-swizzled with the row
 	static_assert(TILE_BYTES % (WAVES * 64) == 0 && TPB >= 4 && TPB % PIECE == 0, "every thread moves whole pieces of a block");
 	__shared__ __attribute__((aligned(16))) unsigned char xs[2][TILE_BYTES];
-	__shared__ __attribute__((aligned(16))) unsigned char os[WAVES][32 * OUT_STRIDE];
+	extern __shared__ __attribute__((aligned(16))) unsigned char os[];   // [2][32 * OUT_STRIDE]
 
 	const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 	const int n = lane & 31, half = lane >> 5;
 	const int64_t col0   = ((int64_t)blockIdx.y * WAVES + wave) * 32;  // first (gate) column of this wavefront
 	const bool    active = col0 < N;  // wavefronts past the last column only help to move x
 
-	// weight fragments (A operand): lane (column n, g = half), step s: W^T[col][16s + 8g .. +7]; wt is [2N, K] ([N, K]) row-major
+	// weight fragments (A operand): lane (row n, g = half), step s: W^T[col][16s + 8g .. +7]; wt is [2N, K] ([N, K]) row-major.  Row
+	// r = 8 a + 4 g + e is column 16 g + 4 a + e of the tile, so that a lane's sixteen results are consecutive columns.
+	const int64_t wcol = col0 + 16 * ((n >> 2) & 1) + 4 * (n >> 3) + (n & 3);
 	u32x4 wa[KS], wb[GATED ? KS : 1];
 #pragma unroll
 	for(int s = 0; s < KS; s++) {
 		wa[s] = u32x4{0u, 0u, 0u, 0u};
 		if(GATED) wb[s] = u32x4{0u, 0u, 0u, 0u};
 		if(active) {
-			wa[s] = *reinterpret_cast<const u32x4*>(wt + (col0 + n) * K + 16 * s + 8 * half);
-			if(GATED) wb[s] = *reinterpret_cast<const u32x4*>(wt + (N + col0 + n) * K + 16 * s + 8 * half);
+			wa[s] = *reinterpret_cast<const u32x4*>(wt + wcol * K + 16 * s + 8 * half);
+			if(GATED) wb[s] = *reinterpret_cast<const u32x4*>(wt + (N + wcol) * K + 16 * s + 8 * half);
 		}
 	}
 
@@ -101,10 +105,17 @@ __global__ void __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu
 	// operand reads (lane = row n, chunk 2s + half, swizzled) and the output patch
 	const int            x_rd  = n * ROW_BYTES;
 	const int            sw    = n & 7;
-	unsigned char* const patch = os[wave];
-	const int            p_wr  = n * OUT_STRIDE + half * 8;
-	const int            p_rd  = (lane >> 2) * OUT_STRIDE + (lane & 3) * 16;
-	const int            o_off = (int)(((lane >> 2) * N + col0 + (lane & 3) * 8) * 2);  // bytes from the block's first row (N < 2^20 checked by the launcher)
+	// this lane's two chunks of the output tile (row n, columns 32 wave + 16 half ..), and the chunks it stores: 1 KB per wavefront and
+	// load, consecutive lanes on consecutive chunks of a row
+	constexpr int CPRO = WAVES * 4, RPS = 64 / CPRO > 0 ? 64 / CPRO : 1;   // chunks per row; rows per store (a row is at most one store)
+	static_assert(CPRO <= 64 && 32 % (WAVES * RPS) == 0, "whole rows per store");
+	constexpr int STORES = 32 / (WAVES * RPS);
+	const int     p_wr[2] = {n * OUT_STRIDE + (((4 * wave + 2 * half) ^ (n & 7)) << 4), n * OUT_STRIDE + (((4 * wave + 2 * half + 1) ^ (n & 7)) << 4)};
+	const int     s_row = wave * RPS + lane / CPRO, s_ch = lane % CPRO;   // (+ WAVES * RPS rows per further store)
+	const int64_t scol  = (int64_t)blockIdx.y * WAVES * 32 + s_ch * 8;
+	const int     p_rd  = s_row * OUT_STRIDE + ((s_ch ^ (s_row & 7)) << 4);
+	static_assert((WAVES * RPS) % 8 == 0, "the swizzle repeats from store to store");
+	const int     o_off = scol < N ? (int)((s_row * N + scol) * 2) : 0x7FFF0000;  // bytes from the block's first row (N < 2^20 checked by the launcher)
 
 	int64_t blk = blockIdx.x;
 	if(blk >= n_blocks) return;  // (whole workgroup)
@@ -112,11 +123,24 @@ __global__ void __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu
 	publish(0, staged);
 	__syncthreads();
 	int   buf = 0;
-	u32x4 sv[2] = {u32x4{0u, 0u, 0u, 0u}, u32x4{0u, 0u, 0u, 0u}};  // the data of the two stores of a block
+	u32x4 sv[STORES];  // the data of the stores of a block
+#pragma unroll
+	for(int i = 0; i < STORES; i++) sv[i] = u32x4{0u, 0u, 0u, 0u};
+	auto store_block = [&](int64_t b, int obuf) {   // the finished tile of block b, whole rows
+		const __amdgpu_buffer_rsrc_t orsrc =
+			__builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<unsigned char*>(out) + (b < 0 ? 0 : b) * 32 * N * 2, 0, b < 0 ? 0 : (int)(rows_in(b) * N * 2), 0x00020000);
+		typedef __attribute__((ext_vector_type(4))) unsigned int store_t;
+#pragma unroll
+		for(int i = 0; i < STORES; i++) sv[i] = *reinterpret_cast<const u32x4*>(os + obuf * (32 * OUT_STRIDE) + p_rd + i * (WAVES * RPS * OUT_STRIDE));
+#pragma unroll
+		for(int i = 0; i < STORES; i++) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(store_t, sv[i]), orsrc, o_off + (int)(i * WAVES * RPS * N * 2), 0, NT ? 2 : 0);
+	};
+	int64_t prev = -1;
 	for(; blk < n_blocks; blk += gridDim.x) {
 		const int64_t next     = blk + gridDim.x;
 		const bool    has_next = next < n_blocks;  // (uniform)
 		staged = fetch(has_next ? next : blk);       // in flight during this block's matrix work (the last block is fetched again: no branch)
+		store_block(prev, buf ^ 1);                  // (its tile is complete since the barrier; before the first block: nothing)
 		const unsigned char* const xb = xs[buf] + x_rd;
 		f32x16 ga, va;
 #pragma unroll
@@ -127,33 +151,29 @@ __global__ void __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu
 			ga = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, wa[s]), __builtin_bit_cast(bf16x8, xf), ga, 0, 0, 0);
 			if(GATED) va = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, wb[s]), __builtin_bit_cast(bf16x8, xf), va, 0, 0, 0);
 		}
-		// silu(a) * b, rounded to bf16, into this wavefront's patch: lane (row n, half) owns columns 8*g4 + 4*half .. +3
+		// silu(a) * b, rounded to bf16, into the output tile: lane (row n, half) owns columns 16 half .. +15 of its wavefront's 32
 #pragma unroll
-		for(int g4 = 0; g4 < 4; g4++) {
-			float o[4];
+		for(int z = 0; z < 2; z++) {
+			u32x4 w;
 #pragma unroll
-			for(int r = 0; r < 4; r++) {
-				const float a = ga[4 * g4 + r];
-				o[r] = GATED ? a * va[4 * g4 + r] * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-a * LOG2E)) : a;
+			for(int k = 0; k < 4; k++) {
+				float o[2];
+#pragma unroll
+				for(int r = 0; r < 2; r++) {
+					const float a = ga[8 * z + 2 * k + r];
+					o[r] = GATED ? a * va[8 * z + 2 * k + r] * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-a * LOG2E)) : a;
+				}
+				w[k] = pack_bf16x2(o[0], o[1]);
 			}
-			*reinterpret_cast<u32x2*>(patch + p_wr + g4 * 16) = u32x2{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
+			*reinterpret_cast<u32x4*>(os + buf * (32 * OUT_STRIDE) + p_wr[z]) = w;
 		}
-		// (the same wavefront writes and reads the patch, and its LDS operations complete in order; the wave barriers
-		// only keep the compiler from moving the reads above the writes, or the next block's writes above the reads)
-		__builtin_amdgcn_wave_barrier();
-		asm volatile("" : "+v"(sv[0]), "+v"(sv[1]));  // sv's registers stay reserved from the previous block's stores up to here
-		sv[0] = *reinterpret_cast<const u32x4*>(patch + p_rd);
-		sv[1] = *reinterpret_cast<const u32x4*>(patch + p_rd + 16 * OUT_STRIDE);
-		__builtin_amdgcn_wave_barrier();
-		const __amdgpu_buffer_rsrc_t orsrc = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<unsigned char*>(out) + blk * 32 * N * 2, 0, active ? (int)(rows_in(blk) * N * 2) : 0, 0x00020000);
-		typedef __attribute__((ext_vector_type(4))) unsigned int store_t;
-		__builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(store_t, sv[0]), orsrc, o_off, 0, 0);
-		__builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(store_t, sv[1]), orsrc, o_off + (int)(16 * N * 2), 0, 0);
 		// publish the next block (its LDS buffer was last read before the previous barrier)
 		publish(buf ^ 1, staged);
 		__syncthreads();
+		prev = blk;
 		buf ^= 1;
 	}
+	store_block(prev, buf ^ 1);
 }
 
 }  // namespace
@@ -179,17 +199,20 @@ int launch_rows_times_weights(const void* x, const void* weight_t, void* out, in
 	auto*         op = static_cast<uint16_t*>(out);
 	// persistent workgroups: about sixteen resident wavefronts per compute unit
 	auto go = [&](auto kern, int waves) {
+		const size_t smem = (size_t)2 * 32 * waves * 64;
 		const unsigned gy   = (unsigned)((col_tiles + waves - 1) / waves);
 		const int64_t  want = (int64_t)256 * (GLU_MAX_WAVES / waves) / gy > 0 ? (int64_t)256 * (GLU_MAX_WAVES / waves) / gy : 1;
-		hipLaunchKernelGGL(kern, dim3((unsigned)(n_blocks < want ? n_blocks : want), gy), dim3(waves * 64), 0, s, xp, wp, op, M, N);
+		hipLaunchKernelGGL(kern, dim3((unsigned)(n_blocks < want ? n_blocks : want), gy), dim3(waves * 64), smem, s, xp, wp, op, M, N);
 	};
-	if(col_tiles <= 4 && !gated) {  // narrow plain products (the attention blocks' output projection): 4-wave workgroups, four per compute unit
-		if(K == 128) go(glu_kernel<8, 4, false>, 4);
-		else go(glu_kernel<4, 4, false>, 4);
-	} else {
-		if(K == 128) gated ? go(glu_kernel<8, GLU_MAX_WAVES, true>, GLU_MAX_WAVES) : go(glu_kernel<8, GLU_MAX_WAVES, false>, GLU_MAX_WAVES);
-		else gated ? go(glu_kernel<4, GLU_MAX_WAVES, true>, GLU_MAX_WAVES) : go(glu_kernel<4, GLU_MAX_WAVES, false>, GLU_MAX_WAVES);
-	}
+	// an output that exceeds the 256 MB of the memory-side cache leaves nothing there for whoever reads it: it is written past the caches
+	const bool nt = M * N * 2 > ((int64_t)256 << 20);
+	auto pick = [&](auto ks_c) {
+		constexpr int KS = decltype(ks_c)::value;
+		if(gated) nt ? go(glu_kernel<KS, GLU_MAX_WAVES, true, true>, GLU_MAX_WAVES) : go(glu_kernel<KS, GLU_MAX_WAVES, true, false>, GLU_MAX_WAVES);
+		else if(col_tiles <= 4) go(glu_kernel<KS, 4, false, false>, 4);   // narrow plain products (the attention blocks' output projection): 4-wave workgroups, four per compute unit
+		else go(glu_kernel<KS, GLU_MAX_WAVES, false, false>, GLU_MAX_WAVES);
+	};
+	K == 128 ? pick(std::integral_constant<int, 8>{}) : pick(std::integral_constant<int, 4>{});
 	return launch_status();
 }
 

@@ -233,3 +233,18 @@ def test_grid_block_projected_form(af3, N, transpose):
         want = want.transpose(0, 1)
     err = (out.float() - want).abs()
     assert err.max() <= 3e-2 * max(1.0, float(want.abs().max())) and err.norm() <= 1e-2 * want.norm()
+
+
+@pytest.mark.parametrize("M,K,N", [(1, 64, 32), (33, 128, 480), (65, 64, 544), (524289 + 31, 64, 256), (262145, 128, 544)])
+def test_glu_whole_row_stores(af3, M, K, N):
+    """Outputs narrower and wider than a workgroup's 512 columns, partial blocks of rows, and outputs beyond 256 MB (their stores bypass the caches)."""
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    x = torch.randn(M, K, generator=g, device="cuda", dtype=torch.bfloat16)
+    w = torch.randn(K, 2 * N, generator=g, device="cuda", dtype=torch.bfloat16) * K ** -0.5
+    print("case", M, K, N, flush=True)
+    out = af3.gated_linear_unit_cpp(x, w)
+    torch.cuda.synchronize()
+    for rows in (slice(0, 4096), slice(max(0, M - 4096), M), slice(M // 2, M // 2 + 4096)):
+        a, b = (x[rows].float() @ w.float()).chunk(2, dim=-1)
+        want = torch.nn.functional.silu(a) * b
+        assert (out[rows].float() - want).abs().max() <= 2 ** -7 * want.abs().max()
