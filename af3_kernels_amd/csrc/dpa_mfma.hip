@@ -166,6 +166,10 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 	constexpr int  NBUF       = LOADERS ? AHEAD + 3 : 3;
 	constexpr int  RING_BYTES = BRING ? (KS2 ? NW / 2 : NW) * NBUF * SLOT_BYTES : 0;  // (KS2: one ring per pair of wavefronts)
 	constexpr int  MASK_BASE  = LDS_SETS * 2 * NBUF * TILE_BYTES + RING_BYTES;
+	// The output gate's rows of a workgroup of four wavefronts that load for themselves wait in the K/V buffers that the tile behind the
+	// last one would take; elsewhere behind the tile list.  (With 8 KB of their own a workgroup no longer shared its compute unit with a
+	// second one: 128 x 4 x 128 x 32 with a gate 13.1 us.)
+	constexpr bool GATE_IN_TILE = DP == 32 && NW == 4 && !SPLIT && !FUSED && KSL == 0;
 	static_assert(!(L2DOM && BMODE != 0), "the log2 variant reads its bias from the workspace");
 	static_assert(FUSED || (LOADERS ? NI % 4 == 0 : NW <= NI), "every wavefront that loads fetches a whole number of 1 KB pieces of each tile");
 	static_assert(!LOADERS || (!SPLIT && !FUSED), "loading wavefronts serve workgroups that share their tiles");
@@ -702,8 +706,8 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 		// ---- output gate: fetched into LDS now, by loads that write LDS directly and hold no registers, and read in the
 		// epilogue.  (Loading it in the epilogue exposed a full memory latency per workgroup: 8 % of the kernel's time.)
 		// The first tile wait of the prologue below also covers these loads: they are older. ----
-		unsigned char* const gate_lds = smem + gate_base + wblk * (32 * DP * 2);
-		if(!FUSED && p.gate && (SPLIT ? wave == 0 : sub == 0)) {  // (the wavefronts that write results)
+		unsigned char* gate_lds = smem + gate_base + wblk * (32 * DP * 2);
+		auto           load_gate = [&]() {
 			const u32x4   g_rsrc = raw_rsrc(static_cast<const uint16_t*>(p.gate) + b * p.gate_stride[0] + h * p.gate_stride[1], (uint32_t)(((L - 1) * p.gate_stride[2] + D) * 2));
 			constexpr int RPL    = 512 / DP;  // rows per 1 KB wave load
 			const int     g_row  = lane / CPR, g_c = lane % CPR;
@@ -714,7 +718,15 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 				const int     voff = (g_c * 8 < D && row < L) ? (int)(row * p.gate_stride[2] * 2) + g_c * 16 : 0x7FFF0000;  // past the range: nothing is fetched
 				lds_dma_b128(g_rsrc, lds_addr_of(gate_lds) + t * 1024, voff);
 			}
-		}
+		};
+		// (GATE_IN_TILE: 2 KB per wavefront in the place of tile my_n, requested where that tile would be)
+		auto gate_to_tile = [&](int buf) {
+			if constexpr(GATE_IN_TILE) {
+				gate_lds = (wave < 2 ? k_lds : v_lds) + buf * TILE_BYTES + (wave & 1) * 2048;
+				if(p.gate) load_gate();
+			}
+		};
+		if(!FUSED && !GATE_IN_TILE && p.gate && (SPLIT ? wave == 0 : sub == 0)) load_gate();  // (the wavefronts that write results)
 
 		// fragment read: lane (n, half) takes chunk 4*sub + 2*c2 + half of row n
 		const int b_rd = (n * 128 + (((n & 7) ^ half) << 4)) ^ (sub << 6);  // (KS2: chunks 4..7 of a row hold keys 32..63)
@@ -1057,6 +1069,12 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 					load_tile(kt1_first, 1);
 					load_bias_tile(kt1_first, 1);
 				}
+			} else {
+				if(GATE_IN_TILE && guessed1) {   // (every wavefront's part of the guessed second tile has landed before the gate takes its place)
+					asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+					__syncthreads();
+				}
+				gate_to_tile(1);
 			}
 #pragma unroll
 			for(int f = 0; f < 4; f++) bfrag[f] = u32x4{0u, 0u, 0u, 0u};
@@ -1127,7 +1145,7 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 				if(it + 2 < my_n) {
 					load_tile(kt2, bufnn);
 					load_bias_tile(kt2, bufnn);  // (its slot held tile it-1, last read in the stage above)
-				}
+				} else if(it + 2 == my_n) gate_to_tile(bufnn);
 				// sub-tile (it, 1): next is (it+1, 0) in the next buffer (harmless stale data after the last tile)
 				stage(ic<0>{}, off_next, mask_rd + kt1 * mask_stride, off_cur, ic<1>{}, kt1, ic<1>{}, bufn * SLOT_BYTES, 0, 0, 0, kt1);
 				if(!BIAS_LATE) load_bias_frags(kt2, ic<0>{});
@@ -1358,7 +1376,7 @@ static size_t lds_bytes(const af3_dpa_params& p) {
 	const size_t writers  = SPLIT ? 1 : KS2 ? NW / 2 : NW;  // wavefronts that own a block of query rows
 	constexpr size_t NBUF = KSL == 1 ? 5 : KSL ? 4 : 3;  // (as in the kernel)
 	return (size_t)(SPLIT ? NW : 1) * 2 * NBUF * KT * DP * 2 + (BMODE >= 2 ? (KS2 ? NW / 2 : NW) * NBUF * bias_slot_bytes(BMODE) : 0) + (n_ktiles * KT + 64) * 4 + n_ktiles * 2 + 16 +
-		   (p.gate ? writers * 32 * DP * 2 : 0);
+		   (p.gate && !(DP == 32 && NW == 4 && !SPLIT && KSL == 0) ? writers * 32 * DP * 2 : 0);  // (GATE_IN_TILE)
 }
 
 template <int DP, int NW, bool L2DOM, int BMODE, bool SPLIT = false, int KSL = 0>
