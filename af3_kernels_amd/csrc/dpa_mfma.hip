@@ -134,7 +134,9 @@ constexpr int bias_slot_bytes(int bmode) { return bmode == 3 ? 4096 + 128 : 4096
 // stage's LDS operands can be fetched at the end of the stage before), so that the NW computing ones never stand still behind a load that the
 // compute unit's load path has not taken in yet.  Requires NW even, no SPLIT, not FUSED.  (KSL = 1.  KSL = 2: the four
 // loading wavefronts and the ring of four tiles for workgroups of NW wavefronts with a query block each -- the form that
-// single rows of head_dim 48 or 64 take.)
+// long single rows of head_dim 56 or 64 take.  KSL = 3: pairs at head_dim up to 48 padded to 64, eight of them and four loading
+// wavefronts in the 168 registers of three wavefronts per SIMD: three contraction chunks instead of four, P.V at the end of its own
+// stage, a ring of four tiles.)
 // FUSED: the grid-attention variant.  One workgroup = one (batch, head); q, k, v and the gate are not
 // read from memory but projected in the kernel from the input rows x[b] (C channels) with the four
 // weight matrices of this head, K and V of ALL keys stay in LDS for the whole workgroup, and each
@@ -145,13 +147,15 @@ template <int DP, int NW, bool L2DOM, int BMODE, bool SPLIT, bool FUSED, int KSL
 // results to ordinary VGPRs instead of AGPRs, which every softmax operand would have to be copied out of;
 // the key-split variants are limited to fewer than 2 wavefronts per SIMD by their LDS buffers anyway)
 __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdgpu_waves_per_eu(FUSED ? (NW <= 4 ? 3 : (NW + 3) / 4) : KSL ? (NW + 7) / 4 : DP == 32 && !SPLIT ? (L2DOM ? 4 : 3) : 2))) dpa_mfma_bf16_kernel(af3_dpa_params p, int n_qtiles, int64_t n_groups, fused_grid_args fa) {
-	constexpr int NC         = DP / 16;            // contraction chunks of QK^T
+	constexpr int NC         = KSL == 3 ? 3 : DP / 16;  // contraction chunks of QK^T (KSL == 3: head_dim up to 48)
 	constexpr int NDB        = DP / 32;            // 32-row blocks of O^T
 	constexpr int CPR        = DP / 8;             // 16-byte chunks per K/V row
 	constexpr int TILE_BYTES = KT * DP * 2;
 	constexpr int NI         = TILE_BYTES / 1024;  // 1 KB wave loads per tile and tensor
 	constexpr int RPI        = 512 / DP;           // tile rows covered by one wave load
-	constexpr bool KS2       = KSL == 1;           // pairs of wavefronts on shared tiles (with loading wavefronts)
+	constexpr bool KS2       = KSL == 1 || KSL == 3;  // pairs of wavefronts on shared tiles (with loading wavefronts)
+	constexpr bool OPS_AHEAD = KSL == 1;           // ... that fetch a stage's LDS operands at the end of the stage before (KSL == 3: a ring of four)
+	constexpr bool PV_LATE   = KSL == 3;           // P.V of a sub-tile closes its own stage (its V^T fragments and packed probabilities are not carried over: registers)
 	constexpr bool LOADERS   = KSL != 0;           // four more wavefronts issue the tile loads (KSL == 2: one computing wavefront per query block)
 	constexpr int QT         = SPLIT ? 32 : KS2 ? NW * 16 : NW * 32;
 	constexpr int  LDS_SETS   = SPLIT ? NW : 1;  // private K/V buffer sets
@@ -162,7 +166,7 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 	// tile buffers of the K/V ring and slots of a bias ring.  With loading wavefronts the loads run two tiles ahead; KS2 in
 	// addition has every tile in LDS one barrier before its first use, so that a stage's LDS operands are fetched at the end of
 	// the stage before it (AHEAD: the tile that has landed when iteration j passes its barrier is j + AHEAD).
-	constexpr int  AHEAD      = KS2 ? 2 : 1;
+	constexpr int  AHEAD      = OPS_AHEAD ? 2 : 1;
 	constexpr int  NBUF       = LOADERS ? AHEAD + 3 : 3;
 	constexpr int  RING_BYTES = BRING ? (KS2 ? NW / 2 : NW) * NBUF * SLOT_BYTES : 0;  // (KS2: one ring per pair of wavefronts)
 	constexpr int  MASK_BASE  = LDS_SETS * 2 * NBUF * TILE_BYTES + RING_BYTES;
@@ -984,7 +988,7 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 		// k_next / mask_next_addr / ring_next (KS2): where the operands of the stage after this one are; ring_kt: the tile whose bias the ring slot read here holds
 		auto stage = [&](auto subn_c, int k_off, int mask_addr_next, int v_off, auto subc_c, int bias_kt, auto bias_sub_c, int ring_off, int k_next, int mask_next_addr, int ring_next, int ring_kt) {
 			constexpr int SUBN = decltype(subn_c)::value, SUBC = decltype(subc_c)::value, FB = 2 * SUBN;
-			if constexpr(!KS2) fetch_operands(subn_c, k_off, mask_addr_next, ring_off, ring_kt);
+			if constexpr(!OPS_AHEAD) fetch_operands(subn_c, k_off, mask_addr_next, ring_off, ring_kt);
 			maskA[0] = mask_next;
 			u32x4  pcur[2];
 			f32x16 sn;
@@ -996,21 +1000,25 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 #define AF3_CHUNK_END() __builtin_amdgcn_sched_barrier(0)
 			AF3_CHUNK_END();
 			// O^T += V^T . P^T of the previous sub-tile, exp2 of this one
+			if constexpr(!PV_LATE) {
 #pragma unroll
-			for(int db = 0; db < NDB; db++)
-				oacc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vprev[0][db]), __builtin_bit_cast(bf16x8, pprev[0]), oacc[db], 0, 0, 0);
+				for(int db = 0; db < NDB; db++)
+					oacc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vprev[0][db]), __builtin_bit_cast(bf16x8, pprev[0]), oacc[db], 0, 0, 0);
+			}
 			exp_part(sc, pcur, ic<0>{}, ic<2>{});
 			AF3_CHUNK_END();
+			if constexpr(!PV_LATE) {
 #pragma unroll
-			for(int db = 0; db < NDB; db++)
-				oacc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vprev[1][db]), __builtin_bit_cast(bf16x8, pprev[1]), oacc[db], 0, 0, 0);
+				for(int db = 0; db < NDB; db++)
+					oacc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vprev[1][db]), __builtin_bit_cast(bf16x8, pprev[1]), oacc[db], 0, 0, 0);
+			}
 			exp_part(sc, pcur, ic<2>{}, ic<2>{});
 			AF3_CHUNK_END();
 			// S^T of the next sub-tile
 			sn = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, kf[0]), qf[0], sn, 0, 0, 0);
 			// V^T fragments of this sub-tile for the next stage's PV product: issued as soon as the two PV
 			// MFMAs above have consumed the previous fragments, a whole stage before their use
-			read_vfrags(v_off, SUBC);
+			if constexpr(!PV_LATE) read_vfrags(v_off, SUBC);
 			exp_part(sc, pcur, ic<4>{}, ic<2>{});
 			AF3_CHUNK_END();
 			sn = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, kf[1]), qf[1], sn, 0, 0, 0);
@@ -1034,7 +1042,8 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 			AF3_CHUNK_END();
 #undef AF3_CHUNK_END
 			rowsum_mfma(pcur[1]);
-			if constexpr(KS2) fetch_operands(subn_c, k_next, mask_next_addr, ring_next, ring_kt);  // (this stage's have been consumed)
+			if constexpr(PV_LATE) read_vfrags(v_off, SUBC);
+			if constexpr(OPS_AHEAD) fetch_operands(subn_c, k_next, mask_next_addr, ring_next, ring_kt);  // (this stage's have been consumed)
 			// The running sum stays below L * 2^REF_SLACK <= 2^25 while every probability respects the
 			// reference, so this also catches a single probability near or beyond the limit (inf, NaN).  A sum that is still
 			// zero (log2 variant: leading sub-tiles of dropped keys, or live logits so far below the initial reference that
@@ -1047,8 +1056,16 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 				rowsum_mfma(pcur[1]);
 			}
 			sc       = sn;
-			pprev[0] = pcur[0];
-			pprev[1] = pcur[1];
+			if constexpr(PV_LATE) {
+#pragma unroll
+				for(int cp = 0; cp < 2; cp++)
+#pragma unroll
+					for(int db = 0; db < NDB; db++)
+						oacc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vprev[cp][db]), __builtin_bit_cast(bf16x8, pcur[cp]), oacc[db], 0, 0, 0);
+			} else {
+				pprev[0] = pcur[0];
+				pprev[1] = pcur[1];
+			}
 		};
 
 		// ---- which live tiles this wavefront walks: all of them, or every NW-th one when splitting ----
@@ -1088,7 +1105,7 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 			if constexpr(KS2) {
 				const int kt1_first = __builtin_amdgcn_readfirstlane(live_at(1));
 				load_bias_frags(kt1_first, ic<0>{});                                                // this wavefront's next sub-tile is in the next tile
-				fetch_operands(ic<0>{}, TILE_BYTES, mask_rd + kt1_first * mask_stride, SLOT_BYTES, kt1_first);  // operands of the first stage: second tile of the walk, buffer 1
+				if constexpr(OPS_AHEAD) fetch_operands(ic<0>{}, TILE_BYTES, mask_rd + kt1_first * mask_stride, SLOT_BYTES, kt1_first);  // operands of the first stage: second tile of the walk, buffer 1
 			} else if(BIAS_LATE) load_bias_frags(kt0, ic<1>{});
 			else if(my_n > 1) load_bias_frags(__builtin_amdgcn_readfirstlane(live_at(1)), ic<0>{});
 
@@ -1107,11 +1124,11 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 					// reads issued, from the buffer of tile it+1) may stay in flight.  LDS reads return in issue order.  (The counter
 					// also counts scalar memory loads, which do not: this relies on the loop holding none -- every kernel argument
 					// is in registers before the loop, and the compiler has no reason to fetch one again while none is spilled.)
-					constexpr int OPERAND_READS = NC + 1 + (BRING ? RAGGED ? 4 : 2 : 0);
+					constexpr int OPERAND_READS = OPS_AHEAD ? NC + 1 + (BRING ? RAGGED ? 4 : 2 : 0) : 0;
 					asm volatile("s_waitcnt lgkmcnt(%0)\n\ts_barrier" ::"n"(OPERAND_READS) : "memory");
 					const int kt3_v = live_at(it + 3);  // (behind the barrier, which would wait for this read)
 					stage(ic<0>{}, bufn * TILE_BYTES, mask_rd + kt1 * mask_stride, buf * TILE_BYTES, ic<0>{}, kt2, ic<0>{}, bufn * SLOT_BYTES, bufnn * TILE_BYTES, mask_rd + kt2 * mask_stride,
-						  bufnn * SLOT_BYTES, kt2);
+						  bufnn * SLOT_BYTES, OPS_AHEAD ? kt2 : kt1);
 					buf = bufn;
 					kt  = kt1;
 					kt1 = kt2;
@@ -1156,6 +1173,7 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 			}
 		}
 		// the last sub-tile's PV product
+		if constexpr(!PV_LATE)
 #pragma unroll
 		for(int cp = 0; cp < 2; cp++)
 #pragma unroll
@@ -1372,7 +1390,7 @@ constexpr size_t LDS_LIMIT = 160 * 1024;  // per workgroup on gfx950
 template <int DP, int NW, int BMODE, bool SPLIT, int KSL = 0>
 static size_t lds_bytes(const af3_dpa_params& p) {
 	const size_t n_ktiles = (size_t)((p.L + KT - 1) / KT);
-	constexpr bool   KS2  = KSL == 1;
+	constexpr bool   KS2  = KSL == 1 || KSL == 3;
 	const size_t writers  = SPLIT ? 1 : KS2 ? NW / 2 : NW;  // wavefronts that own a block of query rows
 	constexpr size_t NBUF = KSL == 1 ? 5 : KSL ? 4 : 3;  // (as in the kernel)
 	return (size_t)(SPLIT ? NW : 1) * 2 * NBUF * KT * DP * 2 + (BMODE >= 2 ? (KS2 ? NW / 2 : NW) * NBUF * bias_slot_bytes(BMODE) : 0) + (n_ktiles * KT + 64) * 4 + n_ktiles * 2 + 16 +
@@ -1381,7 +1399,7 @@ static size_t lds_bytes(const af3_dpa_params& p) {
 
 template <int DP, int NW, bool L2DOM, int BMODE, bool SPLIT = false, int KSL = 0>
 static int launch_one(const af3_dpa_params& p, hipStream_t s) {
-	constexpr int QT       = SPLIT ? 32 : KSL == 1 ? NW * 16 : NW * 32;
+	constexpr int QT       = SPLIT ? 32 : KSL == 1 || KSL == 3 ? NW * 16 : NW * 32;
 	const int     n_qtiles = (int)((p.L + QT - 1) / QT);
 	const int64_t n_groups = p.B * p.H;
 	const int64_t blocks   = ((n_groups + 7) / 8) * 8 * n_qtiles;
@@ -1485,7 +1503,9 @@ static int launch_nw(const af3_dpa_params& p, hipStream_t s) {
 		//   a pair per workgroup           7.0    8.5   18.6   22.1   36.9   41.7
 		//   two pairs on shared tiles      7.5    9.2   11.0   13.4   27.7   31.3
 		//   one wavefront per block, x 4   8.3   11.6   14.9   18.1   21.3   24.6
-		// (Pairs and the last form have four loading wavefronts.  Four pairs at head_dim 48 do not fit in LDS.)
+		//   four pairs (KSL 3)                                        19.5   21.3
+		// (Pairs and the one-per-block form have four loading wavefronts.  With the registers of the other pairs' form -- four
+		// contraction chunks, P.V a stage late -- four pairs at head_dim 48 spilled 18 registers: 32.5 us at L = 1536.)
 		const int64_t wg64 = groups * ((p.L + 63) / 64), wg128 = groups * ((p.L + 127) / 128);
 		if constexpr(DP == 32) {
 			if(blocks1 <= 256 && ktiles >= 4 && lds_bytes<DP, 4, BMODE, true>(p) <= LDS_LIMIT) return launch_one<DP, 4, L2DOM, BMODE, true>(p, s);
@@ -1494,6 +1514,9 @@ static int launch_nw(const af3_dpa_params& p, hipStream_t s) {
 		if(wg64 <= 256 && lds_bytes<DP, 4, BMODE, false, 1>(p) <= LDS_LIMIT) return launch_one<DP, 4, L2DOM, BMODE, false, 1>(p, s);
 		if constexpr(DP == 32) {
 			if(wg128 <= 256 && lds_bytes<DP, 8, BMODE, false, 1>(p) <= LDS_LIMIT) return launch_one<DP, 8, L2DOM, BMODE, false, 1>(p, s);
+		}
+		if constexpr(DP == 64 && BMODE >= 2) {
+			if(p.D <= 48 && wg128 <= 256 && lds_bytes<DP, 8, BMODE, false, 3>(p) <= LDS_LIMIT) return launch_one<DP, 8, L2DOM, BMODE, false, 3>(p, s);
 		}
 		if(wg128 <= 256 && lds_bytes<DP, 4, BMODE, false, 2>(p) <= LDS_LIMIT) return launch_one<DP, 4, L2DOM, BMODE, false, 2>(p, s);
 		return launch_one<DP, 4, L2DOM, BMODE>(p, s);

@@ -24,7 +24,8 @@ def f32np(t):
     (16, 513, 48, 1, 0),                                          # two pairs, head_dim padded to 64
     (16, 515, 24, 1, 1),                                          # pairs on shared tiles, four computing wavefronts
     (16, 1027, 24, 0, 0), (16, 1024, 24, 7, 1),                   # ... eight
-    (16, 1027, 48, 0, 1),                                         # loading wavefronts, one query block each
+    (16, 1027, 48, 0, 1), (16, 1032, 40, 0, 0), (16, 1090, 48, 6, 0),   # eight, head_dim up to 48 padded to 64, P.V in its own stage
+    (16, 1027, 56, 0, 1), (16, 1032, 64, 0, 0),                   # loading wavefronts, one query block each
     (16, 2051, 24, 0, 0), (16, 2050, 48, 1, 0),                   # four wavefronts that load for themselves
 ])
 def test_single_row_bias_at_any_address(af3, oracle, H, L, D, pad, first):
