@@ -4,6 +4,8 @@
 // (src/csrc/xsmm_functors.h:139-145, :838-885).  The e4m3 path has no reference behaviour to
 // follow (src/csrc/xsmm_functors.h:218-226 asserts "not implemented"); it implements OCP e4m3fn
 // with round-to-nearest-even and saturation, which is what gfx950's v_cvt_pk_fp8_f32 does.
+#include <algorithm>
+
 #include "common.hpp"
 
 namespace af3 {
@@ -480,9 +482,11 @@ extern "C" int af3_quantize_qkv_fp8_e4m3(const void* q, const void* k, const voi
 	qa.dst_lo[0] = static_cast<uint8_t*>(q_lo), qa.dst_lo[1] = static_cast<uint8_t*>(k_lo), qa.dst_lo[2] = nullptr;
 	qa.rows = B * H * L, qa.cols = D, qa.rows_per_matrix = L, qa.v_row_stride = v8t_row_stride;
 	qa.pre_scale[0] = q_pre_scale, qa.pre_scale[1] = qa.pre_scale[2] = 1.f;
-	// (quantise: a thread of the dense paths takes 8 elements per trip; two trips per thread, so that the three tensors'
-	// workgroups -- each of which first folds its tensor's partial maxima -- are all resident at once for the usual sizes)
-	const dim3 ga(AMAX3_BLOCKS, 3), gq(ew_blocks(n / 32, 1024), 3);
+	// (quantise: a thread of the dense paths takes 8 elements per trip.  One trip per thread up to two workgroups per compute unit
+	// and tensor -- few elements in few workgroups of four trips each took 4.7 us --, four trips beyond, so that the three tensors'
+	// workgroups, each of which first folds its tensor's partial maxima, are all resident at once for the usual sizes)
+	const int64_t qb = ew_blocks(n / 32, 1024);
+	const dim3    ga(AMAX3_BLOCKS, 3), gq((unsigned)(qb >= 512 ? qb : std::min<int64_t>(ew_blocks(n / 8, 1024), 512)), 3);
 	if(sd == AF3_F32) {
 		hipLaunchKernelGGL(amax3_kernel<false>, ga, dim3(EW_THREADS), 0, s, aa, scratch);
 		hipLaunchKernelGGL(quantize3_kernel<false>, gq, dim3(EW_THREADS), 0, s, qa, scratch, descales);
