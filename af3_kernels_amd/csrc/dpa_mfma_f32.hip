@@ -32,8 +32,8 @@
 // extreme magnitude take the exact form: products alone, maximum, rescaling.
 //
 // Semantics are the reference harness's (examples/dot_product_attention.py:20-43): a dropped key's
-// logit is replaced by -1e9 (its bias is; products up to 64 vanish beside it), so its weight is exactly 0 unless every key of the row is dropped, in
-// which case the row is the mean of V; keys past L weigh 0.
+// finished logit is replaced by -1e9, whatever its K row and bias hold, so its weight is exactly 0 unless every key of the row is
+// dropped, in which case the row is the mean of V; keys past L weigh 0.
 #include "mfma_helpers.hpp"
 
 namespace af3 {
@@ -41,7 +41,7 @@ namespace {
 
 constexpr int   F32_KT    = 32;         // keys per tile
 constexpr int   F32_MAX_L = 16384;      // tile words and tile list live in LDS
-constexpr float DROPPED   = -1.0e9f;    // what masked_fill puts in a dropped key's place
+constexpr float DROPPED   = -1.0e9f * LOG2E;   // what masked_fill puts in a dropped key's place, in log2 units
 constexpr float F32_FLOOR = -3.0e38f;   // a logit of -inf counts as this, so that a tile of such keys leaves a finite maximum
 constexpr float FAST_MAX  = 0x1p20f;    // largest |reference| the fast form takes
 
@@ -80,7 +80,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DP
 	const int       n_tiles   = (int)((p.L + F32_KT - 1) / F32_KT);
 	uint32_t* const live_bits = reinterpret_cast<uint32_t*>(smem + 4 * KS * TILE);
 	int16_t* const  live_list = reinterpret_cast<int16_t*>(live_bits + n_tiles);
-	__shared__ int  s_nlive, s_all;
+	__shared__ int  s_nlive;
 
 	// workgroup -> (batch row, head, query tile); consecutive workgroups go round the 8 XCDs, so the
 	// query tiles of one (b, h) are kept on one XCD and share its L2 copy of K and V
@@ -202,15 +202,14 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DP
 			if(keepit) live_list[cnt + rank] = (int16_t)kt;
 			cnt += __builtin_popcountll(bal);
 		}
-		if(lane == 0) s_nlive = cnt, s_all = any ? 0 : 1;
+		if(lane == 0) s_nlive = cnt;
 	}
 	__syncthreads();
-	const int  nlive       = __builtin_amdgcn_readfirstlane(s_nlive);
-	const bool all_dropped = __builtin_amdgcn_readfirstlane(s_all) != 0;
+	const int nlive = __builtin_amdgcn_readfirstlane(s_nlive);
 
 	u32x4 qf[3][NC];
 	{
-		const float qmul = all_dropped ? 0.f : p.softmax_scale * LOG2E;  // (all dropped: products of exactly 0, so that every logit is exactly the same)
+		const float qmul = p.softmax_scale * LOG2E;
 #pragma unroll
 		for(int c = 0; c < NC; c++)
 #pragma unroll
@@ -221,9 +220,9 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DP
 				qf[0][c][e] = hi, qf[1][c][e] = mid, qf[2][c][e] = lo;
 			}
 	}
-	// ... with DROPPED in the place of a dropped key's bias: the tile's word of live keys is wave-uniform, register i's condition
+	// DROPPED in the place of a dropped key's finished logit: the tile's word of live keys is wave-uniform, register i's condition
 	// is two of its bits, one per half-wave
-	auto drop_keys = [&](int kt, f32x4 (&bs)[4]) {
+	auto drop_keys = [&](int kt, f32x16& s) {
 		const uint32_t live  = (uint32_t)__builtin_amdgcn_readfirstlane((int)live_bits[kt]);
 		const int      past  = (int)((int64_t)(kt + 1) * F32_KT - L);          // keys of this tile that lie past L
 		const uint32_t in    = past > 0 ? 0xffffffffu >> past : 0xffffffffu;  // (past < 32)
@@ -233,9 +232,9 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DP
 		for(int i = 0; i < 16; i++) {
 			const int      k0   = 8 * (i / 4) + i % 4;
 			const uint64_t cond = (uint64_t)(uint32_t)((int)(kept << (31 - k0)) >> 31) | (uint64_t)(uint32_t)((int)(kept << (31 - (k0 + 4))) >> 31) << 32;
-			float          x    = bs[i / 4][i % 4];
+			float          x    = s[i];
 			asm("v_cndmask_b32 %0, %1, %2, %3" : "=v"(x) : "v"(DROPPED), "v"(x), "s"(cond));
-			bs[i / 4][i % 4] = x;
+			s[i] = x;
 		}
 	};
 
@@ -313,16 +312,16 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DP
 	bool exact_only = false;  // (wave-uniform)
 	// the probabilities of a tile in the exact form, moving the reference to the running maximum
 	auto exact_probabilities = [&](int kt, int buf, f32x4 (&bs)[4]) -> f32x16 {
-		drop_keys(kt, bs);
 		f32x16 s;
 #pragma unroll
 		for(int i = 0; i < 16; i++) s[i] = 0.f;
 		s = products(buf, s);
+#pragma unroll
+		for(int i = 0; i < 16; i++) s[i] = fmaxf(__builtin_fmaf(bs[i / 4][i % 4], LOG2E, s[i]), F32_FLOOR);
+		drop_keys(kt, s);
 		float mx = -INFINITY;
 #pragma unroll
 		for(int i = 0; i < 16; i++) {
-			const float bi = bs[i / 4][i % 4];
-			s[i] = fmaxf(__builtin_fmaf(bi, LOG2E, s[i]), F32_FLOOR);
 			if((int64_t)kt * F32_KT + 8 * (i / 4) + 4 * half + i % 4 >= L) s[i] = -INFINITY;
 			mx = fmaxf(mx, s[i]);
 		}
@@ -358,11 +357,11 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DP
 			f32x16 pr;
 			bool   exact = FIRST || exact_only;
 			if(!exact) {
-				drop_keys(kt, bias_t);
 #pragma unroll
 				for(int i = 0; i < 16; i++) pr[i] = __builtin_fmaf(bias_t[i / 4][i % 4], LOG2E, -m_run);
 				fetch_bias(ktn, bias_t);
 				pr = products(buf * KS + ks, pr);
+				drop_keys(kt, pr);  // (|m_run| is at most FAST_MAX: weight 0)
 				float psum = 0.f;
 #pragma unroll
 				for(int i = 0; i < 16; i++) {

@@ -249,3 +249,26 @@ def test_glu_whole_row_stores(af3, M, K, N):
         a, b = (x[rows].float() @ w.float()).chunk(2, dim=-1)
         want = torch.nn.functional.silu(a) * b
         assert (out[rows].float() - want).abs().max() <= 2 ** -7 * want.abs().max()
+
+
+FP32_FORMS = [(1, 2, 97, 32), (5, 4, 385, 32), (16, 4, 385, 32), (3, 4, 161, 64), (33, 8, 131, 32), (40, 8, 97, 64), (3, 2, 95, 20)]   # (every launch form of the fp32 kernel)
+
+
+@pytest.mark.parametrize("B,H,L,D", FP32_FORMS)
+@pytest.mark.parametrize("garbage", [1e10, -1e10, 1e30, float("inf"), float("nan")])
+def test_fp32_dropped_keys_are_replaced_whatever_they_hold(af3, oracle, B, H, L, D, garbage):
+    """masked_fill replaces the finished logit of a dropped key: what K holds there has no weight, in tiles with and without live
+    keys; a batch row without any live key is the mean of V."""
+    g = torch.Generator().manual_seed(L + D)
+    q, k, v = (torch.randn(B, H, L, D, generator=g) for _ in range(3))
+    bias = torch.randn(H, L, L, generator=g)
+    keep = torch.rand(B, L, generator=g) < 0.7
+    keep[:, L - 1] = True
+    keep[0, 40:70] = False
+    if B > 1:
+        keep[1] = False
+    dirty = torch.where(keep[:, None, :, None], k, torch.tensor(garbage))
+    out = af3.dot_product_attention_cpp(q.cuda(), dirty.cuda(), v.cuda(), keep.cuda(), bias.cuda())
+    torch.cuda.synchronize()
+    want = oracle.dpa_formula(f32np(q), f32np(k), f32np(v), keep.numpy(), f32np(bias))
+    assert np.abs(f32np(out) - want).max() <= 2e-5
