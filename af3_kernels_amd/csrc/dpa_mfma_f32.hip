@@ -5,11 +5,14 @@
 // Products of fp32 numbers on the bf16 matrix instructions.  An fp32 number is the exact sum of three bf16 numbers --
 // hi = bf16(x), mid = bf16(x - hi), lo = bf16(x - hi - mid), 3 x 8 significant bits -- and of the nine products of two such
 // sums the six largest are kept (hi.hi, hi.mid, mid.hi, mid.mid, hi.lo, lo.hi), accumulated in fp32; the three dropped ones
-// are below 2^-23 of the product (the scheme is published: Henry, Tang, Heinecke, "Leveraging the bfloat16 artificial
+// are below 2^-23 of the product where the fp32 instructions' is exact (the scheme is published: Henry, Tang, Heinecke, "Leveraging the bfloat16 artificial
 // intelligence datatype for higher-precision computations", 2019).  v_mfma_f32_32x32x16_bf16 multiplies 16-deep in 32
 // clocks where v_mfma_f32_32x32x2_f32 multiplies 2-deep in 64: six products cost 3/8 of the fp32 instructions' time.
-// Errors against fp64, unit-variance inputs (2 x 4 x 768 x 32): rms 4.4e-8, largest 7.7e-7; with the fp32 instructions it was
-// 5.3e-8 and 1.1e-6 (fewer, deeper instructions round the accumulator less often).
+// Errors against 64 bits, relative 2-norm, this form / the fp32 instructions, over 2..64 x 4 x 64..768 x 32, head_dim 4..64 and
+// 1 x 4 x 2000 x 32: unit-variance inputs 1.6e-7..4.3e-7 / 2.2e-7..8.2e-7, q times 16 3.9e-7..9.5e-7 / 4.6e-7..1.3e-6, biases
+// times 10 1.6e-7..2.3e-7 / 1.9e-7..3.8e-7, biases that grow by 40 along the row 2.1e-7..5.4e-7 / 3.0e-7..5.2e-7 (fewer, deeper
+// instructions round the accumulator less often).  Rows whose biases carry an offset of some hundreds or thousands: 0.14 to 1.41
+// times the fp32 instructions', by where the offset lies between two powers of two in either domain.
 // Measured (64 x 4 x 768 x 32): 234 us with the fp32 instructions (53 % of their peak), 131 us in this form.
 //
 // Same transposed formulation as the bf16 kernel: S^T[key][q] = K.Q^T, so that in the 32x32
@@ -24,9 +27,10 @@
 // the split of 16 probabilities per lane), so four wavefronts per SIMD (128 registers) overlap the two; 64 x 4 x 768 x 32 runs
 // 0.9 PFLOP/s of bf16 instructions, two thirds of what a large bf16 matrix product reaches.
 //
-// The logit is s + bias, in log2 units (q carries the factor).  The products accumulate on top of fma(bias, log2 e, -m), m
-// the row's softmax reference: bias and reference cancel in one rounding before any product joins them, so a row whose
-// biases carry an offset keeps its precision, and p = exp2(accumulator).  The reference is
+// The logit is s + bias, in log2 units (q carries the factor).  p = exp2(fma(bias, log2 e, -m) + s), m the row's softmax
+// reference: bias and reference cancel in one rounding before the finished products join them, so a row whose biases carry
+// an offset keeps its precision.  (Products accumulated on top of bias minus reference are rounded at that magnitude, up to 30
+// where the reference is left behind, once per matrix instruction: up to four times the error at the same speed.)  The reference is
 // the running maximum of the first tile; later tiles only check that their row sums have not run away from it (optimistic
 // softmax).  A tile that fails the check, the first tile, and every tile of a wavefront that holds a reference of
 // extreme magnitude take the exact form: products alone, maximum, rescaling.
@@ -360,7 +364,12 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DP
 #pragma unroll
 				for(int i = 0; i < 16; i++) pr[i] = __builtin_fmaf(bias_t[i / 4][i % 4], LOG2E, -m_run);
 				fetch_bias(ktn, bias_t);
-				pr = products(buf * KS + ks, pr);
+				f32x16 s;
+#pragma unroll
+				for(int i = 0; i < 16; i++) s[i] = 0.f;
+				s = products(buf * KS + ks, s);
+#pragma unroll
+				for(int i = 0; i < 16; i++) pr[i] += s[i];
 				drop_keys(kt, pr);  // (|m_run| is at most FAST_MAX: weight 0)
 				float psum = 0.f;
 #pragma unroll
