@@ -33,7 +33,8 @@
 // where the reference is left behind, once per matrix instruction: up to four times the error at the same speed.)  The reference is
 // the running maximum of the first tile; later tiles only check that their row sums have not run away from it (optimistic
 // softmax).  A tile that fails the check, the first tile, and every tile of a wavefront that holds a reference of
-// extreme magnitude take the exact form: products alone, maximum, rescaling.
+// extreme magnitude take the exact form: products alone, maximum, rescaling.  Infinities and NaN do not survive the split
+// into terms: where a result is not finite the wavefront repeats its walk on the fp32 matrix instructions.
 //
 // Semantics are the reference harness's (examples/dot_product_attention.py:20-43): a dropped key's
 // finished logit is replaced by -1e9, whatever its K row and bias hold, so its weight is exactly 0 unless every key of the row is
@@ -314,14 +315,13 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DP
 		}
 	};
 	bool exact_only = false;  // (wave-uniform)
-	// the probabilities of a tile in the exact form, moving the reference to the running maximum
-	auto exact_probabilities = [&](int kt, int buf, f32x4 (&bs)[4]) -> f32x16 {
-		f32x16 s;
+	// the probabilities of a tile, from its products s, in the exact form, moving the reference to the running maximum
+	auto exact_probabilities = [&](int kt, f32x16 s, const f32x4 (&bs)[4]) -> f32x16 {
 #pragma unroll
-		for(int i = 0; i < 16; i++) s[i] = 0.f;
-		s = products(buf, s);
-#pragma unroll
-		for(int i = 0; i < 16; i++) s[i] = fmaxf(__builtin_fmaf(bs[i / 4][i % 4], LOG2E, s[i]), F32_FLOOR);
+		for(int i = 0; i < 16; i++) {
+			s[i] = __builtin_fmaf(bs[i / 4][i % 4], LOG2E, s[i]);
+			s[i] = s[i] < F32_FLOOR ? F32_FLOOR : s[i];  // (NaN stays)
+		}
 		drop_keys(kt, s);
 		float mx = -INFINITY;
 #pragma unroll
@@ -382,7 +382,9 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DP
 			}
 			if(exact) {  // (wave-uniform)
 				if(!FIRST) fetch_bias(kt, bias_t);  // (once more)
-				pr = exact_probabilities(kt, buf * KS + ks, bias_t);
+#pragma unroll
+				for(int i = 0; i < 16; i++) pr[i] = 0.f;
+				pr = exact_probabilities(kt, products(buf * KS + ks, pr), bias_t);
 				float psum = 0.f;
 #pragma unroll
 				for(int i = 0; i < 16; i++) psum += pr[i];
@@ -397,6 +399,62 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DP
 	};
 	step(ic<1>{}, 0);
 	for(int j = 1; j < n_steps; j++) step(ic<0>{}, j);
+	// What is needed from here on comes from its sources once more, out of the compiler's sight: kept from the start, arguments and
+	// row numbers cost the loop above ten registers, and a fourth wavefront per SIMD.
+	typedef __attribute__((address_space(4))) const af3_dpa_params kernarg;
+	kernarg* a  = (kernarg*)__builtin_amdgcn_kernarg_segment_ptr();  // (p is the first argument)
+	int      ln = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+	asm volatile("" : "+s"(a));
+	asm volatile("" : "+v"(ln));
+	const int     on = ln & 31, ohalf = ln >> 5;
+	const int64_t orow = (int64_t)qtile * (NQ * 32) + wblk * 32 + on;
+
+	// ---- something is not finite: an infinity or NaN in the inputs (its bf16 terms are an infinity and NaN, and their products
+	// are NaN where the formula has an infinity or a weight of zero), a value that rounds up to one, a sum that overflows under a
+	// reference left behind.  This wavefront walks its tiles once more, alone, with the fp32 matrix instructions on
+	// operands straight from memory and the exact form throughout: what then is not finite is so in the formula. ----
+	float finite = l_run * 0.f;  // (0, or NaN)
+#pragma unroll
+	for(int db = 0; db < NDB; db++)
+#pragma unroll
+		for(int i = 0; i < 16; i++) finite = __builtin_fmaf(oacc[db][i], 0.f, finite);
+	if(__ballot(!(finite == 0.f))) {
+		m_run = -INFINITY, l_run = 0.f;
+#pragma unroll
+		for(int db = 0; db < NDB; db++)
+#pragma unroll
+			for(int i = 0; i < 16; i++) oacc[db][i] = 0.f;
+		const int          cols = (int)a->D, k_bytes = (int)(a->k_stride[2] * 4), v_bytes = (int)(a->v_stride[2] * 4);
+		const float        scale = a->softmax_scale * LOG2E;
+		const float* const qp = static_cast<const float*>(a->q) + b * a->q_stride[0] + h * a->q_stride[1] + (orow < a->L ? orow : 0) * a->q_stride[2];
+#pragma unroll 1
+		for(int j = ks; j < nlive; j += KS) {
+			kt = tile_at(j);
+			fetch_bias(kt, bias_t);
+			f32x16 pr;
+#pragma unroll
+			for(int i = 0; i < 16; i++) pr[i] = 0.f;
+#pragma unroll 1
+			for(int t = 0; t < DP / 2; t++) {  // A: K[key n][d], B: q[row n][d] of column d = t + DP / 2 half
+				const int   d  = t + DP / 2 * ohalf;
+				const float kx = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(k_rsrc, d < cols ? (kt * F32_KT + on) * k_bytes + d * 4 : 0x40000000, 0, 0));
+				const float qx = d < cols ? qp[d] * scale : 0.f;
+				pr = __builtin_amdgcn_mfma_f32_32x32x2f32(kx, qx, pr, 0, 0, 0);
+			}
+			pr = exact_probabilities(kt, pr, bias_t);
+#pragma unroll
+			for(int i = 0; i < 16; i++) {  // A: V[key of register i][column n], B: its probability
+				l_run += pr[i];
+#pragma unroll
+				for(int db = 0; db < NDB; db++) {
+					const int   col = 32 * db + on;
+					const float vx  = __uint_as_float(
+						__builtin_amdgcn_raw_buffer_load_b32(v_rsrc, col < cols ? (kt * F32_KT + 8 * (i / 4) + 4 * ohalf + i % 4) * v_bytes + col * 4 : 0x40000000, 0, 0));
+					oacc[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(vx, pr[i], oacc[db], 0, 0, 0);
+				}
+			}
+		}
+	}
 	if constexpr(KS > 1) {
 		// ---- merge the partial results of the KS wavefronts of a query block (the tile buffers are dead) ----
 		float* const mred = reinterpret_cast<float*>(smem);           // [NW][32] references
@@ -433,17 +491,18 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DP
 	// ---- epilogue: O^T register i of block db is head column 32*db + 8*(i/4) + 4*half + i%4 ----
 	const float l_tot = l_run + other_half(l_run);
 	const float inv   = 1.f / l_tot;
-	if(row_ok) {
-		float* op = static_cast<float*>(p.out) + b * p.out_stride[0] + h * p.out_stride[1] + qrow * p.out_stride[2];
+	if(orow < a->L) {
+		float* const       op = static_cast<float*>(a->out) + b * a->out_stride[0] + h * a->out_stride[1] + orow * a->out_stride[2];
+		const float* const gp = a->gate ? static_cast<const float*>(a->gate) + b * a->gate_stride[0] + h * a->gate_stride[1] + orow * a->gate_stride[2] : nullptr;
 #pragma unroll
 		for(int db = 0; db < NDB; db++)
 #pragma unroll
 			for(int r4 = 0; r4 < 4; r4++) {
-				const int d0 = 32 * db + 8 * r4 + 4 * half;
-				if(d0 < D) {
+				const int d0 = 32 * db + 8 * r4 + 4 * ohalf;
+				if(d0 < a->D) {
 					float4 w = {oacc[db][4 * r4] * inv, oacc[db][4 * r4 + 1] * inv, oacc[db][4 * r4 + 2] * inv, oacc[db][4 * r4 + 3] * inv};
-					if(p.gate) {  // out *= sigmoid(gate)
-						const float4 g = *reinterpret_cast<const float4*>(static_cast<const float*>(p.gate) + b * p.gate_stride[0] + h * p.gate_stride[1] + qrow * p.gate_stride[2] + d0);
+					if(gp) {  // out *= sigmoid(gate)
+						const float4 g = *reinterpret_cast<const float4*>(gp + d0);
 						w.x *= sigmoidf_fast(g.x), w.y *= sigmoidf_fast(g.y), w.z *= sigmoidf_fast(g.z), w.w *= sigmoidf_fast(g.w);
 					}
 					*reinterpret_cast<float4*>(op + d0) = w;

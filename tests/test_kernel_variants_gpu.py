@@ -291,3 +291,40 @@ def test_fp32_biases_join_finished_products(af3, B, H, L, D, kind, bound):
     s = (q.double() @ k.double().transpose(-1, -2).contiguous()) * D ** -0.5 + bias.double()
     want = s.masked_fill(~keep[:, None, None, :], -1e9).softmax(-1) @ v.double()
     assert (out.double() - want).norm() <= bound * want.norm()
+
+
+@pytest.mark.parametrize("B,H,L,D", FP32_FORMS)
+@pytest.mark.parametrize("kind", ["k+inf", "k-inf", "k nan", "q inf", "v+inf", "v both", "v huge", "v ramp", "bias+inf"])
+def test_fp32_infinities_act_as_in_the_formula(af3, B, H, L, D, kind):
+    """Infinities and NaN of live keys: the logit or sum they make in the formula, NaN rows where that has NaN, every other row and
+    column as without them.  Finite values beyond bf16's largest, and sums that only overflow under a reference left behind, stay finite."""
+    g = torch.Generator().manual_seed(L + D)
+    q, k, v = (torch.randn(B, H, L, D, generator=g) for _ in range(3))
+    bias = torch.randn(H, L, L, generator=g)
+    keep = torch.rand(B, L, generator=g) < 0.8
+    j, j2 = L // 2, L - 1                       # keys of two tiles, both live
+    keep[:, [j, j2]] = True
+    inf, b, h = float("inf"), B - 1, H - 1
+    if kind[0] == "k":
+        k[b, h, j, 1] = {"k+inf": inf, "k-inf": -inf, "k nan": float("nan")}[kind]
+    elif kind == "q inf":
+        q[b, h, 3, 2] = inf
+    elif kind == "bias+inf":
+        bias[h, 5, j] = inf
+    elif kind == "v ramp":
+        v *= 1e35
+        bias += torch.linspace(0.0, 20.0, L)
+    else:
+        v[b, h, j, 1] = inf if kind != "v huge" else 3.4e38
+        if kind == "v both":
+            v[b, h, j2, 1] = -inf
+    print("case", B, H, L, D, kind, flush=True)
+    out = af3.dot_product_attention_cpp(q.cuda(), k.cuda(), v.cuda(), keep.cuda(), bias.cuda()).cpu()
+    s = (q.double() @ k.double().transpose(-1, -2)) * D ** -0.5 + bias.double()
+    want = s.masked_fill(~keep[:, None, None, :], -1e9).softmax(-1) @ v.double()
+    assert torch.equal(out.isnan(), want.isnan()) and torch.equal(out.isinf(), want.isinf())
+    assert torch.equal(out[out.isinf()] > 0, want[want.isinf()] > 0)
+    assert bool(out.isfinite().all()) == (kind in ("v huge", "v ramp"))
+    ok = want.isfinite()
+    size = v.double().abs().where(v.isfinite(), torch.zeros((), dtype=torch.float64)).amax(2, keepdim=True).clamp(min=1.0).expand_as(want)
+    assert ((out.double() - want).abs()[ok] <= 2e-5 * size[ok]).all()
