@@ -560,7 +560,8 @@ bool mfma_f32_eligible(const af3_dpa_params& p) {
 	if(p.bias && p.bias_dtype != AF3_F32) return false;
 	if(p.D > 64 || p.D % 4 != 0 || p.L > F32_MAX_L) return false;
 	// buffer addressing of one (batch row, head) slab uses 32-bit byte offsets
-	if(p.L * p.k_stride[2] * 4 >= 0x40000000LL || p.L * p.v_stride[2] * 4 >= 0x40000000LL || (p.bias && p.L * p.bias_stride[1] * 4 >= 0x7ff00000LL)) return false;
+	const int64_t rows = (p.L + F32_KT - 1) / F32_KT * F32_KT;  // (those of the last tile that lie past L among them)
+	if(rows * p.k_stride[2] * 4 >= 0x40000000LL || rows * p.v_stride[2] * 4 >= 0x40000000LL || (p.bias && p.L * p.bias_stride[1] * 4 >= 0x7ff00000LL)) return false;
 	if(p.gate && ((reinterpret_cast<uintptr_t>(p.gate) & 15) || p.gate_stride[0] % 4 || p.gate_stride[1] % 4 || p.gate_stride[2] % 4)) return false;
 	const void* ptrs[4] = {p.q, p.k, p.v, p.out};
 	for(const void* ptr : ptrs)

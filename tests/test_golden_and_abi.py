@@ -131,6 +131,12 @@ def test_kernel_selection_is_host_only_and_follows_alignment():
     assert sel(ctypes.byref(_params(io_dtype=0, mma_dtype=0, out_dtype=0, bias_dtype=0))) == 3   # fp32 storage -> fp32 MFMA
     assert sel(ctypes.byref(_params(io_dtype=0, mma_dtype=0, out_dtype=0, bias_dtype=0, k=0x2004))) == 0   # rows not 16-byte aligned
     assert sel(ctypes.byref(_params(io_dtype=0, mma_dtype=0, out_dtype=0, bias_dtype=0, force_generic=1))) == 0
+    # rows of the last tile that lie past L: their offsets, too, must fit the 32 bits of the fp32 kernel's loads
+    wide = (ctypes.c_int64 * 3)(0, 0, 50_000_000)
+    fp32 = dict(io_dtype=0, mma_dtype=0, out_dtype=0, bias_dtype=0)
+    assert sel(ctypes.byref(_params(L=5, k_stride=wide, **fp32))) == 0 and sel(ctypes.byref(_params(L=5, v_stride=wide, **fp32))) == 0
+    wide = (ctypes.c_int64 * 3)(0, 0, 8_000_000)
+    assert sel(ctypes.byref(_params(L=5, k_stride=wide, v_stride=wide, **fp32))) == 3
     assert sel(ctypes.byref(_params(L=-1))) == -3
 
 
