@@ -4,9 +4,11 @@ There is no fallback: if the library is missing, loading raises and every op fai
 """
 import ctypes
 import os
+import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libaf3_dpa.so")
+HOST_PATH = os.path.join(_HERE, "_host.so")
 
 AF3_F32, AF3_BF16, AF3_FP8_E4M3, AF3_FP8_E5M2 = 0, 1, 2, 3
 ABI_VERSION = 4
@@ -90,16 +92,30 @@ def load():
     return _lib
 
 
-class _MissingHost:
-    def __getattr__(self, name):
-        raise ImportError(f"{os.path.join(_HERE, '_host.so')} is missing: build it with `python -m af3_kernels_amd.build`.")
+class _Host:
+    """The native host side of the entry points (csrc/host.cpp), looked for when it is first needed: a package that is built after
+    its import works from then on.  While `_host.so` alone is missing every call is answered None, which sends it to the Python
+    implementation (a warning says so, once); without the kernels' library a call raises, as load() does."""
+    FUSED_WEIGHT, Q_BIAS_ROW, OUT_PROJ_T, GLU_T = 1, 2, 3, 4   # as in host.cpp
+    _warned = False
+
+    def __getattr__(self, name):   # (reached until the module's functions are in this object)
+        load()
+        if os.path.exists(HOST_PATH):
+            import torch  # noqa: F401 -- its libraries must be loaded first
+            from . import _host
+            self.__dict__.update((k, v) for k, v in vars(_host).items() if not k.startswith("__"))
+            return getattr(_host, name)
+        if not _Host._warned:
+            _Host._warned = True
+            warnings.warn(f"{HOST_PATH} is missing: calls are prepared in Python, which takes 10 to 40 us more each; build it with `python -m af3_kernels_amd.build`", RuntimeWarning)
+        return lambda *args: None
 
 
 def load_host():
-    """The native host side of the entry points (csrc/host.cpp).  A package that has not been built yet can still be imported
-    (to build it); the first call then says what is missing."""
-    if not os.path.exists(os.path.join(_HERE, "_host.so")):
-        return _MissingHost()
+    """The native host side where it is built already (its functions are then the module's own), else a stand-in that finds it later."""
+    if not (os.path.exists(HOST_PATH) and os.path.exists(LIB_PATH)):
+        return _Host()
     load()
     import torch  # noqa: F401 -- its libraries must be loaded first
     from . import _host

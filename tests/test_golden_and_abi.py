@@ -482,3 +482,50 @@ def test_traffic_digest_follows_the_code_and_not_its_commentary():
         text = open(os.path.join(ROOT, "profiles", fname)).read()
         assert "kernel_code_sha256: " + digest in text, f"profiles/{fname} was collected with other kernel code: re-collect the counters"
         assert bench.measured_traffic_bytes(name) > 0
+
+
+def test_a_package_built_after_its_import_works(tmp_path):
+    """Import, build, call in one process (what `python __graft_entry__.py smoke` does on a fresh checkout), and a package whose native host
+    side did not build: its calls are prepared in Python."""
+    import shutil
+    import subprocess
+    import sys
+    pkg = os.path.join(ROOT, "af3_kernels_amd")
+    (tmp_path / "af3_kernels_amd").mkdir()
+    for f in os.listdir(pkg):
+        if f.endswith(".py"):
+            shutil.copy(os.path.join(pkg, f), tmp_path / "af3_kernels_amd")
+    program = f"""
+import os, warnings
+import torch
+import af3_kernels_amd as af3
+from af3_kernels_amd import ops
+q = torch.zeros(1, 1, 4, 8)
+w = torch.zeros(8, 8)
+calls = (lambda: af3.dot_product_attention_cpp(q, q, q, None, None), lambda: af3.dot_product_attention_fp8(q, q, q, None, None), lambda: af3.gated_linear_unit_cpp(q, w),
+         lambda: af3.self_attention_cpp(q[0, 0], None, None, w, w, w, w, w, 1))
+def answers():
+    out = []
+    for call in calls:
+        try:
+            call()
+            out.append("none")
+        except (ImportError, RuntimeError) as e:
+            out.append(type(e).__name__ + (": device" if "device tensors" in str(e) else ""))
+    return set(out)
+assert answers() == {{"ImportError"}}, answers()
+here = os.path.dirname(af3.__file__)
+with warnings.catch_warnings(record=True) as seen:
+    warnings.simplefilter("always")
+    os.symlink({os.path.join(pkg, "libaf3_dpa.so")!r}, os.path.join(here, "libaf3_dpa.so"))
+    assert answers() == {{"RuntimeError: device"}}, answers()
+    assert len(seen) == 1 and "_host.so" in str(seen[0].message)
+import shutil
+shutil.copy({os.path.join(pkg, "_host.so")!r}, here)
+assert answers() == {{"RuntimeError: device"}}, answers()
+assert type(vars(ops._host)["attention"]).__name__ == "builtin_function_or_method"
+from af3_kernels_amd import _host
+assert all(getattr(ops._host, n) == getattr(_host, n) for n in ("FUSED_WEIGHT", "Q_BIAS_ROW", "OUT_PROJ_T", "GLU_T"))
+"""
+    r = subprocess.run([sys.executable, "-c", program], cwd=tmp_path, capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
