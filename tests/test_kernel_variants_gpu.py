@@ -328,3 +328,15 @@ def test_fp32_infinities_act_as_in_the_formula(af3, B, H, L, D, kind):
     ok = want.isfinite()
     size = v.double().abs().where(v.isfinite(), torch.zeros((), dtype=torch.float64)).amax(2, keepdim=True).clamp(min=1.0).expand_as(want)
     assert ((out.double() - want).abs()[ok] <= 2e-5 * size[ok]).all()
+
+
+@pytest.mark.parametrize("generic", [False, True])
+def test_output_gate_in_float32(af3, generic):
+    """sigmoid of gates from 5 to 18 (times 1): half an ulp of 1 + e is 2^-24, of the quotient 2^-25, and what the exponential is off by stays
+    below 0.04 * 2^-24 there.  (A reciprocal good to one ulp: 1.66 * 2^-24.)"""
+    from af3_kernels_amd import ops
+    gate = torch.linspace(5, 18, 4096 * 32, device="cuda").view(1, 1, 4096, 32)
+    one = torch.ones_like(gate)
+    out = ops._dpa_forward_impl(one, one, one, None, None, ops._DTYPE_CODE[torch.float32], generic, gate=gate)
+    torch.cuda.synchronize()
+    assert (out.double() - torch.sigmoid(gate.double())).abs().max() <= 1.54 * 2 ** -24
