@@ -72,6 +72,12 @@ SYMBOLS = {
     "af3_abi_version": (ctypes.c_int, []),
 }
 
+# ... and those that only this package's two host sides call (not part of the ABI)
+INTERNAL_SYMBOLS = {
+    "af3_project_suits": (ctypes.c_int, [i64, i64, i64]),
+    "af3_project": (ctypes.c_int, [vp, vp, vp, vp, i64, i64, i64, i32, vp]),
+}
+
 _lib = None
 
 
@@ -83,7 +89,7 @@ def load():
                 f"{LIB_PATH} is missing: build it with `python -m af3_kernels_amd.build` (hipcc, gfx950). "
                 "There is no CPU or PyTorch fallback for these ops.")
         lib = ctypes.CDLL(LIB_PATH)
-        for name, (res, args) in SYMBOLS.items():
+        for name, (res, args) in (SYMBOLS | INTERNAL_SYMBOLS).items():
             fn = getattr(lib, name)
             fn.restype, fn.argtypes = res, args
         if lib.af3_abi_version() != ABI_VERSION:

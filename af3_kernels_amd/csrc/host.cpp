@@ -14,6 +14,7 @@
 
 #include <ATen/core/Tensor.h>
 #include <ATen/hip/EmptyTensor.h>
+#include <ATen/ops/clone.h>
 #include <ATen/ops/linear.h>
 #include <ATen/ops/matmul.h>
 #include <c10/hip/HIPCachingAllocator.h>
@@ -280,9 +281,10 @@ int attend(const Tensor& y, int64_t B, int64_t N, int64_t head, const key_mask& 
 Tensor project(const Tensor& x, int64_t M, const Tensor& weight, const Tensor* row, int dev, int& rc) {
 	const int64_t K = weight.size(1), N = weight.size(0);
 	rc = AF3_OK;
-	if(x.scalar_type() == at::kBFloat16 && weight.is_contiguous() && af3_project_suits(M, N, K) && reinterpret_cast<uintptr_t>(x.const_data_ptr()) % 16 == 0) {
-		Tensor y = new_tensor({M, N}, at::kBFloat16, dev);
-		rc = af3_project(x.const_data_ptr(), weight.const_data_ptr(), row ? row->const_data_ptr() : nullptr, y.data_ptr(), M, N, K, 0, current_stream(dev));
+	if(x.scalar_type() == at::kBFloat16 && weight.is_contiguous() && af3_project_suits(M, N, K)) {
+		const Tensor rows = reinterpret_cast<uintptr_t>(x.const_data_ptr()) % 16 == 0 ? x : x.clone();
+		Tensor       y    = new_tensor({M, N}, at::kBFloat16, dev);
+		rc = af3_project(rows.const_data_ptr(), weight.const_data_ptr(), row ? row->const_data_ptr() : nullptr, y.data_ptr(), M, N, K, 0, current_stream(dev));
 		return y;
 	}
 	return at::linear(x.dim() == 2 ? x : x.reshape({M, K}), weight, row ? *row : Tensor());

@@ -135,10 +135,21 @@ def _check_weights(C: int, head: int, ws):
 
 
 def _project(rows: torch.Tensor, ws, q_bias: Optional[torch.Tensor], head: int) -> torch.Tensor:
-    """Stage 1: [rows, C] . [C, 4C] -> per token and head (k | v | q | gate).  The q bias of the diffusion op
-    rides the GEMM's epilogue."""
+    """Stage 1: [rows, C] . [C, 4C] -> per token and head (k | v | q | gate).  The diffusion op, whose q bias is added on the way,
+    takes this library's kernel by the rule of the native host side (the same bits whichever prepares the call); a library GEMM otherwise."""
     W = _fused_weight(ws, head, rows.dtype)
-    return torch.nn.functional.linear(rows, W, None if q_bias is None else _q_bias_row(q_bias, head, rows.dtype))
+    if q_bias is None:
+        return torch.nn.functional.linear(rows, W)
+    row = _q_bias_row(q_bias, head, rows.dtype)
+    lib, (M, K), N = _lib.load(), rows.shape, W.shape[0]
+    if rows.dtype == torch.bfloat16 and lib.af3_project_suits(M, N, K):
+        if not rows.is_contiguous() or rows.data_ptr() % 16:
+            rows = rows.clone(memory_format=torch.contiguous_format)
+        y = torch.empty(M, N, dtype=rows.dtype, device=rows.device)
+        with ops._on_device(rows.device):
+            _lib.check(lib.af3_project(rows.data_ptr(), W.data_ptr(), row.data_ptr(), y.data_ptr(), M, N, K, 0, ops._stream_ptr(rows.device)), "af3_project")
+        return y
+    return torch.nn.functional.linear(rows, W, row)
 
 
 def _attend(y: torch.Tensor, B: int, N: int, head: int, mask, bias) -> torch.Tensor:

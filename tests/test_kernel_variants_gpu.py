@@ -340,3 +340,22 @@ def test_output_gate_in_float32(af3, generic):
     out = ops._dpa_forward_impl(one, one, one, None, None, ops._DTYPE_CODE[torch.float32], generic, gate=gate)
     torch.cuda.synchronize()
     assert (out.double() - torch.sigmoid(gate.double())).abs().max() <= 1.54 * 2 ** -24
+
+
+@pytest.mark.parametrize("S,N,C,head", [(1, 48, 128, 4), (1, 64, 384, 16), (1, 200, 384, 16), (5, 300, 768, 16), (1, 130, 96, 4), (1, 2048, 768, 16)])
+def test_self_attention_has_the_same_bits_on_every_route(af3, S, N, C, head):
+    """The first call on a set of weights, later ones, a mask that is not bool, tokens that are not contiguous or not aligned: prepared by the native host side
+    or in Python, the same kernels (among the shapes: products that this library computes and one it leaves to the library GEMM)."""
+    g = torch.Generator(device="cuda").manual_seed(N)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda", dtype=torch.bfloat16)
+    x = r(N, C) if S == 1 else r(S, N, C)
+    ws = [af3.vnni_repack_tensor(r(C, C) * C ** -0.5, 2, C // head) for _ in range(4)]
+    qb, bias, mask = r(C), r(head, N, N), torch.rand(N, generator=g, device="cuda") < 0.9
+    call = lambda x, mask: af3.self_attention_cpp(x, mask, bias, ws[0], qb, ws[1], ws[2], ws[3], head)
+    first = call(x, mask)
+    assert torch.equal(first, call(x, mask))
+    assert torch.equal(first, call(x, mask.float()))
+    assert torch.equal(first, call(torch.cat([x, x], -1)[..., :C], mask))
+    odd = torch.empty(x.numel() + 1, device="cuda", dtype=torch.bfloat16)[1:].view(x.shape).copy_(x)   # off a 16-byte boundary
+    if S * N * 4 * C * C <= 6e9 and C % 64 == 0:   # (a library GEMM may choose by the address)
+        assert torch.equal(first, call(odd, mask)) and torch.equal(first, call(odd, mask.float()))
