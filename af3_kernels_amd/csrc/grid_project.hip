@@ -44,8 +44,8 @@ struct grid_project_args {
 	int64_t         x_stride_i, x_stride_j;   // elements
 	const uint16_t *gamma, *beta, *wb;        // [128], [128], [4, 128]
 	const uint32_t* w[4];                     // k, v, q, gate: weight^T in panel layout [head][64][32][2]
-	uint16_t*       out[4];                   // k, v, q, gate: [B, 4, N, 32]
-	uint16_t*       bias;                     // [4, n_i, n_j]
+	uint16_t*       out[4];                   // k, v, q, gate: [B, 4, N, 32] (null: the bias alone)
+	uint16_t*       bias;                     // [4, n_i, n_j] (null: the projections alone)
 	int             n_i, n_j, turned, split;
 	float           eps, q_scale;
 };
@@ -58,7 +58,7 @@ __global__ void __launch_bounds__(GP_WAVES * 64) __attribute__((amdgpu_waves_per
 	const int      blocks_per_row = (a.n_j + 31) / 32;
 	const int64_t  n_blocks = (int64_t)a.n_i * blocks_per_row;
 	// split: this workgroup projects for head blockIdx % 4 alone (a quarter of the weights, four times the workgroups per block)
-	const int      h0 = a.split ? (int)(blockIdx.x & 3) : 0, h1 = a.split ? h0 + 1 : 4;
+	const int      h0 = a.split ? (int)(blockIdx.x & 3) : 0, h1 = a.split ? h0 + 1 : a.out[0] ? 4 : 0;
 	const int      wgs = a.split ? (int)(gridDim.x >> 2) : (int)gridDim.x, wg = a.split ? (int)(blockIdx.x >> 2) : (int)blockIdx.x;
 	const int64_t  step = (int64_t)wgs * GP_WAVES;
 	int64_t        u = (int64_t)wave * wgs + wg;   // (first one block per workgroup, then two, ...)
@@ -142,7 +142,7 @@ __global__ void __launch_bounds__(GP_WAVES * 64) __attribute__((amdgpu_waves_per
 		if(u + step < n_blocks) load(u + step);   // (under way during this block's products)
 
 		// ---- pair bias: every row of the operand is one of the four heads', so that every lane has all four values of its token ----
-		if(h0 == 0) {
+		if(h0 == 0 && a.bias) {
 			f32x16 acc;
 #pragma unroll
 			for(int k = 0; k < 16; k++) acc[k] = 0.f;
@@ -204,11 +204,13 @@ __global__ void __launch_bounds__(GP_WAVES * 64) __attribute__((amdgpu_waves_per
 using namespace af3;
 
 // For the Python entry points' native host side (host.cpp); not part of the ABI.  pair [n_i, n_j, 128] (strides in elements), ln_weight,
-// ln_bias [128], proj [4, 128], q/k/v/gate weights in panel layout, all bf16; outputs as in the kernel.
+// ln_bias [128], proj [4, 128], q/k/v/gate weights in panel layout, all bf16; outputs as in the kernel (q, k, v and gate, or bias, may be null).
 extern "C" int af3_grid_project(const void* pair, const int64_t* pair_stride, const void* ln_weight, const void* ln_bias, float eps, const void* proj, const void* wq, const void* wk, const void* wv,
 								const void* wg, int64_t n_i, int64_t n_j, int32_t turned, float q_scale, void* q, void* k, void* v, void* gate, void* bias, void* stream) {
-	for(const void* p : {pair, ln_weight, ln_bias, proj, wq, wk, wv, wg, (const void*)q, (const void*)k, (const void*)v, (const void*)gate, (const void*)bias})
+	for(const void* p : {pair, ln_weight, ln_bias, proj, wq, wk, wv, wg})
 		if(!p) return AF3_ERR_NULL_POINTER;
+	const bool projected = q && k && v && gate;
+	if(!projected && (!bias || q || k || v || gate)) return AF3_ERR_NULL_POINTER;
 	if(n_i <= 0 || n_j <= 0 || n_i > (1 << 20) || n_j > (1 << 20) || n_i * ((n_j + 31) / 32) >= ((int64_t)1 << 31)) return AF3_ERR_BAD_SHAPE;
 	for(const void* p : {pair, ln_weight, ln_bias, proj})
 		if(reinterpret_cast<uintptr_t>(p) & 15) return AF3_ERR_BAD_ARGUMENT;
@@ -226,7 +228,7 @@ extern "C" int af3_grid_project(const void* pair, const int64_t* pair_stride, co
 	const int64_t blocks = n_i * ((n_j + 31) / 32);
 	// Few blocks (up to three of the twelve wavefronts of every compute unit): a workgroup per head, which shares the products among four times the
 	// wavefronts and loads a quarter of the weights.
-	a.split = blocks <= 64 * GP_WAVES ? 1 : 0;
+	a.split = projected && blocks <= 64 * GP_WAVES ? 1 : 0;
 	const int64_t wgs = a.split ? 4 * (blocks < 64 ? blocks : 64) : blocks < 256 ? blocks : 256;
 	if(hipFuncSetAttribute(reinterpret_cast<const void*>(grid_project_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, GP_LDS) != hipSuccess) return AF3_ERR_LAUNCH;
 	hipLaunchKernelGGL(grid_project_kernel, dim3((unsigned)wgs), dim3(GP_WAVES * 64), GP_LDS, static_cast<hipStream_t>(stream), a);

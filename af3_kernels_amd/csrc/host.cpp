@@ -477,33 +477,63 @@ PyObject* py_layernorm_pair_bias(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 // LayerNorm, pair bias and projections in one kernel (128 channels in 4 heads, bfloat16), then the attention launch on q, k, v and the
-// gate [B, 4, N, 32]: into `gated` [B, N, C]; 1 where this form does not take the tensors.
+// gate [B, 4, N, 32] and the output projection.
 bool grid_projected_ok(const ln_args& r, const Tensor* const (&ws)[4]) {
 	const auto odd = [](const Tensor* t, int to) { return reinterpret_cast<uintptr_t>(t->const_data_ptr()) % to != 0; };
 	return r.pair->size(2) == 128 && r.proj->size(0) == 4 && r.pair->scalar_type() == at::kBFloat16 && r.pair->stride(0) % 8 == 0 && r.pair->stride(1) % 8 == 0 && !odd(r.pair, 16) &&
 		   !odd(r.gamma, 16) && !odd(r.beta, 16) && !odd(r.proj, 16) && !odd(ws[0], 4) && !odd(ws[1], 4) && !odd(ws[2], 4) && !odd(ws[3], 4);
 }
-int grid_projected(const ln_args& r, const key_mask& m, const Tensor* const (&ws)[4], bool turned, int64_t hint, bool exact, Tensor& gated, int dev) {
-	const int64_t n_i = r.pair->size(0), n_j = r.pair->size(1), B = turned ? n_j : n_i, N = turned ? n_i : n_j, each = n_i * n_j * 128;
-	const at::DataPtr mem = new_scratch((4 * each + 4 * n_i * n_j) * 2);
-	auto* const       q = static_cast<uint16_t*>(mem.get());
-	uint16_t *const   k = q + each, *const v = k + each, *const gate = v + each, *const bias = gate + each;
-	gated = new_tensor({B, N, 128}, at::kBFloat16, dev);
-	af3_dpa_params p = block(B, 4, N, 32, AF3_BF16, hint);
-	p.q = q, p.k = k, p.v = v, p.gate = gate, p.out = gated.data_ptr(), p.bias = bias;
-	const int64_t st[3] = {4 * N * 32, N * 32, 32}, so[3] = {N * 128, 32, 128};
-	for(int i = 0; i < 3; i++) p.q_stride[i] = p.k_stride[i] = p.v_stride[i] = p.gate_stride[i] = st[i], p.out_stride[i] = so[i];
-	p.bias_stride[0] = n_i * n_j, p.bias_stride[1] = n_j, p.bias_dtype = AF3_BF16;
-	p.key_mask = m.ptr, p.key_mask_stride_b = m.stride;
-	const at::DataPtr work = workspace_for(p, exact);
-	// The whole scale of the logits goes into q where it is projected, in fp32: one rounding.  What is left for the attention
-	// kernel is 1 in its own units (a product with it gives the same bits back).
-	const float log2e = 1.4426950408889634f, q_scale = af3_dpa_log2_domain(&p) ? p.softmax_scale * log2e : p.softmax_scale;
-	p.softmax_scale = q_scale == p.softmax_scale ? 1.f : 1.f / log2e;
+// Where the memory for q, k, v and the gate of the whole call is not there, they go in slabs of batch rows of at most 256 MB, after a
+// pass over the whole pair tensor for the bias, which every slab needs (N = 640 414 -> 488 us, 1024 1316 -> 1450).
+constexpr int64_t GRID_SLAB_BYTES = (int64_t)256 << 20;
+int grid_projected_rows(const ln_args& r, const key_mask& m, const Tensor* const (&ws)[4], bool turned, int64_t hint, bool exact, const Tensor& out_weight, int64_t rows, Tensor& out, int dev) {
+	const int64_t n_i = r.pair->size(0), n_j = r.pair->size(1), B = turned ? n_j : n_i, N = turned ? n_i : n_j, each = rows * N * 128;
+	const bool    whole = rows == B;
+	at::DataPtr   mem = new_scratch((4 * each + 4 * n_i * n_j) * 2), rows_out = new_scratch(each * 2);
+	auto* const     q = static_cast<uint16_t*>(mem.get());
+	uint16_t *const k = q + each, *const v = k + each, *const gate = v + each, *const bias = gate + each;
+	if(!whole) out = new_tensor({B, N, 128}, at::kBFloat16, dev);
 	const int64_t ps[2] = {r.pair->stride(0), r.pair->stride(1)};
-	const int     rc = af3_grid_project(r.pair->const_data_ptr(), ps, r.gamma->const_data_ptr(), r.beta->const_data_ptr(), r.eps, r.proj->const_data_ptr(), ws[0]->const_data_ptr(),
-										ws[1]->const_data_ptr(), ws[2]->const_data_ptr(), ws[3]->const_data_ptr(), n_i, n_j, turned, q_scale, q, k, v, gate, bias, current_stream(dev));
-	return rc != AF3_OK ? rc : af3_dpa_forward(&p, current_stream(dev));
+	const auto project_rows = [&](int64_t b0, int64_t count, float q_scale, bool with_rows, bool with_bias) {
+		const auto* x = static_cast<const uint16_t*>(r.pair->const_data_ptr()) + b0 * ps[turned ? 1 : 0];
+		return af3_grid_project(x, ps, r.gamma->const_data_ptr(), r.beta->const_data_ptr(), r.eps, r.proj->const_data_ptr(), ws[0]->const_data_ptr(), ws[1]->const_data_ptr(), ws[2]->const_data_ptr(),
+								ws[3]->const_data_ptr(), turned ? N : count, turned ? count : N, turned, q_scale, with_rows ? q : nullptr, with_rows ? k : nullptr, with_rows ? v : nullptr,
+								with_rows ? gate : nullptr, with_bias ? bias : nullptr, current_stream(dev));
+	};
+	int rc = whole ? AF3_OK : project_rows(0, B, 1.f, false, true);
+	for(int64_t b0 = 0; b0 < B && rc == AF3_OK; b0 += rows) {
+		const int64_t  count = B - b0 < rows ? B - b0 : rows;
+		af3_dpa_params p = block(count, 4, N, 32, AF3_BF16, hint);
+		p.q = q, p.k = k, p.v = v, p.gate = gate, p.out = rows_out.get(), p.bias = bias;
+		const int64_t st[3] = {4 * N * 32, N * 32, 32}, so[3] = {N * 128, 32, 128};
+		for(int i = 0; i < 3; i++) p.q_stride[i] = p.k_stride[i] = p.v_stride[i] = p.gate_stride[i] = st[i], p.out_stride[i] = so[i];
+		p.bias_stride[0] = n_i * n_j, p.bias_stride[1] = n_j, p.bias_dtype = AF3_BF16;
+		p.key_mask = m.ptr ? m.ptr + b0 * m.stride : nullptr, p.key_mask_stride_b = m.stride;
+		{
+			const at::DataPtr work = workspace_for(p, exact);
+			// The whole scale of the logits goes into q where it is projected, in fp32: one rounding.  What is left for the attention
+			// kernel is 1 in its own units (a product with it gives the same bits back).
+			const float log2e = 1.4426950408889634f, q_scale = af3_dpa_log2_domain(&p) ? p.softmax_scale * log2e : p.softmax_scale;
+			p.softmax_scale = q_scale == p.softmax_scale ? 1.f : 1.f / log2e;
+			rc = project_rows(b0, count, q_scale, true, whole);
+			if(rc == AF3_OK) rc = af3_dpa_forward(&p, current_stream(dev));
+		}
+		if(rc != AF3_OK) break;
+		if(whole) mem = at::DataPtr(), out = new_tensor({B, N, 128}, at::kBFloat16, dev);   // (the result may take the place of what is no longer needed)
+		rc = af3_linear(rows_out.get(), out_weight.const_data_ptr(), static_cast<uint16_t*>(out.data_ptr()) + b0 * N * 128, count * N, 128, out_weight.size(0), AF3_BF16, current_stream(dev));
+	}
+	return rc;
+}
+int grid_projected(const ln_args& r, const key_mask& m, const Tensor* const (&ws)[4], bool turned, int64_t hint, bool exact, const Tensor& out_weight, Tensor& out, int dev) {
+	const int64_t B = r.pair->size(turned ? 1 : 0), N = r.pair->size(turned ? 0 : 1), fit = GRID_SLAB_BYTES / (N * 1024) / 32 * 32;
+	const int64_t rows = fit < 32 ? 32 : fit;
+	if(rows < B) {
+		try {
+			return grid_projected_rows(r, m, ws, turned, hint, exact, out_weight, B, out, dev);
+		} catch(const c10::OutOfMemoryError&) {
+		}
+	}
+	return grid_projected_rows(r, m, ws, turned, hint, exact, out_weight, rows < B ? rows : B, out, dev);
 }
 
 // grid_block(pair, ln_weight, ln_bias, eps, proj_weight, mask, wq, wk, wv, wg, out_proj, head, transpose, least (batch row, head) pairs of
@@ -528,24 +558,24 @@ PyObject* py_grid_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
 	int    rc;
 	{
 		without_gil g;
-		Tensor normed, bias, gated;
-		const bool projected = grid_projected_ok(r, ws);
-		rc = projected ? grid_projected(r, m, ws, turned, hint, exact, gated, dev) : ln_pair_bias(r, normed, bias, dev);
-		if(rc == AF3_OK && !projected) {
-			const Tensor rows = turned ? normed.transpose(0, 1) : normed;
-			rc = B * head >= least && !exact ? grid_kernel(rows, m, &bias, ws, head, gated, dev) : 1;
-			if(rc == 1 && fused.defined()) {
-				const Tensor y = at::linear(rows.reshape({B * N, C}), fused);
-				if(y.scalar_type() == normed.scalar_type() && y.is_contiguous()) {
-					gated = new_tensor({B, N, C}, y.scalar_type(), dev);
-					rc    = attend(y, B, N, head, m, &bias, gated, hint, exact, dev);
+		if(grid_projected_ok(r, ws)) rc = grid_projected(r, m, ws, turned, hint, exact, out_weight, out, dev);
+		else {
+			Tensor normed, bias, gated;
+			rc = ln_pair_bias(r, normed, bias, dev);
+			if(rc == AF3_OK) {
+				const Tensor rows = turned ? normed.transpose(0, 1) : normed;
+				rc = B * head >= least && !exact ? grid_kernel(rows, m, &bias, ws, head, gated, dev) : 1;
+				if(rc == 1 && fused.defined()) {
+					const Tensor y = at::linear(rows.reshape({B * N, C}), fused);
+					if(y.scalar_type() == normed.scalar_type() && y.is_contiguous()) {
+						gated = new_tensor({B, N, C}, y.scalar_type(), dev);
+						rc    = attend(y, B, N, head, m, &bias, gated, hint, exact, dev);
+					}
 				}
 			}
+			if(rc == AF3_OK) rc = narrow_linear(gated, out_weight, out, dev);
 		}
-		if(rc == AF3_OK) {
-			rc = narrow_linear(gated, out_weight, out, dev);
-			if(turned && rc == AF3_OK) out = out.transpose(0, 1);
-		}
+		if(turned && rc == AF3_OK) out = out.transpose(0, 1);
 	}
 	return rc == 1 ? none() : answer(rc, std::move(out));
 	END_HANDLE_TH_ERRORS

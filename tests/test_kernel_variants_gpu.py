@@ -199,12 +199,8 @@ def test_fp8_bias_forms_and_tile_flags(af3, B, H, L, D, mask_kind, compensated):
     assert bool(((out.float() - want).abs() <= bound).all())
 
 
-@pytest.mark.parametrize("transpose", [False, True])
-@pytest.mark.parametrize("N", [1, 2, 31, 33, 64, 97, 150, 161, 200, 229, 330])
-def test_grid_block_projected_form(af3, N, transpose):
-    """The grid block (projections in one pass, attention, output projection) against the same steps in float32, with bf16 roundings where
-    the block stores bf16: partial token blocks, heads in separate workgroups and together, query tiles with idle wavefronts, gate rows of one to
-    four batch rows, both orientations."""
+def grid_block_case(af3, N, transpose):
+    """(module, pair, mask, its result in float32 with bf16 roundings where the block stores bf16)"""
     g = torch.Generator(device="cuda").manual_seed(N)
     mod = af3.GridSelfAttentionCpp(128, 4, transpose).to("cuda", torch.bfloat16).eval().requires_grad_(False)
     for name, p in mod.named_parameters():
@@ -214,11 +210,6 @@ def test_grid_block_projected_form(af3, N, transpose):
     keep[:, 0] = True
     if N > 2:
         keep[1] = False   # a row without any live key
-    print("case", N, transpose, flush=True)
-    out = mod(pair, keep)
-    again = mod(pair, keep)
-    torch.cuda.synchronize()
-    assert torch.equal(out, again)
     bf = lambda t: t.to(torch.bfloat16).float()
     f = lambda m: m.weight.float()
     x = bf(torch.nn.functional.layer_norm(pair.float(), (128,), f(mod.act_norm), mod.act_norm.bias.float(), mod.act_norm.eps))
@@ -232,8 +223,46 @@ def test_grid_block_projected_form(af3, N, transpose):
     want = torch.nn.functional.linear(bf(o.transpose(1, 2).reshape(N, N, 128)), f(mod.output_projection))
     if transpose:
         want = want.transpose(0, 1)
+    return mod, pair, keep, want
+
+
+@pytest.mark.parametrize("transpose", [False, True])
+@pytest.mark.parametrize("N", [1, 2, 31, 33, 64, 97, 150, 161, 200, 229, 330])
+def test_grid_block_projected_form(af3, N, transpose):
+    """The grid block (projections in one pass, attention, output projection) against the same steps in float32, with bf16 roundings where
+    the block stores bf16: partial token blocks, heads in separate workgroups and together, query tiles with idle wavefronts, gate rows of one to
+    four batch rows, both orientations."""
+    mod, pair, keep, want = grid_block_case(af3, N, transpose)
+    print("case", N, transpose, flush=True)
+    out = mod(pair, keep)
+    again = mod(pair, keep)
+    torch.cuda.synchronize()
+    assert torch.equal(out, again)
     err = (out.float() - want).abs()
     assert err.max() <= 3e-2 * max(1.0, float(want.abs().max())) and err.norm() <= 1e-2 * want.norm()
+
+
+@pytest.mark.parametrize("N,transpose", [(641, False), (700, False), (700, True)])
+def test_grid_block_where_memory_is_short(af3, N, transpose):
+    """The projections of the whole call take four times the pair tensor; where that is not there the block runs in slabs of batch
+    rows, in the memory of a result, a slab of 256 MB, its gated rows and a bias, with room for a rewritten bias."""
+    mod, pair, keep, want = grid_block_case(af3, N, transpose)
+    free = mod(pair, keep)
+    need = N * N * (256 + 8) + (256 << 20) * 5 // 4 + 4 * 4 * 704 ** 2 + (24 << 20)
+    assert need < N * N * (5 * 256 + 8)
+    want, free = want.cpu(), free.cpu()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    print("case", N, transpose, flush=True)
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + need) / total)
+    try:
+        out = mod(pair, keep).cpu()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    err = (out.float() - want).abs()
+    assert err.max() <= 3e-2 * max(1.0, float(want.abs().max())) and err.norm() <= 1e-2 * want.norm()
+    assert (out.float() - free.float()).norm() <= 4e-3 * want.norm()
 
 
 @pytest.mark.parametrize("M,K,N", [(1, 64, 32), (33, 128, 480), (65, 64, 544), (524289 + 31, 64, 256), (262145, 128, 544)])
