@@ -115,8 +115,8 @@ PyObject* answer(int rc, Tensor&& out) { return rc == AF3_OK ? wrap(std::move(ou
 
 // ---- matrices derived from weights ------------------------------------------------------------------------------------
 // Remembered for as long as their sources are the same live tensors at the same version, address and layout.  The weak
-// reference keeps a source's address from being handed to another tensor, so the address alone identifies it.  Bounded:
-// past MAX_DERIVED entries, and whenever a source has died, entries go.  Guarded by the GIL.
+// reference keeps a source's address from being handed to another tensor, so the address alone identifies it.  An entry goes with
+// its first source (fused.py hears of that and calls forget_source); past MAX_DERIVED entries all go.  Guarded by the GIL.
 constexpr size_t MAX_DERIVED = 1024;
 using derived_key = std::array<uintptr_t, 5>;   // what (tag), up to four sources
 struct key_hash {
@@ -162,12 +162,14 @@ const Tensor* derived_of(int64_t tag, PyObject* const* o, Py_ssize_t n) {
 	}
 	return &it->second.value;
 }
-// remember(tag, value, source...)
+// remember(tag, value, source...): True for a new entry, None where it is there already or the tensors cannot be remembered
 PyObject* py_remember(PyObject*, PyObject* const* a, Py_ssize_t n) {
 	HANDLE_TH_ERRORS
 	derived_key   k;
 	const Tensor* value = n >= 3 ? tensor_of(a[1]) : nullptr;
 	if(!value || !make_key(PyLong_AsLongLong(a[0]), a + 2, n - 2, k)) return none();
+	const Tensor* known = derived_of(PyLong_AsLongLong(a[0]), a + 2, n - 2);
+	if(known && known->is_same(*value)) return none();
 	for(auto it = g_derived->begin(); it != g_derived->end();) {
 		bool dead = false;
 		for(const source& s : it->second.sources) dead = dead || s.ref.expired();
@@ -181,8 +183,25 @@ PyObject* py_remember(PyObject*, PyObject* const* a, Py_ssize_t n) {
 		d.sources.push_back(source{c10::weak_intrusive_ptr<c10::TensorImpl>(t.getIntrusivePtr()), t.const_data_ptr(), (int64_t)t._version(), t.scalar_type(), t.sizes().vec(), t.strides().vec()});
 	}
 	(*g_derived)[k] = std::move(d);
-	return none();
+	Py_RETURN_TRUE;
 	END_HANDLE_TH_ERRORS
+}
+// recalls(tag, source...): whether a matrix is remembered for these
+PyObject* py_recalls(PyObject*, PyObject* const* a, Py_ssize_t n) {
+	HANDLE_TH_ERRORS
+	return PyBool_FromLong(n >= 2 && derived_of(PyLong_AsLongLong(a[0]), a + 1, n - 1) != nullptr);
+	END_HANDLE_TH_ERRORS
+}
+// forget_source(address of a source's TensorImpl, as Tensor._cdata gives it)
+PyObject* py_forget_source(PyObject*, PyObject* const* a, Py_ssize_t n) {
+	const uintptr_t source = n == 1 ? (uintptr_t)PyLong_AsUnsignedLongLong(a[0]) : 0;
+	if(PyErr_Occurred()) return nullptr;
+	for(auto it = g_derived->begin(); it != g_derived->end();) {
+		bool uses = false;
+		for(size_t i = 1; i < it->first.size(); i++) uses = uses || it->first[i] == source;
+		it = source && uses ? g_derived->erase(it) : std::next(it);
+	}
+	return none();
 }
 PyObject* py_forget(PyObject*, PyObject*) {
 	g_derived->clear();
@@ -618,6 +637,8 @@ PyMethodDef methods[] = {
 	AF3_FN(layernorm_pair_bias, "layernorm_pair_bias(pair, ln_weight, ln_bias, eps, proj_weight)"),
 	AF3_FN(gated_linear_unit, "gated_linear_unit(x, weight, tag)"),
 	AF3_FN(remember, "remember(tag, value, source...): a matrix derived from weights"),
+	AF3_FN(recalls, "recalls(tag, source...): whether one is remembered for these"),
+	AF3_FN(forget_source, "forget_source(address): drops what was derived from this tensor"),
 	{"forget", py_forget, METH_NOARGS, "forget(): drops every remembered matrix"},
 	{nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", "native host side of the entry points", -1, methods, nullptr, nullptr, nullptr, nullptr};

@@ -87,10 +87,31 @@ def clear_weight_cache() -> None:
         _host.forget()
 
 
-def _remember(what: int, head: int, dtype: torch.dtype, value: torch.Tensor, *sources) -> torch.Tensor:
-    """Leaves a matrix derived from weights where the native path of the next call finds it."""
-    _host.remember(what | head << 8 | ops._DTYPE_CODE[dtype] << 40, value, *sources)
+_SOURCES = {}   # address of a remembered matrix's source (its TensorImpl) -> weak reference to it
+
+
+def _source_died(address: int) -> None:
+    with _CACHE_LOCK:
+        _SOURCES.pop(address, None)
+        for k in [k for k, (refs, _, _) in list(_W_CACHE.items()) if any(r() is None for r in refs)]:
+            _W_CACHE.pop(k, None)
+        _host.forget_source(address)
+
+
+def _remember(tag: int, value: torch.Tensor, *sources) -> torch.Tensor:
+    """Leaves a matrix derived from weights where the native path of the next call finds it, until the first of its sources goes."""
+    if _host.remember(tag, value, *sources):
+        with _CACHE_LOCK:
+            for t in sources:
+                address = t._cdata
+                known = _SOURCES.get(address)
+                if known is None or known() is not t:
+                    _SOURCES[address] = weakref.ref(t, lambda _, address=address: _source_died(address))
     return value
+
+
+def _tag(what: int, head: int, dtype: torch.dtype) -> int:
+    return what | head << 8 | ops._DTYPE_CODE[dtype] << 40
 
 
 def _fused_weight(ws, head: int, dtype: torch.dtype) -> torch.Tensor:
@@ -103,7 +124,7 @@ def _fused_weight(ws, head: int, dtype: torch.dtype) -> torch.Tensor:
         K = C // head
         q, k, v, g = (_unpack_panels(w, head).to(dtype).view(C, head, K) for w in ws)
         return torch.stack((k, v, q, g), dim=2).reshape(C, 4 * C).t().contiguous()
-    return _remember(_host.FUSED_WEIGHT, head, dtype, _cached(tuple(ws), (head, dtype), make), *ws)
+    return _remember(_tag(_host.FUSED_WEIGHT, head, dtype), _cached(tuple(ws), (head, dtype), make), *ws)
 
 
 def _q_bias_row(q_bias: torch.Tensor, head: int, dtype: torch.dtype) -> torch.Tensor:
@@ -114,14 +135,12 @@ def _q_bias_row(q_bias: torch.Tensor, head: int, dtype: torch.dtype) -> torch.Te
         row = torch.zeros(head, 4, K, dtype=dtype, device=q_bias.device)
         row[:, 2] = q_bias.reshape(head, K).to(dtype)
         return row.view(4 * C)
-    return _remember(_host.Q_BIAS_ROW, head, dtype, _cached((q_bias,), (head, dtype, "q_bias"), make), q_bias)
+    return _remember(_tag(_host.Q_BIAS_ROW, head, dtype), _cached((q_bias,), (head, dtype, "q_bias"), make), q_bias)
 
 
 def _out_proj_t(out_proj: torch.Tensor) -> torch.Tensor:
     """The output projection in nn.Linear layout [out, in], left where the native path finds it."""
-    w = _cached((out_proj,), ("out_proj",), lambda: out_proj.t().contiguous())
-    _host.remember(_host.OUT_PROJ_T, w, out_proj)
-    return w
+    return _remember(_host.OUT_PROJ_T, _cached((out_proj,), ("out_proj",), lambda: out_proj.t().contiguous()), out_proj)
 
 
 def _check_weights(C: int, head: int, ws):
@@ -483,8 +502,7 @@ def gated_linear_unit_cpp(x: torch.Tensor, weight: torch.Tensor, vnni_repacked: 
         with ops._on_device(x.device):
             _lib.check(_lib.load().af3_silu_mul(y.data_ptr(), out.data_ptr(), y.shape[0], N, ops._DTYPE_CODE[x.dtype], ops._stream_ptr(x.device)), "af3_silu_mul")
         return out.view(*lead, N)
-    wt = _cached((weight,), (bool(vnni_repacked), N_BLK, "glu"), lambda: _plain_weight(weight, vnni_repacked, N_BLK).t().contiguous())
-    _host.remember(tag, wt, weight)
+    wt = _remember(tag, _cached((weight,), (bool(vnni_repacked), N_BLK, "glu"), lambda: _plain_weight(weight, vnni_repacked, N_BLK).t().contiguous()), weight)
     x2 = x.reshape(-1, K)
     if not x2.is_contiguous() or x2.data_ptr() % 16:
         x2 = x2.contiguous()

@@ -367,6 +367,32 @@ def test_derived_weight_cache_follows_tensor_identity_and_version():
     assert len(calls) == n + 1 and torch.equal(third, torch.zeros(4))
 
 
+def test_matrices_remembered_for_the_native_host_side_go_with_their_sources():
+    """What the native host side of the entry points finds: kept while every source lives unchanged, registered once, and given back -- the
+    Python cache's copy too -- when the first source dies."""
+    import gc
+    import weakref
+    from af3_kernels_amd import fused
+    fused.clear_weight_cache()
+    host = fused._host
+    a, b = torch.arange(6.0), torch.ones(3)
+    assert host.recalls(7, a, b) is False
+    value = fused._remember(7, fused._cached((a, b), ("pair",), lambda: torch.cat([a, b])), a, b)
+    assert host.recalls(7, a, b) and not host.recalls(7, b, a) and not host.recalls(8, a, b) and not host.recalls(7, a)
+    assert host.remember(7, value, a, b) is None              # (there already: nothing is registered or swept)
+    a.add_(1.0)
+    assert not host.recalls(7, a, b)
+    assert host.remember(7, value, a, b) is True and host.recalls(7, a, b)
+    gone, sources = weakref.ref(value), len(fused._SOURCES)
+    del value
+    gc.collect()
+    assert gone() is not None
+    del a
+    gc.collect()
+    assert gone() is None and len(fused._SOURCES) == sources - 1 and not any("pair" in k for k in fused._W_CACHE)
+    fused.clear_weight_cache()
+
+
 def test_no_device_is_reported_as_such_before_anything_is_launched():
     """Without a gfx950 as the current device (this test runs where there is no GPU at all) a well-formed call
     returns AF3_ERR_NO_DEVICE_CODE from the host-side check; nothing is enqueued."""
