@@ -437,8 +437,8 @@ class GridSelfAttentionCpp(torch.nn.Module):
         if self.first_run:
             self._packed_weights()
         out = self._native_block(pair, mask)
-        if out is None and self.out_proj.is_cuda:   # (the first call: the closing projection's matrix is not where the native path looks for it)
-            _out_proj_t(self.out_proj)
+        if out is None and pair.dtype == torch.bfloat16 and self.c_pair in (64, 128) and pair.is_cuda and not _host.recalls(_host.OUT_PROJ_T, self.out_proj):
+            _out_proj_t(self.out_proj)   # (the first call: the closing projection's matrix was not where the native path looks for it)
             out = self._native_block(pair, mask)
         if out is not None:
             return out if out.__class__ is not int else _lib.check(out, "grid attention block")

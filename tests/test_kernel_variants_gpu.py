@@ -388,3 +388,27 @@ def test_self_attention_has_the_same_bits_on_every_route(af3, S, N, C, head):
     odd = torch.empty(x.numel() + 1, device="cuda", dtype=torch.bfloat16)[1:].view(x.shape).copy_(x)   # off a 16-byte boundary
     if S * N * 4 * C * C <= 6e9 and C % 64 == 0:   # (a library GEMM may choose by the address)
         assert torch.equal(first, call(odd, mask)) and torch.equal(first, call(odd, mask.float()))
+
+
+@pytest.mark.parametrize("C,head,dtype,attempts", [(128, 4, torch.float32, 1), (96, 4, torch.bfloat16, 1), (128, 4, torch.bfloat16, 2)])
+def test_grid_block_asks_the_native_host_side_once(af3, monkeypatch, C, head, dtype, attempts):
+    """A call that the native block does not take (here by its type, its channels, or a mask that is not bool) goes to Python after one attempt and
+    derives nothing that it does not read; only the first call on a set of weights it may take asks twice."""
+    from af3_kernels_amd import fused
+    seen = []
+
+    class Counting:
+        def __getattr__(self, name):
+            fn = getattr(host, name)
+            return (lambda *a: seen.append(name) or fn(*a)) if callable(fn) else fn
+
+    host = fused._host
+    monkeypatch.setattr(fused, "_host", Counting())
+    mod = af3.GridSelfAttentionCpp(C, head).to("cuda", dtype).eval().requires_grad_(False)
+    pair, keep = torch.randn(40, 40, C, device="cuda").to(dtype), torch.ones(40, 40, device="cuda")
+    mod(pair, keep)
+    assert seen.count("grid_block") == attempts
+    del seen[:]
+    mod(pair, keep)
+    assert seen.count("grid_block") == 1
+    assert host.recalls(host.OUT_PROJ_T, mod.out_proj) == (attempts == 2)
