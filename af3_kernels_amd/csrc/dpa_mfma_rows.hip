@@ -627,7 +627,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 				const int     vc = buf + R * (2 * TILE_R);
 				const bool    fr = decltype(first_c)::value != 0 && t == (int)((first_tiles >> (8 * (R < ROWS ? R : 0))) & 0xffu);
 				if constexpr(R == ROWS - 2) {
-					asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+					// (with two rows the V^T fragments of tile t - 1 may still be on their way: they are consumed in this step; with more
+					// rows an earlier step of this tile has consumed them)
+					if constexpr(ROWS == 2) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+					else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
 					step(r_c, first_c, anydrop_c, fr, k2, m1, vc, [&](auto s_c) {
 						constexpr int S = decltype(s_c)::value;
 						if constexpr(S == 1) {

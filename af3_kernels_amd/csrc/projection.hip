@@ -99,7 +99,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) p
 	const int x_rd = (wm * A * 32 + n) * 128, w_rd = X_BYTES + (wn * B * 32 + n) * 128;
 	int buf = 0;
 	for(int s = 0; s < slabs; s++) {
-		asm volatile("s_barrier" ::: "memory");   // slab s is in LDS; every wavefront is done with slab s - 1
+		asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // slab s is in LDS; every wavefront's reads of slab s - 1 have returned
 		const unsigned char* const base = smem + buf * SLAB_BYTES;
 #pragma unroll
 		for(int c = 0; c < SLAB / 16; c++) {

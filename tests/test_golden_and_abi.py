@@ -555,3 +555,21 @@ assert all(getattr(ops._host, n) == getattr(_host, n) for n in ("FUSED_WEIGHT", 
 """
     r = subprocess.run([sys.executable, "-c", program], cwd=tmp_path, capture_output=True, text=True)
     assert r.returncode == 0, r.stderr
+
+
+def test_hand_written_barriers_wait_for_lds_reads():
+    """A barrier that hands a tile's LDS buffer back to those who refill it must find this wavefront's reads of that tile returned: a
+    barrier in inline assembly says so itself (lgkmcnt), not the place where the compiler consumes them.  Without one stand only the
+    barriers of wavefronts that read no LDS (projection.hip: the loading wavefronts, two; dpa_mfma_rows.hip: a wavefront without
+    query rows) and that of the shared-bias kernel with three or four rows, whose reads an earlier step, held in order by
+    assembly statements, has consumed."""
+    import re
+    src = os.path.join(ROOT, "af3_kernels_amd", "csrc")
+    bare = {}
+    for name in sorted(os.listdir(src)):
+        if name.endswith((".hip", ".hpp")):
+            text = open(os.path.join(src, name)).read()
+            n = sum("lgkmcnt(" not in a for a in re.findall(r'asm volatile\("([^;]*?s_barrier[^;]*?)"\s*:', text))
+            if n:
+                bare[name] = n
+    assert bare == {"dpa_mfma_rows.hip": 2, "projection.hip": 2}
