@@ -399,13 +399,13 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DP
 	};
 	step(ic<1>{}, 0);
 	for(int j = 1; j < n_steps; j++) step(ic<0>{}, j);
-	// What is needed from here on comes from its sources once more, out of the compiler's sight: kept from the start, arguments and
-	// row numbers cost the loop above ten registers, and a fourth wavefront per SIMD.
-	typedef __attribute__((address_space(4))) const af3_dpa_params kernarg;
-	kernarg* a  = (kernarg*)__builtin_amdgcn_kernarg_segment_ptr();  // (p is the first argument)
-	int      ln = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
-	asm volatile("" : "+s"(a));
-	asm volatile("" : "+v"(ln));
+	// Row numbers from here on come from the lane's number once more, out of the compiler's sight where the loop above has no
+	// registers to spare: kept from the start they cost it a fourth wavefront per SIMD.
+	int ln = lane;
+	if constexpr(KS == 1) {
+		ln = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+		asm volatile("" : "+v"(ln));
+	}
 	const int     on = ln & 31, ohalf = ln >> 5;
 	const int64_t orow = (int64_t)qtile * (NQ * 32) + wblk * 32 + on;
 
@@ -424,9 +424,9 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DP
 		for(int db = 0; db < NDB; db++)
 #pragma unroll
 			for(int i = 0; i < 16; i++) oacc[db][i] = 0.f;
-		const int          cols = (int)a->D, k_bytes = (int)(a->k_stride[2] * 4), v_bytes = (int)(a->v_stride[2] * 4);
-		const float        scale = a->softmax_scale * LOG2E;
-		const float* const qp = static_cast<const float*>(a->q) + b * a->q_stride[0] + h * a->q_stride[1] + (orow < a->L ? orow : 0) * a->q_stride[2];
+		const int          cols = (int)p.D, k_bytes = (int)(p.k_stride[2] * 4), v_bytes = (int)(p.v_stride[2] * 4);
+		const float        scale = p.softmax_scale * LOG2E;
+		const float* const qp = static_cast<const float*>(p.q) + b * p.q_stride[0] + h * p.q_stride[1] + (orow < p.L ? orow : 0) * p.q_stride[2];
 #pragma unroll 1
 		for(int j = ks; j < nlive; j += KS) {
 			kt = tile_at(j);
@@ -491,15 +491,15 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DP
 	// ---- epilogue: O^T register i of block db is head column 32*db + 8*(i/4) + 4*half + i%4 ----
 	const float l_tot = l_run + other_half(l_run);
 	const float inv   = 1.f / l_tot;
-	if(orow < a->L) {
-		float* const       op = static_cast<float*>(a->out) + b * a->out_stride[0] + h * a->out_stride[1] + orow * a->out_stride[2];
-		const float* const gp = a->gate ? static_cast<const float*>(a->gate) + b * a->gate_stride[0] + h * a->gate_stride[1] + orow * a->gate_stride[2] : nullptr;
+	if(orow < p.L) {
+		float* const       op = static_cast<float*>(p.out) + b * p.out_stride[0] + h * p.out_stride[1] + orow * p.out_stride[2];
+		const float* const gp = p.gate ? static_cast<const float*>(p.gate) + b * p.gate_stride[0] + h * p.gate_stride[1] + orow * p.gate_stride[2] : nullptr;
 #pragma unroll
 		for(int db = 0; db < NDB; db++)
 #pragma unroll
 			for(int r4 = 0; r4 < 4; r4++) {
 				const int d0 = 32 * db + 8 * r4 + 4 * ohalf;
-				if(d0 < a->D) {
+				if(d0 < p.D) {
 					float4 w = {oacc[db][4 * r4] * inv, oacc[db][4 * r4 + 1] * inv, oacc[db][4 * r4 + 2] * inv, oacc[db][4 * r4 + 3] * inv};
 					if(gp) {  // out *= sigmoid(gate)
 						const float4 g = *reinterpret_cast<const float4*>(gp + d0);
