@@ -10,9 +10,8 @@ libaf3_dpa.so (hand-written HIP for gfx950) through the C ABI of include/af3_dpa
 Inputs must live on a ROCm device; CPU tensors raise.  The attention core (`dot_product_attention_cpp`, the fp8 variant,
 the casts, pad and repack helpers) runs in the HIP library or not at all: there is no CPU path and no PyTorch fallback, and
 a missing library raises at first use.  The callers around the core compose it with library matrix products where a plain
-GEMM is the right tool (the wide projection of the three-launch path, output projections and `Linear` layers wider than
-128 columns: hipBLASLt through torch) and, for shapes outside their HIP kernels (other channel counts, float32), run the
-reference module's own torch ops on the device; each function's docstring names its limits.
+GEMM is the right tool (the projection of the three-launch path where it is large or float32, output projections and `Linear` layers
+wider than 128 columns: hipBLASLt through torch); each function's docstring names its limits.
 """
 from . import _lib
 from .fused import GridSelfAttentionCpp, Linear, _attention_cpp, clear_weight_cache, gated_linear_unit_cpp, layernorm_pair_bias, self_attention_cpp  # noqa: F401

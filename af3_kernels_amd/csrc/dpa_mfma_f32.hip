@@ -13,7 +13,7 @@
 // times 10 1.6e-7..2.3e-7 / 1.9e-7..3.8e-7, biases that grow by 40 along the row 2.1e-7..5.4e-7 / 3.0e-7..5.2e-7 (fewer, deeper
 // instructions round the accumulator less often).  Rows whose biases carry an offset of some hundreds or thousands: 0.14 to 1.41
 // times the fp32 instructions', by where the offset lies between two powers of two in either domain.
-// Measured (64 x 4 x 768 x 32): 234 us with the fp32 instructions (53 % of their peak), 131 us in this form.
+// Measured (64 x 4 x 768 x 32): 234 us with the fp32 instructions (53 % of their peak), 131 to 139 us by box in this form.
 //
 // Same transposed formulation as the bf16 kernel: S^T[key][q] = K.Q^T, so that in the 32x32
 // accumulator layout a lane (q = lane%32, half = lane/32) holds 16 keys of ONE query row
@@ -533,7 +533,8 @@ int launch(const af3_dpa_params& p, hipStream_t s) {
 //   two, 128 query rows           9.1    31.0    31.2    18.6    31.6*   18.8*   14.2*   63.4    26.7   189.7
 //   four, 64 query rows           7.6    20.5    20.7*   13.4*   39.8    25.5    19.7    61.2    37.7   238.3
 //   four, 32 query rows           7.4*   18.4*   35.1    22.5    52.5    33.2    35.3   105.7    69.6   416.5
-// (fp32 matrix instructions, one wavefront per block, before: 2x128 13 us, 64x768 234 us.)  Rows of less than four tiles do
+// (fp32 matrix instructions, one wavefront per block, before: 2x128 13 us, 64x768 234 us.  With biases joining finished products the forms
+// taken measure 2x128 7.4, 8x384 13.0, 32x256 13.2, 16x384 17.4, 16x768 47.7, 64x768 131.6.)  Rows of less than four tiles do
 // not gain from a split.
 template <int DP>
 int launch_dp(const af3_dpa_params& p, hipStream_t s) {

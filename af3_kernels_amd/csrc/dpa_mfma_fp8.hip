@@ -1,5 +1,5 @@
-// fp8 (OCP e4m3) matrix-core attention kernel for gfx950: both products on
-// v_mfma_f32_32x32x16_fp8_fp8 with fp32 accumulation, bf16 bias, bf16 or fp32 output.
+// fp8 (OCP e4m3) matrix-core attention kernel for gfx950: both products on the e4m3 matrix instructions (64-deep for K.Q^T where
+// head_dim allows, 16-deep otherwise) with fp32 accumulation, bf16 bias, bf16 or fp32 output.
 //
 // The reference has no fp8 path (its e4m3 converters are "not implemented" asserts,
 // src/csrc/xsmm_functors.h:218-226); this kernel computes the same formula as
@@ -30,7 +30,7 @@
 //     below and shifted when read (element by element before).
 //   * 39 KB of LDS and 128 registers: four workgroups of four wavefronts per compute unit.
 // us per call with its two quantising launches (12 to 14 us), 16 heads of 24, before / now: 5x1536 89.0/71.3, 8x1536 133.6/104.9, 8x1301 (ragged
-// rows) -/101.7, 8x1000 66.7/54.2, 5x300 37.9/20.3, 1x1536 42.1/34.2.  Measured on the way: the bias loads are 13 us of the
+// rows) -/101.7, 8x1000 66.7/54.2, 5x300 37.9/20.3, 1x1536 42.1/34.2 (boxes differ: 5x1536 72 to 75).  Measured on the way: the bias loads are 13 us of the
 // 57 that the kernel takes at 5x1536, the exponentials 4; four workgroups per compute unit instead of three changed nothing, nor did
 // pinning the matrix instructions between the exponentials: the vector port is busy three quarters of the time.
 #include "mfma_helpers.hpp"

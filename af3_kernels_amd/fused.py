@@ -7,11 +7,13 @@
     gated_linear_unit_cpp  src/af3_kernels/__init__.py:21-28    -> gated_linear_unit_impl (gated_linear_unit.cpp:20-80)
     Linear                 src/af3_kernels/__init__.py:138-163  -> linear_impl            (gated_linear_unit.cpp:82-129)
 
-On the GPU the grid op in AlphaFold 3's shape (bfloat16, 128 channels, 4 heads) is ONE kernel for the projections,
-the attention and the gate (af3_grid_attention_forward: q, k, v and the gate never touch device memory) followed by
-the output projection (af3_linear).  Every other shape, and the diffusion op, is three launches:
-  1. ONE library GEMM for the four projections: x [rows, C] . W [C, 4C], output columns ordered
-     (head, [k, v, q, gate], channel)  (hipBLASLt through torch: a plain GEMM is library territory);
+On the GPU the module in AlphaFold 3's shape (bfloat16, 128 channels, 4 heads) is one pass over the pair tensor for LayerNorm, pair
+bias and projections, the shared-bias attention kernel with the gate in its epilogue, and the output projection (csrc/host.cpp,
+csrc/grid_project.hip); _attention_cpp in that shape is ONE kernel for the projections, the attention and the gate
+(af3_grid_attention_forward: q, k, v and the gate never touch device memory) followed by the output projection
+(af3_linear).  Every other shape, and the diffusion op, is three launches:
+  1. ONE product for the four projections: x [rows, C] . W [C, 4C], output columns ordered (head, [k, v, q, gate], channel): for
+     the diffusion op this library's kernel up to 6e9 multiply-adds (csrc/projection.hip), a library GEMM otherwise;
   2. the attention kernel, reading q, k, v and the gate where that GEMM left them (no
      "b n (h d) -> b h n d" copies), adding bias and mask, and applying sigmoid(gate) in its
      epilogue while writing straight into the "b n (h d)" layout;
@@ -392,7 +394,8 @@ def layernorm_pair_bias(pair: torch.Tensor, ln_weight: torch.Tensor, ln_bias: to
 
 class GridSelfAttentionCpp(torch.nn.Module):
     """Same constructor, parameters and forward as the reference module (src/af3_kernels/Attention.py:23-82):
-    LayerNorm and the pair-bias projection are one kernel (layernorm_pair_bias), the rest is _attention_cpp."""
+    in AlphaFold 3's shape LayerNorm, pair bias and projections are one kernel, attention and output projection one each (the
+    native block); other calls are layernorm_pair_bias and _attention_cpp."""
 
     def __init__(self, c_pair: int = 128, num_head: int = 4, transpose: bool = False):
         super().__init__()

@@ -309,8 +309,8 @@ def dot_product_attention_cpp(
     af3_kernels.dot_product_attention_cpp (src/af3_kernels/__init__.py:31-52).
 
     q, k, v [B,H,L,D]; bias [H,L,L] (or pre-padded [H,M,M]); mask [L], [B,L] or [B,1,1,L],
-    truthy = attend.  float32 inputs run in fp32 FMA arithmetic, bfloat16 inputs on the bf16
-    matrix cores with fp32 accumulation.  As in the reference, k, v and bias are cast to q's
+    truthy = attend.  float32 inputs run to float32 precision (three-term bf16 products on the matrix
+    cores, or vector FMA), bfloat16 inputs on the bf16 matrix cores, both with fp32 accumulation.  As in the reference, k, v and bias are cast to q's
     dtype.  Unlike the reference, q is left untouched and a fresh tensor is returned; a 1-D
     mask is broadcast over the batch (the harness semantics, examples/dot_product_attention.py:
     34-37).  use_flash_attention / BLK_SZ / FLASH_SZ are accepted and ignored: they tune CPU

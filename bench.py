@@ -217,7 +217,7 @@ def bench_fused(args, case):
             kbytes = case.head * case.N * case.N * 2 + 5 * case.N * case.C * 2 + case.N
             ach = kbytes / (kernel_ms * 1e-3) / 1e9
             roofline = {"bound": "hbm", "achieved": round(ach, 1), "peak": PEAK_HBM_GBS, "unit": "GB/s", "frac": round(ach / PEAK_HBM_GBS, 4), "traffic": None,
-                        "kernel": "attention kernel with the gate in its epilogue (of projection GEMM + attention)", "algorithmic_bytes_per_launch": kbytes, **timing}
+                        "kernel": "attention kernel with the gate in its epilogue (of projection + attention)", "algorithmic_bytes_per_launch": kbytes, **timing}
         else:
             ach = case.flops_attention / (kernel_ms * 1e-3) / 1e12
             roofline = {"bound": "mfma", "achieved": round(ach, 1), "peak": PEAK_TFLOPS["bf16"], "unit": "TFLOP/s", "frac": round(ach / PEAK_TFLOPS["bf16"], 4),
@@ -230,7 +230,7 @@ def bench_fused(args, case):
             "warmup": args.warmup, "ms_per_step": round(ms_per_step, 4), "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "bf16",
             "data": "synthetic",
             "config": {"workload": f"{case.name}: rows [{case.B}, {case.N}, {case.C}] head={case.head} bf16, Bernoulli({case.keep}) key mask; "
-                                   f"{'one kernel + output projection GEMM' if one_kernel else 'projection GEMM + attention kernel' + (' + output projection GEMM' if case.kind == 'grid' else '')}",
+                                   f"{'one kernel + output projection GEMM' if one_kernel else 'projection + attention kernel' + (' + output projection GEMM' if case.kind == 'grid' else '')}",
                        "flops": case.flops},
             "roofline": roofline}
     if not args.no_cpu_baseline:
