@@ -109,6 +109,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 	const int     n_t_all  = (int)((L + KT_R - 1) / KT_R);
 	uint16_t* const mask_tab = reinterpret_cast<uint16_t*>(smem + MASK_BASE);
 	__shared__ int  s_last[4];  // index of the last live key + 1 of each batch row (0: every key dropped)
+	__shared__ int  s_again;    // some wavefront's walk has to be repeated carefully
 	__shared__ int  s_first[4]; // index of the first key tile of each batch row that holds a live key
 
 	// ---- workgroup -> (group of batch rows, head, query tile): all query tiles of one (group, head) get ids congruent
@@ -141,7 +142,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 		__syncthreads();
 	}
 
-	if constexpr(STAGED) {  // (chunks past L are never fetched: what the slots hold there must be finite)
+	if(STAGED && L % KT_R != 0) {  // (chunks past L are never fetched: what the slots hold there must be finite)
 		for(int i = tid; i < NW * 4096 / 16; i += NW * 64) reinterpret_cast<u32x4*>(smem + SLOT_BASE)[i] = u32x4{0u, 0u, 0u, 0u};
 		__syncthreads();
 	}
@@ -332,6 +333,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 		}
 		if(lane == 0) s_last[r] = last, s_first[r] = first;
 	}
+	if(tid == 0) s_again = 0;
 	asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wavefront's pieces of the first tile and its bias fragment have landed
 	__syncthreads();                                    // the mask table and the first tile are complete
 	// keys behind the last live key of every row carry weight 0 and are not walked; a row without live keys needs them all
@@ -378,8 +380,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 	// finite value their A holds contributes nothing.
 	u32x2 maskA = {0u, 0x3F803F80u};
 	u32x2 maskB[ROWS];
-#pragma unroll
-	for(int r = 0; r < ROWS; r++) maskB[r] = u32x2{half == 0 ? 0x3F80u : 0u, 0u};
 
 	// ---- per-lane LDS read offsets inside a (buffer, batch row) block ----
 	int k_rd[2];
@@ -399,14 +399,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 	// ---- online-softmax state: one query row per lane and batch row (the two half-waves hold disjoint keys) ----
 	float  m_ref[ROWS];   // reference maximum, log2 units, exactly m_hi + m_lo of two bf16 values
 	float  lsum[ROWS];    // the row sum (complete: the same value in both half-waves)
+	float  rs_prev;       // the previous step's share of it (quick walk)
 	f32x16 oacc[ROWS];
-#pragma unroll
-	for(int r = 0; r < ROWS; r++) {
-		m_ref[r] = 0.f;
-		lsum[r]  = 0.f;
-#pragma unroll
-		for(int i = 0; i < 16; i++) oacc[r][i] = 0.f;
-	}
 
 	// Row sums on the matrix pipe (see dpa_mfma.hip): a 16x16x32 MFMA whose A operand is this 0/1 pattern leaves, in
 	// register 0 of every lane, the sum of the 16 packed probabilities of that lane's own query row over both half-waves.
@@ -446,6 +440,20 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
 		for(int i = 0; i < 16; i++) oacc[R][i] *= alpha;
 	};
+	// The quick walk's first tile: every batch row has a live key in it, nothing is accumulated, and each query's reference is the
+	// maximum of its logits.  The mask instruction once more, without mask values, subtracts it.
+	auto first_reference = [&](auto r_c, f32x16& s) {
+		constexpr int R = decltype(r_c)::value;
+		float mx = fmaxf(fmaxf(s[0], s[1]), s[2]);
+#pragma unroll
+		for(int i = 3; i < 15; i += 2) mx = fmaxf(fmaxf(mx, s[i]), s[i + 1]);
+		mx = half_swap_max(fmaxf(mx, s[15]));
+		const float neg_hi = __uint_as_float(pack_bf16x2(0.f, -mx));   // (the high half is the rounded value; the low one is zero)
+		const float neg_lo = -mx - neg_hi;
+		if(half == 0) maskB[R][1] = pack_bf16x2(neg_hi, neg_lo);
+		const u32x2 ones = {0u, 0x3F803F80u};
+		s = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(__builtin_bit_cast(s16x4, ones), __builtin_bit_cast(s16x4, maskB[R]), s, 0, 0, 0);
+	};
 	auto exp_part = [&](const f32x16& s, u32x4 (&pf)[2], auto i0_c, auto n_c) {
 		constexpr int I0 = decltype(i0_c)::value, N = decltype(n_c)::value;
 #pragma unroll
@@ -462,8 +470,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 	// first K.Q^T instruction).
 	f32x16 sc, bias_frag;
 	u32x4  kf[2];
-	u32x4  pprev[2] = {u32x4{0u, 0u, 0u, 0u}, u32x4{0u, 0u, 0u, 0u}};
-	u32x4  vprev[2] = {u32x4{0u, 0u, 0u, 0u}, u32x4{0u, 0u, 0u, 0u}};
+	u32x4  pprev[2], vprev[2];
 #pragma unroll
 	for(int i = 0; i < 16; i++) bias_frag[i] = 0.f;
 	// the next tile's bias fragment -> registers: from the slot, or (direct mode) from the raw bf16 pieces loaded a tile ago:
@@ -512,16 +519,18 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 	// k_addr2: LDS byte address of the K tile of the step after the next; m_addr: (per lane) of the next step's mask
 	// entries; v_addr: of this step's V tile; hook(i): run behind the i-th matrix instruction of the step (i = 0..4; 1 is the
 	// first K.Q^T instruction of the next step).
-	// FIRST: a leading tile, in which a row that meets its first live key (`force`, wave-uniform) fixes its softmax reference.  ANYDROP: some batch row of this group has no
-	// live key (it then takes no bias: a wave-uniform branch the common instantiation does not carry).
-	auto step = [&](auto r_c, auto first_c, auto anydrop_c, bool force, int k_addr2, int m_addr, int v_addr, auto&& hook) {
+	// FIRST: a leading tile, in which a row that meets its first live key (`force`, wave-uniform) fixes its softmax reference.  CAREFUL: the walk that tests every step's row
+	// sums, and whose batch rows may lack live keys (they then take no bias: a wave-uniform branch that the quick walk does not carry).
+	auto step = [&](auto r_c, auto first_c, auto careful_c, bool force, int k_addr2, int m_addr, int v_addr, auto&& hook) {
 		constexpr int  R = decltype(r_c)::value, RN = (R + 1) % ROWS, RP = (R + ROWS - 1) % ROWS;
-		constexpr bool FIRST = decltype(first_c)::value != 0, ANYDROP = decltype(anydrop_c)::value != 0;
-		if constexpr(FIRST) rereference(r_c, sc, force);
+		constexpr bool FIRST = decltype(first_c)::value != 0, CAREFUL = decltype(careful_c)::value != 0;
+		if constexpr(FIRST && CAREFUL) rereference(r_c, sc, force);
+		else if constexpr(FIRST) first_reference(r_c, sc);
 		maskA[0] = *reinterpret_cast<const uint16_t*>(smem + m_addr);
 		u32x4  pcur[2];
 		f32x16 sn;
 		f32x4  rs = {0.f, 0.f, 0.f, 0.f};
+		if constexpr(!CAREFUL) lsum[RP] += rs_prev;
 		// The order below is the order the instructions are meant to issue in: one matrix instruction, then a slice of the
 		// vector work, so that consecutive matrix instructions belong to different chains.  Matrix intrinsics are pure
 		// values to the compiler and would drift to wherever their consumers are; each slice therefore ends with an empty
@@ -554,7 +563,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
 			for(int i = 0; i < 16; i++) z[i] = 0.f;
 			bool with_bias = HAS_BIAS;
-			if constexpr(ANYDROP) with_bias = HAS_BIAS && !dropped[RN];  // (wave-uniform)
+			if constexpr(CAREFUL) with_bias = HAS_BIAS && !dropped[RN];  // (wave-uniform)
 			if(with_bias) sn = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, kf[0]), qf[RN][0], bias_frag, 0, 0, 0);
 			else sn = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, kf[0]), qf[RN][0], z, 0, 0, 0);
 		}
@@ -596,15 +605,19 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 #undef AF3_PIN2
 #undef AF3_PIN3
 		rs = rowsum(rs, pcur[1]);
-		// This step's sum stays below 32 * 2^REF_SLACK while every probability respects the reference, so the test also
-		// catches a single probability near or beyond the limit (inf, NaN).
-		if(__ballot(!(rs[0] < PSUM_LIMIT))) {  // rare
-			rereference(r_c, sc, false);
-			exp_part(sc, pcur, ic<0>{}, ic<16>{});
-			rs = rowsum(f32x4{0.f, 0.f, 0.f, 0.f}, pcur[0]);
-			rs = rowsum(rs, pcur[1]);
+		if constexpr(CAREFUL) {
+			// This step's sum stays below 32 * 2^REF_SLACK while every probability respects the reference, so the test also
+			// catches a single probability near or beyond the limit (inf, NaN).
+			if(__ballot(!(rs[0] < PSUM_LIMIT))) {  // rare
+				rereference(r_c, sc, false);
+				exp_part(sc, pcur, ic<0>{}, ic<16>{});
+				rs = rowsum(f32x4{0.f, 0.f, 0.f, 0.f}, pcur[0]);
+				rs = rowsum(rs, pcur[1]);
+			}
+			lsum[R] += rs[0];
+		} else {
+			rs_prev = rs[0];   // (added a step later: nothing waits for the matrix pipe here)
 		}
-		lsum[R] += rs[0];
 		sc       = sn;
 		pprev[0] = pcur[0];
 		pprev[1] = pcur[1];
@@ -616,7 +629,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 	// t - 1, whose buffer tile t + 2 then overwrites.  That step's first matrix instruction is the last reader of bias
 	// fragment t: behind it the fragment registers take fragment t + 1, and the slot (once those reads have returned: the
 	// last step's first matrix instruction waits for them) or the raw-piece registers are refilled with fragment t + 2.
-	auto tile = [&](auto first_c, auto anydrop_c, int t, int buf, int bufn, int bufnn) {
+	auto tile = [&](auto first_c, auto careful_c, int t, int buf, int bufn, int bufnn) {
 		const int m0 = mask_rd + t * (ROWS * 64);
 		auto one = [&](auto r_c) {
 			constexpr int R = decltype(r_c)::value;
@@ -631,7 +644,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 					// rows an earlier step of this tile has consumed them)
 					if constexpr(ROWS == 2) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 					else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-					step(r_c, first_c, anydrop_c, fr, k2, m1, vc, [&](auto s_c) {
+					step(r_c, first_c, careful_c, fr, k2, m1, vc, [&](auto s_c) {
 						constexpr int S = decltype(s_c)::value;
 						if constexpr(S == 1) {
 							load_tile_or_gate(t + 2, bufnn);
@@ -641,19 +654,19 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 						}
 					});
 				} else if constexpr(R == ROWS - 1) {
-					step(r_c, first_c, anydrop_c, fr, k2, m1, vc, [&](auto s_c) {
+					step(r_c, first_c, careful_c, fr, k2, m1, vc, [&](auto s_c) {
 						constexpr int S = decltype(s_c)::value;
 						if constexpr(S == 1) load_bias(t + 2);   // (behind this step's first K.Q^T instruction, which has waited for the slot's reads)
 					});
 				} else {
-					step(r_c, first_c, anydrop_c, fr, k2, m1, vc, [](auto) {});
+					step(r_c, first_c, careful_c, fr, k2, m1, vc, [](auto) {});
 				}
 			}
 		};
 		one(ic<0>{}), one(ic<1>{}), one(ic<2>{}), one(ic<3>{});
 	};
-	auto run = [&](auto anydrop_c) {
-		constexpr bool ANYDROP = decltype(anydrop_c)::value != 0;
+	auto run = [&](auto careful_c) {
+		constexpr bool CAREFUL = decltype(careful_c)::value != 0;
 		// ---- prologue: the second tile and bias fragment, S^T of the first step, K fragments of the second ----
 		// (tile 0 and bias fragment 0 were requested at the top of the kernel and are complete)
 		next_bias_fragment(0);  // fragment 0 -> registers
@@ -665,7 +678,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 		{
 			f32x16 s0;
 #pragma unroll
-			for(int i = 0; i < 16; i++) s0[i] = (HAS_BIAS && !(ANYDROP && dropped[0])) ? bias_frag[i] : 0.f;
+			for(int i = 0; i < 16; i++) s0[i] = (HAS_BIAS && !(CAREFUL && dropped[0])) ? bias_frag[i] : 0.f;
 #pragma unroll
 			for(int c = 0; c < 2; c++) s0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, read_kfrag(k_rd[c])), qf[0][c], s0, 0, 0, 0);
 			maskA[0] = *reinterpret_cast<const uint16_t*>(smem + mask_rd);
@@ -674,40 +687,86 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 			kf[1] = read_kfrag(2 * TILE_R + k_rd[1]);
 		}
 		int buf = 0, t = 0;
-		for(; t <= t_force_max; t++) {   // (one trip unless some row's leading tiles hold dropped keys only)
+		for(; t <= (CAREFUL ? t_force_max : 0); t++) {   // (more than one trip where some row's leading tiles hold dropped keys only)
 			const int bufn = buf == (NBUF_R - 1) * BUF_R ? 0 : buf + BUF_R, bufnn = bufn == (NBUF_R - 1) * BUF_R ? 0 : bufn + BUF_R;
-			tile(ic<1>{}, anydrop_c, t, buf, bufn, bufnn);
+			tile(ic<1>{}, careful_c, t, buf, bufn, bufnn);
 			buf = bufn;
 		}
 		for(; t < n_t; t++) {
 			const int bufn = buf == (NBUF_R - 1) * BUF_R ? 0 : buf + BUF_R, bufnn = bufn == (NBUF_R - 1) * BUF_R ? 0 : bufn + BUF_R;
-			tile(ic<0>{}, anydrop_c, t, buf, bufn, bufnn);
+			tile(ic<0>{}, careful_c, t, buf, bufn, bufnn);
 			buf = bufn;
 		}
 	};
-	if((int64_t)qtile * (NW * 32) + wave * 32 >= L) {
-		// ---- no query row of this wavefront exists (L % 128 != 0, the last query tile): it fetches its batch row's tiles, keeps the
-		// barriers' count -- one per tile -- and leaves the vector and matrix pipes to others ----
-		load_tile(1, BUF_R);
-		int bufnn = 2 * BUF_R;
-		for(int t = 0; t < n_t; t++) {
-			asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-			load_tile(t + 2, bufnn);
-			bufnn = bufnn == (NBUF_R - 1) * BUF_R ? 0 : bufnn + BUF_R;
-		}
-		return;
-	}
-	if(n_t > 0) {
-		bool any_dropped = false;
+	// The key axis is walked without a look at the row sums on the way (a test per step made the wavefront wait for the matrix pipe
+	// and kept the step's logits alive behind it: 768 x 4 x 768 x 32 408 -> 392 us without, 1491 2837 -> 2713, 384 64.9 -> 62.8).  Sums
+	// that end below the careful walk's limit have stayed below it throughout: the results are the careful walk's.  Beyond it they
+	// stand all the same if the sums stay below 2^100 and the results are finite (probabilities and sums are floating-point: a
+	// reference left behind costs them no digits).  Otherwise the whole workgroup -- its wavefronts fetch tiles for one another --
+	// walks once more, carefully, and a workgroup with a batch row without a live key, or without one in its first tile, does so at once.
+	bool careful = t_force_max > 0;
 #pragma unroll
-		for(int r = 0; r < ROWS; r++) any_dropped = any_dropped || dropped[r];
-		if(any_dropped) run(ic<1>{});
-		else run(ic<0>{});
+	for(int r = 0; r < ROWS; r++) careful = careful || dropped[r];   // (the same in every wavefront of the workgroup)
+	const bool no_rows = (int64_t)qtile * (NW * 32) + wave * 32 >= L;
+	auto walk = [&](auto careful_c) {
+		if(no_rows) {
+			// ---- no query row of this wavefront exists (L % 128 != 0, the last query tile): it fetches its batch row's tiles, keeps the
+			// barriers' count -- one per tile -- and leaves the vector and matrix pipes to others ----
+			load_tile(1, BUF_R);
+			int bufnn = 2 * BUF_R;
+			for(int t = 0; t < n_t; t++) {
+				asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+				load_tile(t + 2, bufnn);
+				bufnn = bufnn == (NBUF_R - 1) * BUF_R ? 0 : bufnn + BUF_R;
+			}
+		} else {
+#pragma unroll
+			for(int r = 0; r < ROWS; r++) {
+				m_ref[r] = 0.f;
+				lsum[r]  = 0.f;
+				maskB[r] = u32x2{half == 0 ? 0x3F80u : 0u, 0u};
+#pragma unroll
+				for(int i = 0; i < 16; i++) oacc[r][i] = 0.f;
+			}
+			rs_prev  = 0.f;
+			pprev[0] = pprev[1] = vprev[0] = vprev[1] = u32x4{0u, 0u, 0u, 0u};
+			run(careful_c);
+			lsum[ROWS - 1] += rs_prev;
+			// the last step's P.V product (batch row 3)
+			oacc[ROWS - 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vprev[0]), __builtin_bit_cast(bf16x8, pprev[0]), oacc[ROWS - 1], 0, 0, 0);
+			oacc[ROWS - 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vprev[1]), __builtin_bit_cast(bf16x8, pprev[1]), oacc[ROWS - 1], 0, 0, 0);
+		}
+		asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load may still be writing LDS when the workgroup's allocation is released
+	};
+	if(!careful) {
+		walk(ic<0>{});
+		bool over = false;
+#pragma unroll
+		for(int r = 0; r < ROWS; r++) over = over || !(lsum[r] < PSUM_LIMIT);
+		if(__ballot(row_ok && over)) {   // rare
+			bool bad = false;
+#pragma unroll
+			for(int r = 0; r < ROWS; r++) {
+				float t = lsum[r] * 0x1p28f;   // (infinite from 2^100 on)
+#pragma unroll
+				for(int i = 0; i < 16; i++) t = fmaf(oacc[r][i], 0.f, t);
+				bad = bad || !(t < __builtin_inff());
+			}
+			if(__ballot(row_ok && bad) && lane == 0) s_again = 1;
+		}
+		__syncthreads();
+		if(__builtin_amdgcn_readfirstlane(s_again)) {   // rare
+			careful = true;
+			load_tile(0, 0);
+			load_bias(0);
+			load_bias_direct(0);
+			load_bias_staged(0);
+			asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+			__syncthreads();
+		}
 	}
-	asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load may still be writing LDS when the workgroup's allocation is released
-	// the last step's P.V product (batch row 3)
-	oacc[ROWS - 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vprev[0]), __builtin_bit_cast(bf16x8, pprev[0]), oacc[ROWS - 1], 0, 0, 0);
-	oacc[ROWS - 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vprev[1]), __builtin_bit_cast(bf16x8, pprev[1]), oacc[ROWS - 1], 0, 0, 0);
+	if(careful) walk(ic<1>{});
+	if(no_rows) return;
 
 	// ---- epilogue: O^T register i is head column 8*(i/4) + 4*half + i%4; optional output gate (out *= sigmoid(gate), the
 	// reference's "weighted_avg *= sigmoid(gating_query(pair))", src/csrc/dot_product_attention.cpp:335-349) ----

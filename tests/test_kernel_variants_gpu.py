@@ -412,3 +412,30 @@ def test_grid_block_asks_the_native_host_side_once(af3, monkeypatch, C, head, dt
     mod(pair, keep)
     assert seen.count("grid_block") == 1
     assert host.recalls(host.OUT_PROJ_T, mod.out_proj) == (attempts == 2)
+
+
+@pytest.mark.parametrize("B,H,L,D", [(16, 2, 160, 32), (17, 2, 165, 24), (3, 2, 164, 32), (2, 1, 72, 32), (7, 3, 392, 16)])   # bias staged, from the workspace, read in place; 2 to 4 rows
+@pytest.mark.parametrize("kind", ["45", "60", "68", "120", "60, large v"])
+def test_shared_bias_quick_and_careful_walks(af3, oracle, B, H, L, D, kind):
+    """Logits that rise far above the first tile's: row sums of 2^65 to 2^98 let the walk without sum checks stand, larger ones, results
+    that overflow under the old reference (values of 2^120 at 2^86) send the workgroup through the careful walk."""
+    g = torch.Generator().manual_seed(L + D)
+    q, k, v = (torch.randn(B, H, L, D, generator=g).to(torch.bfloat16) for _ in range(3))
+    bias = torch.randn(H, L, L, generator=g).to(torch.bfloat16)
+    keep = torch.rand(B, L, generator=g) < 0.8
+    keep[:, 0] = keep[:, L - 1] = True
+    rows = [1, 40, L - 1]
+    bias[:, rows, L - 1] = float(kind.split(",")[0])
+    if "large" in kind:
+        v[B - 1, :, L - 1] *= 2.0 ** 120
+    prev = af3.set_rows_kernel("always")
+    try:
+        print("case", B, H, L, D, kind, flush=True)
+        out = f32np(af3.dot_product_attention_cpp(q.cuda(), k.cuda(), v.cuda(), keep.cuda(), bias.cuda()))
+        torch.cuda.synchronize()
+    finally:
+        af3.set_rows_kernel(prev)
+    want = oracle.dpa_formula(f32np(q), f32np(k), f32np(v), keep.numpy(), f32np(bias))
+    assert np.isfinite(out).all()
+    scale = np.maximum(1.0, np.abs(f32np(v)).max(axis=2, keepdims=True) * 2.0 ** -2) if "large" in kind else 1.0   # (of the column's largest value)
+    assert (np.abs(out - want) / scale).max() <= 2e-2
