@@ -77,6 +77,9 @@ bool mfma_rows_can_serve(const af3_dpa_params& p);   // eligible, and its bias c
 int64_t mfma_rows_workspace_bytes(const af3_dpa_params& p);
 bool mfma_rows_suits_a_small_batch(const af3_dpa_params& p);  // fewer than 128 batch rows and a bias that this kernel stages in place
 int launch_dpa_mfma_rows(const af3_dpa_params& p, hipStream_t s);
+// dpa_strip.hip: the bf16 kernel for a bias that is read in place once per batch row; the caller has checked mfma_bf16_eligible
+bool mfma_strip_wanted(const af3_dpa_params& p);
+int launch_dpa_strip(const af3_dpa_params& p, hipStream_t s);
 bool mfma_bf16_eligible(const af3_dpa_params& p);
 int64_t mfma_bf16_workspace_bytes(const af3_dpa_params& p);
 int64_t mfma_bf16_workspace_used(const af3_dpa_params& p);

@@ -1552,6 +1552,7 @@ int launch_dpa_mfma_bf16(const af3_dpa_params& p, hipStream_t s) {
 	const bool batch_limit = p.B >= 2 && (p.workspace || (p.reserved & 4) || (rows_kernel_suits(p) && mfma_rows_workspace_bytes(p) == 0));
 	af3_dpa_params pl = p;
 	pl.reserved       = (int32_t)(batch_limit ? BIAS_LIMIT_BATCH : BIAS_LIMIT_SINGLE);
+	if(mode >= 2 && mfma_strip_wanted(pl)) return launch_dpa_strip(pl, s);
 	auto go = [&](auto dp_c) {
 		constexpr int DP = decltype(dp_c)::value;
 		return l2dom ? launch_nw<DP, true, 0>(pl, s) : mode == 1 ? launch_nw<DP, false, 1>(pl, s) : mode == 2 ? launch_nw<DP, false, 2>(pl, s) : mode == 3 ? launch_nw<DP, false, 3>(pl, s) : launch_nw<DP, false, 0>(pl, s);

@@ -439,3 +439,42 @@ def test_shared_bias_quick_and_careful_walks(af3, oracle, B, H, L, D, kind):
     assert np.isfinite(out).all()
     scale = np.maximum(1.0, np.abs(f32np(v)).max(axis=2, keepdims=True) * 2.0 ** -2) if "large" in kind else 1.0   # (of the column's largest value)
     assert (np.abs(out - want) / scale).max() <= 2e-2
+
+
+@pytest.mark.parametrize("B,H,L,D", [
+    (1, 1, 32, 24), (2, 3, 33, 8), (1, 16, 50, 48), (5, 4, 63, 32), (37, 4, 37, 32),   # four wavefronts, one to three blocks of 16 rows; lengths around a tile
+    (1, 16, 257, 32), (1, 16, 290, 24), (1, 16, 513, 48), (1, 16, 640, 40), (1, 5, 1155, 16),   # eight
+    (1, 16, 769, 24), (1, 16, 900, 24), (1, 16, 1040, 48),                                     # four blocks; two workgroups per compute unit
+    (1, 2, 2050, 48),                                                                          # nine tiles per wavefront
+])
+@pytest.mark.parametrize("kind", ["random", "tail", "one", "none", "low", "high", "v inf"])
+def test_strips(af3, oracle, B, H, L, D, kind):
+    """The kernel for biases read in place: its forms at the edges of tiles and strips, masks that leave wavefronts without a live tile,
+    rows whose sums leave the range of the walk without a reference."""
+    g = torch.Generator().manual_seed(L + D)
+    q, k, v = (torch.randn(B, H, L, D, generator=g).to(torch.bfloat16) for _ in range(3))
+    bias = torch.randn(H, L, L, generator=g).to(torch.bfloat16)
+    keep = torch.rand(B, L, generator=g) < 0.8
+    keep[:, 0] = True
+    if kind == "tail":
+        keep[:, L - L // 3:] = False
+    elif kind in ("one", "none"):
+        keep[:] = False
+        keep[:, L // 2] = kind == "one"
+    elif kind == "low":
+        bias[:, ::3] -= 120
+    elif kind == "high":
+        bias[:, 1::3, L - 1] = 100.0
+        bias[:, 2::5, : L // 2] = 90.0
+        keep[:, L - 1] = True
+    elif kind == "v inf":
+        keep[:, L - 2] = True
+        v[:, :, L - 2, D - 1] = float("inf")
+    print("case", B, H, L, D, kind, flush=True)
+    out = f32np(af3.dot_product_attention_cpp(q.cuda(), k.cuda(), v.cuda(), keep.cuda(), bias.cuda()))
+    if kind == "v inf":   # (weights are positive, unless they round to zero)
+        assert np.isposinf(out[..., D - 1]).mean() > 0.9
+        out, v = out[..., : D - 1], v[..., : D - 1]
+    want = oracle.dpa_formula(f32np(q), f32np(k), f32np(v), keep.numpy(), f32np(bias)) if kind != "v inf" else oracle.dpa_formula(f32np(q), f32np(k), f32np(torch.nn.functional.pad(v, (0, 1))), keep.numpy(), f32np(bias))[..., : D - 1]
+    # (a bias of -120 or 100 leaves its logit steps of 2^-17 or finer; 2e-2 is bf16's budget)
+    assert np.abs(out - want).max() <= 2e-2
