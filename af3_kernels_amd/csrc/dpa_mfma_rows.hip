@@ -122,18 +122,45 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 				 "s"(p.D), "s"(p.key_mask_stride_b), "s"(p.bias_stride[0]), "s"(p.bias_stride[1]));
 	asm volatile("" ::"s"(p.q_stride[0]), "s"(p.q_stride[1]), "s"(p.q_stride[2]), "s"(p.k_stride[0]), "s"(p.k_stride[1]), "s"(p.k_stride[2]), "s"(p.v_stride[0]), "s"(p.v_stride[1]),
 				 "s"(p.v_stride[2]));
-	const int64_t wg    = blockIdx.x;
-	const int     xcd   = (int)(wg & 7);
-	const int64_t slot  = wg >> 3;
-	const int64_t group = (slot / n_qtiles) * 8 + xcd;
-	const int     qtile = (int)(slot % n_qtiles);
-	if(group >= n_groups) return;
-	const int64_t g = group / p.H, h = group % p.H;
+	// (32-bit divisions: a 64-bit one is 150 instructions, i.e. 700 clocks of a start that waits for them)
+	const uint32_t slot = blockIdx.x >> 3, q_div = slot / (uint32_t)n_qtiles, group = q_div * 8 + (blockIdx.x & 7);
+	const int      qtile = (int)(slot - q_div * (uint32_t)n_qtiles);
+	if(group >= (uint32_t)n_groups) return;
+	const int64_t g = group / (uint32_t)p.H, h = group - (uint32_t)g * (uint32_t)p.H;
 	const int64_t b0 = b_first + g * ROWS, b_end = b_first + b_count;   // (rows past b_end repeat the last one and are not stored)
 
 	const int tid = threadIdx.x, lane = tid & 63;
 	const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 	const int n = lane & 31, half = lane >> 5;
+
+	// The start of a workgroup is bound by the number of its instructions (a wavefront issues one in about 4.5 clocks) and by one memory
+	// latency; of the 25 k clocks around the walk of 12 tiles at L = 384 it was half.  Hence 32-bit divisions, a mask table written four keys
+	// at a time without a length-specific unroll, its last and first live key from ballots, and everything that needs no other
+	// wavefront's data in front of the barrier.  H = 4, D = 32: L = 384, B = 384 62.8 -> 61.5 us, L = 768 392 -> 386, L = 1491 (mask rows at
+	// odd addresses, once read byte by byte) 2713 -> 2590.
+	// ---- key-mask bytes of batch row `wave`, requested before anything else: four keys per lane and load at any address (the last four of
+	// a row that L ends in the middle of are shifted), up to 2048 keys in flight ----
+	const bool           mask_vec = L >= 4;
+	const int64_t        mask_row = b0 + (wave < ROWS ? wave : 0) < b_end ? b0 + (wave < ROWS ? wave : 0) : b_end - 1;
+	const uint8_t* const keep     = p.key_mask ? p.key_mask + mask_row * p.key_mask_stride_b : nullptr;
+	constexpr int MASK_CHUNKS = 8;
+	uint32_t      mraw[MASK_CHUNKS];
+	auto load_mask = [&](int c) -> uint32_t {   // chunk c: keys 256 c + 4 lane .. + 3, as they lie in memory
+		const int key0 = 256 * c + 4 * lane;
+		return *reinterpret_cast<const u32_bytes*>(keep + (key0 + 4 <= (int)L ? key0 : (int)L - 4));
+	};
+	auto mask_of = [&](int c, uint32_t w) -> uint32_t {   // ... zeros from L on
+		const int over = 256 * c + 4 * lane + 4 - (int)L;
+		return over <= 0 ? w : over < 4 ? w >> (8 * over) : 0u;
+	};
+	auto request_mask = [&](int c0) {
+#pragma unroll
+		for(int c = 0; c < MASK_CHUNKS; c++) {
+			mraw[c] = 0x01010101u;
+			if(keep && 256 * (c0 + c) < (int)L) mraw[c] = load_mask(c0 + c);
+		}
+	};
+	if(mask_vec && wave < ROWS) request_mask(0);
 
 	// ---- zero the tile buffers when a load can leave parts of them unwritten (padded head columns, rows past L):
 	// stale LDS contents there must be finite ----
@@ -247,8 +274,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 	};
 
 	// ---- everything the walk needs before its first step is requested here in one go, so that the workgroup pays one
-	// memory latency, not a chain of them: the first K and V tiles and the first bias fragment (straight into LDS), the raw
-	// q rows, and the key-mask bytes ----
+	// memory latency, not a chain of them: the first K and V tiles, the first bias fragment (straight into LDS)
+	// and the raw q rows ----
 	load_tile(0, 0);
 	load_bias(0);
 	load_bias_direct(0);
@@ -266,63 +293,51 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 		}
 	}
 
-	// ---- key-mask table: entry = additive mask value of (tile, batch row, key) as bf16 bits; wavefront w fills row w.
-	// With 4-byte aligned mask rows a lane takes four keys per load and all loads of the row are in flight together. ----
+	// ---- key-mask table: entry = additive mask value of (tile, batch row, key) as bf16 bits; wavefront w fills row w ----
 	const int n_keys_tab = (n_t_all + 1) * KT_R;
 	if(wave < ROWS) {
-		const int      r    = wave;
-		const int64_t  br   = b0 + r < b_end ? b0 + r : b_end - 1;
-		const uint8_t* keep = p.key_mask ? p.key_mask + br * p.key_mask_stride_b : nullptr;
-		int            last = 0, first = -1;   // (first: wave-uniform, from ballots)
-		const bool     vec  = !keep || (((reinterpret_cast<uintptr_t>(p.key_mask) | (uintptr_t)p.key_mask_stride_b | (uintptr_t)L) & 3) == 0);
-		if(vec) {
-			constexpr int MAXC = MAX_L_ROWS / 256 + 1;   // chunks of 256 keys (4 per lane) that cover the table
-			uint32_t      mraw[MAXC];
-#pragma unroll
-			for(int c = 0; c < MAXC; c++) {
+		const int r    = wave;
+		int       last = 0, first = -1;   // (wave-uniform)
+		if(mask_vec) {
+			auto write_chunk = [&](int c, uint32_t m) {
 				const int key0 = 256 * c + 4 * lane;
-				mraw[c]        = 0u;
-				if(256 * c < L) mraw[c] = !keep ? 0x01010101u : (key0 < L ? *reinterpret_cast<const uint32_t*>(keep + key0) : 0u);
-			}
-			auto write_chunks = [&](bool all_live) {
-#pragma unroll
-				for(int c = 0; c < MAXC; c++) {
-					const int key0 = 256 * c + 4 * lane;
-					if(256 * c >= n_keys_tab) break;
-					uint32_t e[4];
-#pragma unroll
-					for(int j = 0; j < 4; j++) {
-						const bool in   = key0 + j < L;
-						const bool live = in && (all_live || ((mraw[c] >> (8 * j)) & 0xffu) != 0);
-						e[j]            = live ? 0u : (in ? (uint32_t)MASK_DROPPED_BF16 : (uint32_t)MASK_OUT_OF_RANGE_BF16);
-						if(live && !all_live) last = key0 + j + 1;
-					}
-					if(key0 < n_keys_tab) *reinterpret_cast<u32x2*>(mask_tab + ((key0 >> 5) * ROWS + r) * 32 + (key0 & 31)) = u32x2{e[0] | (e[1] << 16), e[2] | (e[3] << 16)};
+				if(key0 >= n_keys_tab) return;
+				const uint32_t gone = (~(((m & 0x7f7f7f7fu) + 0x7f7f7f7fu) | m) >> 7) & 0x01010101u;   // 1 in the bytes that are zero
+				uint32_t       lo = ((gone & 1u) | ((gone & 0x100u) << 8)) * MASK_DROPPED_BF16, hi = (((gone >> 16) & 1u) | ((gone >> 24) << 16)) * MASK_DROPPED_BF16;
+				if(key0 + 4 > (int)L) {
+					const int in = (int)L - key0;   // keys of this lane in front of L
+					constexpr uint32_t OUT = MASK_OUT_OF_RANGE_BF16;
+					lo = in >= 2 ? lo : in == 1 ? (lo & 0xffffu) | (OUT << 16) : OUT | (OUT << 16);
+					hi = in == 3 ? (hi & 0xffffu) | (OUT << 16) : OUT | (OUT << 16);
 				}
+				*reinterpret_cast<u32x2*>(mask_tab + ((key0 >> 5) * ROWS + r) * 32 + (key0 & 31)) = u32x2{lo, hi};
 			};
+			for(int c0 = 0; 256 * c0 < n_keys_tab; c0 += MASK_CHUNKS) {
+				if(c0 > 0) request_mask(c0);
 #pragma unroll
-			for(int c = MAXC - 1; c >= 0; c--) {   // a lane's four keys of chunk c lie in tile 8 c + lane / 8
-				const unsigned long long bal = __ballot(mraw[c] != 0u);   // (chunks at or beyond L hold zeros)
-				if(bal) first = 8 * c + (__builtin_ctzll(bal) >> 3);
-			}
-			write_chunks(false);
-#pragma unroll
-			for(int off = 32; off >= 1; off >>= 1) {
-				const int o = __shfl_xor(last, off);
-				last        = o > last ? o : last;
+				for(int c = 0; c < MASK_CHUNKS; c++) {
+					if(256 * (c0 + c) >= n_keys_tab) break;
+					const uint32_t           mc  = mask_of(c0 + c, mraw[c]);
+					const unsigned long long bal = __ballot(mc != 0u);   // a lane's four keys of chunk c lie in tile 8 c + lane / 8
+					if(bal) {
+						const int      top = 63 - __builtin_clzll(bal);
+						const uint32_t m   = __builtin_amdgcn_readlane(mc, top);
+						last               = 256 * (c0 + c) + 4 * top + ((31 - __builtin_clz(m)) >> 3) + 1;
+						if(first < 0) first = 8 * (c0 + c) + (__builtin_ctzll(bal) >> 3);
+					}
+					write_chunk(c0 + c, mc);
+				}
 			}
 			// A batch row without any live key yields the mean over all L keys (masked_fill(-1e9) + softmax in
 			// examples/dot_product_attention.py:37-39): its keys count as live, and q and the bias are dropped for it
 			// below, so that all its logits are exactly equal.
-			if(last == 0) {
-				write_chunks(true);
-				last = 0;
-			}
+			if(last == 0)
+				for(int c = 0; 256 * c < n_keys_tab; c++) write_chunk(c, 0x01010101u);
 		} else {
 			for(int base = 0; base < n_keys_tab; base += 64) {
 				const int  key  = base + lane;
 				const bool in   = key < L;
-				const bool live = in && keep[in ? key : 0] != 0;
+				const bool live = in && (!keep || keep[in ? key : 0] != 0);
 				if(key < n_keys_tab) mask_tab[((key >> 5) * ROWS + r) * 32 + (key & 31)] = live ? (uint16_t)0 : (in ? MASK_DROPPED_BF16 : MASK_OUT_OF_RANGE_BF16);
 				const unsigned long long bal = __ballot(live);
 				if(bal) last = base + 64 - __builtin_clzll(bal);
@@ -334,45 +349,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 		if(lane == 0) s_last[r] = last, s_first[r] = first;
 	}
 	if(tid == 0) s_again = 0;
-	asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wavefront's pieces of the first tile and its bias fragment have landed
-	__syncthreads();                                    // the mask table and the first tile are complete
-	// keys behind the last live key of every row carry weight 0 and are not walked; a row without live keys needs them all
-	// The softmax reference of a batch row is fixed by the first tile that holds a live key of that row (a tile of dropped
-	// keys says nothing about the row's logits): tiles up to the last such tile over the group's rows (normally tile 0 alone)
-	// run the variant of the tile code that can do so.
-	int  l_eff = 0, t_force_max = 0;
-	bool dropped[ROWS];
-	uint32_t first_tiles = 0;   // byte r: the first tile of batch row r that holds a live key (at most 128 tiles)
-#pragma unroll
-	for(int r = 0; r < ROWS; r++) {
-		const int last = __builtin_amdgcn_readfirstlane(s_last[r]);
-		dropped[r]     = last == 0;
-		const int need = dropped[r] ? (int)L : last;
-		l_eff          = need > l_eff ? need : l_eff;
-		const int ft   = dropped[r] ? 0 : __builtin_amdgcn_readfirstlane(s_first[r]);
-		first_tiles |= (uint32_t)ft << (8 * r);
-		t_force_max    = ft > t_force_max ? ft : t_force_max;
-	}
-	n_t = (l_eff + KT_R - 1) / KT_R;
-
-	// Q fragments (B operand of S^T = K.Q^T): lane (q = n, g = half) holds q[q][16c + 8g .. +7], scaled by
-	// softmax_scale * log2 e in fp32 and rounded once to bf16 (the reference rounds the scaled q too,
-	// src/csrc/dot_product_attention.cpp:95-98).  A batch row without live keys gets q = 0.
-	bf16x8 qf[ROWS][2];
-#pragma unroll
-	for(int r = 0; r < ROWS; r++) {
-		const float qmul = dropped[r] ? 0.f : p.softmax_scale * LOG2E;
-#pragma unroll
-		for(int c = 0; c < 2; c++) {
-			u32x4 sc4;
-#pragma unroll
-			for(int j = 0; j < 4; j++) {
-				const uint32_t w = qraw[r][c][j];
-				sc4[j] = pack_bf16x2(bf16_bits_to_f32(w & 0xffffu) * qmul, bf16_bits_to_f32(w >> 16) * qmul);
-			}
-			qf[r][c] = __builtin_bit_cast(bf16x8, sc4);
-		}
-	}
 	// Operands of the mask MFMA (v_mfma_f32_32x32x8_bf16: four contraction slots per half-wave, two registers per operand).
 	// A (per key): slot 0 = the key's mask value (from the table, zero-extended), slots 2 and 3 = 1.0.
 	// B (per query): slot 0 = 1.0, slots 2 and 3 = -m_hi and -m_lo, the softmax reference of this lane's query row as two
@@ -396,12 +372,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 	const int mask_rd = MASK_BASE + n * 2;               // + ((tile * ROWS + row) * 32) * 2
 	const int slot_rd = SLOT_BASE + wave * 4096 + lane * 16;  // + 1024 per group of four accumulator registers
 
-	// ---- online-softmax state: one query row per lane and batch row (the two half-waves hold disjoint keys) ----
-	float  m_ref[ROWS];   // reference maximum, log2 units, exactly m_hi + m_lo of two bf16 values
-	float  lsum[ROWS];    // the row sum (complete: the same value in both half-waves)
-	float  rs_prev;       // the previous step's share of it (quick walk)
-	f32x16 oacc[ROWS];
-
 	// Row sums on the matrix pipe (see dpa_mfma.hip): a 16x16x32 MFMA whose A operand is this 0/1 pattern leaves, in
 	// register 0 of every lane, the sum of the 16 packed probabilities of that lane's own query row over both half-waves.
 	u32x4 ones_a;
@@ -411,6 +381,55 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 		const uint32_t w   = on ? 0x3F803F80u : 0u;
 		ones_a = u32x4{w, w, w, w};
 	}
+
+	// Q fragments (B operand of S^T = K.Q^T): lane (q = n, g = half) holds q[q][16c + 8g .. +7], scaled by
+	// softmax_scale * log2 e in fp32 and rounded once to bf16 (the reference rounds the scaled q too,
+	// src/csrc/dot_product_attention.cpp:95-98).
+	bf16x8 qf[ROWS][2];
+#pragma unroll
+	for(int r = 0; r < ROWS; r++) {
+		const float qmul = p.softmax_scale * LOG2E;
+#pragma unroll
+		for(int c = 0; c < 2; c++) {
+			u32x4 sc4;
+#pragma unroll
+			for(int j = 0; j < 4; j++) {
+				const uint32_t w = qraw[r][c][j];
+				sc4[j] = pack_bf16x2(bf16_bits_to_f32(w & 0xffffu) * qmul, bf16_bits_to_f32(w >> 16) * qmul);
+			}
+			qf[r][c] = __builtin_bit_cast(bf16x8, sc4);
+		}
+	}
+	asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wavefront's pieces of the first tile and its bias fragment have landed
+	__syncthreads();                                    // the mask table and the first tile are complete
+	// keys behind the last live key of every row carry weight 0 and are not walked; a row without live keys needs them all
+	// The softmax reference of a batch row is fixed by the first tile that holds a live key of that row (a tile of dropped
+	// keys says nothing about the row's logits): tiles up to the last such tile over the group's rows (normally tile 0 alone)
+	// run the variant of the tile code that can do so.
+	int  l_eff = 0, t_force_max = 0;
+	bool dropped[ROWS];
+	uint32_t first_tiles = 0;   // byte r: the first tile of batch row r that holds a live key (at most 128 tiles)
+#pragma unroll
+	for(int r = 0; r < ROWS; r++) {
+		const int last = __builtin_amdgcn_readfirstlane(s_last[r]);
+		dropped[r]     = last == 0;
+		const int need = dropped[r] ? (int)L : last;
+		l_eff          = need > l_eff ? need : l_eff;
+		const int ft   = dropped[r] ? 0 : __builtin_amdgcn_readfirstlane(s_first[r]);
+		first_tiles |= (uint32_t)ft << (8 * r);
+		t_force_max    = ft > t_force_max ? ft : t_force_max;
+	}
+	n_t = (l_eff + KT_R - 1) / KT_R;
+
+	// a batch row without live keys gets q = 0
+#pragma unroll
+	for(int r = 0; r < ROWS; r++)
+		if(dropped[r]) qf[r][0] = qf[r][1] = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
+	// ---- online-softmax state: one query row per lane and batch row (the two half-waves hold disjoint keys) ----
+	float  m_ref[ROWS];   // reference maximum, log2 units, exactly m_hi + m_lo of two bf16 values
+	float  lsum[ROWS];    // the row sum (complete: the same value in both half-waves)
+	float  rs_prev;       // the previous step's share of it (quick walk)
+	f32x16 oacc[ROWS];
 
 	// Move the reference of batch row R for every query whose maximum is not within REF_SLACK of it (all queries when
 	// `force`), rescale what has been accumulated and re-express s relative to the new reference.

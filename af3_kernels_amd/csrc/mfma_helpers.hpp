@@ -18,6 +18,7 @@ typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
 typedef __attribute__((ext_vector_type(4), aligned(2))) uint32_t u32x4_any;
 typedef __attribute__((ext_vector_type(2), aligned(2))) uint32_t u32x2_any;
 typedef __attribute__((ext_vector_type(4), aligned(4))) float    f32x4_any;
+typedef __attribute__((aligned(1))) uint32_t u32_bytes;
 template <int V>
 using ic = std::integral_constant<int, V>;
 

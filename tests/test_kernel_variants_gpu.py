@@ -441,6 +441,32 @@ def test_shared_bias_quick_and_careful_walks(af3, oracle, B, H, L, D, kind):
     assert (np.abs(out - want) / scale).max() <= 2e-2
 
 
+@pytest.mark.parametrize("B,H,L,D", [(3, 2, 1, 32), (2, 1, 3, 16), (4, 2, 4, 32), (3, 2, 37, 32), (2, 2, 255, 24), (3, 1, 257, 32), (2, 1, 2047, 32), (2, 1, 2049, 32), (3, 1, 2306, 16)])
+@pytest.mark.parametrize("kind", ["random", "last", "head", "middle", "none", "bytes", "no mask"])
+def test_shared_bias_mask_rows(af3, oracle, B, H, L, D, kind):
+    """The shared-bias kernel's key masks: rows shorter than one load, at odd addresses, ending inside a load, longer than what is requested
+    ahead; the only live keys at either end; batch rows without any; keep bytes other than 1."""
+    g = torch.Generator().manual_seed(L + D)
+    q, k, v = (torch.randn(B, H, L, D, generator=g).to(torch.bfloat16) for _ in range(3))
+    bias = torch.randn(H, L, L, generator=g).to(torch.bfloat16)
+    keep = torch.rand(B, L + 1, generator=g)[:, 1:] < 0.8
+    if kind != "random":
+        keep[1] = False
+        keep[1, {"last": slice(L - 1, L), "head": slice(0, 1), "middle": slice(L // 2, L // 2 + 2)}.get(kind, slice(0, 0))] = True
+    dev = keep.to(torch.uint8).mul(0x80).cuda().view(torch.bool) if kind == "bytes" else keep.cuda()
+    prev = af3.set_rows_kernel("always")
+    try:
+        print("case", B, H, L, D, kind, flush=True)
+        out = f32np(af3.dot_product_attention_cpp(q.cuda(), k.cuda(), v.cuda(), None if kind == "no mask" else dev, bias.cuda()))
+        torch.cuda.synchronize()
+    finally:
+        af3.set_rows_kernel(prev)
+    if kind == "no mask":
+        keep = torch.ones(B, L, dtype=torch.bool)
+    want = oracle.dpa_formula(f32np(q), f32np(k), f32np(v), keep.numpy(), f32np(bias))
+    assert np.abs(out - want).max() <= 2e-2   # (bf16 q, k, v and probabilities; |v| < 5)
+
+
 @pytest.mark.parametrize("B,H,L,D", [
     (1, 1, 32, 24), (2, 3, 33, 8), (1, 16, 50, 48), (5, 4, 63, 32), (37, 4, 37, 32),   # four wavefronts, one to three blocks of 16 rows; lengths around a tile
     (1, 16, 257, 32), (1, 16, 290, 24), (1, 16, 513, 48), (1, 16, 640, 40), (1, 5, 1155, 16),   # eight
