@@ -13,7 +13,7 @@
 // whose diagonal is 1/alpha (a power of two, exact in bf16), the key mask a third MFMA, in tiles that drop a key;
 // P^T = exp(logit - m) * 2^8 is quantised to e4m3 in registers (values in (0, 256], e4m3 tops out at
 // 448) and is the B operand of O^T += V8^T . P^T.  The row maximum m is the true running maximum
-// (no slack: P must stay below the e4m3 range), the row sum is taken over the quantised P, on the matrix pipe.
+// (no slack: P must stay below the e4m3 range, and the largest P, exactly 256, is rounded best), the row sum is taken over the quantised P, on the matrix pipe.
 //
 // What bounds it: the vector port (16 fma, 16 exponentials, 8 packs, a dozen maxima and, while maxima still move, 17 products
 // per 32 x 32 logits), then the matrix pipe (256 to 288 clocks), shared by up to four wavefronts per SIMD; everything else must
@@ -59,7 +59,7 @@ __device__ __forceinline__ float max3(float a, float b, float c) {   // (written
 // BMODE: 0 = no bias, 1 = element by element (a head's slab beyond 32-bit offsets), 2 = through LDS, rows of whole aligned
 // 16-byte chunks, 3 = through LDS, rows that start at any element.
 template <int DP, bool COMP, bool ONES, int BMODE>
-__global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(DP == 32 ? 4 : 3))) dpa_mfma_fp8_kernel(af3_dpa_params p, int n_qtiles, int64_t n_groups) {
+__global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(DP == 32 ? 4 : 3))) dpa_mfma_fp8_kernel(af3_dpa_params p, int n_qtiles, int n_units, int per_xcd) {
 	constexpr int NDB      = DP / 32;       // 32-row blocks of O^T
 	constexpr int K_TILE1  = KT8 * DP;      // bytes of one K tile
 	constexpr int K_TILE   = K_TILE1 * (COMP ? 2 : 1);  // hi tile followed by the residual tile
@@ -77,20 +77,26 @@ __global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(D
 	int16_t* const       live_list = reinterpret_cast<int16_t*>(mask_tab + n_ktiles * KT8) + 4;
 	int32_t* const       counts    = reinterpret_cast<int32_t*>(mask_tab + n_ktiles * KT8);   // [0] any live key, [1] tiles to walk (a static array would cost 1 KB)
 
-	// workgroup -> (batch, head, query tile), all query tiles of one (batch, head) on one XCD
+	// workgroup -> (batch row, head, query tile)
 	// the kernel arguments that the start of a workgroup needs, requested in one batch (otherwise: the launch counts, a wait,
 	// the early exit, and only then the fields of p -- memory latencies in a row that a small launch cannot hide)
-	asm volatile("" ::"s"(n_qtiles), "s"(n_groups), "s"(p.q), "s"(p.k), "s"(p.v), "s"(p.bias), "s"(p.key_mask), "s"(p.H), "s"(p.L), "s"(p.D), "s"(p.key_mask_stride_b),
+	asm volatile("" ::"s"(n_qtiles), "s"(n_units), "s"(per_xcd), "s"(p.B), "s"(p.q), "s"(p.k), "s"(p.v), "s"(p.bias), "s"(p.key_mask), "s"(p.H), "s"(p.L), "s"(p.D), "s"(p.key_mask_stride_b),
 				 "s"(p.bias_stride[0]), "s"(p.bias_stride[1]), "s"(p.device_descales), "s"(p.k_lo));
 	asm volatile("" ::"s"(p.q_stride[0]), "s"(p.q_stride[1]), "s"(p.q_stride[2]), "s"(p.k_stride[0]), "s"(p.k_stride[1]), "s"(p.k_stride[2]), "s"(p.v_stride[0]), "s"(p.v_stride[1]),
 				 "s"(p.v_stride[2]));
-	const int64_t wg    = blockIdx.x;
-	const int     xcd   = (int)(wg & 7);
-	const int64_t slot  = wg >> 3;
-	const int64_t group = (slot / n_qtiles) * 8 + xcd;
-	const int     qtile = (int)(slot % n_qtiles);
-	if(group >= n_groups) return;
-	const int64_t b = group / p.H, h = group % p.H;
+	uint32_t       b_u, h_u, qtile_u;
+	const uint32_t xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+	if(per_xcd > 0) {   // blocks of query rows in one run per XCD, the batch rows of a block next to each other
+		const uint32_t part = slot / (uint32_t)p.B, block = xcd * (uint32_t)per_xcd + part;
+		if(block >= (uint32_t)n_units) return;
+		h_u = block / (uint32_t)n_qtiles, qtile_u = block - h_u * (uint32_t)n_qtiles, b_u = slot - part * (uint32_t)p.B;
+	} else {   // (batch row, head) pairs dealt to the XCDs, a pair's query tiles next to each other
+		const uint32_t part = slot / (uint32_t)n_qtiles, group = part * 8 + xcd;
+		if(group >= (uint32_t)n_units) return;
+		b_u = group / (uint32_t)p.H, h_u = group - b_u * (uint32_t)p.H, qtile_u = slot - part * (uint32_t)n_qtiles;
+	}
+	const int64_t b = b_u, h = h_u;
+	const int     qtile = (int)qtile_u;
 
 	const int     tid = threadIdx.x, lane = tid & 63;
 	const int     wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -385,8 +391,7 @@ __global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(D
 		constexpr int I = decltype(i_c)::value;
 		const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[4 * I], c_exp, -mc)), p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[4 * I + 1], c_exp, -mc));
 		const float p2 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[4 * I + 2], c_exp, -mc)), p3 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[4 * I + 3], c_exp, -mc));
-		int w;
-		asm("" : "=v"(w));   // (both halves are written)
+		int w = __float_as_int(p0);   // (both halves are written)
 		w = __builtin_amdgcn_cvt_pk_fp8_f32(p0, p1, w, false);
 		w = __builtin_amdgcn_cvt_pk_fp8_f32(p2, p3, w, true);
 		pf[I >> 1][I & 1] = (uint32_t)w;
@@ -408,9 +413,9 @@ __global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(D
 		mx0 = max3(mx0, sc[6], sc[7]), mx1 = max3(mx1, sc[8], sc[9]);
 		mx0 = max3(mx0, sc[10], sc[11]), mx1 = max3(mx1, sc[12], sc[13]);
 		mx0 = max3(mx0, sc[14], sc[15]);
-		mx0 = fmaxf(mx0, mx1);
+		mx0 = max3(mx0, mx1, m_run);
 		const auto  sw    = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx0), __float_as_uint(mx0), false, false);
-		const float m_new = max3(m_run, __uint_as_float(sw[0]), __uint_as_float(sw[1]));
+		const float m_new = max3(mx0, __uint_as_float(sw[0]), __uint_as_float(sw[1]));
 		if(__ballot(m_new > m_run)) {   // (the first time from -inf: the factor is 0, and nothing has been accumulated)
 			const float a = __builtin_amdgcn_exp2f((m_run - m_new) * c_exp);
 			if constexpr(!ONES) lacc[0] *= a;
@@ -562,13 +567,17 @@ template <int DP, bool COMP, bool ONES, int BMODE>
 int launch8(const af3_dpa_params& p, hipStream_t s) {
 	const int     n_qtiles = (int)((p.L + NW8 * 32 - 1) / (NW8 * 32));
 	const int     n_ktiles = (int)((p.L + KT8 - 1) / KT8);
-	const int64_t n_groups = p.B * p.H;
-	const int64_t blocks   = ((n_groups + 7) / 8) * 8 * n_qtiles;
+	// The batch rows share the bias: with a bias to share, the workgroups of one block of query rows run side by side on one XCD, whose L2
+	// then serves all but the first of them.  Fewer than 64 such blocks fill the XCDs unevenly and are dealt by (batch row, head).
+	// (16 heads of 24, 1536 rows, us per call, pairs / blocks: 5 batch rows 76.8 / 75.2, 8 106.9 / 102.5; 8 of 1301 102.0 / 100.2.)
+	const int64_t n_blocks = p.H * n_qtiles, n_groups = p.B * p.H;
+	const int64_t per_xcd  = p.bias && p.B > 1 && n_blocks >= 64 ? (n_blocks + 7) / 8 : 0;
+	const int64_t blocks   = per_xcd > 0 ? per_xcd * 8 * p.B : (n_groups + 7) / 8 * 8 * n_qtiles;
 	if(blocks <= 0 || blocks > 0x7fffffffLL) return AF3_ERR_BAD_SHAPE;
 	const size_t smem = (size_t)3 * (COMP ? 3 : 2) * KT8 * DP + (BMODE >= 2 ? NW8 * 2 * BIAS_HALF8 : 0) + (size_t)n_ktiles * KT8 * 2 + (size_t)n_ktiles * 2 + 16;
 	auto         kern = dpa_mfma_fp8_kernel<DP, COMP, ONES, BMODE>;
 	if(smem > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) return AF3_ERR_LAUNCH;
-	hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW8 * 64), smem, s, p, n_qtiles, n_groups);
+	hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW8 * 64), smem, s, p, n_qtiles, (int)(per_xcd > 0 ? n_blocks : n_groups), (int)per_xcd);
 	return launch_status();
 }
 template <int DP, bool COMP, bool ONES>

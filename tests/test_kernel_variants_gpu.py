@@ -170,6 +170,21 @@ def test_projection_forms(af3, M, N, K, form, with_row):
     assert bool((out[M] == 7.0).all())
 
 
+@pytest.mark.parametrize("B,H,L,D", [(2, 64, 20, 24), (3, 33, 130, 24), (2, 9, 1000, 16), (5, 16, 512, 32), (7, 13, 641, 48)])   # from 64 blocks of 128 rows on, numbers of them that 8 does not divide
+def test_fp8_batch_rows_side_by_side(af3, B, H, L, D):
+    """Workgroups dealt by blocks of query rows compute what those of single batch rows do, dealt by heads: the same bits."""
+    g = torch.Generator().manual_seed(L + D)
+    q, k, v = (torch.randn(B, H, L, D, generator=g).clamp(-3.9, 3.9).to(torch.bfloat16).cuda() for _ in range(3))
+    for t in (q, k, v):
+        t[:, 0, 0, 0] = 4.0   # (one scale for every batch row)
+    bias = torch.randn(H, L, L, generator=g).to(torch.bfloat16).cuda()
+    keep = (torch.rand(L, generator=g) < 0.8).cuda()
+    print("case", B, H, L, D, flush=True)
+    out = af3.dot_product_attention_fp8(q, k, v, keep, bias)
+    for b in range(B):
+        assert torch.equal(out[b:b + 1], af3.dot_product_attention_fp8(q[b:b + 1], k[b:b + 1], v[b:b + 1], keep, bias))
+
+
 @pytest.mark.parametrize("compensated", [True, False])
 @pytest.mark.parametrize("B,H,L,D,mask_kind", [
     (1, 1, 1, 24, "none"), (2, 3, 33, 24, "random"), (1, 2, 64, 32, "none"), (2, 2, 65, 16, "tail"), (3, 2, 127, 48, "random"), (1, 3, 128, 64, "tail"),
