@@ -44,7 +44,7 @@ constexpr int NW8   = 4;     // wavefronts per workgroup (32 query rows each)
 constexpr int MAX_L8 = 8192;
 constexpr float P_SHIFT = 8.f;  // P is stored as p * 2^8
 constexpr int BIAS_HALF8 = 2048 + 128;   // 32 rows x 32 keys of bf16, and one dword per row behind them (rows that start at any element)
-constexpr int16_t TILE_FULL = 0x4000;    // flag in a tile list entry: no key of the tile is dropped
+constexpr int TILE_FULL = 0x4000;    // flag beside a tile's number: no key of the tile is dropped
 typedef __attribute__((ext_vector_type(8))) int i32x8;
 
 __device__ __forceinline__ float max3(float a, float b, float c) {   // (written out: fmaxf quiets its operands first)
@@ -69,13 +69,12 @@ __global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(D
 	constexpr bool RING    = BMODE >= 2, RAGGED = BMODE == 3;
 
 	extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-	// [3][K tile, V^T tile] [two half slots of bias per wavefront] [mask table: bf16 bits per key] [tile list]
+	// [3][K tile, V^T tile] [two half slots of bias per wavefront] [mask table: bf16 bits per key] [tile flags]
 	constexpr int        SLOT_BASE = 3 * TILE;
 	constexpr int        MASK_BASE = SLOT_BASE + (RING ? NW8 * 2 * BIAS_HALF8 : 0);
 	uint16_t* const      mask_tab  = reinterpret_cast<uint16_t*>(smem + MASK_BASE);
 	const int            n_ktiles  = (int)((p.L + KT8 - 1) / KT8);
-	int16_t* const       live_list = reinterpret_cast<int16_t*>(mask_tab + n_ktiles * KT8) + 4;
-	int32_t* const       counts    = reinterpret_cast<int32_t*>(mask_tab + n_ktiles * KT8);   // [0] any live key, [1] tiles to walk (a static array would cost 1 KB)
+	uint8_t* const       tile_flags = reinterpret_cast<uint8_t*>(mask_tab + n_ktiles * KT8);   // per tile: bit 0 a live key, bit 1 a key that is not
 
 	// workgroup -> (batch row, head, query tile)
 	// the kernel arguments that the start of a workgroup needs, requested in one batch (otherwise: the launch counts, a wait,
@@ -188,21 +187,28 @@ __global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(D
 			if(half == 0) lds_dma_b32(b_rsrc, slot_addr + sub * BIAS_HALF8 + 2048, b_tail + off);
 	};
 
-	// ---- requested first: the key-mask bytes (four keys per lane and load where rows allow), q, and -- once the buffers are cleared -- the
-	// first tile and its bias, on the guess that it holds a live key ----
-	const uint8_t* keep     = p.key_mask ? p.key_mask + b * p.key_mask_stride_b : nullptr;
-	const bool     mask_vec = !keep || (((reinterpret_cast<uintptr_t>(p.key_mask) | (uintptr_t)p.key_mask_stride_b | (uintptr_t)L) & 3) == 0);
-	const int      n_chunks = (n_ktiles * KT8 + 255) / 256;
-	uint32_t       mraw[2];
-	auto request_mask = [&](int c0) {
+	// ---- requested first: the first tile and its bias (on the guess that it holds a live key), the key-mask bytes, q, the scales.  A workgroup's
+	// start is bound by these latencies and by its instructions (a lone wavefront issues one in about 4.5 clocks): hence no barrier
+	// in front of the loads, four mask bytes at a time at any address, and no list of tiles but a bit for each.  16 heads of 24, us
+	// per call before / after: 1x128 12.3 / 11.7, 5x300 19.1 / 18.4, 2x777 27.1 / 25.9, 8x1301 99.0 / 97.0, 5x1536 70.0 / 69.5 ----
+	load_tile(0, 0);
+	load_bias(0, 0);
+	load_bias(0, 1);
+	const uint8_t* const keep     = p.key_mask ? p.key_mask + b * p.key_mask_stride_b : nullptr;
+	const bool           mask_vec = L >= 4;   // four keys per lane and load at any address (the last four of a row that L ends in the middle of are shifted)
+	const int            n_chunks = (n_ktiles * KT8 + 255) / 256;
+	uint32_t             mraw[2];
+	auto request_mask = [&](int c0) {   // chunk c: keys 256 c + 4 lane .. + 3
 #pragma unroll
 		for(int i = 0; i < 2; i++) {
-			const int64_t key0 = (int64_t)(c0 + i * NW8) * 256 + 4 * lane;
-			mraw[i]            = 0u;
-			if(c0 + i * NW8 < n_chunks) mraw[i] = !keep ? 0x01010101u : (key0 < L ? *reinterpret_cast<const uint32_t*>(keep + key0) : 0u);
+			const int key0 = (c0 + i * NW8) * 256 + 4 * lane;
+			mraw[i]        = 0x01010101u;
+			if(keep && (c0 + i * NW8) * 256 < (int)L) mraw[i] = *reinterpret_cast<const u32_bytes*>(keep + (key0 + 4 <= (int)L ? key0 : (int)L - 4));
 		}
 	};
 	if(mask_vec) request_mask(wave);
+	float dq = p.q_descale, dk = p.k_descale, dv = p.v_descale;   // real = stored * descale
+	if(p.device_descales) dq = p.device_descales[0], dk = p.device_descales[1], dv = p.device_descales[2];
 	// q operands of the 64-deep instruction: lane (q, g = half) holds columns [32 g, ..) of q8 and q_lo (DP = 64), or all 32 columns
 	// of q8 in both half-waves (not compensated: in the lower) and of q_lo in the lower (DP = 32); zeros elsewhere
 	i32x8 qa, qb;
@@ -217,20 +223,24 @@ __global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(D
 			qa[2 * c] = (int)x[0], qa[2 * c + 1] = (int)x[1], qb[2 * c] = (int)y[0], qb[2 * c + 1] = (int)y[1];
 		}
 	}
-	for(int i = tid; i < SLOT_BASE / 16; i += NW8 * 64) reinterpret_cast<u32x4*>(smem)[i] = u32x4{0u, 0u, 0u, 0u};
-	__syncthreads();
-	load_tile(0, 0);
-	load_bias(0, 0);
-	load_bias(0, 1);
-	if constexpr(ONES) {   // (e4m3 1.0; no load writes these rows)
-		if(tid < 96) {
-			const int buf = tid >> 5, r = (tid >> 4) & 1, w = tid & 15;
-			reinterpret_cast<uint32_t*>(smem + buf * TILE + K_TILE + (D + 4 * r) * KT8)[w] = 0x38383838u;
+	// what no load writes of the tiles: head columns past the chunk that holds the last one (zeros: a stale byte there must not be a NaN
+	// pattern) and rows from D on of V^T (zeros, and for the row sums e4m3 1.0 in rows D and D + 4)
+	if(tid < (DP - D) * (KT8 / 16)) {   // (at most 96)
+		const uint32_t w = ONES && ((tid >> 2) & ~4) == 0 ? 0x38383838u : 0u;
+#pragma unroll
+		for(int buf = 0; buf < 3; buf++) reinterpret_cast<u32x4*>(smem + buf * TILE + K_TILE + D * KT8)[tid] = u32x4{w, w, w, w};
+	}
+	if(D <= DP - 16) {
+		for(int i = tid; i < 3 * K_TILE / 16; i += NW8 * 64) {
+			const int buf = i / (K_TILE / 16), u = i - buf * (K_TILE / 16), row = (u / KCPR) % KT8;
+			if((((u % KCPR) ^ k_sw(row)) << 4) >= D) reinterpret_cast<u32x4*>(smem + buf * TILE)[u] = u32x4{0u, 0u, 0u, 0u};
 		}
 	}
 
-	// ---- key-mask table, flags of the tiles with a live key, list of those tiles ----
-	auto flag_of = [&](bool any_live, bool any_not) -> int16_t { return (int16_t)((any_live ? 1 : 0) | (any_not ? 0 : TILE_FULL)); };
+	const float alpha = dq * dk * p.softmax_scale;  // logits = alpha * (q8 . k8) + bias
+	const float c_exp = alpha * LOG2E;              // exp(logit - m) = exp2(acc*c_exp - m_acc*c_exp), m_acc in accumulator units
+
+	// ---- key-mask table and tile flags ----
 	if(mask_vec) {
 		for(int c0 = wave; c0 < n_chunks; c0 += 2 * NW8) {
 			if(c0 != wave) request_mask(c0);
@@ -238,58 +248,48 @@ __global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(D
 			for(int i = 0; i < 2; i++) {
 				const int c = c0 + i * NW8;
 				if(c >= n_chunks) break;
-				const int key0 = c * 256 + 4 * lane;
-				uint32_t  e[4];
-				bool      any = false, all = true;
-#pragma unroll
-				for(int j = 0; j < 4; j++) {
-					const bool in   = key0 + j < (int)L;
-					const bool live = in && ((mraw[i] >> (8 * j)) & 0xffu) != 0;
-					any             = any || live, all = all && live;
-					e[j]            = live ? 0u : (in ? (uint32_t)MASK_DROPPED_BF16 : (uint32_t)MASK_OUT_OF_RANGE_BF16);
+				const int key0 = c * 256 + 4 * lane, over = key0 + 4 - (int)L;
+				uint32_t  m    = mraw[i];
+				if(over > 0) m = over < 4 ? m >> (8 * over) : 0u;
+				const uint32_t gone = (~(((m & 0x7f7f7f7fu) + 0x7f7f7f7fu) | m) >> 7) & 0x01010101u;   // 1 in the bytes that are zero
+				uint32_t       lo = ((gone & 1u) | ((gone & 0x100u) << 8)) * MASK_DROPPED_BF16, hi = (((gone >> 16) & 1u) | ((gone >> 24) << 16)) * MASK_DROPPED_BF16;
+				if(over > 0) {
+					constexpr uint32_t OUT = MASK_OUT_OF_RANGE_BF16;   // keys from L on
+					lo = over <= 2 ? lo : over == 3 ? (lo & 0xffffu) | (OUT << 16) : OUT | (OUT << 16);
+					hi = over == 1 ? (hi & 0xffffu) | (OUT << 16) : OUT | (OUT << 16);
 				}
-				if(key0 < n_ktiles * KT8) *reinterpret_cast<u32x2*>(mask_tab + key0) = u32x2{e[0] | (e[1] << 16), e[2] | (e[3] << 16)};
-				const unsigned long long bal = __ballot(any), baln = __ballot(!all);   // 16 lanes per tile
-				if(lane < 4 && 4 * c + lane < n_ktiles) live_list[4 * c + lane] = flag_of(((bal >> (16 * lane)) & 0xffffull) != 0, ((baln >> (16 * lane)) & 0xffffull) != 0);
+				if(key0 < n_ktiles * KT8) *reinterpret_cast<u32x2*>(mask_tab + key0) = u32x2{lo, hi};
+				const unsigned long long bal = __ballot(m != 0u), baln = __ballot(gone != 0u);   // 16 lanes per tile (keys from L on are gone)
+				if(lane < 4 && 4 * c + lane < n_ktiles) tile_flags[4 * c + lane] = (uint8_t)((((bal >> (16 * lane)) & 0xffffull) != 0 ? 1 : 0) | (((baln >> (16 * lane)) & 0xffffull) != 0 ? 2 : 0));
 			}
 		}
-	} else {
-		for(int kt = wave; kt < n_ktiles; kt += NW8) {
-			const int64_t key  = (int64_t)kt * KT8 + lane;
-			const bool    in   = key < L;
-			const bool    live = in && keep[in ? key : 0] != 0;
-			mask_tab[kt * KT8 + lane] = live ? (uint16_t)0 : (in ? MASK_DROPPED_BF16 : MASK_OUT_OF_RANGE_BF16);
-			const unsigned long long bal = __ballot(live);
-			if(lane == 0) live_list[kt] = flag_of(bal != 0, bal != ~0ull);
-		}
+	} else if(wave == 0) {   // (a single tile)
+		const bool in = lane < (int)L, live = in && (!keep || keep[in ? lane : 0] != 0);
+		mask_tab[lane] = live ? (uint16_t)0 : (in ? MASK_DROPPED_BF16 : MASK_OUT_OF_RANGE_BF16);
+		const bool any = __ballot(live) != 0;
+		if(lane == 0) tile_flags[0] = any ? 3 : 2;
 	}
 	__syncthreads();
-	if(wave == 0) {
-		bool any_live = false;
-		for(int base = 0; base < n_ktiles; base += 64) any_live = any_live || __ballot(base + lane < n_ktiles && (live_list[base + lane] & 1) != 0) != 0;
-		const bool all = !any_live;   // no key is live: every tile is kept, the result is the mean over all L keys
-		int        cnt = 0;
-		for(int base = 0; base < n_ktiles; base += 64) {
-			const int     kt     = base + lane;
-			const int16_t f      = kt < n_ktiles ? live_list[kt] : (int16_t)0;
-			const bool    keepit = kt < n_ktiles && (all || (f & 1) != 0);
-			const unsigned long long bal = __ballot(keepit);
-			const int rank = __builtin_amdgcn_mbcnt_hi((unsigned)(bal >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)bal, 0));
-			__builtin_amdgcn_wave_barrier();
-			if(keepit) live_list[cnt + rank] = (int16_t)(kt | (f & TILE_FULL));
-			cnt += __builtin_popcountll(bal);
-		}
-		if(lane == 0) counts[0] = any_live ? 1 : 0, counts[1] = cnt;
+	// the tiles to walk, as bits (at most 128 tiles)
+	unsigned long long todo[2], part[2];
+#pragma unroll
+	for(int i = 0; i < 2; i++) {
+		const int f = 64 * i + lane < n_ktiles ? tile_flags[64 * i + lane] : 2;
+		todo[i] = __ballot((f & 1) != 0), part[i] = __ballot((f & 2) != 0);
 	}
-	__syncthreads();
-	const int  nlive       = __builtin_amdgcn_readfirstlane(counts[1]);
-	const bool all_dropped = __builtin_amdgcn_readfirstlane(counts[0]) == 0;
-
-	// scales: real = stored * descale
-	float dq = p.q_descale, dk = p.k_descale, dv = p.v_descale;
-	if(p.device_descales) dq = p.device_descales[0], dk = p.device_descales[1], dv = p.device_descales[2];
-	const float alpha = dq * dk * p.softmax_scale;  // logits = alpha * (q8 . k8) + bias
-	const float c_exp = alpha * LOG2E;              // exp(logit - m) = exp2(acc*c_exp - m_acc*c_exp), m_acc in accumulator units
+	const bool all_dropped = (todo[0] | todo[1]) == 0;   // no key is live: every tile is walked, the result is the mean over all L keys
+	if(all_dropped) todo[0] = __ballot(lane < n_ktiles), todo[1] = __ballot(64 + lane < n_ktiles);
+	const int nlive = __builtin_popcountll(todo[0]) + __builtin_popcountll(todo[1]);
+	int       entry_last = 0;
+	auto next_entry = [&]() -> int {   // the next tile's number and flag; behind the last one: that one again
+		const int i = todo[0] == 0 ? 1 : 0;
+		if(todo[i] != 0) {
+			const int t = __builtin_ctzll(todo[i]);
+			entry_last  = (64 * i + t) | ((part[i] >> t) & 1 ? 0 : TILE_FULL);
+			todo[i] &= todo[i] - 1;
+		}
+		return entry_last;
+	};
 
 	if(all_dropped) {
 #pragma unroll
@@ -476,8 +476,7 @@ __global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(D
 	};
 
 	// ---- prologue: first tile, its first logits; second tile under way ----
-	auto entry_at = [&](int j) -> int { return __builtin_amdgcn_readfirstlane((int)live_list[j < nlive ? j : nlive - 1]); };
-	int entry = entry_at(0), entry1 = entry_at(1);
+	int entry = next_entry(), entry1 = next_entry();
 	if((entry & ~TILE_FULL) != 0) {   // (the guess was wrong; loads land in issue order)
 		load_tile(entry & ~TILE_FULL, 0);
 		load_bias(entry & ~TILE_FULL, 0);
@@ -511,7 +510,7 @@ __global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(D
 		const int  kt = entry & ~TILE_FULL, kt1 = entry1 & ~TILE_FULL;
 		const int  nxt = cur == 2 * TILE ? 0 : cur + TILE, nxt2 = nxt == 2 * TILE ? 0 : nxt + TILE;
 		const bool has1 = it + 1 < nlive, has2 = it + 2 < nlive;
-		const int  entry2 = entry_at(it + 2);
+		const int  entry2 = next_entry();
 		// the second half of this tile's bias has landed (younger: tile it + 1 and the first half of its bias)
 		if(has1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(KV_MIN + BIAS_LOADS) : "memory");
 		else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -574,7 +573,7 @@ int launch8(const af3_dpa_params& p, hipStream_t s) {
 	const int64_t per_xcd  = p.bias && p.B > 1 && n_blocks >= 64 ? (n_blocks + 7) / 8 : 0;
 	const int64_t blocks   = per_xcd > 0 ? per_xcd * 8 * p.B : (n_groups + 7) / 8 * 8 * n_qtiles;
 	if(blocks <= 0 || blocks > 0x7fffffffLL) return AF3_ERR_BAD_SHAPE;
-	const size_t smem = (size_t)3 * (COMP ? 3 : 2) * KT8 * DP + (BMODE >= 2 ? NW8 * 2 * BIAS_HALF8 : 0) + (size_t)n_ktiles * KT8 * 2 + (size_t)n_ktiles * 2 + 16;
+	const size_t smem = (size_t)3 * (COMP ? 3 : 2) * KT8 * DP + (BMODE >= 2 ? NW8 * 2 * BIAS_HALF8 : 0) + (size_t)n_ktiles * KT8 * 2 + (size_t)((n_ktiles + 15) & ~15);
 	auto         kern = dpa_mfma_fp8_kernel<DP, COMP, ONES, BMODE>;
 	if(smem > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) return AF3_ERR_LAUNCH;
 	hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW8 * 64), smem, s, p, n_qtiles, (int)(per_xcd > 0 ? n_blocks : n_groups), (int)per_xcd);

@@ -170,6 +170,30 @@ def test_projection_forms(af3, M, N, K, form, with_row):
     assert bool((out[M] == 7.0).all())
 
 
+@pytest.mark.parametrize("B,H,L,D", [(1, 1, 1, 8), (1, 2, 3, 24), (2, 1, 4, 40), (1, 2, 63, 16), (1, 1, 257, 32), (2, 1, 1026, 24), (1, 1, 4161, 24), (1, 1, 8192, 24)])
+@pytest.mark.parametrize("kind", ["random", "first", "last", "one tile", "none", "bytes", "no mask"])
+def test_fp8_mask_rows(af3, B, H, L, D, kind):
+    """Mask rows shorter than one load, ending inside a load, of more than 64 tiles; rows with one live key or none; keep bytes other than 1."""
+    g = torch.Generator().manual_seed(L + D)
+    q, k, v = (torch.randn(B, H, L, D, generator=g).to(torch.bfloat16).cuda() for _ in range(3))
+    bias = torch.randn(H, L, L, generator=g).to(torch.bfloat16).cuda()
+    keep = torch.rand(L + 1, generator=g)[1:] < 0.8
+    if kind in ("first", "last", "one tile", "none"):
+        keep[:] = False
+        keep[{"first": slice(0, 1), "last": slice(L - 1, L), "one tile": slice(L // 2, L // 2 + 3), "none": slice(0, 0)}[kind]] = True
+    dev = keep.to(torch.uint8).mul(0x80).cuda().view(torch.bool) if kind == "bytes" else keep.cuda()
+    print("case", B, H, L, D, kind, flush=True)
+    out = af3.dot_product_attention_fp8(q, k, v, None if kind == "no mask" else dev, bias)
+    torch.cuda.synchronize()
+    keep = torch.ones(L, dtype=torch.bool) if kind == "no mask" else keep
+    vd, vs = af3.quantize_fp8_e4m3(v)
+    s = (q.float() * D ** -0.5).matmul(k.float().transpose(-1, -2).contiguous()) + bias.float()
+    p = (s.masked_fill(~keep.cuda(), float("-inf")) if keep.any() else torch.zeros_like(s)).softmax(-1)
+    # e4m3 weights: each within 2^-4 of itself, as in the test of the bias forms
+    bound = 2 ** -4 * p.matmul((vd.float() * vs).abs()) + 2e-2
+    assert bool(((out.float() - p.matmul(vd.float() * vs)).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("B,H,L,D", [(2, 64, 20, 24), (3, 33, 130, 24), (2, 9, 1000, 16), (5, 16, 512, 32), (7, 13, 641, 48)])   # from 64 blocks of 128 rows on, numbers of them that 8 does not divide
 def test_fp8_batch_rows_side_by_side(af3, B, H, L, D):
     """Workgroups dealt by blocks of query rows compute what those of single batch rows do, dealt by heads: the same bits."""
