@@ -58,8 +58,10 @@ __device__ __forceinline__ float max3(float a, float b, float c) {   // (written
 // ONES: head_dim < DP, row sums through P.V; otherwise two 16x16x32 instructions per 32 keys.
 // BMODE: 0 = no bias, 1 = element by element (a head's slab beyond 32-bit offsets), 2 = through LDS, rows of whole aligned
 // 16-byte chunks, 3 = through LDS, rows that start at any element.
-template <int DP, bool COMP, bool ONES, int BMODE>
-__global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(DP == 32 ? 4 : 3))) dpa_mfma_fp8_kernel(af3_dpa_params p, int n_qtiles, int n_units, int per_xcd) {
+// KS: 1, or the number of parts that the tiles of a block of query rows are dealt to, each with wavefronts and buffers of its own
+// (for launches of few workgroups); their sums are merged through LDS at the end.
+template <int DP, bool COMP, bool ONES, int BMODE, int KS>
+__global__ void __launch_bounds__(KS * NW8 * 64) __attribute__((amdgpu_waves_per_eu(DP == 32 ? 4 : KS == 1 ? 3 : 2))) dpa_mfma_fp8_kernel(af3_dpa_params p, int n_qtiles, int n_units, int per_xcd) {
 	constexpr int NDB      = DP / 32;       // 32-row blocks of O^T
 	constexpr int K_TILE1  = KT8 * DP;      // bytes of one K tile
 	constexpr int K_TILE   = K_TILE1 * (COMP ? 2 : 1);  // hi tile followed by the residual tile
@@ -69,9 +71,9 @@ __global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(D
 	constexpr bool RING    = BMODE >= 2, RAGGED = BMODE == 3;
 
 	extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-	// [3][K tile, V^T tile] [two half slots of bias per wavefront] [mask table: bf16 bits per key] [tile flags]
-	constexpr int        SLOT_BASE = 3 * TILE;
-	constexpr int        MASK_BASE = SLOT_BASE + (RING ? NW8 * 2 * BIAS_HALF8 : 0);
+	// [KS][3][K tile, V^T tile] [two half slots of bias per wavefront] [mask table: bf16 bits per key] [tile flags]
+	constexpr int        SLOT_BASE = KS * 3 * TILE;
+	constexpr int        MASK_BASE = SLOT_BASE + (RING ? KS * NW8 * 2 * BIAS_HALF8 : 0);
 	uint16_t* const      mask_tab  = reinterpret_cast<uint16_t*>(smem + MASK_BASE);
 	const int            n_ktiles  = (int)((p.L + KT8 - 1) / KT8);
 	uint8_t* const       tile_flags = reinterpret_cast<uint8_t*>(mask_tab + n_ktiles * KT8);   // per tile: bit 0 a live key, bit 1 a key that is not
@@ -98,7 +100,8 @@ __global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(D
 	const int     qtile = (int)qtile_u;
 
 	const int     tid = threadIdx.x, lane = tid & 63;
-	const int     wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+	const int     wave_all = __builtin_amdgcn_readfirstlane(tid >> 6), wave = wave_all % NW8, part = wave_all / NW8;
+	const int     buf0 = part * 3 * TILE;   // this part's first buffer
 	const int     n = lane & 31, half = lane >> 5;
 	const int64_t L = p.L;
 	const int     D = (int)p.D;
@@ -160,7 +163,7 @@ __global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(D
 	const int       b_odd  = RAGGED ? (int)(b_base & 2) : 0;
 	const u32x4     b_rsrc = raw_rsrc(reinterpret_cast<const void*>(b_base - b_odd), RING ? (uint32_t)((((L - 1) * p.bias_stride[1] + L) * 2 + b_odd + 3) & ~3ll) : 0u);
 	const int       b_row_bytes = (int)(p.bias_stride[1] * 2), q0 = qtile * (NW8 * 32) + wave * 32;
-	const uint32_t  slot_addr   = lds0 + SLOT_BASE + wave * (2 * BIAS_HALF8);
+	const uint32_t  slot_addr   = lds0 + SLOT_BASE + wave_all * (2 * BIAS_HALF8);
 	constexpr int   BIAS_LOADS  = RAGGED ? 3 : RING ? 2 : 0;
 	int b_voff[2] = {0, 0}, b_tail = 0;
 	const int b_chunk = (lane & 3) ^ ((lane >> 4) & 3);   // (row 16 j + lane / 4)
@@ -187,13 +190,14 @@ __global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(D
 			if(half == 0) lds_dma_b32(b_rsrc, slot_addr + sub * BIAS_HALF8 + 2048, b_tail + off);
 	};
 
-	// ---- requested first: the first tile and its bias (on the guess that it holds a live key), the key-mask bytes, q, the scales.  A workgroup's
+	// ---- requested first: the first tile and its bias (on the guess that the tiles up to it hold live keys), the key-mask bytes, q, the scales.  A workgroup's
 	// start is bound by these latencies and by its instructions (a lone wavefront issues one in about 4.5 clocks): hence no barrier
 	// in front of the loads, four mask bytes at a time at any address, and no list of tiles but a bit for each.  16 heads of 24, us
 	// per call before / after: 1x128 12.3 / 11.7, 5x300 19.1 / 18.4, 2x777 27.1 / 25.9, 8x1301 99.0 / 97.0, 5x1536 70.0 / 69.5 ----
-	load_tile(0, 0);
-	load_bias(0, 0);
-	load_bias(0, 1);
+	const int guess = part < n_ktiles ? part : 0;
+	load_tile(guess, buf0);
+	load_bias(guess, 0);
+	load_bias(guess, 1);
 	const uint8_t* const keep     = p.key_mask ? p.key_mask + b * p.key_mask_stride_b : nullptr;
 	const bool           mask_vec = L >= 4;   // four keys per lane and load at any address (the last four of a row that L ends in the middle of are shifted)
 	const int            n_chunks = (n_ktiles * KT8 + 255) / 256;
@@ -201,12 +205,12 @@ __global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(D
 	auto request_mask = [&](int c0) {   // chunk c: keys 256 c + 4 lane .. + 3
 #pragma unroll
 		for(int i = 0; i < 2; i++) {
-			const int key0 = (c0 + i * NW8) * 256 + 4 * lane;
+			const int key0 = (c0 + i * (KS * NW8)) * 256 + 4 * lane;
 			mraw[i]        = 0x01010101u;
-			if(keep && (c0 + i * NW8) * 256 < (int)L) mraw[i] = *reinterpret_cast<const u32_bytes*>(keep + (key0 + 4 <= (int)L ? key0 : (int)L - 4));
+			if(keep && (c0 + i * (KS * NW8)) * 256 < (int)L) mraw[i] = *reinterpret_cast<const u32_bytes*>(keep + (key0 + 4 <= (int)L ? key0 : (int)L - 4));
 		}
 	};
-	if(mask_vec) request_mask(wave);
+	if(mask_vec) request_mask(wave_all);
 	float dq = p.q_descale, dk = p.k_descale, dv = p.v_descale;   // real = stored * descale
 	if(p.device_descales) dq = p.device_descales[0], dk = p.device_descales[1], dv = p.device_descales[2];
 	// q operands of the 64-deep instruction: lane (q, g = half) holds columns [32 g, ..) of q8 and q_lo (DP = 64), or all 32 columns
@@ -228,10 +232,10 @@ __global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(D
 	if(tid < (DP - D) * (KT8 / 16)) {   // (at most 96)
 		const uint32_t w = ONES && ((tid >> 2) & ~4) == 0 ? 0x38383838u : 0u;
 #pragma unroll
-		for(int buf = 0; buf < 3; buf++) reinterpret_cast<u32x4*>(smem + buf * TILE + K_TILE + D * KT8)[tid] = u32x4{w, w, w, w};
+		for(int buf = 0; buf < 3 * KS; buf++) reinterpret_cast<u32x4*>(smem + buf * TILE + K_TILE + D * KT8)[tid] = u32x4{w, w, w, w};
 	}
 	if(D <= DP - 16) {
-		for(int i = tid; i < 3 * K_TILE / 16; i += NW8 * 64) {
+		for(int i = tid; i < KS * 3 * K_TILE / 16; i += KS * NW8 * 64) {
 			const int buf = i / (K_TILE / 16), u = i - buf * (K_TILE / 16), row = (u / KCPR) % KT8;
 			if((((u % KCPR) ^ k_sw(row)) << 4) >= D) reinterpret_cast<u32x4*>(smem + buf * TILE)[u] = u32x4{0u, 0u, 0u, 0u};
 		}
@@ -242,11 +246,11 @@ __global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(D
 
 	// ---- key-mask table and tile flags ----
 	if(mask_vec) {
-		for(int c0 = wave; c0 < n_chunks; c0 += 2 * NW8) {
-			if(c0 != wave) request_mask(c0);
+		for(int c0 = wave_all; c0 < n_chunks; c0 += 2 * KS * NW8) {
+			if(c0 != wave_all) request_mask(c0);
 #pragma unroll
 			for(int i = 0; i < 2; i++) {
-				const int c = c0 + i * NW8;
+				const int c = c0 + i * (KS * NW8);
 				if(c >= n_chunks) break;
 				const int key0 = c * 256 + 4 * lane, over = key0 + 4 - (int)L;
 				uint32_t  m    = mraw[i];
@@ -263,7 +267,7 @@ __global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(D
 				if(lane < 4 && 4 * c + lane < n_ktiles) tile_flags[4 * c + lane] = (uint8_t)((((bal >> (16 * lane)) & 0xffffull) != 0 ? 1 : 0) | (((baln >> (16 * lane)) & 0xffffull) != 0 ? 2 : 0));
 			}
 		}
-	} else if(wave == 0) {   // (a single tile)
+	} else if(wave_all == 0) {   // (a single tile)
 		const bool in = lane < (int)L, live = in && (!keep || keep[in ? lane : 0] != 0);
 		mask_tab[lane] = live ? (uint16_t)0 : (in ? MASK_DROPPED_BF16 : MASK_OUT_OF_RANGE_BF16);
 		const bool any = __ballot(live) != 0;
@@ -271,25 +275,33 @@ __global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(D
 	}
 	__syncthreads();
 	// the tiles to walk, as bits (at most 128 tiles)
-	unsigned long long todo[2], part[2];
+	unsigned long long todo[2], some[2];
 #pragma unroll
 	for(int i = 0; i < 2; i++) {
 		const int f = 64 * i + lane < n_ktiles ? tile_flags[64 * i + lane] : 2;
-		todo[i] = __ballot((f & 1) != 0), part[i] = __ballot((f & 2) != 0);
+		todo[i] = __ballot((f & 1) != 0), some[i] = __ballot((f & 2) != 0);
 	}
 	const bool all_dropped = (todo[0] | todo[1]) == 0;   // no key is live: every tile is walked, the result is the mean over all L keys
 	if(all_dropped) todo[0] = __ballot(lane < n_ktiles), todo[1] = __ballot(64 + lane < n_ktiles);
-	const int nlive = __builtin_popcountll(todo[0]) + __builtin_popcountll(todo[1]);
+	const int n_todo = __builtin_popcountll(todo[0]) + __builtin_popcountll(todo[1]);
+	const int nlive  = (n_todo - part + KS - 1) / KS, n_most = (n_todo + KS - 1) / KS;   // tiles of this part and of the first; they differ by one at most
 	int       entry_last = 0;
-	auto next_entry = [&]() -> int {   // the next tile's number and flag; behind the last one: that one again
+	auto pop = [&]() -> int {   // the next tile's number and flag; behind the last one: that one again
 		const int i = todo[0] == 0 ? 1 : 0;
 		if(todo[i] != 0) {
 			const int t = __builtin_ctzll(todo[i]);
-			entry_last  = (64 * i + t) | ((part[i] >> t) & 1 ? 0 : TILE_FULL);
+			entry_last  = (64 * i + t) | ((some[i] >> t) & 1 ? 0 : TILE_FULL);
 			todo[i] &= todo[i] - 1;
 		}
 		return entry_last;
 	};
+	auto next_entry = [&]() -> int {   // ... of this part
+		const int e = pop();
+#pragma unroll
+		for(int i = 1; i < KS; i++) pop();
+		return e;
+	};
+	for(int i = 0; i < part; i++) pop();
 
 	if(all_dropped) {
 #pragma unroll
@@ -315,7 +327,7 @@ __global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(D
 	const bool           has_bias = BMODE != 0 && !all_dropped;
 	const unsigned char* bias_row = BMODE == 1 ? static_cast<const unsigned char*>(p.bias) + (h * p.bias_stride[0] + (row_ok ? qrow : 0) * p.bias_stride[1]) * 2 : nullptr;
 	// half slot -> the two fragments of 32 keys: lane (n, half), fragment c2: keys 16 c2 + 8 half .. + 7 of query row n
-	const int b_rd    = SLOT_BASE + wave * (2 * BIAS_HALF8) + n * 64, b_sw = (n >> 2) & 3;
+	const int b_rd    = SLOT_BASE + wave_all * (2 * BIAS_HALF8) + n * 64, b_sw = (n >> 2) & 3;
 	const int b_shift = RAGGED ? 8 * ((b_odd + (int)(row_ok ? qrow : L - 1) * b_row_bytes) & 2) : 0;
 	u32x4     bfrag[2] = {u32x4{0u, 0u, 0u, 0u}, u32x4{0u, 0u, 0u, 0u}};
 	auto read_bias = [&](int kt, int sub) {
@@ -477,8 +489,8 @@ __global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(D
 
 	// ---- prologue: first tile, its first logits; second tile under way ----
 	int entry = next_entry(), entry1 = next_entry();
-	if((entry & ~TILE_FULL) != 0) {   // (the guess was wrong; loads land in issue order)
-		load_tile(entry & ~TILE_FULL, 0);
+	if((entry & ~TILE_FULL) != guess) {   // (the guess was wrong; loads land in issue order)
+		load_tile(entry & ~TILE_FULL, buf0);
 		load_bias(entry & ~TILE_FULL, 0);
 		load_bias(entry & ~TILE_FULL, 1);
 	}
@@ -488,15 +500,15 @@ __global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(D
 		read_bias(kt0, 0);
 		asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 		if(nlive > 1) {
-			load_tile(entry1 & ~TILE_FULL, TILE);
+			load_tile(entry1 & ~TILE_FULL, buf0 + TILE);
 			load_bias(entry1 & ~TILE_FULL, 0);
 		}
 #pragma unroll
 		for(int i = 0; i < 16; i++) sc[i] = 0.f;
-		const i32x8 ka = read_k(0, 0);
+		const i32x8 ka = read_k(buf0, 0);
 		sc = kq(ka, qa, sc);
 		if constexpr(COMP) {
-			if constexpr(DP == 64) sc = kq(read_k(0, 1), qa, sc);
+			if constexpr(DP == 64) sc = kq(read_k(buf0, 1), qa, sc);
 			sc = kq(ka, qb, sc);
 		}
 		if constexpr(BMODE != 0) sc = bias_mfma(bias_mfma(sc, 0), 1);
@@ -505,10 +517,10 @@ __global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(D
 	}
 	// Tile `it` is in buffer it % 3.  Order of this wavefront's loads: tile it + 1 (behind the barrier of iteration it - 1), its
 	// first half of bias (in the second stage of it - 1), its second half (in the first stage of it), tile it + 2, ...
-	int cur = 0;
+	int cur = buf0;
 	for(int it = 0; it < nlive; it++) {
 		const int  kt = entry & ~TILE_FULL, kt1 = entry1 & ~TILE_FULL;
-		const int  nxt = cur == 2 * TILE ? 0 : cur + TILE, nxt2 = nxt == 2 * TILE ? 0 : nxt + TILE;
+		const int  nxt = cur == buf0 + 2 * TILE ? buf0 : cur + TILE, nxt2 = nxt == buf0 + 2 * TILE ? buf0 : nxt + TILE;
 		const bool has1 = it + 1 < nlive, has2 = it + 2 < nlive;
 		const int  entry2 = next_entry();
 		// the second half of this tile's bias has landed (younger: tile it + 1 and the first half of its bias)
@@ -535,6 +547,39 @@ __global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(D
 		entry = entry1, entry1 = entry2, cur = nxt;
 	}
 
+	if constexpr(KS > 1) {
+		if(nlive < n_most) asm volatile("s_barrier" ::: "memory");   // (the barrier of the other parts' last tile)
+		// the other parts' O, l and m to the first, [wavefront of those][register / 4][lane] x 16 bytes
+		constexpr int REGS4 = 4 * NDB + 1;
+		static_assert((KS - 1) * NW8 * REGS4 * 1024 <= MASK_BASE, "the partial sums fit the buffers");
+		f32x4* const at = reinterpret_cast<f32x4*>(smem) + (part > 0 ? wave_all - NW8 : wave) * (REGS4 * 64) + lane;
+		__syncthreads();   // everyone is done with the buffers
+		if(part > 0) {
+#pragma unroll
+			for(int db = 0; db < NDB; db++)
+#pragma unroll
+				for(int i = 0; i < 4; i++) at[(4 * db + i) * 64] = f32x4{oacc[db][4 * i], oacc[db][4 * i + 1], oacc[db][4 * i + 2], oacc[db][4 * i + 3]};
+			at[4 * NDB * 64] = f32x4{m_run, lacc[0], 0.f, 0.f};
+		}
+		__syncthreads();
+		if(part > 0) return;
+#pragma unroll
+		for(int o = 0; o < KS - 1; o++) {   // (a part without tiles: m = -inf, factor 0)
+			const f32x4* const from = at + o * (NW8 * REGS4 * 64);
+			const f32x4        ml   = from[4 * NDB * 64];
+			const float        m_new = fmaxf(m_run, ml[0]), a = __builtin_amdgcn_exp2f((m_run - m_new) * c_exp), f = __builtin_amdgcn_exp2f((ml[0] - m_new) * c_exp);
+			m_run   = m_new;
+			lacc[0] = lacc[0] * a + ml[1] * f;
+#pragma unroll
+			for(int db = 0; db < NDB; db++)
+#pragma unroll
+				for(int i = 0; i < 4; i++) {
+					const f32x4 x = from[(4 * db + i) * 64];
+#pragma unroll
+					for(int j = 0; j < 4; j++) oacc[db][4 * i + j] = oacc[db][4 * i + j] * a + x[j] * f;
+				}
+		}
+	}
 	// epilogue: out = O * dv / l   (l was summed over p * 2^8, the same factor O carries; both half-waves are in it)
 	float l_tot = lacc[0];
 	if constexpr(ONES) {
@@ -562,8 +607,8 @@ __global__ void __launch_bounds__(NW8 * 64) __attribute__((amdgpu_waves_per_eu(D
 	}
 }
 
-template <int DP, bool COMP, bool ONES, int BMODE>
-int launch8(const af3_dpa_params& p, hipStream_t s) {
+template <int DP, bool COMP, bool ONES, int BMODE, int KS>
+int launch8_parts(const af3_dpa_params& p, hipStream_t s) {
 	const int     n_qtiles = (int)((p.L + NW8 * 32 - 1) / (NW8 * 32));
 	const int     n_ktiles = (int)((p.L + KT8 - 1) / KT8);
 	// The batch rows share the bias: with a bias to share, the workgroups of one block of query rows run side by side on one XCD, whose L2
@@ -573,11 +618,25 @@ int launch8(const af3_dpa_params& p, hipStream_t s) {
 	const int64_t per_xcd  = p.bias && p.B > 1 && n_blocks >= 64 ? (n_blocks + 7) / 8 : 0;
 	const int64_t blocks   = per_xcd > 0 ? per_xcd * 8 * p.B : (n_groups + 7) / 8 * 8 * n_qtiles;
 	if(blocks <= 0 || blocks > 0x7fffffffLL) return AF3_ERR_BAD_SHAPE;
-	const size_t smem = (size_t)3 * (COMP ? 3 : 2) * KT8 * DP + (BMODE >= 2 ? NW8 * 2 * BIAS_HALF8 : 0) + (size_t)n_ktiles * KT8 * 2 + (size_t)((n_ktiles + 15) & ~15);
-	auto         kern = dpa_mfma_fp8_kernel<DP, COMP, ONES, BMODE>;
+	const size_t smem = (size_t)KS * (3 * (COMP ? 3 : 2) * KT8 * DP + (BMODE >= 2 ? NW8 * 2 * BIAS_HALF8 : 0)) + (size_t)n_ktiles * KT8 * 2 + (size_t)((n_ktiles + 15) & ~15);
+	auto         kern = dpa_mfma_fp8_kernel<DP, COMP, ONES, BMODE, KS>;
 	if(smem > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) return AF3_ERR_LAUNCH;
-	hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NW8 * 64), smem, s, p, n_qtiles, (int)(per_xcd > 0 ? n_blocks : n_groups), (int)per_xcd);
+	hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(KS * NW8 * 64), smem, s, p, n_qtiles, (int)(per_xcd > 0 ? n_blocks : n_groups), (int)per_xcd);
 	return launch_status();
+}
+template <int DP, bool COMP, bool ONES, int BMODE>
+int launch8(const af3_dpa_params& p, hipStream_t s) {
+	// Launches of few workgroups: two parts.  A lone wavefront of a SIMD takes 1070 clocks for a stage, of which its 175 instructions are 790,
+	// two take 1330 for both; from two workgroups per compute unit on there is nothing left to fill, and a part of one or two tiles
+	// is not worth its merge.  16 heads of 24, us per call, one part / two: 1x128 11.9/12.0, 1x256 14.1/13.5, 1x512 18.4/16.4, 2x777 25.5/22.9,
+	// 1x1536 33.8/27.5, 2x1536 42.5/39.4, 8x512 25.9/25.5, but 8x300 22.6/24.0, 3x1301 50.7/55.0, 3x1536 53.1/56.5.  Four parts are slower than two
+	// throughout (1x512 18.2, 1x1536 28.3).  Head_dim above 32 (one such workgroup per compute unit): 16 heads of 48, 1x777 29.2/26.0, 1x1536
+	// 40.9/34.3, 2x1200 43.7/49.9.
+	if constexpr(BMODE >= 2) {
+		const int64_t n_wg = p.B * p.H * ((p.L + NW8 * 32 - 1) / (NW8 * 32)), n_ktiles = (p.L + KT8 - 1) / KT8;
+		if(n_ktiles >= 3 && (n_wg <= 256 || (DP == 32 && n_wg <= 512 && n_ktiles >= 8))) return launch8_parts<DP, COMP, ONES, BMODE, 2>(p, s);
+	}
+	return launch8_parts<DP, COMP, ONES, BMODE, 1>(p, s);
 }
 template <int DP, bool COMP, bool ONES>
 int launch8_bias(const af3_dpa_params& p, hipStream_t s) {

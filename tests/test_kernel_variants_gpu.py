@@ -170,7 +170,8 @@ def test_projection_forms(af3, M, N, K, form, with_row):
     assert bool((out[M] == 7.0).all())
 
 
-@pytest.mark.parametrize("B,H,L,D", [(1, 1, 1, 8), (1, 2, 3, 24), (2, 1, 4, 40), (1, 2, 63, 16), (1, 1, 257, 32), (2, 1, 1026, 24), (1, 1, 4161, 24), (1, 1, 8192, 24)])
+@pytest.mark.parametrize("B,H,L,D", [(1, 1, 1, 8), (1, 2, 3, 24), (2, 1, 4, 40), (1, 2, 63, 16), (1, 1, 257, 32), (2, 1, 1026, 24), (1, 1, 4161, 24), (1, 1, 8192, 24),
+                                     (66, 8, 130, 24), (17, 8, 450, 16), (6, 16, 705, 32), (3, 16, 770, 48)])   # launches of many workgroups: keys not in parts
 @pytest.mark.parametrize("kind", ["random", "first", "last", "one tile", "none", "bytes", "no mask"])
 def test_fp8_mask_rows(af3, B, H, L, D, kind):
     """Mask rows shorter than one load, ending inside a load, of more than 64 tiles; rows with one live key or none; keep bytes other than 1."""
@@ -196,7 +197,8 @@ def test_fp8_mask_rows(af3, B, H, L, D, kind):
 
 @pytest.mark.parametrize("B,H,L,D", [(2, 64, 20, 24), (3, 33, 130, 24), (2, 9, 1000, 16), (5, 16, 512, 32), (7, 13, 641, 48)])   # from 64 blocks of 128 rows on, numbers of them that 8 does not divide
 def test_fp8_batch_rows_side_by_side(af3, B, H, L, D):
-    """Workgroups dealt by blocks of query rows compute what those of single batch rows do, dealt by heads: the same bits."""
+    """Workgroups dealt by blocks of query rows compute what those of single batch rows do, dealt by heads and perhaps with the keys in parts (whose
+    maxima differ, and with them the roundings of the e4m3 weights)."""
     g = torch.Generator().manual_seed(L + D)
     q, k, v = (torch.randn(B, H, L, D, generator=g).clamp(-3.9, 3.9).to(torch.bfloat16).cuda() for _ in range(3))
     for t in (q, k, v):
@@ -205,8 +207,12 @@ def test_fp8_batch_rows_side_by_side(af3, B, H, L, D):
     keep = (torch.rand(L, generator=g) < 0.8).cuda()
     print("case", B, H, L, D, flush=True)
     out = af3.dot_product_attention_fp8(q, k, v, keep, bias)
+    # independent weight errors of at most 2^-4 on each side: sum p v e has at most 2^-4 of the rms of sum p v for random v, twice that for both
+    # (a block in the wrong place: 2^0.5 of it)
     for b in range(B):
-        assert torch.equal(out[b:b + 1], af3.dot_product_attention_fp8(q[b:b + 1], k[b:b + 1], v[b:b + 1], keep, bias))
+        one = af3.dot_product_attention_fp8(q[b:b + 1], k[b:b + 1], v[b:b + 1], keep, bias).float()
+        for i in range(0, L, 128):
+            assert (out[b:b + 1, :, i:i + 128].float() - one[:, :, i:i + 128]).norm() <= 2 ** -3 * one[:, :, i:i + 128].norm()
 
 
 @pytest.mark.parametrize("compensated", [True, False])
