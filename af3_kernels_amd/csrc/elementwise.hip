@@ -5,6 +5,7 @@
 // follow (src/csrc/xsmm_functors.h:218-226 asserts "not implemented"); it implements OCP e4m3fn
 // with round-to-nearest-even and saturation, which is what gfx950's v_cvt_pk_fp8_f32 does.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.hpp"
 
@@ -134,6 +135,19 @@ __global__ void __launch_bounds__(EW_THREADS) cvt_e5m2_kernel(const uint8_t* __r
 	}
 }
 
+// maximum over a wavefront, in every lane: without the cross-lane network of LDS, whose six passes are a chain of 700 clocks
+__device__ __forceinline__ float wave_max(float a) {
+	auto dpp = [&](auto ctrl) { a = fmaxf(a, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(a), decltype(ctrl)::value, 0xf, 0xf, true))); };
+	dpp(std::integral_constant<int, 0xB1>{});    // lane ^ 1
+	dpp(std::integral_constant<int, 0x4E>{});    // lane ^ 2
+	dpp(std::integral_constant<int, 0x141>{});   // mirrored within 8
+	dpp(std::integral_constant<int, 0x140>{});   // mirrored within 16
+	const auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(a), false, false);
+	a            = fmaxf(__uint_as_float(x[0]), __uint_as_float(x[1]));
+	const auto y = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(a), false, false);
+	return fmaxf(__uint_as_float(y[0]), __uint_as_float(y[1]));
+}
+
 // ---- per-tensor amax -------------------------------------------------------------------------
 // 16-byte loads, wave then workgroup reduction, one atomic per workgroup (a few hundred atomics on
 // the one result word instead of one per wavefront).
@@ -146,19 +160,24 @@ __device__ __forceinline__ float block_amax(const void* __restrict__ src, int64_
 	const bool    vec  = (reinterpret_cast<uintptr_t>(src) & 15) == 0;
 	const int64_t nvec = vec ? n / PER : 0;
 	float         a    = 0.f;  // fmaxf drops NaN operands: a NaN element does not poison the scale
-	for(int64_t i = tid0; i < nvec; i += stride) {
-		const u32x4 w = static_cast<const u32x4*>(src)[i];
+	// four loads under way at a time (one memory latency for all): trips past the end repeat the thread's first element
+	for(int64_t i = tid0; i < nvec; i += 4 * stride) {
+		u32x4 w[4];
 #pragma unroll
-		for(int j = 0; j < 4; j++) {
-			if(SRC_BF16) a = fmaxf(a, fmaxf(fabsf(bf16_bits_to_f32(w[j] & 0xffffu)), fabsf(bf16_bits_to_f32(w[j] >> 16))));
-			else a = fmaxf(a, fabsf(__uint_as_float(w[j])));
-		}
+		for(int u = 0; u < 4; u++) w[u] = static_cast<const u32x4*>(src)[i + u * stride < nvec ? i + u * stride : i];
+#pragma unroll
+		for(int u = 0; u < 4; u++)
+#pragma unroll
+			for(int j = 0; j < 4; j++) {
+				if(SRC_BF16) a = fmaxf(a, fmaxf(fabsf(bf16_bits_to_f32(w[u][j] & 0xffffu)), fabsf(bf16_bits_to_f32(w[u][j] >> 16))));
+				else a = fmaxf(a, fabsf(__uint_as_float(w[u][j])));
+			}
 	}
 	for(int64_t i = nvec * PER + tid0; i < n; i += stride) {
 		const float f = SRC_BF16 ? bf16_bits_to_f32(static_cast<const uint16_t*>(src)[i]) : static_cast<const float*>(src)[i];
 		a = fmaxf(a, fabsf(f));
 	}
-	for(int o = 32; o > 0; o >>= 1) a = fmaxf(a, __shfl_xor(a, o));
+	a = wave_max(a);
 	if((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = a;
 	__syncthreads();
 	if(threadIdx.x == 0)
@@ -198,11 +217,12 @@ __device__ __forceinline__ float fp8_pow2_scale(float amax, float pre_scale) {
 	return ldexpf(1.f, e);
 }
 
-template <bool SRC_BF16>
+// multiplier(): pre_scale * scale, called once, behind the first loads (what it takes to find the scale runs under their latency)
+template <bool SRC_BF16, typename Multiplier>
 __device__ __forceinline__ void quantize_e4m3_body(const void* __restrict__ src, uint8_t* __restrict__ dst, int64_t rows, int64_t cols, int64_t src_row_stride,
-													 int transpose, int64_t rows_per_matrix, int64_t dst_row_stride, float pre_scale, float scale,
+													 int transpose, int64_t rows_per_matrix, int64_t dst_row_stride, Multiplier multiplier,
 													 uint8_t* __restrict__ dst_lo) {
-	const float   mul    = pre_scale * scale;
+	float         mul    = 0.f;
 	const int64_t stride = (int64_t)gridDim.x * EW_THREADS;
 	auto          ld     = [&](int64_t r, int64_t c) -> float {
         const int64_t i = r * src_row_stride + c;
@@ -222,16 +242,26 @@ __device__ __forceinline__ void quantize_e4m3_body(const void* __restrict__ src,
 		// dense rows on both sides: the tensor is one run of elements; one thread = 8 consecutive elements (16- or 2 x 16-byte
 		// loads, 8-byte stores), no index arithmetic beyond the running offset
 		const int total8 = (int)((rows * cols) >> 3), step = (int)stride;
-		for(int i = (int)(blockIdx.x * EW_THREADS + threadIdx.x); i < total8; i += step) {
+		constexpr int NV = SRC_BF16 ? 1 : 2;
+		u32x4         w[NV], w_next[NV];
+		auto          load = [&](int i, u32x4 (&to)[NV]) {
+#pragma unroll
+			for(int u = 0; u < NV; u++) to[u] = static_cast<const u32x4*>(src)[NV * (i < total8 ? i : 0) + u];   // (total8 > 0, or the loop does not run)
+		};
+		const int i0 = (int)(blockIdx.x * EW_THREADS + threadIdx.x);
+		if(total8 > 0) load(i0, w_next);
+		mul = multiplier();
+		for(int i = i0; i < total8; i += step) {
 			float f[8];
-			if(SRC_BF16) {
-				const u32x4 w = static_cast<const u32x4*>(src)[i];
 #pragma unroll
-				for(int j = 0; j < 4; j++) f[2 * j] = bf16_bits_to_f32(w[j] & 0xffffu), f[2 * j + 1] = bf16_bits_to_f32(w[j] >> 16);
+			for(int u = 0; u < NV; u++) w[u] = w_next[u];
+			load(i < total8 - step ? i + step : 0, w_next);
+			if constexpr(SRC_BF16) {
+#pragma unroll
+				for(int j = 0; j < 4; j++) f[2 * j] = bf16_bits_to_f32(w[0][j] & 0xffffu), f[2 * j + 1] = bf16_bits_to_f32(w[0][j] >> 16);
 			} else {
-				const u32x4 w0 = static_cast<const u32x4*>(src)[2 * i], w1 = static_cast<const u32x4*>(src)[2 * i + 1];
 #pragma unroll
-				for(int j = 0; j < 4; j++) f[j] = __uint_as_float(w0[j]), f[4 + j] = __uint_as_float(w1[j]);
+				for(int j = 0; j < 4; j++) f[j] = __uint_as_float(w[0][j]), f[4 + j] = __uint_as_float(w[NV - 1][j]);
 			}
 #pragma unroll
 			for(int j = 0; j < 8; j++) f[j] = fminf(fmaxf(f[j] * mul, -448.f), 448.f);
@@ -252,6 +282,7 @@ __device__ __forceinline__ void quantize_e4m3_body(const void* __restrict__ src,
 		}
 	} else if(!transpose) {
 		// one thread = 4 consecutive columns of one row (cols % 4 == 0 is checked by the launcher)
+		mul = multiplier();
 		const int64_t cq = cols >> 2, total = rows * cq;
 		for(int64_t i = (int64_t)blockIdx.x * EW_THREADS + threadIdx.x; i < total; i += stride) {
 			const int64_t r = i / cq, c = (i % cq) << 2;
@@ -287,16 +318,19 @@ __device__ __forceinline__ void quantize_e4m3_body(const void* __restrict__ src,
 			// consecutive bytes of one output row; consecutive wavefronts take the column blocks of the same 64 row quads, so
 			// the rows they share are fetched by one compute unit (in different workgroups they would be fetched once per XCD).
 			const uint32_t cb_n = (uint32_t)(cols >> 3), rq_u = (uint32_t)rq, rq_b = (rq_u + 63) >> 6, items = (uint32_t)n_mat * rq_b * cb_n * 64;
+			bool first = true;
 			for(uint32_t i = blockIdx.x * EW_THREADS + threadIdx.x; i < items; i += (uint32_t)stride) {
 				const uint32_t wi = i >> 6, cb = wi % cb_n, r4 = ((wi / cb_n) % rq_b) * 64 + (i & 63);
-				if(r4 >= rq_u) continue;
-				const int64_t mat = wi / (cb_n * rq_b), r = mat * rows_per_matrix + ((int64_t)r4 << 2), left = rows_per_matrix - ((int64_t)r4 << 2);
+				const int64_t  mat = wi / (cb_n * rq_b), r = mat * rows_per_matrix + ((int64_t)r4 << 2), left = rows_per_matrix - ((int64_t)r4 << 2);
 				u32x4          w[4];
 #pragma unroll
 				for(int k = 0; k < 4; k++) {
 					w[k] = u32x4{0u, 0u, 0u, 0u};
 					if(left > k) w[k] = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(src) + (r + k) * src_row_stride + (cb << 3));
 				}
+				if(first) mul = multiplier();   // (a wavefront's lanes run the same trips: items is a multiple of 64)
+				first = false;
+				if(r4 >= rq_u) continue;
 				uint8_t* const d0 = dst + (mat * cols + (cb << 3)) * dst_row_stride + ((int64_t)r4 << 2);
 #pragma unroll
 				for(int j = 0; j < 8; j++) {
@@ -314,8 +348,10 @@ __device__ __forceinline__ void quantize_e4m3_body(const void* __restrict__ src,
 				}
 			}
 		} else if(total < ((int64_t)1 << 31) && stride < ((int64_t)1 << 30)) {
+			mul = multiplier();
 			for(uint32_t i = blockIdx.x * EW_THREADS + threadIdx.x; i < (uint32_t)total; i += (uint32_t)stride) element(i, (uint32_t)cols, (uint32_t)rq);
 		} else {
+			mul = multiplier();
 			for(int64_t i = (int64_t)blockIdx.x * EW_THREADS + threadIdx.x; i < total; i += stride) element(i, cols, rq);
 		}
 	}
@@ -327,11 +363,13 @@ __global__ void __launch_bounds__(EW_THREADS) quantize_e4m3_kernel(const void* _
 																	 float pre_scale, const float* amax, float* descale_out, uint8_t* __restrict__ dst_lo) {
 	const float scale = fp8_pow2_scale(*amax, pre_scale);
 	if(blockIdx.x == 0 && threadIdx.x == 0 && descale_out) *descale_out = 1.f / scale;
-	quantize_e4m3_body<SRC_BF16>(src, dst, rows, cols, src_row_stride, transpose, rows_per_matrix, dst_row_stride, pre_scale, scale, dst_lo);
+	quantize_e4m3_body<SRC_BF16>(src, dst, rows, cols, src_row_stride, transpose, rows_per_matrix, dst_row_stride, [&]() { return pre_scale * scale; }, dst_lo);
 }
 
 // q, k and v of one attention call in one launch (blockIdx.y): q and k as they are (plus residuals),
-// v transposed; each workgroup first folds its tensor's partial maxima from amax3_kernel.
+// v transposed; each wavefront folds its tensor's partial maxima from amax3_kernel for itself, under the latency of its first loads.
+// (Short launches: what they wait for counts.  With the maxima folded by shuffles and through LDS before the first load, and one load at a
+// time in both launches, us for the two: 1x16x128x24 6.5 / now 6.2, 2x16x777x24 9.1 / 8.4, 5x16x1536x24 14.0 / 13.3.)
 struct Quant3Args {
 	const void* src[3];
 	uint8_t*    dst[3];
@@ -341,23 +379,17 @@ struct Quant3Args {
 };
 template <bool SRC_BF16>
 __global__ void __launch_bounds__(EW_THREADS) quantize3_kernel(Quant3Args a, const float* __restrict__ partials, float* __restrict__ descales) {
-	__shared__ float red[EW_THREADS / 64];
-	__shared__ float s_amax;
 	const int t = blockIdx.y;
-	static_assert(AMAX3_BLOCKS == EW_THREADS, "one partial per thread");
-	float m = partials[t * AMAX3_BLOCKS + threadIdx.x];
-	for(int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
-	if((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
-	__syncthreads();
-	if(threadIdx.x == 0) {
-		for(int w = 1; w < EW_THREADS / 64; w++) m = fmaxf(m, red[w]);
-		s_amax = m;
-	}
-	__syncthreads();
-	const float scale = fp8_pow2_scale(s_amax, a.pre_scale[t]);
-	if(blockIdx.x == 0 && threadIdx.x == 0) descales[t] = 1.f / scale;
+	static_assert(AMAX3_BLOCKS == 4 * 64, "four partial maxima per lane: every wavefront folds them for itself");
+	typedef __attribute__((ext_vector_type(4), aligned(4))) float f32x4_any;   // (the caller's floats start at any of them)
+	const f32x4 m4 = *reinterpret_cast<const f32x4_any*>(partials + t * AMAX3_BLOCKS + 4 * (threadIdx.x & 63));
+	auto multiplier = [&]() -> float {
+		const float scale = fp8_pow2_scale(wave_max(fmaxf(fmaxf(m4[0], m4[1]), fmaxf(m4[2], m4[3]))), a.pre_scale[t]);
+		if(blockIdx.x == 0 && threadIdx.x == 0) descales[t] = 1.f / scale;
+		return a.pre_scale[t] * scale;
+	};
 	const bool tr = t == 2;
-	quantize_e4m3_body<SRC_BF16>(a.src[t], a.dst[t], a.rows, a.cols, a.cols, tr ? 1 : 0, a.rows_per_matrix, tr ? a.v_row_stride : a.cols, a.pre_scale[t], scale, a.dst_lo[t]);
+	quantize_e4m3_body<SRC_BF16>(a.src[t], a.dst[t], a.rows, a.cols, a.cols, tr ? 1 : 0, a.rows_per_matrix, tr ? a.v_row_stride : a.cols, multiplier, a.dst_lo[t]);
 }
 
 // ---- pad / repack ----------------------------------------------------------------------------

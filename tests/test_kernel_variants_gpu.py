@@ -195,6 +195,23 @@ def test_fp8_mask_rows(af3, B, H, L, D, kind):
     assert bool(((out.float() - p.matmul(vd.float() * vs)).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,H,L,D", [(1, 1, 1, 8), (1, 1, 5, 8), (1, 3, 77, 24), (2, 16, 515, 24), (3, 16, 1536, 24), (5, 16, 1541, 24), (5, 16, 1536, 32)])   # up to more than four loads per thread
+def test_fp8_scale_sees_every_element(af3, B, H, L, D, dtype):
+    """One large element of v anywhere: a maximum that missed it would clamp it.  With q = 0 and no bias the output is the mean of v, here 2^10 / L."""
+    q, k = torch.zeros(B, H, L, D, dtype=dtype, device="cuda"), torch.ones(B, H, L, D, dtype=dtype, device="cuda")
+    n = q.numel()
+    for at in sorted({0, n - 1, n // 2, n - 9 if n > 9 else 0, (1 << 19) % n, min(n - 1, 3 * (1 << 19) + 5)}):
+        v = torch.zeros(n, dtype=dtype, device="cuda")
+        v[at] = 1024.0
+        print("case", B, H, L, D, at, flush=True)
+        out = af3.dot_product_attention_fp8(q, k, v.view(B, H, L, D), None, None)
+        b, h, d = at // (H * L * D), at // (L * D) % H, at % D
+        want = torch.zeros(B, H, 1, D, device="cuda")
+        want[b, h, 0, d] = 1024.0 / L
+        assert bool(((out.float() - want).abs() <= 2 ** -8 * want).all())
+
+
 @pytest.mark.parametrize("B,H,L,D", [(2, 64, 20, 24), (3, 33, 130, 24), (2, 9, 1000, 16), (5, 16, 512, 32), (7, 13, 641, 48)])   # from 64 blocks of 128 rows on, numbers of them that 8 does not divide
 def test_fp8_batch_rows_side_by_side(af3, B, H, L, D):
     """Workgroups dealt by blocks of query rows compute what those of single batch rows do, dealt by heads and perhaps with the keys in parts (whose
