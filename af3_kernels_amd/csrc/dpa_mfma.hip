@@ -194,7 +194,6 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 	// unfused variants with an output gate: the gate rows of each wavefront's query block, [32][DP] bf16, behind the tile list
 	const int            gate_base = (mask_base + (n_ktiles * KT + 64) * 4 + n_ktiles * 2 + 15) & ~15;
 	int16_t* const       live_list = reinterpret_cast<int16_t*>(mask_tab + n_ktiles * KT + 64);
-	__shared__ int       s_nvalid, s_nlive;
 
 	// ---- workgroup -> (batch, head, query tile).  Workgroups are handed to the 8 XCDs round
 	// robin, so all query tiles of one (batch, head) are given ids that are congruent mod 8:
@@ -207,15 +206,13 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 				 "s"(p.bias_stride[0]), "s"(p.bias_stride[1]), "s"(p.reserved));
 	asm volatile("" ::"s"(p.q_stride[0]), "s"(p.q_stride[1]), "s"(p.q_stride[2]), "s"(p.k_stride[0]), "s"(p.k_stride[1]), "s"(p.k_stride[2]), "s"(p.v_stride[0]), "s"(p.v_stride[1]),
 				 "s"(p.v_stride[2]));
-	const int64_t wg    = blockIdx.x;
-	const int     xcd   = (int)(wg & 7);
-	const int64_t slot  = wg >> 3;
-	const int64_t group = (slot / n_qtiles) * 8 + xcd;
-	const int     qtile = (int)(slot % n_qtiles);
-	if(!FUSED && group >= n_groups) return;
+	// (32-bit divisions: the launcher keeps the grid below 2^31, and a 64-bit one is 150 instructions of a start that waits for them)
+	const uint32_t xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, q_div = slot / (uint32_t)n_qtiles, group = q_div * 8 + xcd;
+	const int      qtile = (int)(slot - q_div * (uint32_t)n_qtiles);
+	if(!FUSED && group >= (uint32_t)n_groups) return;
 	// FUSED (4 heads): an XCD serves two heads -- their bias (2.4 MB) stays in its 4 MB L2 -- and the two
 	// workgroups that read the same rows x[b] through that L2 are neighbours in dispatch order.
-	const int64_t b = FUSED ? (slot >> 1) * 4 + (xcd >> 1) : group / p.H, h = FUSED ? 2 * (xcd & 1) + (slot & 1) : group % p.H;
+	const int64_t b = FUSED ? (slot >> 1) * 4 + (xcd >> 1) : group / (uint32_t)p.H, h = FUSED ? 2 * (xcd & 1) + (slot & 1) : group - (uint32_t)b * (uint32_t)p.H;
 	if(FUSED && b >= p.B) return;
 
 	const int     tid = threadIdx.x, lane = tid & 63;
@@ -363,20 +360,22 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 			lds_dma_b128(b_rsrc, bring_addr + slot_i * SLOT_BYTES + j * 1024, off);
 		}
 	};
-	// ---- key-mask bytes: requested first.  With 4-byte aligned mask rows
-	// a lane takes four keys per load (a chunk of 256 keys = four tiles per wavefront and load) and all of a wavefront's
+	// ---- key-mask bytes: requested first.  A lane takes four keys per load at any address (the last four of a row that L ends in the
+	// middle of are shifted; a chunk of 256 keys = four tiles per wavefront and load) and all of a wavefront's
 	// loads -- up to eight per pass -- are in flight together: one memory latency, not one per tile (a single row's walk
-	// is short enough for that to show). ----
-	const uint8_t* keep     = p.key_mask ? p.key_mask + b * p.key_mask_stride_b : nullptr;
-	const bool     mask_vec = !keep || (((reinterpret_cast<uintptr_t>(p.key_mask) | (uintptr_t)p.key_mask_stride_b | (uintptr_t)L) & 3) == 0);
-	const int      n_chunks = (n_ktiles * KT + 255) / 256;
-	uint32_t       mraw[8];
+	// is short enough for that to show).  With the mask of a length that is no multiple of four read byte by byte, 64-bit divisions and the
+	// list of tiles always compacted, us per call before / now: 16 heads of 24, 1x1491 20.9 / 20.1; 16 heads of 48, 1x1291 22.5 / 21.1, 1x1536
+	// 21.9 / 20.9. ----
+	const uint8_t* const keep     = p.key_mask ? p.key_mask + b * p.key_mask_stride_b : nullptr;
+	const bool           mask_vec = L >= 4;
+	const int            n_chunks = (n_ktiles * KT + 255) / 256;
+	uint32_t             mraw[8];
 	auto request_mask = [&](int c0) {
 #pragma unroll
 		for(int i = 0; i < 8; i++) {
-			const int64_t key0 = (int64_t)(c0 + i * NW) * 256 + 4 * lane;
-			mraw[i]            = 0u;
-			if(c0 + i * NW < n_chunks) mraw[i] = !keep ? 0x01010101u : (key0 < L ? *reinterpret_cast<const uint32_t*>(keep + key0) : 0u);
+			const int key0 = (c0 + i * NW) * 256 + 4 * lane;
+			mraw[i]        = 0x01010101u;
+			if(keep && (c0 + i * NW) * 256 < (int)L) mraw[i] = *reinterpret_cast<const u32_bytes*>(keep + (key0 + 4 <= (int)L ? key0 : (int)L - 4));
 		}
 	};
 	if(mask_vec && !is_loader) request_mask(wave);
@@ -429,62 +428,61 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 			for(int i = 0; i < 8; i++) {
 				const int c = c0 + i * NW;
 				if(c >= n_chunks) break;
-				const int64_t key0 = (int64_t)c * 256 + 4 * lane;
-				u32x4         e;
-				bool          any = false;
+				const int key0 = c * 256 + 4 * lane, over = key0 + 4 - (int)L;
+				uint32_t  m    = mraw[i];
+				if(over > 0) m = over < 4 ? m >> (8 * over) : 0u;
+				const uint32_t gone = (~(((m & 0x7f7f7f7fu) + 0x7f7f7f7fu) | m) >> 7) & 0x01010101u;   // 1 in the bytes that are zero
+				u32x4          e;
 #pragma unroll
-				for(int j = 0; j < 4; j++) {
-					const bool in   = key0 + j < L;
-					const bool live = in && ((mraw[i] >> (8 * j)) & 0xffu) != 0;
-					any             = any || live;
-					e[j]            = (live ? 0u : (in ? (uint32_t)MASK_DROPPED_BF16 : (uint32_t)MASK_OUT_OF_RANGE_BF16)) | (L2DOM ? 0x3F800000u : 0u);
+				for(int j = 0; j < 4; j++) e[j] = ((0u - ((gone >> (8 * j)) & 1u)) & (uint32_t)MASK_DROPPED_BF16) | (L2DOM ? 0x3F800000u : 0u);
+				if(over > 0) {
+#pragma unroll
+					for(int j = 0; j < 4; j++)
+						if(j >= 4 - over) e[j] = (uint32_t)MASK_OUT_OF_RANGE_BF16 | (L2DOM ? 0x3F800000u : 0u);
 				}
-				if(key0 < (int64_t)n_ktiles * KT) *reinterpret_cast<u32x4*>(mask_tab + key0) = e;
-				const unsigned long long bal = __ballot(any);   // 16 lanes per tile
-				if(lane < 4 && 4 * c + lane < n_ktiles) {
-					const bool tile_live = ((bal >> (16 * lane)) & 0xffffull) != 0;
-					live_list[4 * c + lane] = tile_live ? 1 : 0;
-				}
+				if(key0 < n_ktiles * KT) *reinterpret_cast<u32x4*>(mask_tab + key0) = e;
+				const unsigned long long bal = __ballot(m != 0u);   // 16 lanes per tile
+				if(lane < 4 && 4 * c + lane < n_ktiles) live_list[4 * c + lane] = ((bal >> (16 * lane)) & 0xffffull) != 0 ? (int16_t)(4 * c + lane) : (int16_t)-1;
 			}
 		}
-	} else {
-		for(int kt = wave; kt < n_ktiles; kt += NW) {
-			const int64_t  key  = (int64_t)kt * KT + lane;
-			const bool     in   = key < L;
-			const bool     live = in && keep[in ? key : 0] != 0;
-			const uint32_t mv   = live ? 0u : (in ? (uint32_t)MASK_DROPPED_BF16 : (uint32_t)MASK_OUT_OF_RANGE_BF16);
-			mask_tab[kt * KT + lane] = mv | (L2DOM ? 0x3F800000u : 0u);
-			const unsigned long long bal = __ballot(live);
-			if(lane == 0) {
-				live_list[kt] = bal ? 1 : 0;
+	} else if(wave == 0) {   // (a single tile)
+		const bool in = lane < (int)L, live = in && (!keep || keep[in ? lane : 0] != 0);
+		mask_tab[lane] = (live ? 0u : (in ? (uint32_t)MASK_DROPPED_BF16 : (uint32_t)MASK_OUT_OF_RANGE_BF16)) | (L2DOM ? 0x3F800000u : 0u);
+		const bool any = __ballot(live) != 0;
+		if(lane == 0) live_list[0] = any ? 0 : -1;
+	}
+	__syncthreads();
+	// The live tiles are the first ones of the row as often as not, and then the list stands as it is.  Otherwise it is compacted
+	// (wavefront 0, 64 tiles per pass: rank = number of live tiles below).  If no key of this batch row is live every
+	// tile is kept: the result is then the mean over all L keys.
+	int  nlive = 0;
+	bool in_place = true;
+	for(int base = 0; base < n_ktiles; base += 64) {
+		const unsigned long long bal = __ballot(base + lane < n_ktiles && live_list[base + lane] >= 0);
+		if(bal) in_place = in_place && nlive == base && (bal & (bal + 1)) == 0;
+		nlive += __builtin_popcountll(bal);
+	}
+	const bool any_live = nlive != 0;
+	if(!in_place || !any_live) {
+		__syncthreads();   // (every wavefront has seen the list as it was)
+		if(wave == 0) {
+			int cnt = 0;
+			for(int base = 0; base < n_ktiles; base += 64) {
+				const int  kt     = base + lane;
+				const bool keepit = kt < n_ktiles && (!any_live || live_list[kt] >= 0);
+				const unsigned long long bal = __ballot(keepit);
+				const int rank = __builtin_amdgcn_mbcnt_hi((unsigned)(bal >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)bal, 0));
+				__builtin_amdgcn_wave_barrier();  // all entries of this pass are read before any is written (cnt + rank <= kt)
+				if(keepit) live_list[cnt + rank] = (int16_t)kt;
+				cnt += __builtin_popcountll(bal);
 			}
 		}
+		__syncthreads();
+		if(!any_live) nlive = n_ktiles;
 	}
-	__syncthreads();
-	// Compact the flags into a list of live tile indices (wavefront 0, 64 tiles per pass: rank =
-	// number of live tiles below).  If no key of this batch row is live every tile is kept: the
-	// result is then the mean over all L keys.
-	if(wave == 0) {
-		bool any_live = false;
-		for(int base = 0; base < n_ktiles; base += 64) any_live = any_live || __ballot(base + lane < n_ktiles && live_list[base + lane] != 0) != 0;
-		const bool all = !any_live;
-		int        cnt = 0;
-		for(int base = 0; base < n_ktiles; base += 64) {
-			const int  kt   = base + lane;
-			const bool keepit = kt < n_ktiles && (all || live_list[kt] != 0);
-			const unsigned long long bal = __ballot(keepit);
-			const int rank = __builtin_amdgcn_mbcnt_hi((unsigned)(bal >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)bal, 0));
-			__builtin_amdgcn_wave_barrier();  // all flags of this pass are read before any index is written (cnt + rank <= kt)
-			if(keepit) live_list[cnt + rank] = (int16_t)kt;
-			cnt += __builtin_popcountll(bal);
-		}
-		if(lane == 0) s_nlive = cnt, s_nvalid = any_live ? 1 : 0;
-	}
-	__syncthreads();
-	const int nlive = __builtin_amdgcn_readfirstlane(s_nlive);
 	// A batch row without any live key: q and the bias are dropped so that every logit is exactly
 	// the mask constant and the weights come out uniform whatever the accumulation order.
-	const bool all_dropped = __builtin_amdgcn_readfirstlane(s_nvalid) == 0;
+	const bool all_dropped = !any_live;
 
 	if constexpr(LOADERS) {
 		if(is_loader) {

@@ -529,6 +529,34 @@ def test_shared_bias_mask_rows(af3, oracle, B, H, L, D, kind):
     assert np.abs(out - want).max() <= 2e-2   # (bf16 q, k, v and probabilities; |v| < 5)
 
 
+@pytest.mark.parametrize("B,H,L,D,with_bias", [(1, 2, 1, 64, True), (1, 2, 3, 56, True), (2, 1, 4, 32, False), (1, 1, 65, 64, True), (1, 2, 255, 56, True), (5, 4, 300, 32, False), (1, 1, 1027, 64, True), (2, 2, 770, 24, False), (1, 1, 4161, 64, True), (1, 1, 8190, 64, False)])
+@pytest.mark.parametrize("kind", ["random", "tail", "last", "head", "late", "gap", "none", "bytes", "no mask"])
+def test_one_row_mask_rows(af3, oracle, B, H, L, D, with_bias, kind):
+    """The one-row kernel's key masks: rows shorter than one load, at odd addresses, ending inside a load, of more than 64 tiles; live tiles that
+    are the first of the row, or not; batch rows without any; keep bytes other than 1."""
+    g = torch.Generator().manual_seed(L + D)
+    q, k, v = (torch.randn(B, H, L, D, generator=g).to(torch.bfloat16) for _ in range(3))
+    bias = torch.randn(H, L, L, generator=g).to(torch.bfloat16) if with_bias else None
+    keep = torch.rand(B, L + 1, generator=g)[:, 1:] < 0.8
+    if kind in ("last", "head", "none"):
+        keep[B - 1] = False
+        keep[B - 1, {"last": slice(L - 1, L), "head": slice(0, 1), "none": slice(0, 0)}[kind]] = True
+    elif kind in ("tail", "late", "gap"):
+        keep[:, {"tail": slice(L - L // 3, L), "late": slice(0, L // 3), "gap": slice(L // 4, L // 2)}[kind]] = False
+    dev = keep.to(torch.uint8).mul(0x80).cuda().view(torch.bool) if kind == "bytes" else keep.cuda()
+    prev = af3.set_rows_kernel("never")
+    try:
+        print("case", B, H, L, D, kind, flush=True)
+        out = f32np(af3.dot_product_attention_cpp(q.cuda(), k.cuda(), v.cuda(), None if kind == "no mask" else dev, bias.cuda() if with_bias else None))
+        torch.cuda.synchronize()
+    finally:
+        af3.set_rows_kernel(prev)
+    if kind == "no mask":
+        keep = torch.ones(B, L, dtype=torch.bool)
+    want = oracle.dpa_formula(f32np(q), f32np(k), f32np(v), keep.numpy(), f32np(bias) if with_bias else np.zeros((H, L, L), np.float32))
+    assert np.abs(out - want).max() <= 2e-2   # (bf16 q, k, v and probabilities; |v| < 5)
+
+
 @pytest.mark.parametrize("B,H,L,D", [
     (1, 1, 32, 24), (2, 3, 33, 8), (1, 16, 50, 48), (5, 4, 63, 32), (37, 4, 37, 32),   # four wavefronts, one to three blocks of 16 rows; lengths around a tile
     (1, 16, 257, 32), (1, 16, 290, 24), (1, 16, 513, 48), (1, 16, 640, 40), (1, 5, 1155, 16),   # eight
