@@ -85,7 +85,6 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DP
 	const int       n_tiles   = (int)((p.L + F32_KT - 1) / F32_KT);
 	uint32_t* const live_bits = reinterpret_cast<uint32_t*>(smem + 4 * KS * TILE);
 	int16_t* const  live_list = reinterpret_cast<int16_t*>(live_bits + n_tiles);
-	__shared__ int  s_nlive;
 
 	// workgroup -> (batch row, head, query tile); consecutive workgroups go round the 8 XCDs, so the
 	// query tiles of one (b, h) are kept on one XCD and share its L2 copy of K and V
@@ -95,13 +94,11 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DP
 				 "s"(p.bias_stride[0]), "s"(p.bias_stride[1]));
 	asm volatile("" ::"s"(p.q_stride[0]), "s"(p.q_stride[1]), "s"(p.q_stride[2]), "s"(p.k_stride[0]), "s"(p.k_stride[1]), "s"(p.k_stride[2]), "s"(p.v_stride[0]), "s"(p.v_stride[1]),
 				 "s"(p.v_stride[2]));
-	const int64_t wg    = blockIdx.x;
-	const int     xcd   = (int)(wg & 7);
-	const int64_t slot  = wg >> 3;
-	const int64_t group = (slot / n_qtiles) * 8 + xcd;
-	const int     qtile = (int)(slot % n_qtiles);
-	if(group >= n_groups) return;
-	const int64_t b = group / p.H, h = group % p.H;
+	// (32-bit divisions: the launcher keeps the grid below 2^31)
+	const uint32_t slot = blockIdx.x >> 3, q_div = slot / (uint32_t)n_qtiles, group = q_div * 8 + (blockIdx.x & 7);
+	const int      qtile = (int)(slot - q_div * (uint32_t)n_qtiles);
+	if(group >= (uint32_t)n_groups) return;
+	const int64_t b = group / (uint32_t)p.H, h = group - (uint32_t)b * (uint32_t)p.H;
 
 	const int     tid = threadIdx.x, lane = tid & 63;
 	const int     wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -148,6 +145,23 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DP
 			*reinterpret_cast<u32x2*>(dst + 2 * TERM) = u32x2{l0, l1};
 		}
 	};
+	// ---- key-mask bytes, requested first: four keys per lane at any address (the last four of a row that L ends in the middle of are
+	// shifted), 256 keys = eight tiles per wavefront and load, four loads under way.  (A byte per lane and a tile per half-wave and load,
+	// the list of tiles always compacted, 64-bit divisions: us per call before / now, B x 4 heads x L x 32: 2x128 7.39 / 6.59, 8x384 12.97 / 12.16,
+	// 64x256 21.6 / 21.1, 64x768 134.4 / 131.0.) ----
+	const uint8_t* const keep     = p.key_mask ? p.key_mask + b * p.key_mask_stride_b : nullptr;
+	const bool           mask_vec = L >= 4;
+	const int            n_chunks = (n_tiles * F32_KT + 255) / 256;
+	uint32_t             mraw[4];
+	auto request_mask = [&](int c0) {
+#pragma unroll
+		for(int i = 0; i < 4; i++) {
+			const int key0 = (c0 + i * NW) * 256 + 4 * lane;
+			mraw[i]        = 0x01010101u;
+			if(keep && (c0 + i * NW) * 256 < (int)L) mraw[i] = *reinterpret_cast<const u32_bytes*>(keep + (key0 + 4 <= (int)L ? key0 : (int)L - 4));
+		}
+	};
+	if(mask_vec) request_mask(wave);
 	const int guess = mv_sub < n_tiles ? mv_sub : n_tiles - 1;
 	fetch_tile(guess);  // (the guess that the leading tiles hold live keys: in flight while the mask is read)
 
@@ -187,30 +201,53 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DP
 	fetch_bias(guess_kt, bias_t);
 
 	// ---- live keys of every tile and the list of tiles with at least one ----
-	const uint8_t* keep = p.key_mask ? p.key_mask + b * p.key_mask_stride_b : nullptr;
-	for(int kt = wave * 2 + half; kt < n_tiles + 1; kt += 2 * NW) {  // one half-wave per tile (the last pass may hold one tile only)
-		const int64_t            key  = (int64_t)kt * F32_KT + n;
-		const bool               live = kt < n_tiles && key < L && (keep ? keep[key] != 0 : true);
-		const unsigned long long bal  = __ballot(live);
-		if(n == 0 && kt < n_tiles) live_bits[kt] = half ? (uint32_t)(bal >> 32) : (uint32_t)bal;
-	}
-	__syncthreads();
-	if(wave == 0) {  // compact the flags into tile indices; a batch row without live keys keeps every tile
-		bool any = false;
-		for(int base = 0; base < n_tiles; base += 64) any = any || __ballot(base + lane < n_tiles && live_bits[base + lane] != 0) != 0;
-		int cnt = 0;
-		for(int base = 0; base < n_tiles; base += 64) {
-			const int  kt     = base + lane;
-			const bool keepit = kt < n_tiles && (!any || live_bits[kt] != 0);
-			const unsigned long long bal = __ballot(keepit);
-			const int rank = __builtin_amdgcn_mbcnt_hi((unsigned)(bal >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)bal, 0));
-			if(keepit) live_list[cnt + rank] = (int16_t)kt;
-			cnt += __builtin_popcountll(bal);
+	if(mask_vec) {
+		for(int c0 = wave; c0 < n_chunks; c0 += 4 * NW) {
+			if(c0 != wave) request_mask(c0);
+#pragma unroll
+			for(int i = 0; i < 4; i++) {
+				const int c = c0 + i * NW;
+				if(c >= n_chunks) break;
+				const int over = c * 256 + 4 * lane + 4 - (int)L;
+				uint32_t  m    = mraw[i];
+				if(over > 0) m = over < 4 ? m >> (8 * over) : 0u;
+				// one bit per byte that is not zero, four of them side by side, eight lanes' together in the tile's word
+				const uint32_t live = ((((m & 0x7f7f7f7fu) + 0x7f7f7f7fu) | m) >> 7) & 0x01010101u;
+				int            w    = (int)(((live * 0x01020408u) >> 24) << (4 * (lane & 7)));
+				w |= __builtin_amdgcn_update_dpp(0, w, 0xB1, 0xf, 0xf, true);    // lane ^ 1
+				w |= __builtin_amdgcn_update_dpp(0, w, 0x4E, 0xf, 0xf, true);    // lane ^ 2
+				w |= __builtin_amdgcn_update_dpp(0, w, 0x141, 0xf, 0xf, true);   // mirrored within 8
+				if((lane & 7) == 0 && 8 * c + (lane >> 3) < n_tiles) live_bits[8 * c + (lane >> 3)] = (uint32_t)w, live_list[8 * c + (lane >> 3)] = (int16_t)(8 * c + (lane >> 3));
+			}
 		}
-		if(lane == 0) s_nlive = cnt;
+	} else if(wave == 0) {   // (a single tile)
+		const unsigned long long bal = __ballot(lane < (int)L && (!keep || keep[lane < (int)L ? lane : 0] != 0));
+		if(lane == 0) live_bits[0] = (uint32_t)bal, live_list[0] = 0;
 	}
 	__syncthreads();
-	const int nlive = __builtin_amdgcn_readfirstlane(s_nlive);
+	// the list of the tiles to walk: as it stands if they are the first ones of the row or if no key is live (every tile then), otherwise compacted
+	int  nlive = 0;
+	bool in_place = true;
+	for(int base = 0; base < n_tiles; base += 64) {
+		const unsigned long long bal = __ballot(base + lane < n_tiles && live_bits[base + lane] != 0);
+		if(bal) in_place = in_place && nlive == base && (bal & (bal + 1)) == 0;
+		nlive += __builtin_popcountll(bal);
+	}
+	if(nlive == 0) nlive = n_tiles;
+	if(!in_place) {
+		if(wave == 0) {
+			int cnt = 0;
+			for(int base = 0; base < n_tiles; base += 64) {
+				const int  kt     = base + lane;
+				const bool keepit = kt < n_tiles && live_bits[kt] != 0;
+				const unsigned long long bal = __ballot(keepit);
+				const int rank = __builtin_amdgcn_mbcnt_hi((unsigned)(bal >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)bal, 0));
+				if(keepit) live_list[cnt + rank] = (int16_t)kt;
+				cnt += __builtin_popcountll(bal);
+			}
+		}
+		__syncthreads();
+	}
 
 	u32x4 qf[3][NC];
 	{

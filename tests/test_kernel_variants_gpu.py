@@ -557,6 +557,30 @@ def test_one_row_mask_rows(af3, oracle, B, H, L, D, with_bias, kind):
     assert np.abs(out - want).max() <= 2e-2   # (bf16 q, k, v and probabilities; |v| < 5)
 
 
+@pytest.mark.parametrize("B,H,L,D", [(1, 2, 1, 32), (2, 1, 3, 8), (2, 2, 4, 64), (1, 2, 31, 32), (3, 4, 255, 32), (2, 1, 1026, 20), (1, 1, 4161, 32), (70, 4, 130, 32), (1, 1, 8190, 16)])
+@pytest.mark.parametrize("kind", ["random", "tail", "last", "head", "late", "gap", "none", "bytes", "no mask"])
+def test_fp32_mask_rows(af3, oracle, B, H, L, D, kind):
+    """The fp32 matrix kernel's key masks: rows shorter than one load, at odd addresses, ending inside a load, of more than 64 tiles; live tiles that
+    are the first of the row, or not; batch rows without any; keep bytes other than 1."""
+    g = torch.Generator().manual_seed(L + D)
+    q, k, v = (torch.randn(B, H, L, D, generator=g) for _ in range(3))
+    bias = torch.randn(H, L, L, generator=g)
+    keep = torch.rand(B, L + 1, generator=g)[:, 1:] < 0.8
+    if kind in ("last", "head", "none"):
+        keep[B - 1] = False
+        keep[B - 1, {"last": slice(L - 1, L), "head": slice(0, 1), "none": slice(0, 0)}[kind]] = True
+    elif kind in ("tail", "late", "gap"):
+        keep[:, {"tail": slice(L - L // 3, L), "late": slice(0, L // 3), "gap": slice(L // 4, L // 2)}[kind]] = False
+    dev = keep.to(torch.uint8).mul(0x80).cuda().view(torch.bool) if kind == "bytes" else keep.cuda()
+    print("case", B, H, L, D, kind, flush=True)
+    out = af3.dot_product_attention_cpp(q.cuda(), k.cuda(), v.cuda(), None if kind == "no mask" else dev, bias.cuda()).cpu().numpy()
+    torch.cuda.synchronize()
+    if kind == "no mask":
+        keep = torch.ones(B, L, dtype=torch.bool)
+    want = oracle.dpa_formula(q.numpy(), k.numpy(), v.numpy(), keep.numpy(), bias.numpy())
+    assert np.abs(out - want).max() <= 1e-4   # (the fp32 tier)
+
+
 @pytest.mark.parametrize("B,H,L,D", [
     (1, 1, 32, 24), (2, 3, 33, 8), (1, 16, 50, 48), (5, 4, 63, 32), (37, 4, 37, 32),   # four wavefronts, one to three blocks of 16 rows; lengths around a tile
     (1, 16, 257, 32), (1, 16, 290, 24), (1, 16, 513, 48), (1, 16, 640, 40), (1, 5, 1155, 16),   # eight
