@@ -1502,10 +1502,11 @@ static int launch_nw(const af3_dpa_params& p, hipStream_t s) {
 		//   two pairs on shared tiles      7.5    9.2   11.0   13.4   27.7   31.3
 		//   one wavefront per block, x 4   8.3   11.6   14.9   18.1   21.3   24.6
 		//   four pairs (KSL 3)                                        19.5   21.3
+		// (bf16 biases with head_dim up to 48 come here only beyond what dpa_strip.hip takes: fewer than 32 keys, long or scattered rows.)
 		// (Pairs and the one-per-block form have four loading wavefronts.  With the registers of the other pairs' form -- four
 		// contraction chunks, P.V a stage late -- four pairs at head_dim 48 spilled 18 registers: 32.5 us at L = 1536.)
 		const int64_t wg64 = groups * ((p.L + 63) / 64), wg128 = groups * ((p.L + 127) / 128);
-		if constexpr(DP == 32) {
+		if constexpr(DP == 32 && BMODE == 1) {   // (bf16 biases: such launches are the strip kernel's)
 			if(blocks1 <= 256 && ktiles >= 4 && lds_bytes<DP, 4, BMODE, true>(p) <= LDS_LIMIT) return launch_one<DP, 4, L2DOM, BMODE, true>(p, s);
 		}
 		if(blocks1 <= 256) return launch_one<DP, 2, L2DOM, BMODE, false, 1>(p, s);

@@ -548,7 +548,7 @@ __global__ void __launch_bounds__(KS * NW8 * 64) __attribute__((amdgpu_waves_per
 	}
 
 	if constexpr(KS > 1) {
-		if(nlive < n_most) asm volatile("s_barrier" ::: "memory");   // (the barrier of the other parts' last tile)
+		if(nlive < n_most) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // (the barrier of the other parts' last tile)
 		// the other parts' O, l and m to the first, [wavefront of those][register / 4][lane] x 16 bytes
 		constexpr int REGS4 = 4 * NDB + 1;
 		static_assert((KS - 1) * NW8 * REGS4 * 1024 <= MASK_BASE, "the partial sums fit the buffers");
