@@ -29,9 +29,10 @@
 //     ahead (16-byte loads from 32 rows per instruction before); rows that start at any element are fetched from the dword
 //     below and shifted when read (element by element before).
 //   * 39 KB of LDS and 128 registers: four workgroups of four wavefronts per compute unit.
-// us per call with its two quantising launches (12 to 14 us), 16 heads of 24, before / now: 5x1536 89.0/71.3, 8x1536 133.6/104.9, 8x1301 (ragged
-// rows) -/101.7, 8x1000 66.7/54.2, 5x300 37.9/20.3, 1x1536 42.1/34.2 (boxes differ: 5x1536 72 to 75).  Measured on the way: the bias loads are 13 us of the
-// 57 that the kernel takes at 5x1536, the exponentials 4; four workgroups per compute unit instead of three changed nothing, nor did
+//   * Workgroups in an order that lets batch rows share the bias, tiles in two parts where workgroups are few: see launch8_parts, launch8.
+// us per call with its two quantising launches (6 to 13 us), 16 heads of 24, 16-deep products / these forms, workgroups by heads and one part / now:
+// 5x1536 89.0/71.3/68.4, 8x1536 133.6/104.9/101, 8x1301 (ragged rows) -/101.7/97, 8x1000 66.7/54.2/54, 5x300 37.9/20.3/17.5, 1x1536 42.1/34.2/27.6 (boxes
+// differ: 5x1536 68 to 71).  Measured on the way: with the bias streamed once per batch row its loads were 13 us of 57 at 5x1536, the exponentials 4; four workgroups per compute unit instead of three changed nothing, nor did
 // pinning the matrix instructions between the exponentials: the vector port is busy three quarters of the time.
 #include "mfma_helpers.hpp"
 
@@ -615,8 +616,9 @@ int launch8_parts(const af3_dpa_params& p, hipStream_t s) {
 	// then serves all but the first of them.  Fewer than 64 such blocks fill the XCDs unevenly and are dealt by (batch row, head).
 	// (16 heads of 24, 1536 rows, us per call, pairs / blocks: 5 batch rows 76.8 / 75.2, 8 106.9 / 102.5; 8 of 1301 102.0 / 100.2.)
 	const int64_t n_blocks = p.H * n_qtiles, n_groups = p.B * p.H;
-	const int64_t per_xcd  = p.bias && p.B > 1 && n_blocks >= 64 ? (n_blocks + 7) / 8 : 0;
-	const int64_t blocks   = per_xcd > 0 ? per_xcd * 8 * p.B : (n_groups + 7) / 8 * 8 * n_qtiles;
+	const int64_t side_by  = (n_blocks + 7) / 8 * 8 * p.B;
+	const int64_t per_xcd  = p.bias && p.B > 1 && n_blocks >= 64 && side_by <= 0x7fffffffLL ? (n_blocks + 7) / 8 : 0;
+	const int64_t blocks   = per_xcd > 0 ? side_by : (n_groups + 7) / 8 * 8 * n_qtiles;
 	if(blocks <= 0 || blocks > 0x7fffffffLL) return AF3_ERR_BAD_SHAPE;
 	const size_t smem = (size_t)KS * (3 * (COMP ? 3 : 2) * KT8 * DP + (BMODE >= 2 ? NW8 * 2 * BIAS_HALF8 : 0)) + (size_t)n_ktiles * KT8 * 2 + (size_t)((n_ktiles + 15) & ~15);
 	auto         kern = dpa_mfma_fp8_kernel<DP, COMP, ONES, BMODE, KS>;
