@@ -52,13 +52,14 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 	constexpr int NO = KIND == 0 ? ND : ND + 1; // ... of O: the row sums in a block of their own, or in column 24
 	constexpr int NV = KIND == 2 ? 3 : 2;       // 1 KB loads of a K or V tile
 	constexpr int R  = NB * 16;                 // query rows of the strip
+	constexpr bool LO = KIND == 1;              // q's second term meets K in matrix instructions of its own
 	constexpr int PC = KIND == 2 ? 52 : 36;     // floats of a row's partial sums in LDS
 	constexpr int SUM_COL = KIND == 0 ? 24 : 16 * ND;
 	constexpr int NT = ANY ? (NB + 3) / 4 : 0;  // loads of the dwords that follow the rows of a tile's bias (64 rows each)
 	constexpr int WAVE_LDS = 2 * NB * 1024 + 2 * NV * 1024 + 2 * NT * 256 + 32;   // of a wavefront's own: two tiles of the bias, one of K and of V, constants
 	extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
 	// [tiles and constants of each wavefront | partial sums (in the same place, later)] [q, as the matrix instructions take it] [key-mask tables: 128 B per tile]
-	constexpr int TILES = NW * WAVE_LDS, PARTS = NW * R * PC * 4, Q_AT = TILES > PARTS ? TILES : PARTS, Q_ROW = KS * 64 + 16, MASK_AT = Q_AT + R * Q_ROW;
+	constexpr int TILES = NW * WAVE_LDS, PARTS = NW * R * PC * 4, Q_AT = TILES > PARTS ? TILES : PARTS, Q_ROW = KS * 64 + 16, MASK_AT = Q_AT + (LO ? 2 : 1) * R * Q_ROW;
 	__shared__ float s_max[NW * R];
 	__shared__ int   s_bad;
 
@@ -80,12 +81,14 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 	// ---- requests that the compiler waits for: q (a thread takes a 16-byte chunk of a row of the strip, padding included: what the
 	// range checks keep out is zero), and the key mask of this wavefront's tiles (wave, wave + NW, ...) ----
 	constexpr int QN = (R * 4 * KS + NW * 64 - 1) / (NW * 64);
+	const int DC = D >> 3;   // 16-byte chunks of a q, K or V row
+	auto q_chunk = [&](int ch) __attribute__((always_inline)) { return ch < DC ? ch : ch - DC; };   // (chunk DC + c of an operand: the second term of chunk c)
 	const __amdgpu_buffer_rsrc_t q_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(qp), 0, (L - 1) * p.q_row + D * 2, 0x00020000);
 	u32x4 qraw[QN];
 #pragma unroll
 	for(int j = 0; j < QN; j++) {
 		const int i = tid + j * NW * 64, ch = i % (4 * KS);
-		qraw[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(q_rsrc, ch * 8 < D ? (strip * R + i / (4 * KS)) * p.q_row + ch * 16 : 0x40000000, 0, 0));
+		qraw[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(q_rsrc, q_chunk(ch) < DC ? (strip * R + i / (4 * KS)) * p.q_row + q_chunk(ch) * 16 : 0x40000000, 0, 0));
 	}
 	const int last_k0 = L - KT_S, my_all = (n_tiles - wave + NW - 1) / NW;   // (0 or less: no tile)
 	const __amdgpu_buffer_rsrc_t m_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(keep), 0, masked ? L : 0, 0x00020000);
@@ -100,7 +103,6 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 	// ---- loads that write LDS directly.  A wavefront's tiles are its own: nothing but its own waits orders them.  The last tile of a
 	// length that is no multiple of 32 starts at key L - 32; its first keys, seen before, are masked out of it. ----
 	const int b_base = wave * WAVE_LDS, k_base = b_base + 2 * NB * 1024, v_base = k_base + NV * 1024, t_base = v_base + NV * 1024, const_base = t_base + 2 * NT * 256;
-	const int DC = D >> 3;   // 16-byte chunks of a K or V row
 	// K: place i of half h holds key 8 (i / 4) + 4 h + i % 4; with 2, 4 or 6 chunks a row the chunks of some rows are swapped, so that the 16 rows
 	// of a fragment read always meet 16 different places of the banks
 	const int  swap_shift = DC == 4 ? 2 : 3, swap_mask = DC == 4 ? 3 : DC & 1 ? 0 : 1;
@@ -175,7 +177,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 #pragma unroll
 		for(int hf = 0; hf < 2; hf++) {
 			const int ch = 4 * st + g;
-			k_rd[st][hf] = ch < DC ? k_base + (16 * hf + i16) * (DC * 16) + ((ch ^ ((i16 >> swap_shift) & swap_mask)) << 4) : ZEROS_AT;
+			k_rd[st][hf] = q_chunk(ch) < DC ? k_base + (16 * hf + i16) * (DC * 16) + ((q_chunk(ch) ^ ((i16 >> swap_shift) & swap_mask)) << 4) : ZEROS_AT;
 		}
 #pragma unroll
 	for(int d = 0; d < ND; d++)
@@ -191,17 +193,26 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 	const int t_half = g < 3 ? NB * 1024 : NT * 256, t_blk = g < 3 ? 1024 : 64;
 	const int b_rd = b_base + i16 * 64 + ((g ^ ((i16 >> 2) & 3)) << 4);
 
-	// q to LDS, scaled and rounded once
+	// q to LDS, scaled, as two bf16 terms as far as there is room: the second one of the first columns takes the columns behind head_dim, where
+	// K's operand repeats those columns, or (head_dim 32: none) all of it goes through matrix instructions of its own.  (Rounded once, the
+	// rms error against 64 bits was 1 to 8 % above that of the one-row kernel, whose reference makes a row's largest weight exactly
+	// 1; now, one-row kernel / here: 37 x 4 x 37 x 32 8.2e-4 / 7.5e-4, 16 heads of 24 x 768 2.8e-4 / 2.7e-4, 16 heads of 48 x 128 5.4e-4 / 5.4e-4.  The second terms cost nothing, at head_dim
+	// 32 3 % of a call.)
 #pragma unroll
 	for(int j = 0; j < QN; j++) {
 		const int i = tid + j * NW * 64, row = i / (4 * KS), ch = i % (4 * KS);
-		u32x4     w;
+		u32x4     hi, lo;
 #pragma unroll
 		for(int e = 0; e < 4; e++) {
 			const uint32_t raw = qraw[j][e];
-			w[e] = pack_bf16x2(bf16_bits_to_f32(raw & 0xffffu) * p.scale, bf16_bits_to_f32(raw >> 16) * p.scale);
+			const float    x = bf16_bits_to_f32(raw & 0xffffu) * p.scale, y = bf16_bits_to_f32(raw >> 16) * p.scale;
+			const uint32_t h2 = pack_bf16x2(x, y);
+			hi[e] = h2, lo[e] = pack_bf16x2(x - bf16_bits_to_f32(h2 & 0xffffu), y - bf16_bits_to_f32(h2 >> 16));
 		}
-		if(i < R * 4 * KS) *reinterpret_cast<u32x4*>(smem + Q_AT + row * Q_ROW + ch * 16) = w;
+		if(i < R * 4 * KS) {
+			*reinterpret_cast<u32x4*>(smem + Q_AT + row * Q_ROW + ch * 16) = ch < DC ? hi : lo;
+			if constexpr(LO) *reinterpret_cast<u32x4*>(smem + Q_AT + (R + row) * Q_ROW + ch * 16) = lo;
+		}
 	}
 
 	// ---- key-mask table of this wavefront's tiles: what is added to a key's logits.  Tiles behind the last one with a live key are not walked. ----
@@ -215,11 +226,14 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 	}
 	asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 	__syncthreads();   // q
-	bf16x8 qf[NB][KS];
+	bf16x8 qf[NB][KS], ql[NB];   // (ql: LO only)
 #pragma unroll
 	for(int c = 0; c < NB; c++)
 #pragma unroll
-		for(int s = 0; s < KS; s++) qf[c][s] = *reinterpret_cast<const bf16x8*>(smem + Q_AT + (16 * c + i16) * Q_ROW + s * 64 + g * 16);
+		for(int s = 0; s < KS; s++) {
+			qf[c][s] = *reinterpret_cast<const bf16x8*>(smem + Q_AT + (16 * c + i16) * Q_ROW + s * 64 + g * 16);
+			if constexpr(LO) ql[c] = *reinterpret_cast<const bf16x8*>(smem + Q_AT + (R + 16 * c + i16) * Q_ROW + g * 16);
+		}
 
 	auto read_k = [&](bf16x8 (&kf)[2][KS], f32x4 (&mk)[2], int i) __attribute__((always_inline)) {   // i: of this wavefront's tiles
 #pragma unroll
@@ -298,6 +312,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 					s[hf] = mfma(__builtin_bit_cast(bf16x8, sel[hf]), bb, mk[hf]);
 #pragma unroll
 					for(int st = 0; st < KS; st++) s[hf] = mfma(kf[hf][st], qf[0][st], s[hf]);
+					if constexpr(LO) s[hf] = mfma(kf[hf][0], ql[0], s[hf]);
 				}
 			}
 			if constexpr(NB > 1) b_next = read_b(0, 1, k0_0);
@@ -332,12 +347,14 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 				}
 				__builtin_amdgcn_sched_barrier(0);
 				o[CP][0] = mfma(vf[0], pp, o[CP][0]);
-				sn[0] = mfma(__builtin_bit_cast(bf16x8, sel[0]), bb, mk[0]);
+				if constexpr(LO) sn[0] = mfma(__builtin_bit_cast(bf16x8, sel[0]), bb, mfma(kf[0][0], ql[CN], mk[0]));
+				else sn[0] = mfma(__builtin_bit_cast(bf16x8, sel[0]), bb, mk[0]);
 				ex(ic<0>{});
 				AF3_PIN(pc[0]); AF3_PIN(sn[0][0]);
 				__builtin_amdgcn_sched_barrier(0);
 				o[CP][1] = mfma(vf[1], pp, o[CP][1]);
-				sn[1] = mfma(__builtin_bit_cast(bf16x8, sel[1]), bb, mk[1]);
+				if constexpr(LO) sn[1] = mfma(__builtin_bit_cast(bf16x8, sel[1]), bb, mfma(kf[1][0], ql[CN], mk[1]));
+				else sn[1] = mfma(__builtin_bit_cast(bf16x8, sel[1]), bb, mk[1]);
 				ex(ic<1>{});
 				AF3_PIN(pc[1]); AF3_PIN(sn[1][0]);
 				__builtin_amdgcn_sched_barrier(0);
@@ -491,6 +508,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 							f32x4 s = mfma(__builtin_bit_cast(bf16x8, sel[hf]), bb, mk[hf]);
 #pragma unroll
 							for(int st = 0; st < KS; st++) s = mfma(kf[hf][st], qf[c][st], s);
+							if constexpr(LO) s = mfma(kf[hf][0], ql[c], s);
 							mx[c] = fmaxf(fmaxf(fmaxf(mx[c], s[0]), s[1]), fmaxf(s[2], s[3]));
 						}
 					}
@@ -524,10 +542,10 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 template <int NB, int KIND, bool ANY, int NW>
 static int launch_strip_n(const af3_dpa_params& p, hipStream_t s) {
 	constexpr int R = NB * 16, NT = ANY ? (NB + 3) / 4 : 0, tiles = NW * ((2 * NB + (KIND == 2 ? 6 : 4)) * 1024 + 2 * NT * 256 + 32), parts = NW * R * (KIND == 2 ? 52 : 36) * 4;
-	const int     smem = (tiles > parts ? tiles : parts) + R * ((KIND == 2 ? 128 : 64) + 16) + (((int)p.L + KT_S - 1) / KT_S + NW) * 128;
+	const int     smem = (tiles > parts ? tiles : parts) + (KIND == 1 ? 2 : 1) * R * ((KIND == 2 ? 128 : 64) + 16) + (((int)p.L + KT_S - 1) / KT_S + NW) * 128;
 	auto          kern = dpa_strip_bf16_kernel<NB, KIND, ANY, NW>;
 	if(smem > 160 * 1024 - NW * R * 4 - 64) return AF3_ERR_BAD_SHAPE;
-	if(smem > 40 * 1024) {
+	if(smem > 64 * 1024 - NW * R * 4 - 64) {   // (the call costs the host 0.7 us)
 		if(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem) != hipSuccess) return AF3_ERR_LAUNCH;
 	}
 	const int  out_size = p.out_dtype == AF3_F32 ? 4 : 2;

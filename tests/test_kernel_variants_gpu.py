@@ -581,6 +581,24 @@ def test_fp32_mask_rows(af3, oracle, B, H, L, D, kind):
     assert np.abs(out - want).max() <= 1e-4   # (the fp32 tier)
 
 
+@pytest.mark.parametrize("B,H,L,D", [(2, 4, 40, 8), (1, 16, 200, 16), (9, 4, 57, 32), (2, 4, 512, 32), (1, 5, 1155, 16)])
+def test_strips_do_not_round_q(af3, oracle, B, H, L, D):
+    """head_dim 8 and 16 (q's second term in the padding), 32 (in instructions of its own): what is rounded is each weight, once, the row sum's
+    weights with it, and the result."""
+    g = torch.Generator().manual_seed(L + D)
+    q, k, v = (torch.randn(B, H, L, D, generator=g).mul(m).to(torch.bfloat16) for m in (6.0, 1.0, 1.0))
+    bias = torch.randn(H, L, L, generator=g).to(torch.bfloat16)
+    keep = torch.ones(B, L, dtype=torch.bool)
+    print("case", B, H, L, D, flush=True)
+    out = f32np(af3.dot_product_attention_cpp(q.cuda(), k.cuda(), v.cuda(), keep.cuda(), bias.cuda()))
+    want = oracle.dpa_formula(f32np(q), f32np(k), f32np(v), keep.numpy(), f32np(bias))
+    size = oracle.dpa_formula(f32np(q), f32np(k), np.abs(f32np(v)), keep.numpy(), f32np(bias))
+    # half a unit in the last of eight bits, 2^-8 at most, each: a weight, the sum of the weights, the result; q to 2^-17 (2^-8 / 8 for sums of |q k| up to 2^6)
+    assert (np.abs(out - want) <= 3.125 * 2.0 ** -8 * size + 1e-6).all()
+    # in rms those three are independent and each below a third of its maximum on average
+    assert np.sqrt(np.mean((out - want) ** 2)) <= 2.0 ** -9 * np.sqrt(np.mean(size ** 2))
+
+
 @pytest.mark.parametrize("B,H,L,D", [
     (1, 1, 32, 24), (2, 3, 33, 8), (1, 16, 50, 48), (5, 4, 63, 32), (37, 4, 37, 32),   # four wavefronts, one to three blocks of 16 rows; lengths around a tile
     (1, 16, 257, 32), (1, 16, 290, 24), (1, 16, 513, 48), (1, 16, 640, 40), (1, 5, 1155, 16),   # eight
