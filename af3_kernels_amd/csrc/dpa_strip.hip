@@ -6,8 +6,8 @@
 // one per compute unit -- and its wavefronts take the key tiles (32 keys) of the strip in turn.  The NB blocks of 16 rows are NB
 // independent chains of one wavefront: they share the tile's K, V and mask operands, and while one block's logits are exponentiated
 // the matrix pipe works on its neighbours.  Nothing is shared between wavefronts until the strip's partial sums are added up
-// through LDS at the end, so the walk has no barrier, every operand but V^T goes from memory straight into the registers that the
-// matrix instructions read, and two tiles are under way while one is worked on.
+// through LDS at the end, so the walk has no barrier: every wavefront's bias, K and V travel by loads that write LDS directly, into
+// places of its own, each asked to hold the next tile as soon as it has been read, and are awaited by count.
 //
 // Logits: S^T[key][q] = K . Q^T on v_mfma_f32_16x16x32_bf16 in two halves of 16 keys, on top of the bias as the matrix pipe adds it
 // (a 0/1 selection times the bias rows as they lie in memory: exact), on top of the key mask (the C operand, shared by the strip's
@@ -580,7 +580,7 @@ bool bias_rows_anywhere(const af3_dpa_params& p) { return (reinterpret_cast<uint
 // and beyond that, in two rounds, 29.0 / 32.6 and 32.3 / 40.2 at 1792.  Rows at any address (one more load and LDS read per piece):
 //   head_dim 24   L  65        257       385       513        769          1025         1281         1491
 //                 7.0 / 5.9  8.6 / 6.9  8.6 / 7.4  10.2 / 8.4  12.7 / 11.6  17.8 / 17.2  20.8 / 21.8  22.6 / 23.6
-// Few heads: 4 x 2048 x 24 23.9 / 10.6, 2 x 1500 x 48 29.7 / 9.6.  Batches that read in place: 37 x 4 x 37 x 32 5.4 / 4.9, 2 x 16 x 512 x 24
+// Few heads: 4 x 2048 x 24 23.9 / 10.6, 2 x 1500 x 48 29.7 / 9.6.  Batches that read in place: 37 x 4 x 37 x 32 5.4 / 5.0, 2 x 16 x 512 x 24
 // 8.5 / 7.2, 5 x 16 x 128 x 48 6.7 / 5.6.
 strip_form strip_form_of(const af3_dpa_params& p) {
 	const bool any = bias_rows_anywhere(p);
