@@ -43,25 +43,37 @@ struct strip_args {
 	float          scale;
 };
 
+// A workgroup's LDS, all of it dynamic, as the kernel and its launcher see it:
+// [tiles and constants of each wavefront | partial sums (in the same place, later)] [q, as the matrix instructions take it | rows' maxima (later)] [a flag] [key-mask tables: 128 B per tile]
+template <int NB, int KIND, bool ANY, int NW>
+struct strip_lds {
+	static constexpr int KS = KIND == 2 ? 2 : 1;       // contraction steps of 32 head columns
+	static constexpr int NV = KIND == 2 ? 3 : 2;       // 1 KB loads of a K or V tile
+	static constexpr int R  = NB * 16;                 // query rows of the strip
+	static constexpr int NT = ANY ? (NB + 3) / 4 : 0;  // loads of the dwords that follow the rows of a tile's bias (64 rows each)
+	static constexpr int PC = KIND == 2 ? 52 : 36;     // floats of a row's partial sums
+	static constexpr int WAVE   = 2 * NB * 1024 + 2 * NV * 1024 + 2 * NT * 256 + 32;   // of a wavefront's own: two tiles of the bias, one of K and of V, constants
+	static constexpr int Q_ROW  = KS * 64 + 16;
+	static constexpr int TILES = NW * WAVE, PARTS = NW * R * PC * 4, Q_AT = TILES > PARTS ? TILES : PARTS;
+	static constexpr int FLAG_AT = Q_AT + (KIND == 1 ? 2 : 1) * R * Q_ROW, MASK_AT = FLAG_AT + 16;
+	static_assert(NW * R * 4 <= R * Q_ROW, "the rows' maxima of all wavefronts take no more than q did");
+	static constexpr int bytes(int L) { return MASK_AT + ((L + KT_S - 1) / KT_S + NW) * 128; }
+	static_assert(bytes(MAX_L_MFMA) <= 160 * 1024, "every length that reaches this kernel fits a compute unit");
+};
+
 // KIND: 0 = head_dim up to 24 (row sums in V's column 24), 1 = 32, 2 = 40 and 48 (two contraction steps).  Grid: x = head (with a multiple of 8 heads the strips of one head share an XCD and
 // its L2 copy of K and V), y = strip, z = batch row.
 template <int NB, int KIND, bool ANY, int NW>
 __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) dpa_strip_bf16_kernel(strip_args p) {
-	constexpr int KS = KIND == 2 ? 2 : 1;       // contraction steps of 32 head columns
+	using lds = strip_lds<NB, KIND, ANY, NW>;
+	constexpr int KS = lds::KS, NV = lds::NV, NT = lds::NT, R = lds::R, PC = lds::PC, WAVE_LDS = lds::WAVE, Q_AT = lds::Q_AT, Q_ROW = lds::Q_ROW, MASK_AT = lds::MASK_AT;
 	constexpr int ND = KIND == 2 ? 3 : 2;       // blocks of 16 head columns of V
 	constexpr int NO = KIND == 0 ? ND : ND + 1; // ... of O: the row sums in a block of their own, or in column 24
-	constexpr int NV = KIND == 2 ? 3 : 2;       // 1 KB loads of a K or V tile
-	constexpr int R  = NB * 16;                 // query rows of the strip
 	constexpr bool LO = KIND == 1;              // q's second term meets K in matrix instructions of its own
-	constexpr int PC = KIND == 2 ? 52 : 36;     // floats of a row's partial sums in LDS
 	constexpr int SUM_COL = KIND == 0 ? 24 : 16 * ND;
-	constexpr int NT = ANY ? (NB + 3) / 4 : 0;  // loads of the dwords that follow the rows of a tile's bias (64 rows each)
-	constexpr int WAVE_LDS = 2 * NB * 1024 + 2 * NV * 1024 + 2 * NT * 256 + 32;   // of a wavefront's own: two tiles of the bias, one of K and of V, constants
 	extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-	// [tiles and constants of each wavefront | partial sums (in the same place, later)] [q, as the matrix instructions take it] [key-mask tables: 128 B per tile]
-	constexpr int TILES = NW * WAVE_LDS, PARTS = NW * R * PC * 4, Q_AT = TILES > PARTS ? TILES : PARTS, Q_ROW = KS * 64 + 16, MASK_AT = Q_AT + (LO ? 2 : 1) * R * Q_ROW;
-	__shared__ float s_max[NW * R];
-	__shared__ int   s_bad;
+	float* const s_max = reinterpret_cast<float*>(smem + Q_AT);   // (q is in registers by then)
+	int* const   s_bad = reinterpret_cast<int*>(smem + lds::FLAG_AT);
 
 	asm volatile("" ::"s"(p.q), "s"(p.k), "s"(p.v), "s"(p.bias), "s"(p.mask), "s"(p.q_h), "s"(p.k_h), "s"(p.v_h), "s"(p.bias_h), "s"(p.q_row), "s"(p.k_row), "s"(p.v_row), "s"(p.bias_row), "s"(p.H),
 				 "s"(p.L), "s"(p.D), "s"(p.per_chunk), "s"(p.scale));
@@ -158,7 +170,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 		if(lane < 8) *reinterpret_cast<uint32_t*>(smem + const_base + 4 * lane) = lane == 4 ? 0x3F80u : 0u;
 	};
 	fill();
-	if(tid == 0) s_bad = 0;
+	if(tid == 0) *s_bad = 0;
 
 	// ---- per-lane constants ----
 	u32x4 sel[2];   // half h of the tile's keys: row i picks key 8 (i / 4) + 4 h + i % 4
@@ -478,9 +490,9 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 			else *reinterpret_cast<u32x2*>(at + d0 * 2) = u32x2{pack_bf16x2(t[0], t[1]), pack_bf16x2(t[2], t[3])};
 		}
 		if(with_reference) return;
-		if(__ballot(bad) && lane == 0) s_bad = 1;
+		if(__ballot(bad) && lane == 0) *s_bad = 1;
 		__syncthreads();
-		if(!__builtin_amdgcn_readfirstlane(s_bad)) return;
+		if(!__builtin_amdgcn_readfirstlane(*s_bad)) return;
 		// ---- rare: the rows' maxima, then the walk again, over all tiles (a row without a live key needs them) ----
 		my_n = my_all > 0 ? my_all : 0;
 		fill();
@@ -541,11 +553,11 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 
 template <int NB, int KIND, bool ANY, int NW>
 static int launch_strip_n(const af3_dpa_params& p, hipStream_t s) {
-	constexpr int R = NB * 16, NT = ANY ? (NB + 3) / 4 : 0, tiles = NW * ((2 * NB + (KIND == 2 ? 6 : 4)) * 1024 + 2 * NT * 256 + 32), parts = NW * R * (KIND == 2 ? 52 : 36) * 4;
-	const int     smem = (tiles > parts ? tiles : parts) + (KIND == 1 ? 2 : 1) * R * ((KIND == 2 ? 128 : 64) + 16) + (((int)p.L + KT_S - 1) / KT_S + NW) * 128;
+	using lds = strip_lds<NB, KIND, ANY, NW>;
+	constexpr int R    = lds::R;
+	const int     smem = lds::bytes((int)p.L);
 	auto          kern = dpa_strip_bf16_kernel<NB, KIND, ANY, NW>;
-	if(smem > 160 * 1024 - NW * R * 4 - 64) return AF3_ERR_BAD_SHAPE;
-	if(smem > 64 * 1024 - NW * R * 4 - 64) {   // (the call costs the host 0.7 us)
+	if(smem > 64 * 1024) {   // beyond the default limit: raise it for this kernel (the call costs the host 0.7 us)
 		if(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem) != hipSuccess) return AF3_ERR_LAUNCH;
 	}
 	const int  out_size = p.out_dtype == AF3_F32 ? 4 : 2;

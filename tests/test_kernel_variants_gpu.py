@@ -599,6 +599,26 @@ def test_strips_do_not_round_q(af3, oracle, B, H, L, D):
     assert np.sqrt(np.mean((out - want) ** 2)) <= 2.0 ** -9 * np.sqrt(np.mean(size ** 2))
 
 
+@pytest.mark.parametrize("H,L,D,first", [
+    (2, 7872, 48, 1), (2, 7873, 48, 0), (2, 8096, 48, 1), (2, 8097, 40, 0), (2, 8191, 48, 0), (2, 8192, 48, 1), (2, 8192, 32, 1),   # four blocks, rows at any address: the most LDS a workgroup takes
+    (3, 8192, 48, 0), (2, 8192, 40, 0),                              # two workgroups per compute unit
+    (9, 1953, 48, 0), (1, 3201, 24, 0), (1, 3296, 24, 1), (1, 4640, 16, 0), (1, 8191, 8, 0),   # around and above the 64 KB that a launch gets without asking
+])
+def test_strips_of_long_rows(af3, oracle, H, L, D, first):
+    """Every length up to 8192 is served, whatever part of a compute unit's LDS its mask tables leave."""
+    g = torch.Generator(device="cuda").manual_seed(L + D)
+    q, k, v = (torch.randn(1, H, L, D, generator=g, device="cuda").to(torch.bfloat16) for _ in range(3))
+    bias = torch.randn(first + H * L * L, generator=g, device="cuda", dtype=torch.bfloat16)[first:].view(H, L, L)
+    keep = torch.rand(L, generator=g, device="cuda") < 0.8
+    keep[0] = True
+    print("case", H, L, D, first, flush=True)
+    out = af3.dot_product_attention_cpp(q, k, v, keep, bias)[0, :, ::13].double()
+    torch.cuda.synchronize()
+    s = (q[0, :, ::13].double() @ k[0].double().transpose(-1, -2).contiguous()) * D ** -0.5 + bias[:, ::13].double()
+    want = s.masked_fill(~keep, -1e9).softmax(-1) @ v[0].double()
+    assert (out - want).abs().max() <= 2e-2   # (bf16's budget)
+
+
 @pytest.mark.parametrize("B,H,L,D", [
     (1, 1, 32, 24), (2, 3, 33, 8), (1, 16, 50, 48), (5, 4, 63, 32), (37, 4, 37, 32),   # four wavefronts, one to three blocks of 16 rows; lengths around a tile
     (1, 16, 257, 32), (1, 16, 290, 24), (1, 16, 513, 48), (1, 16, 640, 40), (1, 5, 1155, 16),   # eight
