@@ -503,7 +503,8 @@ def test_shared_bias_quick_and_careful_walks(af3, oracle, B, H, L, D, kind):
     assert (np.abs(out - want) / scale).max() <= 2e-2
 
 
-@pytest.mark.parametrize("B,H,L,D", [(3, 2, 1, 32), (2, 1, 3, 16), (4, 2, 4, 32), (3, 2, 37, 32), (2, 2, 255, 24), (3, 1, 257, 32), (2, 1, 2047, 32), (2, 1, 2049, 32), (3, 1, 2306, 16)])
+@pytest.mark.parametrize("B,H,L,D", [(3, 2, 1, 32), (2, 1, 3, 16), (4, 2, 4, 32), (3, 2, 37, 32), (2, 2, 255, 24), (3, 1, 257, 32), (2, 1, 2047, 32), (2, 1, 2049, 32), (3, 1, 2306, 16),
+                                     (4, 1, 2013, 32), (3, 1, 1984, 32)])   # (the last two: around the 64 KB of LDS that a launch gets without asking)
 @pytest.mark.parametrize("kind", ["random", "last", "head", "middle", "none", "bytes", "no mask"])
 def test_shared_bias_mask_rows(af3, oracle, B, H, L, D, kind):
     """The shared-bias kernel's key masks: rows shorter than one load, at odd addresses, ending inside a load, longer than what is requested
