@@ -210,6 +210,9 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 	// rms error against 64 bits was 1 to 8 % above that of the one-row kernel, whose reference makes a row's largest weight exactly
 	// 1; now, one-row kernel / here: 37 x 4 x 37 x 32 8.2e-4 / 7.5e-4, 16 heads of 24 x 768 2.8e-4 / 2.7e-4, 16 heads of 48 x 128 5.4e-4 / 5.4e-4.  The second terms cost nothing, at head_dim
 	// 32 3 % of a call.)
+	// A column's two terms have one sign, and neither is zero unless q is (or is smaller than 2^-102): the first is truncated, the second a 2^-24th of it above the rest, so
+	// that an infinity in K makes the infinity of the formula of both, never infinity minus infinity or 0 times infinity.
+	const uint32_t first = LO || tid % (4 * KS) >= DC || tid % (4 * KS) + DC < 4 * KS ? 0xffff0000u : ~0u;   // (a column without a second term is rounded)
 #pragma unroll
 	for(int j = 0; j < QN; j++) {
 		const int i = tid + j * NW * 64, row = i / (4 * KS), ch = i % (4 * KS);
@@ -218,8 +221,8 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 		for(int e = 0; e < 4; e++) {
 			const uint32_t raw = qraw[j][e];
 			const float    x = bf16_bits_to_f32(raw & 0xffffu) * p.scale, y = bf16_bits_to_f32(raw >> 16) * p.scale;
-			const uint32_t h2 = pack_bf16x2(x, y);
-			hi[e] = h2, lo[e] = pack_bf16x2(x - bf16_bits_to_f32(h2 & 0xffffu), y - bf16_bits_to_f32(h2 >> 16));
+			const float    xh = __uint_as_float(__float_as_uint(x) & first), yh = __uint_as_float(__float_as_uint(y) & first);
+			hi[e] = pack_bf16x2(xh, yh), lo[e] = pack_bf16x2(__builtin_fmaf(xh, -0x1.fffffep-1f, x), __builtin_fmaf(yh, -0x1.fffffep-1f, y));
 		}
 		if(i < R * 4 * KS) {
 			*reinterpret_cast<u32x4*>(smem + Q_AT + row * Q_ROW + ch * 16) = ch < DC ? hi : lo;

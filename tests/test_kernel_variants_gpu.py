@@ -594,10 +594,42 @@ def test_strips_do_not_round_q(af3, oracle, B, H, L, D):
     out = f32np(af3.dot_product_attention_cpp(q.cuda(), k.cuda(), v.cuda(), keep.cuda(), bias.cuda()))
     want = oracle.dpa_formula(f32np(q), f32np(k), f32np(v), keep.numpy(), f32np(bias))
     size = oracle.dpa_formula(f32np(q), f32np(k), np.abs(f32np(v)), keep.numpy(), f32np(bias))
-    # half a unit in the last of eight bits, 2^-8 at most, each: a weight, the sum of the weights, the result; q to 2^-17 (2^-8 / 8 for sums of |q k| up to 2^6)
+    # half a unit in the last of eight bits, 2^-8 at most, each: a weight, the sum of the weights, the result; q to 2^-16 (2^-8 / 8 for sums of |q k| up to 2^5)
     assert (np.abs(out - want) <= 3.125 * 2.0 ** -8 * size + 1e-6).all()
     # in rms those three are independent and each below a third of its maximum on average
     assert np.sqrt(np.mean((out - want) ** 2)) <= 2.0 ** -9 * np.sqrt(np.mean(size ** 2))
+
+
+@pytest.mark.parametrize("B,H,L,D", [(2, 4, 40, 8), (1, 16, 50, 16), (1, 16, 257, 16), (37, 4, 37, 32), (2, 4, 512, 32), (3, 4, 63, 24), (1, 16, 290, 24), (1, 16, 769, 24), (1, 16, 200, 40), (1, 5, 1155, 40), (1, 16, 50, 48), (1, 16, 513, 48)])
+@pytest.mark.parametrize("kind", ["k+inf", "k-inf", "k nan", "q inf", "v+inf", "v both"])
+def test_strips_infinities_act_as_in_the_formula(af3, B, H, L, D, kind):
+    """Infinities and NaN of live keys in each chunk of eight head columns, with and without a second term of q: NaN rows where the formula has
+    them, every other row as without them."""
+    g = torch.Generator().manual_seed(L + D)
+    q, k, v = (torch.randn(B, H, L, D, generator=g).to(torch.bfloat16) for _ in range(3))
+    bias = torch.randn(H, L, L, generator=g).to(torch.bfloat16)
+    keep = torch.rand(B, L, generator=g) < 0.8
+    at = [(i % B, i % H, (L // 3 + 7 * i) % L, 8 * i + (i + 3) % 8) for i in range(D // 8)]   # (one key per chunk)
+    inf = float("inf")
+    for b, h, j, c in at:
+        keep[b, j] = True
+        if kind[0] == "k":
+            k[b, h, j, c] = {"k+inf": inf, "k-inf": -inf, "k nan": float("nan")}[kind]
+        elif kind == "q inf":
+            q[b, h, j, c] = inf
+        else:
+            v[b, h, j, c] = inf
+            if kind == "v both":
+                keep[b, j - 1] = True
+                v[b, h, j - 1, c] = -inf
+    print("case", B, H, L, D, kind, flush=True)
+    out = af3.dot_product_attention_cpp(q.cuda(), k.cuda(), v.cuda(), keep.cuda(), bias.cuda()).cpu().double()
+    s = (q.double() @ k.double().transpose(-1, -2)) * D ** -0.5 + bias.double()
+    want = s.masked_fill(~keep[:, None, None, :], -1e9).softmax(-1) @ v.double()
+    assert torch.equal(out.isnan(), want.isnan()) and torch.equal(out.isinf(), want.isinf())
+    assert torch.equal(out[out.isinf()] > 0, want[want.isinf()] > 0)
+    ok = want.isfinite()
+    assert ((out - want).abs()[ok] <= 2e-2).all()   # (bf16's budget)
 
 
 @pytest.mark.parametrize("H,L,D,first", [
