@@ -15,9 +15,10 @@
 // order in which ds_read_b64_tr_b16 delivers V^T.  A column of ones in V's padding (or a constant operand) makes the row sums one more
 // column of O.
 //
-// Softmax: the walk subtracts nothing at first.  Sums that end within 2^-60 .. 2^100 with finite results stand (probabilities and
-// sums are floating-point; 2^-60 leaves 66 powers of two below a row's largest probability); otherwise the workgroup finds its
-// rows' maxima in a walk of their own and repeats the walk with them.
+// Softmax: the walk subtracts nothing, or, from rows that look masked through their bias, that bias.  Sums that end within
+// 2^-60 .. 2^100 with finite results stand (probabilities and sums are floating-point; 2^-60 leaves 66 powers of two below a row's
+// largest probability); otherwise the workgroup finds its rows' maxima in a walk of their own and repeats the walk with them (one such
+// row in every strip: 7.4 -> 13.4 us at 16 x 768 x 24, 17.7 -> 41 at 1536).
 //
 // Reference: one (batch, head, query tile) task of src/csrc/dot_product_attention.cpp:88-191.
 #include "mfma_helpers.hpp"
@@ -73,7 +74,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 	constexpr int SUM_COL = KIND == 0 ? 24 : 16 * ND;
 	extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
 	float* const s_max = reinterpret_cast<float*>(smem + Q_AT);   // (q is in registers by then)
-	int* const   s_bad = reinterpret_cast<int*>(smem + lds::FLAG_AT);
+	int* const   s_bad = reinterpret_cast<int*>(smem + lds::FLAG_AT);   // [0]: rows whose sums do not stand; [1]: how many wavefronts took references from samples
 
 	asm volatile("" ::"s"(p.q), "s"(p.k), "s"(p.v), "s"(p.bias), "s"(p.mask), "s"(p.q_h), "s"(p.k_h), "s"(p.v_h), "s"(p.bias_h), "s"(p.q_row), "s"(p.k_row), "s"(p.v_row), "s"(p.bias_row), "s"(p.H),
 				 "s"(p.L), "s"(p.D), "s"(p.per_chunk), "s"(p.scale));
@@ -170,7 +171,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 		if(lane < 8) *reinterpret_cast<uint32_t*>(smem + const_base + 4 * lane) = lane == 4 ? 0x3F80u : 0u;
 	};
 	fill();
-	if(tid == 0) *s_bad = 0;
+	if(tid < 2) s_bad[tid] = 0;
 
 	// ---- per-lane constants ----
 	u32x4 sel[2];   // half h of the tile's keys: row i picks key 8 (i / 4) + 4 h + i % 4
@@ -204,6 +205,8 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 	const int t_rd = g < 3 ? b_base + i16 * 64 + (((g + 1) ^ ((i16 >> 2) & 3)) << 4) : t_base + i16 * 4;   // the dword behind this lane's eight elements
 	const int t_half = g < 3 ? NB * 1024 : NT * 256, t_blk = g < 3 ? 1024 : 64;
 	const int b_rd = b_base + i16 * 64 + ((g ^ ((i16 >> 2) & 3)) << 4);
+	const int s_row = lane < R ? lane : R - 1, s_rd = b_base + s_row * 64 + (((s_row >> 2) & 3) << 4) + 2;   // one bias (the first or second of this wavefront's first tile) of each row
+	const unsigned s_low = strip * R + s_row < L ? 0xC200u : 0xFFFFu;   // -32 (of rows past L: none is lower)
 
 	// q to LDS, scaled, as two bf16 terms as far as there is room: the second one of the first columns takes the columns behind head_dim, where
 	// K's operand repeats those columns, or (head_dim 32: none) all of it goes through matrix instructions of its own.  (Rounded once, the
@@ -300,10 +303,32 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 	};
 	auto wait_loads = [](auto n_c) __attribute__((always_inline)) { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(n_c)::value) : "memory"); };
 
+	// Padded queries masked through the bias would leave the range and have their strips walked three times.  A wavefront that finds a row's
+	// bias below -32 at the head of its first tile looks at two more of each row, one of them the row's own (rows masked but for their
+	// neighbourhood show themselves there), and takes the larger for a reference where both are that low.  (Other wavefronts of the strip
+	// come to the same answer or, where they had no reason to look, to a count that does not match at the end.)  us per call, one-row kernel /
+	// without this / with it: 16 heads of 24 x 768, the last tenth of the rows at -1e9 9.6 / 13.1 / 7.8 (ordinary rows 9.7 / 7.4 / 7.4, rows that
+	// see 64 neighbours - / 7.3 / 7.5), x 1536 19.1 / 31.7 / 18.3, 37 x 4 x 37 x 32 5.6 / 8.3 / 5.5.
 	f32x4 o[NB][NO];
-	float m_ref[NB];   // with_reference: the maximum of this lane's query row of each block
-	bool with_reference = false;
-	for(;;) {
+	float m_ref[NB];   // what the walk with references (REF) takes off this lane's query row of each block
+	int   ref = 0;
+	if(__builtin_expect(__ballot(*reinterpret_cast<const uint16_t*>(smem + s_rd) > s_low) != 0 && my_n > 0, 0)) {   // (bf16 bits; negative NaN as well)
+		int row = strip * R + s_row;
+		asm volatile("" : "+v"(row));   // (none of this is prepared at the start)
+		const bool     in  = row < L;
+		const int      far = in ? row + (L >> 1) : 0, at = in ? row * (int)p.bias_row : 0;
+		const uint32_t r0 = *reinterpret_cast<const uint16_t*>(bias + (uint32_t)(at + (in ? row : 0) * 2)), r1 = *reinterpret_cast<const uint16_t*>(bias + (uint32_t)(at + (far < L ? far : far - L) * 2));
+		const uint32_t lim = p.bias_limit & 0xffffu;   // (as the walk takes them)
+		float          m = fmaxf(bf16_bits_to_f32(r0 < lim ? r0 : lim), bf16_bits_to_f32(r1 < lim ? r1 : lim));
+		m   = in && m < -32.f ? m : 0.f;
+		ref = __builtin_amdgcn_readfirstlane(__ballot(m < 0.f) != 0);
+		if(__ballot(m < MASK_DROPPED)) my_n = my_all;   // (there a dropped key's logit is no lower than the others': all keys count)
+#pragma unroll
+		for(int c = 0; c < NB; c++) m_ref[c] = __shfl(m, 16 * c + i16);
+		if(ref && lane == 0) atomicAdd(s_bad + 1, 1);
+	}
+	auto walk = [&](auto ref_c) __attribute__((always_inline)) {
+		constexpr bool REF = decltype(ref_c)::value;
 #pragma unroll
 		for(int c = 0; c < NB; c++)
 #pragma unroll
@@ -356,7 +381,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 					pc[I] = pack_bf16x2(__builtin_amdgcn_exp2f(s[I >> 1][(I & 1) * 2] * LOG2E), __builtin_amdgcn_exp2f(s[I >> 1][(I & 1) * 2 + 1] * LOG2E));
 				};
 				const bf16x8 pp = __builtin_bit_cast(bf16x8, pprev);
-				if(with_reference) {   // (from the finished logit: where all keys are dropped, all are equal)
+				if constexpr(REF) {   // (from the finished logit: where all keys are dropped, all are equal)
 #pragma unroll
 					for(int e = 0; e < 4; e++) s[0][e] -= m_ref[C], s[1][e] -= m_ref[C];
 				}
@@ -456,9 +481,11 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 			for(int d = 0; d < ND; d++) o[NB - 1][d] = mfma(vf[d], pp, o[NB - 1][d]);
 			if constexpr(KIND > 0) o[NB - 1][ND] = mfma(__builtin_bit_cast(bf16x8, ones), pp, o[NB - 1][ND]);
 		}
+	};
 
-		// ---- the wavefronts' partial sums, added up by all threads: four head columns of a row per thread and trip; optional output
-		// gate (out *= sigmoid(gate)), any row and head strides.  Results leave before it is known whether they stand. ----
+	// ---- the wavefronts' partial sums, added up by all threads: four head columns of a row per thread and trip; optional output
+	// gate (out *= sigmoid(gate)), any row and head strides.  Results leave before it is known whether they stand. ----
+	auto merge = [&]() __attribute__((always_inline)) {   // whether they do not
 		asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (no load may still be writing LDS)
 		__syncthreads();   // (they lie over the tiles)
 		float* const part = reinterpret_cast<float*>(smem) + wave * (R * PC) + i16 * PC + 4 * g;
@@ -492,64 +519,66 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 			if(p.out_f32) *reinterpret_cast<f32x4*>(at + d0 * 4) = t;
 			else *reinterpret_cast<u32x2*>(at + d0 * 2) = u32x2{pack_bf16x2(t[0], t[1]), pack_bf16x2(t[2], t[3])};
 		}
-		if(with_reference) return;
-		if(__ballot(bad) && lane == 0) *s_bad = 1;
+		if(__ballot(bad) && lane == 0) s_bad[0] = 1;
 		__syncthreads();
-		if(!__builtin_amdgcn_readfirstlane(*s_bad)) return;
-		// ---- rare: the rows' maxima, then the walk again, over all tiles (a row without a live key needs them) ----
-		my_n = my_all > 0 ? my_all : 0;
-		fill();
-		{
-			{
-				k_rsrc[2] = k_bytes, v_rsrc[2] = v_bytes, b_rsrc[2] = b_bytes;
-				float mx[NB];
+		const int some = __builtin_amdgcn_readfirstlane(s_bad[0]), looked = __builtin_amdgcn_readfirstlane(s_bad[1]);
+		return (some | looked) != 0 && (some != 0 || looked != (n_tiles < NW ? n_tiles : NW));
+	};
+
+	if(ref) walk(std::true_type{});
+	else walk(std::false_type{});
+	if(!merge()) return;
+
+	// ---- rare: the rows' maxima, then the walk again, over all tiles (a row without a live key needs them) ----
+	my_n = my_all > 0 ? my_all : 0;
+	fill();
+	k_rsrc[2] = k_bytes, v_rsrc[2] = v_bytes, b_rsrc[2] = b_bytes;
+	float mx[NB];
 #pragma unroll
-				for(int c = 0; c < NB; c++) mx[c] = -__builtin_inff();
-				for(int i = 0; i < my_all; i++) {
-					const int at = (wave + NW * i) * KT_S, k0 = at < last_k0 ? at : last_k0;
-					load_k(k0);
+	for(int c = 0; c < NB; c++) mx[c] = -__builtin_inff();
+	for(int i = 0; i < my_all; i++) {
+		const int at = (wave + NW * i) * KT_S, k0 = at < last_k0 ? at : last_k0;
+		load_k(k0);
 #pragma unroll
-					for(int c = 0; c < NB; c++) load_b(k0, 0, c);
-					load_t(k0, 0);
-					wait_loads(ic<0>{});
-					bf16x8 kf[2][KS];
-					f32x4  mk[2];
-					read_k(kf, mk, i);
+		for(int c = 0; c < NB; c++) load_b(k0, 0, c);
+		load_t(k0, 0);
+		wait_loads(ic<0>{});
+		bf16x8 kf[2][KS];
+		f32x4  mk[2];
+		read_k(kf, mk, i);
 #pragma unroll
-					for(int c = 0; c < NB; c++) {
-						const bf16x8 bb = clamped(read_b(0, c, k0));
+		for(int c = 0; c < NB; c++) {
+			const bf16x8 bb = clamped(read_b(0, c, k0));
 #pragma unroll
-						for(int hf = 0; hf < 2; hf++) {
-							f32x4 s = mfma(__builtin_bit_cast(bf16x8, sel[hf]), bb, mk[hf]);
+			for(int hf = 0; hf < 2; hf++) {
+				f32x4 s = mfma(__builtin_bit_cast(bf16x8, sel[hf]), bb, mk[hf]);
 #pragma unroll
-							for(int st = 0; st < KS; st++) s = mfma(kf[hf][st], qf[c][st], s);
-							if constexpr(LO) s = mfma(kf[hf][0], ql[c], s);
-							mx[c] = fmaxf(fmaxf(fmaxf(mx[c], s[0]), s[1]), fmaxf(s[2], s[3]));
-						}
-					}
-					asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (read before the next tile's loads write there)
-				}
-#pragma unroll
-				for(int c = 0; c < NB; c++) {
-					mx[c] = fmaxf(mx[c], __shfl_xor(mx[c], 16));
-					mx[c] = fmaxf(mx[c], __shfl_xor(mx[c], 32));
-					if(g == 0) s_max[wave * R + 16 * c + i16] = mx[c];
-				}
-				__syncthreads();
-#pragma unroll
-				for(int c = 0; c < NB; c++) {
-					float m = s_max[16 * c + i16];
-#pragma unroll
-					for(int w = 1; w < NW; w++) m = fmaxf(m, s_max[w * R + 16 * c + i16]);
-					m_ref[c] = m;
-				}
-				with_reference = true;
-				__syncthreads();
-				load_first();
-				wait_loads(ic<0>{});
+				for(int st = 0; st < KS; st++) s = mfma(kf[hf][st], qf[c][st], s);
+				if constexpr(LO) s = mfma(kf[hf][0], ql[c], s);
+				mx[c] = fmaxf(fmaxf(fmaxf(mx[c], s[0]), s[1]), fmaxf(s[2], s[3]));
 			}
 		}
+		asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (read before the next tile's loads write there)
 	}
+#pragma unroll
+	for(int c = 0; c < NB; c++) {
+		mx[c] = fmaxf(mx[c], __shfl_xor(mx[c], 16));
+		mx[c] = fmaxf(mx[c], __shfl_xor(mx[c], 32));
+		if(g == 0) s_max[wave * R + 16 * c + i16] = mx[c];
+	}
+	__syncthreads();
+#pragma unroll
+	for(int c = 0; c < NB; c++) {
+		float m = s_max[16 * c + i16];
+#pragma unroll
+		for(int w = 1; w < NW; w++) m = fmaxf(m, s_max[w * R + 16 * c + i16]);
+		m_ref[c] = m;
+	}
+	__syncthreads();
+	load_first();
+	wait_loads(ic<0>{});
+	walk(std::true_type{});
+	merge();
 }
 
 }  // namespace

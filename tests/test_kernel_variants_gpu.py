@@ -632,6 +632,40 @@ def test_strips_infinities_act_as_in_the_formula(af3, B, H, L, D, kind):
     assert ((out - want).abs()[ok] <= 2e-2).all()   # (bf16's budget)
 
 
+@pytest.mark.parametrize("B,H,L,D", [(1, 1, 32, 24), (2, 3, 33, 8), (1, 16, 50, 48), (37, 4, 37, 32), (1, 16, 257, 32), (1, 16, 290, 24), (1, 16, 513, 48), (1, 5, 1155, 16), (1, 16, 769, 24), (1, 16, 1040, 48)])
+@pytest.mark.parametrize("kind", ["far", "-1e9", "-inf", "window", "misleading", "scattered"])
+def test_strips_rows_masked_through_the_bias(af3, B, H, L, D, kind):
+    """Query rows whose biases all lie far below zero, rows of which only the neighbourhood of the diagonal does not, and rows
+    whose two samples are no sign of the rest."""
+    g = torch.Generator().manual_seed(L + D)
+    q, k, v = (torch.randn(B, H, L, D, generator=g).to(torch.bfloat16) for _ in range(3))
+    bias = torch.randn(H, L, L, generator=g).to(torch.bfloat16)
+    keep = torch.rand(B, L, generator=g) < 0.8
+    keep[:, L // 3] = True
+    i = torch.arange(L)
+    if kind in ("far", "-1e9", "-inf"):
+        bias[:, L - L // 5:] = {"far": -3.0e4, "-1e9": -1.0e9, "-inf": float("-inf")}[kind]
+    elif kind == "window":
+        keep[:] = True
+        bias[:, (i[:, None] - i[None]).abs() > 20] = -3.0e4
+    elif kind == "misleading":
+        bias[:, i, i] = -3.0e4
+        bias[:, i, (i + L // 2) % L] = -3.0e4
+        bias[:, ::2, : L // 4] = -3.0e4
+    else:
+        bias[:, ::5] = torch.linspace(-300.0, -180.0, L)
+        bias[:, 1::7] -= 45
+    print("case", B, H, L, D, kind, flush=True)
+    out = af3.dot_product_attention_cpp(q.cuda(), k.cuda(), v.cuda(), keep.cuda(), bias.cuda()).cpu().float()
+    # one batch row takes biases down to -2^126, several down to -2^16 (q.k still counts there)
+    lowest = -2.0 ** 126 if B == 1 else -2.0 ** 16
+    s = (q.float() @ k.float().transpose(-1, -2)) * D ** -0.5 + bias.float().clamp(min=lowest)
+    rows = L - L // 5 if kind == "-inf" and B == 1 else L   # (beyond these a dropped key's logit is no lower)
+    s[:, :, :rows].masked_fill_(~keep[:, None, None, :], float("-inf"))
+    want = s.softmax(-1) @ v.float()
+    assert (out - want).abs().max() <= 2e-2   # (bf16's budget; a logit at -3e4 or -2^16 has steps of 2^-9 or 2^-8)
+
+
 @pytest.mark.parametrize("H,L,D,first", [
     (2, 7872, 48, 1), (2, 7873, 48, 0), (2, 8096, 48, 1), (2, 8097, 40, 0), (2, 8191, 48, 0), (2, 8192, 48, 1), (2, 8192, 32, 1),   # four blocks, rows at any address: the most LDS a workgroup takes
     (3, 8192, 48, 0), (2, 8192, 40, 0),                              # two workgroups per compute unit
