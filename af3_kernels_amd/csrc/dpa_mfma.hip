@@ -67,12 +67,11 @@ __device__ __forceinline__ void load_bias8_guarded(const void* bias_row, int64_t
 // (lim: that limit, twice.  Batches that have this kernel or the shared-bias kernel read the bias in place for speed take the
 // latter's limit of -2^16: a query row whose biases all lie beyond it is the softmax of q.k alone, whichever kernel serves it.)
 constexpr uint32_t BIAS_LIMIT_SINGLE = 0xFE80FE80u, BIAS_LIMIT_BATCH = 0xC780C780u;
-typedef __attribute__((ext_vector_type(2))) unsigned short u16x2;
 __device__ __forceinline__ u32x4 bias_frag_finite(u32x4 w, uint32_t lim) {
 #pragma unroll
 	for(int j = 0; j < 4; j++) {
 		const uint32_t x = w[j];  // (a copy: __builtin_bit_cast applied to the vector element itself reads element 0 with this compiler)
-		w[j] = __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2, x), __builtin_bit_cast(u16x2, lim)));
+		w[j] = bias_limited(x, lim);
 	}
 	return w;
 }
@@ -429,9 +428,7 @@ __global__ void __launch_bounds__((NW + (KSL ? 4 : 0)) * 64) __attribute__((amdg
 				const int c = c0 + i * NW;
 				if(c >= n_chunks) break;
 				const int key0 = c * 256 + 4 * lane, over = key0 + 4 - (int)L;
-				uint32_t  m    = mraw[i];
-				if(over > 0) m = over < 4 ? m >> (8 * over) : 0u;
-				const uint32_t gone = (~(((m & 0x7f7f7f7fu) + 0x7f7f7f7fu) | m) >> 7) & 0x01010101u;   // 1 in the bytes that are zero
+				const uint32_t m = keep_bytes_in_row(mraw[i], over), gone = gone_bytes(m);
 				u32x4          e;
 #pragma unroll
 				for(int j = 0; j < 4; j++) e[j] = ((0u - ((gone >> (8 * j)) & 1u)) & (uint32_t)MASK_DROPPED_BF16) | (L2DOM ? 0x3F800000u : 0u);

@@ -208,11 +208,8 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DP
 			for(int i = 0; i < 4; i++) {
 				const int c = c0 + i * NW;
 				if(c >= n_chunks) break;
-				const int over = c * 256 + 4 * lane + 4 - (int)L;
-				uint32_t  m    = mraw[i];
-				if(over > 0) m = over < 4 ? m >> (8 * over) : 0u;
 				// one bit per byte that is not zero, four of them side by side, eight lanes' together in the tile's word
-				const uint32_t live = ((((m & 0x7f7f7f7fu) + 0x7f7f7f7fu) | m) >> 7) & 0x01010101u;
+				const uint32_t live = live_bytes(keep_bytes_in_row(mraw[i], c * 256 + 4 * lane + 4 - (int)L));
 				int            w    = (int)(((live * 0x01020408u) >> 24) << (4 * (lane & 7)));
 				w |= __builtin_amdgcn_update_dpp(0, w, 0xB1, 0xf, 0xf, true);    // lane ^ 1
 				w |= __builtin_amdgcn_update_dpp(0, w, 0x4E, 0xf, 0xf, true);    // lane ^ 2

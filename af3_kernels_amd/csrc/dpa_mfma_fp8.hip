@@ -254,16 +254,8 @@ __global__ void __launch_bounds__(KS * NW8 * 64) __attribute__((amdgpu_waves_per
 				const int c = c0 + i * (KS * NW8);
 				if(c >= n_chunks) break;
 				const int key0 = c * 256 + 4 * lane, over = key0 + 4 - (int)L;
-				uint32_t  m    = mraw[i];
-				if(over > 0) m = over < 4 ? m >> (8 * over) : 0u;
-				const uint32_t gone = (~(((m & 0x7f7f7f7fu) + 0x7f7f7f7fu) | m) >> 7) & 0x01010101u;   // 1 in the bytes that are zero
-				uint32_t       lo = ((gone & 1u) | ((gone & 0x100u) << 8)) * MASK_DROPPED_BF16, hi = (((gone >> 16) & 1u) | ((gone >> 24) << 16)) * MASK_DROPPED_BF16;
-				if(over > 0) {
-					constexpr uint32_t OUT = MASK_OUT_OF_RANGE_BF16;   // keys from L on
-					lo = over <= 2 ? lo : over == 3 ? (lo & 0xffffu) | (OUT << 16) : OUT | (OUT << 16);
-					hi = over == 1 ? (hi & 0xffffu) | (OUT << 16) : OUT | (OUT << 16);
-				}
-				if(key0 < n_ktiles * KT8) *reinterpret_cast<u32x2*>(mask_tab + key0) = u32x2{lo, hi};
+				const uint32_t m = keep_bytes_in_row(mraw[i], over), gone = gone_bytes(m);
+				if(key0 < n_ktiles * KT8) *reinterpret_cast<u32x2*>(mask_tab + key0) = mask_values_bf16(gone, over);
 				const unsigned long long bal = __ballot(m != 0u), baln = __ballot(gone != 0u);   // 16 lanes per tile (keys from L on are gone)
 				if(lane < 4 && 4 * c + lane < n_ktiles) tile_flags[4 * c + lane] = (uint8_t)((((bal >> (16 * lane)) & 0xffffull) != 0 ? 1 : 0) | (((baln >> (16 * lane)) & 0xffffull) != 0 ? 2 : 0));
 			}

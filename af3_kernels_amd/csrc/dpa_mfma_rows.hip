@@ -149,10 +149,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 		const int key0 = 256 * c + 4 * lane;
 		return *reinterpret_cast<const u32_bytes*>(keep + (key0 + 4 <= (int)L ? key0 : (int)L - 4));
 	};
-	auto mask_of = [&](int c, uint32_t w) -> uint32_t {   // ... zeros from L on
-		const int over = 256 * c + 4 * lane + 4 - (int)L;
-		return over <= 0 ? w : over < 4 ? w >> (8 * over) : 0u;
-	};
+	auto mask_of = [&](int c, uint32_t w) -> uint32_t { return keep_bytes_in_row(w, 256 * c + 4 * lane + 4 - (int)L); };
 	auto request_mask = [&](int c0) {
 #pragma unroll
 		for(int c = 0; c < MASK_CHUNKS; c++) {
@@ -302,15 +299,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 			auto write_chunk = [&](int c, uint32_t m) {
 				const int key0 = 256 * c + 4 * lane;
 				if(key0 >= n_keys_tab) return;
-				const uint32_t gone = (~(((m & 0x7f7f7f7fu) + 0x7f7f7f7fu) | m) >> 7) & 0x01010101u;   // 1 in the bytes that are zero
-				uint32_t       lo = ((gone & 1u) | ((gone & 0x100u) << 8)) * MASK_DROPPED_BF16, hi = (((gone >> 16) & 1u) | ((gone >> 24) << 16)) * MASK_DROPPED_BF16;
-				if(key0 + 4 > (int)L) {
-					const int in = (int)L - key0;   // keys of this lane in front of L
-					constexpr uint32_t OUT = MASK_OUT_OF_RANGE_BF16;
-					lo = in >= 2 ? lo : in == 1 ? (lo & 0xffffu) | (OUT << 16) : OUT | (OUT << 16);
-					hi = in == 3 ? (hi & 0xffffu) | (OUT << 16) : OUT | (OUT << 16);
-				}
-				*reinterpret_cast<u32x2*>(mask_tab + ((key0 >> 5) * ROWS + r) * 32 + (key0 & 31)) = u32x2{lo, hi};
+				*reinterpret_cast<u32x2*>(mask_tab + ((key0 >> 5) * ROWS + r) * 32 + (key0 & 31)) = mask_values_bf16(gone_bytes(m), key0 + 4 - (int)L);
 			};
 			for(int c0 = 0; 256 * c0 < n_keys_tab; c0 += MASK_CHUNKS) {
 				if(c0 > 0) request_mask(c0);
@@ -507,8 +496,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 				bias_frag[4 * ld] = v[0], bias_frag[4 * ld + 1] = v[1], bias_frag[4 * ld + 2] = v[2], bias_frag[4 * ld + 3] = v[3];
 			}
 		} else if constexpr(DIRECT || STAGED) {
-			typedef __attribute__((ext_vector_type(2))) unsigned short u16x2;
-			const u16x2 lim = {(unsigned short)0xC780, (unsigned short)0xC780};
+			const uint32_t lim = 0xC780C780u;
 			if constexpr(STAGED) {  // this lane's four 8-byte pieces, keys 8 ld + 4 half .. + 3 of row n: chunk ld at its swizzled place
 #pragma unroll
 				for(int ld = 0; ld < 4; ld++)
@@ -519,7 +507,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
 				for(int j = 0; j < 2; j++) {
 					const uint32_t raw = braw[ld][j];
-					const uint32_t w   = __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2, raw), lim));
+					const uint32_t w   = bias_limited(raw, lim);
 					bias_frag[4 * ld + 2 * j]     = __uint_as_float(w << 16) * LOG2E;
 					bias_frag[4 * ld + 2 * j + 1] = __uint_as_float(w & 0xffff0000u) * LOG2E;
 				}

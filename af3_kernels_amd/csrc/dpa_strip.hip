@@ -290,14 +290,11 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 	};
 	auto mfma = [](const bf16x8& a, const bf16x8& bb, const f32x4& c) __attribute__((always_inline)) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bb, c, 0, 0, 0); };
 	auto clamped = [&](const bias_piece& raw) __attribute__((always_inline)) {
-		typedef __attribute__((ext_vector_type(2))) unsigned short u16x2;
 		u32x4 w;
 #pragma unroll
 		for(int j = 0; j < 4; j++) {
-			const uint32_t lim = p.bias_limit, lo = raw.w[j];
-			uint32_t       x = lo;
-			if constexpr(ANY) x = __builtin_amdgcn_alignbit(j < 3 ? raw.w[j < 3 ? j + 1 : 3] : raw.next, lo, raw.sh);
-			w[j] = __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2, x), __builtin_bit_cast(u16x2, lim)));
+			const uint32_t lo = raw.w[j];
+			w[j] = bias_limited(ANY ? __builtin_amdgcn_alignbit(j < 3 ? raw.w[j < 3 ? j + 1 : 3] : raw.next, lo, raw.sh) : lo, p.bias_limit);
 		}
 		return __builtin_bit_cast(bf16x8, w);
 	};

@@ -1,4 +1,4 @@
-// Device helpers shared by the bf16 matrix-core attention kernels (dpa_mfma.hip, dpa_mfma_rows.hip).
+// Device helpers shared by the matrix-core attention kernels (dpa_mfma.hip, dpa_mfma_rows.hip, dpa_strip.hip, dpa_mfma_fp8.hip, dpa_mfma_f32.hip).
 #pragma once
 #include <type_traits>
 
@@ -19,6 +19,7 @@ typedef __attribute__((ext_vector_type(4), aligned(2))) uint32_t u32x4_any;
 typedef __attribute__((ext_vector_type(2), aligned(2))) uint32_t u32x2_any;
 typedef __attribute__((ext_vector_type(4), aligned(4))) float    f32x4_any;
 typedef __attribute__((aligned(1))) uint32_t u32_bytes;
+typedef __attribute__((ext_vector_type(2))) unsigned short u16x2;
 template <int V>
 using ic = std::integral_constant<int, V>;
 
@@ -42,6 +43,30 @@ __device__ __forceinline__ float half_swap_max(float x) {
 	// lower half of the other, so (x, x) yields {low|low} and {high|high}.
 	auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
 	return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+// ---- key masks, four keep bytes to a word ----
+// what a load at `key + 4 <= L ? key : L - 4` brought for keys from `key` on, `over` = key + 4 - L: zeros from L on
+__device__ __forceinline__ uint32_t keep_bytes_in_row(uint32_t m, int over) {
+	if(over > 0) m = over < 4 ? m >> (8 * over) : 0u;
+	return m;
+}
+// 1 in the bytes that are not zero, and in those that are
+__device__ __forceinline__ uint32_t live_bytes(uint32_t m) { return ((((m & 0x7f7f7f7fu) + 0x7f7f7f7fu) | m) >> 7) & 0x01010101u; }
+__device__ __forceinline__ uint32_t gone_bytes(uint32_t m) { return (~(((m & 0x7f7f7f7fu) + 0x7f7f7f7fu) | m) >> 7) & 0x01010101u; }
+// the additive mask values of four keys, as bf16
+__device__ __forceinline__ u32x2 mask_values_bf16(uint32_t gone, int over) {
+	constexpr uint32_t OUT = MASK_OUT_OF_RANGE_BF16;   // keys from L on
+	uint32_t           lo = ((gone & 1u) | ((gone & 0x100u) << 8)) * MASK_DROPPED_BF16, hi = (((gone >> 16) & 1u) | ((gone >> 24) << 16)) * MASK_DROPPED_BF16;
+	if(over > 0) {
+		lo = over <= 2 ? lo : over == 3 ? (lo & 0xffffu) | (OUT << 16) : OUT | (OUT << 16);
+		hi = over == 1 ? (hi & 0xffffu) | (OUT << 16) : OUT | (OUT << 16);
+	}
+	return u32x2{lo, hi};
+}
+// two biases, limited from below: as unsigned numbers every negative bf16 beyond the limit, -inf and negative NaN included, is larger
+__device__ __forceinline__ uint32_t bias_limited(uint32_t x, uint32_t lim) {
+	return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2, x), __builtin_bit_cast(u16x2, lim)));
 }
 
 // 16 bytes per lane from a raw buffer straight into LDS (lane i lands at lds_addr + 16*i).  Written as
