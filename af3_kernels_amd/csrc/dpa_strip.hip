@@ -243,6 +243,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 		if(bal) my_n = (bal >> 32) && 2 * j + 1 < my_all ? 2 * j + 2 : 2 * j + 1;
 	}
 	asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+	const unsigned long long low = __ballot(*reinterpret_cast<const uint16_t*>(smem + s_rd) > s_low);   // (bf16 bits; negative NaN as well)
 	__syncthreads();   // q
 	bf16x8 qf[NB][KS], ql[NB];   // (ql: LO only)
 #pragma unroll
@@ -309,7 +310,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 	f32x4 o[NB][NO];
 	float m_ref[NB];   // what the walk with references (REF) takes off this lane's query row of each block
 	int   ref = 0;
-	if(__builtin_expect(__ballot(*reinterpret_cast<const uint16_t*>(smem + s_rd) > s_low) != 0 && my_n > 0, 0)) {   // (bf16 bits; negative NaN as well)
+	if(__builtin_expect(low != 0 && my_n > 0, 0)) {
 		int row = strip * R + s_row;
 		asm volatile("" : "+v"(row));   // (none of this is prepared at the start)
 		const bool     in  = row < L;
