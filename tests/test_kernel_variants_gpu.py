@@ -582,12 +582,14 @@ def test_fp32_mask_rows(af3, oracle, B, H, L, D, kind):
     assert np.abs(out - want).max() <= 1e-4   # (the fp32 tier)
 
 
-@pytest.mark.parametrize("B,H,L,D", [(2, 4, 40, 8), (1, 16, 200, 16), (9, 4, 57, 32), (2, 4, 512, 32), (1, 5, 1155, 16)])
-def test_strips_do_not_round_q(af3, oracle, B, H, L, D):
-    """head_dim 8 and 16 (q's second term in the padding), 32 (in instructions of its own): what is rounded is each weight, once, the row sum's
-    weights with it, and the result."""
+@pytest.mark.parametrize("B,H,L,D,whole", [(2, 4, 40, 8, 8), (1, 16, 200, 16, 16), (9, 4, 57, 32, 32), (2, 4, 512, 32, 32), (1, 5, 1155, 16, 16),
+                                           (1, 16, 300, 24, 8), (1, 16, 130, 40, 24), (2, 3, 257, 48, 16)])
+def test_strips_do_not_round_q(af3, oracle, B, H, L, D, whole):
+    """head_dim 8 and 16 (q's second term in the padding), 32 (in instructions of its own) and the columns of 24, 40 and 48 whose second
+    term the padding holds (q is zero in the others): what is rounded is each weight, once, the row sum's weights with it, and the result."""
     g = torch.Generator().manual_seed(L + D)
     q, k, v = (torch.randn(B, H, L, D, generator=g).mul(m).to(torch.bfloat16) for m in (6.0, 1.0, 1.0))
+    q[..., whole:] = 0
     bias = torch.randn(H, L, L, generator=g).to(torch.bfloat16)
     keep = torch.ones(B, L, dtype=torch.bool)
     print("case", B, H, L, D, flush=True)
