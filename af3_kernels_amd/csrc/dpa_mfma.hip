@@ -1499,7 +1499,9 @@ static int launch_nw(const af3_dpa_params& p, hipStream_t s) {
 		//   two pairs on shared tiles      7.5    9.2   11.0   13.4   27.7   31.3
 		//   one wavefront per block, x 4   8.3   11.6   14.9   18.1   21.3   24.6
 		//   four pairs (KSL 3)                                        19.5   21.3
-		// (bf16 biases with head_dim up to 48 come here only beyond what dpa_strip.hip takes: fewer than 32 keys, long or scattered rows.)
+		// That is the choice for fp32 biases and for head_dim above 48.  Of bf16 biases with head_dim up to 48 dpa_strip.hip takes most, and what
+		// comes here is: fewer than 32 keys (a pair per workgroup); K and V rows that lie apart, as in a packed projection, from where eight-wavefront
+		// strips no longer fit one round (16 heads: 769 aligned, 1025 odd); and dense rows beyond 1536 aligned, 1152 odd.
 		// (Pairs and the one-per-block form have four loading wavefronts.  With the registers of the other pairs' form -- four
 		// contraction chunks, P.V a stage late -- four pairs at head_dim 48 spilled 18 registers: 32.5 us at L = 1536.)
 		const int64_t wg64 = groups * ((p.L + 63) / 64), wg128 = groups * ((p.L + 127) / 128);

@@ -148,7 +148,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DP
 	// ---- key-mask bytes, requested first: four keys per lane at any address (the last four of a row that L ends in the middle of are
 	// shifted), 256 keys = eight tiles per wavefront and load, four loads under way.  (A byte per lane and a tile per half-wave and load,
 	// the list of tiles always compacted, 64-bit divisions: us per call before / now, B x 4 heads x L x 32: 2x128 7.39 / 6.59, 8x384 12.97 / 12.16,
-	// 64x256 21.6 / 21.1, 64x768 134.4 / 131.0.) ----
+	// 64x256 21.6 / 21.1, 64x768 135.8 / 134.8: there no more than calls differ by.) ----
 	const uint8_t* const keep     = p.key_mask ? p.key_mask + b * p.key_mask_stride_b : nullptr;
 	const bool           mask_vec = L >= 4;
 	const int            n_chunks = (n_tiles * F32_KT + 255) / 256;

@@ -625,7 +625,8 @@ int launch8(const af3_dpa_params& p, hipStream_t s) {
 	// is not worth its merge.  16 heads of 24, us per call, one part / two: 1x128 11.9/12.0, 1x256 14.1/13.5, 1x512 18.4/16.4, 2x777 25.5/22.9,
 	// 1x1536 33.8/27.5, 2x1536 42.5/39.4, 8x512 25.9/25.5, but 8x300 22.6/24.0, 3x1301 50.7/55.0, 3x1536 53.1/56.5.  Four parts are slower than two
 	// throughout (1x512 18.2, 1x1536 28.3).  Head_dim above 32 (one such workgroup per compute unit): 16 heads of 48, 1x777 29.2/26.0, 1x1536
-	// 40.9/34.3, 2x1200 43.7/49.9.
+	// 40.9/34.3, 2x1200 43.7/49.9.  (Compensated, head_dim 32, rows at any address: 128 registers with 5 spilled in one part, 7 in two;
+	// 16 heads of 32, 1x777 31.6/25.0, 1x1491 50.9/37.0, one part throughout 5x1491 89.6 against 79.7 at an aligned 1496.)
 	if constexpr(BMODE >= 2) {
 		const int64_t n_wg = p.B * p.H * ((p.L + NW8 * 32 - 1) / (NW8 * 32)), n_ktiles = (p.L + KT8 - 1) / KT8;
 		if(n_ktiles >= 3 && (n_wg <= 256 || (DP == 32 && n_wg <= 512 && n_ktiles >= 8))) return launch8_parts<DP, COMP, ONES, BMODE, 2>(p, s);

@@ -2,7 +2,7 @@
 // the token attention of the diffusion transformer, small batches), head_dim up to 48.
 //
 // Such a launch has few query rows (16 heads of 768: 12288, 12 per SIMD), so the query rows are cut fine and the key axis is cut as
-// well: a workgroup owns a strip of NB x 16 query rows of one (batch row, head) -- 48 rows of 768 or 96 of 1536 make 256 workgroups,
+// well: a workgroup owns a strip of NB x 16 query rows of one (batch row, head) -- one to four blocks; 48 rows of 768 make 256 workgroups,
 // one per compute unit -- and its wavefronts take the key tiles (32 keys) of the strip in turn.  The NB blocks of 16 rows are NB
 // independent chains of one wavefront: they share the tile's K, V and mask operands, and while one block's logits are exponentiated
 // the matrix pipe works on its neighbours.  Nothing is shared between wavefronts until the strip's partial sums are added up
@@ -67,6 +67,7 @@ struct strip_lds {
 template <int NB, int KIND, bool ANY, int NW>
 __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) dpa_strip_bf16_kernel(strip_args p) {
 	using lds = strip_lds<NB, KIND, ANY, NW>;
+	static_assert(NB <= 4, "the walk has four slots a tile");
 	constexpr int KS = lds::KS, NV = lds::NV, NT = lds::NT, R = lds::R, PC = lds::PC, WAVE_LDS = lds::WAVE, Q_AT = lds::Q_AT, Q_ROW = lds::Q_ROW, MASK_AT = lds::MASK_AT;
 	constexpr int ND = KIND == 2 ? 3 : 2;       // blocks of 16 head columns of V
 	constexpr int NO = KIND == 0 ? ND : ND + 1; // ... of O: the row sums in a block of their own, or in column 24
@@ -460,7 +461,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 						}
 					}
 				};
-				one(ic<0>{}), one(ic<1>{}), one(ic<2>{}), one(ic<3>{}), one(ic<4>{}), one(ic<5>{}), one(ic<6>{}), one(ic<7>{});
+				one(ic<0>{}), one(ic<1>{}), one(ic<2>{}), one(ic<3>{});
 				half = other;
 				i++, k0_0 = k0_1, k0_1 = k0_2, k0_2 = k0_2 + NW * KT_S < last_k0 ? k0_2 + NW * KT_S : last_k0;
 #pragma unroll
@@ -616,14 +617,17 @@ bool bias_rows_anywhere(const af3_dpa_params& p) { return (reinterpret_cast<uint
 // The lowest strip whose workgroups are all resident at once (a second round pays the start again): eight wavefronts and one workgroup
 // per compute unit, or four and two where three blocks are not enough or the row has so few tiles that eight would idle.  Measured, us per
 // call in a graph replay, one batch row of 16 heads (the kernel of dpa_mfma.hip / here):
-//   head_dim 24   L  64        128       256       384       512       640        768        896         1024        1280         1536
-//                 6.2 / 5.9  6.9 / 6.0  7.0 / 6.4  7.9 / 6.6  8.3 / 7.2  10.4 / 8.6  11.3 / 9.7   12.2 / 11.2  12.8 / 11.9  18.5 / 15.9  22.2 / 19.0
-//   head_dim 48      6.8 / 6.0  7.6 / 6.1  8.4 / 6.4  9.3 / 7.5  10.3 / 8.3  11.8 / 10.1  12.8 / 11.1  13.8 / 12.8  15.0 / 13.8  21.1 / 18.8  24.7 / 22.5
-// and beyond that, in two rounds, 29.0 / 32.6 and 32.3 / 40.2 at 1792.  Rows at any address (one more load and LDS read per piece):
-//   head_dim 24   L  65        257       385       513        769          1025         1281         1491
-//                 7.0 / 5.9  8.6 / 6.9  8.6 / 7.4  10.2 / 8.4  12.7 / 11.6  17.8 / 17.2  20.8 / 21.8  22.6 / 23.6
-// Few heads: 4 x 2048 x 24 23.9 / 10.6, 2 x 1500 x 48 29.7 / 9.6.  Batches that read in place: 37 x 4 x 37 x 32 5.4 / 5.0, 2 x 16 x 512 x 24
-// 8.5 / 7.2, 5 x 16 x 128 x 48 6.7 / 5.6.
+//   head_dim 24   L  64        128       256       384       512       640       768       896         1024        1280        1536
+//                 4.8 / 4.1  5.5 / 4.1  5.7 / 4.7  6.6 / 5.2  6.8 / 5.7  8.9 / 6.4  9.6 / 7.2  10.3 / 9.3  11.2 / 10.4  17.0 / 14.7  19.2 / 17.9
+//   head_dim 48      5.4 / 4.3  6.3 / 4.5  7.2 / 5.2  8.0 / 6.0  8.8 / 6.5  10.3 / 7.9  11.2 / 8.8  12.0 / 11.1  13.5 / 12.6  19.0 / 17.9  21.9 / 21.3
+// and beyond that, in two rounds, 22.1 / 29.3 and 25.9 / 33.7 at 1792.  Rows at any address (one more load and LDS read per piece):
+//   head_dim 24   L  65        257       385       513        769         1025         1153         1281         1491
+//                 5.8 / 4.2  7.3 / 5.5  7.4 / 6.0  8.6 / 6.9  10.2 / 8.8  15.9 / 15.3  16.5 / 17.7  18.9 / 20.4  20.5 / 22.1
+//   head_dim 48   L  65        257       385       513         769          1023         1155         1291         1491
+//                 6.6 / 4.6  7.7 / 6.3  8.6 / 7.0  10.1 / 8.5  11.8 / 10.9  14.6 / 13.9  20.6 / 21.2  22.3 / 23.6  25.0 / 26.2
+// (769 to 1023 there: four blocks on 256 registers, 6 of them spilled.)
+// Few heads: 4 x 2048 x 24 23.7 / 10.6, 2 x 1500 x 48 29.8 / 8.7, 2 x 7871 x 48 269 / 72, 3 x 8192 x 48 262 / 199.  Batches that read in place:
+// 37 x 4 x 37 x 32 5.6 / 5.1, 2 x 16 x 512 x 24 8.5 / 7.1, 5 x 16 x 128 x 48 6.9 / 5.8.
 strip_form strip_form_of(const af3_dpa_params& p) {
 	const bool any = bias_rows_anywhere(p);
 	auto wgs = [&](int nb) { return p.B * p.H * ((p.L + 16 * nb - 1) / (16 * nb)); };
