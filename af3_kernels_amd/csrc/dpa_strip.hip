@@ -75,7 +75,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 	constexpr int SUM_COL = KIND == 0 ? 24 : 16 * ND;
 	extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
 	float* const s_max = reinterpret_cast<float*>(smem + Q_AT);   // (q is in registers by then)
-	int* const   s_bad = reinterpret_cast<int*>(smem + lds::FLAG_AT);   // [0]: rows whose sums do not stand; [1]: how many wavefronts took references from samples
+	int* const   s_bad = reinterpret_cast<int*>(smem + lds::FLAG_AT);   // [0]: rows whose sums do not stand; [1]: how many wavefronts took references from samples; [2..3]: a byte per wavefront, whether its tiles hold a live key
 
 	asm volatile("" ::"s"(p.q), "s"(p.k), "s"(p.v), "s"(p.bias), "s"(p.mask), "s"(p.q_h), "s"(p.k_h), "s"(p.v_h), "s"(p.bias_h), "s"(p.q_row), "s"(p.k_row), "s"(p.v_row), "s"(p.bias_row), "s"(p.H),
 				 "s"(p.L), "s"(p.D), "s"(p.per_chunk), "s"(p.scale));
@@ -236,13 +236,15 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 
 	// ---- key-mask table of this wavefront's tiles: what is added to a key's logits.  Tiles behind the last one with a live key are not walked. ----
 	int  my_n = my_all > 0 ? 1 : 0;
+	bool my_live = false;
 	for(int j = 0; 2 * j < my_all; j++) {
 		const uint32_t m = (j == 0 ? m_first[0] : j == 1 ? m_first[1] : load_mask(j)) | (masked ? 0u : 1u);
 		const int      i = 2 * j + (lane >> 5), seen = ((wave + NW * i) * KT_S + KT_S) - L;   // seen: keys of the last tile that the one before has covered
 		if(i < my_all) *reinterpret_cast<float*>(smem + mask_base + i * 128 + (lane & 31) * 4) = (lane & 31) < seen ? MASK_OUT_OF_RANGE : m ? 0.f : MASK_DROPPED;
 		const unsigned long long bal = __ballot(m != 0u);
-		if(bal) my_n = (bal >> 32) && 2 * j + 1 < my_all ? 2 * j + 2 : 2 * j + 1;
+		if(bal) my_n = (bal >> 32) && 2 * j + 1 < my_all ? 2 * j + 2 : 2 * j + 1, my_live = true;
 	}
+	if(lane == 0) reinterpret_cast<uint8_t*>(s_bad + 2)[wave] = my_live;
 	asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 	const unsigned long long low = __ballot(*reinterpret_cast<const uint16_t*>(smem + s_rd) > s_low);   // (bf16 bits; negative NaN as well)
 	__syncthreads();   // q
@@ -291,12 +293,13 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 		return r;
 	};
 	auto mfma = [](const bf16x8& a, const bf16x8& bb, const f32x4& c) __attribute__((always_inline)) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bb, c, 0, 0, 0); };
+	uint32_t limit = p.bias_limit;
 	auto clamped = [&](const bias_piece& raw) __attribute__((always_inline)) {
 		u32x4 w;
 #pragma unroll
 		for(int j = 0; j < 4; j++) {
 			const uint32_t lo = raw.w[j];
-			w[j] = bias_limited(ANY ? __builtin_amdgcn_alignbit(j < 3 ? raw.w[j < 3 ? j + 1 : 3] : raw.next, lo, raw.sh) : lo, p.bias_limit);
+			w[j] = bias_limited(ANY ? __builtin_amdgcn_alignbit(j < 3 ? raw.w[j < 3 ? j + 1 : 3] : raw.next, lo, raw.sh) : lo, limit);
 		}
 		return __builtin_bit_cast(bf16x8, w);
 	};
@@ -484,6 +487,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 
 	// ---- the wavefronts' partial sums, added up by all threads: four head columns of a row per thread and trip; optional output
 	// gate (out *= sigmoid(gate)), any row and head strides.  Results leave before it is known whether they stand. ----
+	bool live;   // whether the batch row has a live key
 	auto merge = [&]() __attribute__((always_inline)) {   // whether they do not
 		asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (no load may still be writing LDS)
 		__syncthreads();   // (they lie over the tiles)
@@ -520,16 +524,28 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 		}
 		if(__ballot(bad) && lane == 0) s_bad[0] = 1;
 		__syncthreads();
-		const int some = __builtin_amdgcn_readfirstlane(s_bad[0]), looked = __builtin_amdgcn_readfirstlane(s_bad[1]);
-		return (some | looked) != 0 && (some != 0 || looked != (n_tiles < NW ? n_tiles : NW));
+		const u32x4 flags = *reinterpret_cast<const u32x4*>(s_bad);
+		const int   some = __builtin_amdgcn_readfirstlane(flags[0]), looked = __builtin_amdgcn_readfirstlane(flags[1]);
+		live = __builtin_amdgcn_readfirstlane(NW > 4 ? flags[2] | flags[3] : flags[2]) != 0;
+		return !live || ((some | looked) != 0 && (some != 0 || looked != (n_tiles < NW ? n_tiles : NW)));
 	};
 
 	if(ref) walk(std::true_type{});
 	else walk(std::false_type{});
 	if(!merge()) return;
 
-	// ---- rare: the rows' maxima, then the walk again, over all tiles (a row without a live key needs them) ----
+	// ---- rare: the rows' maxima, then the walk again, over all tiles (a row without a live key needs them).  A batch row without a live
+	// key yields the mean over all L keys whatever the dropped logits are: q and the bias (every one is limited to 0) are left out. ----
 	my_n = my_all > 0 ? my_all : 0;
+	if(!live) {
+		limit = 0;
+#pragma unroll
+		for(int c = 0; c < NB; c++) {
+#pragma unroll
+			for(int s = 0; s < KS; s++) qf[c][s] = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
+			if constexpr(LO) ql[c] = qf[c][0];
+		}
+	}
 	fill();
 	k_rsrc[2] = k_bytes, v_rsrc[2] = v_bytes, b_rsrc[2] = b_bytes;
 	float mx[NB];

@@ -668,6 +668,32 @@ def test_strips_rows_masked_through_the_bias(af3, B, H, L, D, kind):
     assert (out - want).abs().max() <= 2e-2   # (bf16's budget; a logit at -3e4 or -2^16 has steps of 2^-9 or 2^-8)
 
 
+@pytest.mark.parametrize("B,H,L,D", [(1, 1, 32, 24), (2, 3, 33, 8), (1, 16, 50, 48), (1, 16, 257, 32), (1, 16, 290, 24), (2, 16, 300, 48), (1, 5, 1155, 16)])
+@pytest.mark.parametrize("kind", ["-inf", "+inf", "nan", "huge", "far", "q"])
+def test_strips_without_a_live_key_give_the_mean(af3, B, H, L, D, kind):
+    """A batch row without a live key: the mean of V over all keys, whatever its logits would have been."""
+    g = torch.Generator().manual_seed(L + D)
+    q, k, v = (torch.randn(B, H, L, D, generator=g).to(torch.bfloat16) for _ in range(3))
+    bias = torch.randn(H, L, L, generator=g).to(torch.bfloat16)
+    if kind == "q":   # (with finite keys)
+        q[:, :, ::3, 1] = float("inf")
+        q[:, :, 1::3] = 1.0e38
+    elif kind == "far":   # (rows that look masked through their bias, down to some of -2^125)
+        bias[:] = -float("inf")
+        i = torch.arange(L)
+        bias[:, i, i] = -(2.0 ** 125)
+    else:
+        at = torch.rand(H, L, L, generator=g) < 0.1
+        bias[at] = {"-inf": -float("inf"), "+inf": float("inf"), "nan": float("nan"), "huge": 2.0 ** 100}[kind]
+    keep = torch.zeros(B, L, dtype=torch.bool)
+    keep[1:] = True
+    print("case", B, H, L, D, kind, flush=True)
+    out = af3.dot_product_attention_cpp(q.cuda(), k.cuda(), v.cuda(), keep.cuda(), bias.cuda()).cpu().double()
+    want = v[0].double().mean(1, keepdim=True).expand(H, L, D)
+    # weights of 1 are exact: fp32 sums and quotient (L 2^-24 of sums of |v| up to 5 on average), the result rounded to bf16
+    assert ((out[0] - want).abs() <= 2.0 ** -8 * want.abs() + L * 2.0 ** -24 * 5).all()
+
+
 @pytest.mark.parametrize("H,L,D,first", [
     (2, 7872, 48, 1), (2, 7873, 48, 0), (2, 8096, 48, 1), (2, 8097, 40, 0), (2, 8191, 48, 0), (2, 8192, 48, 1), (2, 8192, 32, 1),   # four blocks, rows at any address: the most LDS a workgroup takes
     (3, 8192, 48, 0), (2, 8192, 40, 0),                              # two workgroups per compute unit
