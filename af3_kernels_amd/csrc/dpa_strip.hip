@@ -28,6 +28,8 @@ namespace af3 {
 namespace {
 
 constexpr int      KT_S       = 32;   // keys per tile
+// what a dropped key's logit gets: no bias of eight bits brings it near 0, so that the sums of a row without a live key never stand
+constexpr float    DROPPED    = MASK_DROPPED - 0x1p88f;
 
 // What the kernel takes, as the launcher lays it out: a workgroup's start is a chain of scalar instructions that no other work covers
 // and whose code is fetched cold, so nothing is divided and little is multiplied there.
@@ -75,7 +77,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 	constexpr int SUM_COL = KIND == 0 ? 24 : 16 * ND;
 	extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
 	float* const s_max = reinterpret_cast<float*>(smem + Q_AT);   // (q is in registers by then)
-	int* const   s_bad = reinterpret_cast<int*>(smem + lds::FLAG_AT);   // [0]: rows whose sums do not stand; [1]: how many wavefronts took references from samples; [2..3]: a byte per wavefront, whether its tiles hold a live key
+	int* const   s_bad = reinterpret_cast<int*>(smem + lds::FLAG_AT);   // [0]: rows whose sums do not stand; [1]: how many wavefronts took references from samples, + 2^8 for each that took one below a dropped key's logit, + 2^16 if its tiles hold a live key; [2]: wavefronts whose tiles do (second walk)
 
 	asm volatile("" ::"s"(p.q), "s"(p.k), "s"(p.v), "s"(p.bias), "s"(p.mask), "s"(p.q_h), "s"(p.k_h), "s"(p.v_h), "s"(p.bias_h), "s"(p.q_row), "s"(p.k_row), "s"(p.v_row), "s"(p.bias_row), "s"(p.H),
 				 "s"(p.L), "s"(p.D), "s"(p.per_chunk), "s"(p.scale));
@@ -172,7 +174,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 		if(lane < 8) *reinterpret_cast<uint32_t*>(smem + const_base + 4 * lane) = lane == 4 ? 0x3F80u : 0u;
 	};
 	fill();
-	if(tid < 2) s_bad[tid] = 0;
+	if(tid < 3) s_bad[tid] = 0;
 
 	// ---- per-lane constants ----
 	u32x4 sel[2];   // half h of the tile's keys: row i picks key 8 (i / 4) + 4 h + i % 4
@@ -236,15 +238,13 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 
 	// ---- key-mask table of this wavefront's tiles: what is added to a key's logits.  Tiles behind the last one with a live key are not walked. ----
 	int  my_n = my_all > 0 ? 1 : 0;
-	bool my_live = false;
 	for(int j = 0; 2 * j < my_all; j++) {
 		const uint32_t m = (j == 0 ? m_first[0] : j == 1 ? m_first[1] : load_mask(j)) | (masked ? 0u : 1u);
 		const int      i = 2 * j + (lane >> 5), seen = ((wave + NW * i) * KT_S + KT_S) - L;   // seen: keys of the last tile that the one before has covered
-		if(i < my_all) *reinterpret_cast<float*>(smem + mask_base + i * 128 + (lane & 31) * 4) = (lane & 31) < seen ? MASK_OUT_OF_RANGE : m ? 0.f : MASK_DROPPED;
+		if(i < my_all) *reinterpret_cast<float*>(smem + mask_base + i * 128 + (lane & 31) * 4) = (lane & 31) < seen ? MASK_OUT_OF_RANGE : m ? 0.f : DROPPED;
 		const unsigned long long bal = __ballot(m != 0u);
-		if(bal) my_n = (bal >> 32) && 2 * j + 1 < my_all ? 2 * j + 2 : 2 * j + 1, my_live = true;
+		if(bal) my_n = (bal >> 32) && 2 * j + 1 < my_all ? 2 * j + 2 : 2 * j + 1;
 	}
-	if(lane == 0) reinterpret_cast<uint8_t*>(s_bad + 2)[wave] = my_live;
 	asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 	const unsigned long long low = __ballot(*reinterpret_cast<const uint16_t*>(smem + s_rd) > s_low);   // (bf16 bits; negative NaN as well)
 	__syncthreads();   // q
@@ -293,6 +293,11 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 		return r;
 	};
 	auto mfma = [](const bf16x8& a, const bf16x8& bb, const f32x4& c) __attribute__((always_inline)) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bb, c, 0, 0, 0); };
+	auto live_keys = [&]() __attribute__((always_inline)) {   // whether this wavefront's tiles hold any
+		bool any = false;
+		for(int i = lane; i < my_all * KT_S; i += 64) any = any || *reinterpret_cast<const float*>(smem + mask_base + i * 4) == 0.f;
+		return __ballot(any) != 0;
+	};
 	uint32_t limit = p.bias_limit;
 	auto clamped = [&](const bias_piece& raw) __attribute__((always_inline)) {
 		u32x4 w;
@@ -324,10 +329,14 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 		float          m = fmaxf(bf16_bits_to_f32(r0 < lim ? r0 : lim), bf16_bits_to_f32(r1 < lim ? r1 : lim));
 		m   = in && m < -32.f ? m : 0.f;
 		ref = __builtin_amdgcn_readfirstlane(__ballot(m < 0.f) != 0);
-		if(__ballot(m < MASK_DROPPED)) my_n = my_all;   // (there a dropped key's logit is no lower than the others': all keys count)
+		int count = 1;
+		if(__ballot(m < DROPPED)) {   // (there a dropped key's logit is no lower than the others': all keys count, and sums without a live key may look as if they stood)
+			my_n  = my_all;
+			count = live_keys() ? 0x10101 : 0x101;
+		}
 #pragma unroll
 		for(int c = 0; c < NB; c++) m_ref[c] = __shfl(m, 16 * c + i16);
-		if(ref && lane == 0) atomicAdd(s_bad + 1, 1);
+		if(ref && lane == 0) atomicAdd(s_bad + 1, count);
 	}
 	auto walk = [&](auto ref_c) __attribute__((always_inline)) {
 		constexpr bool REF = decltype(ref_c)::value;
@@ -487,7 +496,6 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 
 	// ---- the wavefronts' partial sums, added up by all threads: four head columns of a row per thread and trip; optional output
 	// gate (out *= sigmoid(gate)), any row and head strides.  Results leave before it is known whether they stand. ----
-	bool live;   // whether the batch row has a live key
 	auto merge = [&]() __attribute__((always_inline)) {   // whether they do not
 		asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (no load may still be writing LDS)
 		__syncthreads();   // (they lie over the tiles)
@@ -524,10 +532,8 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 		}
 		if(__ballot(bad) && lane == 0) s_bad[0] = 1;
 		__syncthreads();
-		const u32x4 flags = *reinterpret_cast<const u32x4*>(s_bad);
-		const int   some = __builtin_amdgcn_readfirstlane(flags[0]), looked = __builtin_amdgcn_readfirstlane(flags[1]);
-		live = __builtin_amdgcn_readfirstlane(NW > 4 ? flags[2] | flags[3] : flags[2]) != 0;
-		return !live || ((some | looked) != 0 && (some != 0 || looked != (n_tiles < NW ? n_tiles : NW)));
+		const int some = __builtin_amdgcn_readfirstlane(s_bad[0]), looked = __builtin_amdgcn_readfirstlane(s_bad[1]);
+		return (some | looked) != 0 && (some != 0 || (looked & 0xff) != (n_tiles < NW ? n_tiles : NW) || (looked > 0xff && looked < 0x10000));
 	};
 
 	if(ref) walk(std::true_type{});
@@ -537,7 +543,9 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 	// ---- rare: the rows' maxima, then the walk again, over all tiles (a row without a live key needs them).  A batch row without a live
 	// key yields the mean over all L keys whatever the dropped logits are: q and the bias (every one is limited to 0) are left out. ----
 	my_n = my_all > 0 ? my_all : 0;
-	if(!live) {
+	if(live_keys() && lane == 0) atomicAdd(s_bad + 2, 1);
+	__syncthreads();
+	if(__builtin_amdgcn_readfirstlane(s_bad[2]) == 0) {
 		limit = 0;
 #pragma unroll
 		for(int c = 0; c < NB; c++) {

@@ -635,7 +635,7 @@ def test_strips_infinities_act_as_in_the_formula(af3, B, H, L, D, kind):
 
 
 @pytest.mark.parametrize("B,H,L,D", [(1, 1, 32, 24), (2, 3, 33, 8), (1, 16, 50, 48), (37, 4, 37, 32), (1, 16, 257, 32), (1, 16, 290, 24), (1, 16, 513, 48), (1, 5, 1155, 16), (1, 16, 769, 24), (1, 16, 1040, 48)])
-@pytest.mark.parametrize("kind", ["far", "-1e9", "-inf", "window", "misleading", "scattered"])
+@pytest.mark.parametrize("kind", ["far", "-1e9", "-inf", "-inf, tail", "window", "misleading", "scattered"])
 def test_strips_rows_masked_through_the_bias(af3, B, H, L, D, kind):
     """Query rows whose biases all lie far below zero, rows of which only the neighbourhood of the diagonal does not, and rows
     whose two samples are no sign of the rest."""
@@ -645,8 +645,10 @@ def test_strips_rows_masked_through_the_bias(af3, B, H, L, D, kind):
     keep = torch.rand(B, L, generator=g) < 0.8
     keep[:, L // 3] = True
     i = torch.arange(L)
-    if kind in ("far", "-1e9", "-inf"):
-        bias[:, L - L // 5:] = {"far": -3.0e4, "-1e9": -1.0e9, "-inf": float("-inf")}[kind]
+    if kind in ("far", "-1e9") or "-inf" in kind:
+        bias[:, L - L // 5:] = {"far": -3.0e4, "-1e9": -1.0e9}.get(kind, float("-inf"))
+        if "tail" in kind:   # (wavefronts without a live key beside others that have some)
+            keep[:, L // 3 + 1:] = False
     elif kind == "window":
         keep[:] = True
         bias[:, (i[:, None] - i[None]).abs() > 20] = -3.0e4
@@ -662,7 +664,7 @@ def test_strips_rows_masked_through_the_bias(af3, B, H, L, D, kind):
     # one batch row takes biases down to -2^126, several down to -2^16 (q.k still counts there)
     lowest = -2.0 ** 126 if B == 1 else -2.0 ** 16
     s = (q.float() @ k.float().transpose(-1, -2)) * D ** -0.5 + bias.float().clamp(min=lowest)
-    rows = L - L // 5 if kind == "-inf" and B == 1 else L   # (beyond these a dropped key's logit is no lower)
+    rows = L - L // 5 if "-inf" in kind and B == 1 else L   # (beyond these a dropped key's logit is no lower)
     s[:, :, :rows].masked_fill_(~keep[:, None, None, :], float("-inf"))
     want = s.softmax(-1) @ v.float()
     assert (out - want).abs().max() <= 2e-2   # (bf16's budget; a logit at -3e4 or -2^16 has steps of 2^-9 or 2^-8)
