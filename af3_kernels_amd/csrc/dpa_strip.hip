@@ -541,7 +541,8 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 	if(!merge()) return;
 
 	// ---- rare: the rows' maxima, then the walk again, over all tiles (a row without a live key needs them).  A batch row without a live
-	// key yields the mean over all L keys whatever the dropped logits are: q and the bias (every one is limited to 0) are left out. ----
+	// key yields the mean over all L keys whatever the dropped logits are: q and the bias (every one is limited to 0) are left out (16 heads of
+	// 24 x 768 12.1 us instead of 7.1, x 1536 31.8 instead of 17.1). ----
 	my_n = my_all > 0 ? my_all : 0;
 	if(live_keys() && lane == 0) atomicAdd(s_bad + 2, 1);
 	__syncthreads();
