@@ -16,7 +16,8 @@
 //
 // Work split.  Workgroup = NW wavefronts = NW blocks of 32 query rows of one (group of 4 batch rows, head).  K and V
 // tiles (32 keys x 4 batch rows) are staged in LDS by loads that write LDS directly, four buffers deep, and shared
-// by the NW wavefronts; one workgroup barrier per tile, i.e. per four blocks of logits of every wavefront.
+// by the NW wavefronts; one workgroup barrier per tile, i.e. per four blocks of logits of every wavefront.  A workgroup may
+// walk several query tiles of its group and head one behind the other without coming to rest (plan_chunks).
 #include "mfma_helpers.hpp"
 
 namespace af3 {
@@ -94,11 +95,17 @@ __global__ void __launch_bounds__(256) bias_rows_prepass_kernel(const void* __re
 // 2's cache-line requests, whose lanes each fetch from a row of their own).
 // The launch covers batch rows [b_first, b_first + b_count) in groups of ROWS.
 // GATE: out *= sigmoid(gate) in the epilogue.
+// Per XCD the first n_chunked (group, head) pairs are cut into n_chunks workgroups of q_chunk query tiles, the others into workgroups of one.
+// Whether workgroups may walk several query tiles.  Four batch rows and their gates do not fit the registers between two query tiles (14 spilled ones: the
+// grid block of 768 tokens 637 -> 655 us; with one query tile to a workgroup 633), the in-place form has not been given it.
+constexpr bool several_query_tiles(int rows, int bmode, bool gate) { return bmode != 2 && !(gate && rows == 4); }
 template <int ROWS, int BMODE, bool GATE>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) dpa_rows_bf16_kernel(af3_dpa_params p, int n_qtiles, int64_t n_groups, int64_t b_first, int64_t b_count) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) dpa_rows_bf16_kernel(af3_dpa_params p, int n_qtiles, int64_t n_groups, int64_t b_first, int64_t b_count, int q_chunk,
+																										   int n_chunks, int n_chunked) {
 	static_assert(ROWS >= 2 && ROWS <= 4, "two to four row chains per wavefront");
 	constexpr int  NW       = 4;
 	constexpr bool HAS_BIAS = BMODE != 0, SLOT = BMODE == 1, DIRECT = BMODE == 2, STAGED = BMODE == 3;
+	constexpr bool MULTI    = several_query_tiles(ROWS, BMODE, GATE);
 	constexpr int  BUF_R    = ROWS * 2 * TILE_R;                    // one buffer: [row][K tile | V tile]
 	constexpr int  SLOT_BASE = NBUF_R * BUF_R;                      // per-wavefront bias slots (4 KB each)
 	constexpr int  MASK_BASE = SLOT_BASE + (SLOT || STAGED ? NW * 4096 : 0);
@@ -109,7 +116,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 	const int     n_t_all  = (int)((L + KT_R - 1) / KT_R);
 	uint16_t* const mask_tab = reinterpret_cast<uint16_t*>(smem + MASK_BASE);
 	__shared__ int  s_last[4];  // index of the last live key + 1 of each batch row (0: every key dropped)
-	__shared__ int  s_again;    // some wavefront's walk has to be repeated carefully
+	__shared__ uint32_t s_again;  // query tiles of which some wavefront's walk has to be repeated carefully
 	__shared__ int  s_first[4]; // index of the first key tile of each batch row that holds a live key
 
 	// ---- workgroup -> (group of batch rows, head, query tile): all query tiles of one (group, head) get ids congruent
@@ -118,14 +125,18 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 	// The kernel arguments that the start of a workgroup needs, requested in one batch (the compiler would fetch the launch
 	// counts, wait, test the early exit, and only then request the fields of p, in two more batches: three memory latencies
 	// in a row that the wavefronts of a small launch stand through).
-	asm volatile("" ::"s"(n_qtiles), "s"(n_groups), "s"(b_first), "s"(b_count), "s"(p.q), "s"(p.k), "s"(p.v), "s"(p.bias), "s"(p.key_mask), "s"(p.workspace), "s"(p.H), "s"(p.L),
+	asm volatile("" ::"s"(n_qtiles), "s"(n_groups), "s"(b_first), "s"(b_count), "s"(q_chunk), "s"(n_chunks), "s"(n_chunked), "s"(p.q), "s"(p.k), "s"(p.v), "s"(p.bias), "s"(p.key_mask), "s"(p.workspace), "s"(p.H), "s"(p.L),
 				 "s"(p.D), "s"(p.key_mask_stride_b), "s"(p.bias_stride[0]), "s"(p.bias_stride[1]));
 	asm volatile("" ::"s"(p.q_stride[0]), "s"(p.q_stride[1]), "s"(p.q_stride[2]), "s"(p.k_stride[0]), "s"(p.k_stride[1]), "s"(p.k_stride[2]), "s"(p.v_stride[0]), "s"(p.v_stride[1]),
 				 "s"(p.v_stride[2]));
 	// (32-bit divisions: a 64-bit one is 150 instructions, i.e. 700 clocks of a start that waits for them)
-	const uint32_t slot = blockIdx.x >> 3, q_div = slot / (uint32_t)n_qtiles, group = q_div * 8 + (blockIdx.x & 7);
-	const int      qtile = (int)(slot - q_div * (uint32_t)n_qtiles);
+	const uint32_t slot = blockIdx.x >> 3, chunked = (uint32_t)n_chunked * (uint32_t)n_chunks;
+	const bool     single = slot >= chunked;
+	const uint32_t s_rel = single ? slot - chunked : slot, parts = single ? (uint32_t)n_qtiles : (uint32_t)n_chunks, q_div = s_rel / parts;
+	const uint32_t group = (q_div + (single ? (uint32_t)n_chunked : 0u)) * 8 + (blockIdx.x & 7);
 	if(group >= (uint32_t)n_groups) return;
+	const int chunk = single ? 1 : q_chunk, qtile0 = (int)(s_rel - q_div * parts) * chunk;
+	const int n_q   = qtile0 + chunk <= n_qtiles ? chunk : n_qtiles - qtile0;   // query tiles of this workgroup
 	const int64_t g = group / (uint32_t)p.H, h = group - (uint32_t)g * (uint32_t)p.H;
 	const int64_t b0 = b_first + g * ROWS, b_end = b_first + b_count;   // (rows past b_end repeat the last one and are not stored)
 
@@ -172,8 +183,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 	}
 
 	// ---- per-lane constants ----
-	const int64_t qrow   = (int64_t)qtile * (NW * 32) + wave * 32 + n;
-	const bool    row_ok = qrow < L;
+	const int64_t row00 = (int64_t)qtile0 * (NW * 32) + wave * 32;   // this wavefront's first query row
+	const int     my_q  = row00 + (int64_t)(n_q - 1) * (NW * 32) < L ? n_q : n_q - 1;   // query tiles in which it has rows: all, or all but the last
 	int n_t = 1;   // key tiles to walk: known once the key masks are read; the first tile is always walked
 
 	// ---- tile and bias loaders: loads that write LDS directly (no registers, invisible to the compiler's wait counting;
@@ -192,81 +203,123 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 	const int     k_tile_stride = (int)(KT_R * p.k_stride[2] * 2), v_tile_stride = (int)(KT_R * p.v_stride[2] * 2);
 	const int     k_pc_stride = (int)(16 * p.k_stride[2] * 2), v_pc_stride = (int)(16 * p.v_stride[2] * 2);
 	const uint32_t lds_tiles = lds_addr_of(smem) + wave * (2 * TILE_R);
-	auto load_tile_piece = [&](int t, int buf_off, auto pc_c) {
-		constexpr int PC = decltype(pc_c)::value;
-		if(!loader || t >= n_t) return;   // (no request for a tile the walk stops short of: nothing is in flight when the kernel ends)
-		if constexpr(PC == 0) lds_dma_b128(k_rsrc, lds_tiles + buf_off, k_voff + t * k_tile_stride);
-		if constexpr(PC == 1) lds_dma_b128(k_rsrc, lds_tiles + buf_off + 1024, k_voff + (t * k_tile_stride + k_pc_stride));
-		if constexpr(PC == 2) lds_dma_b128(v_rsrc, lds_tiles + buf_off + TILE_R, v_voff + t * v_tile_stride);
-		if constexpr(PC == 3) lds_dma_b128(v_rsrc, lds_tiles + buf_off + TILE_R + 1024, v_voff + (t * v_tile_stride + v_pc_stride));
+	auto load_tile = [&](int t, int buf_off) {   // (for tiles that will be walked only: nothing is in flight when the kernel ends)
+		if(!loader) return;
+		lds_dma_b128(k_rsrc, lds_tiles + buf_off, k_voff + t * k_tile_stride);
+		lds_dma_b128(k_rsrc, lds_tiles + buf_off + 1024, k_voff + (t * k_tile_stride + k_pc_stride));
+		lds_dma_b128(v_rsrc, lds_tiles + buf_off + TILE_R, v_voff + t * v_tile_stride);
+		lds_dma_b128(v_rsrc, lds_tiles + buf_off + TILE_R + 1024, v_voff + (t * v_tile_stride + v_pc_stride));
 	};
-	auto load_tile = [&](int t, int buf_off) {
-		load_tile_piece(t, buf_off, ic<0>{}), load_tile_piece(t, buf_off, ic<1>{}), load_tile_piece(t, buf_off, ic<2>{}), load_tile_piece(t, buf_off, ic<3>{});
+	// (The arguments of what happens once or twice per query tile are loaded again where they are used: kept through the walk, they are spilled.)
+	using args_t = const __attribute__((address_space(4))) af3_dpa_params*;
+	auto args = []() __attribute__((always_inline)) -> args_t {
+		args_t a = (args_t)__builtin_amdgcn_kernarg_segment_ptr();
+		asm volatile("" : "+s"(a));
+		return a;
 	};
 	// Output gate: the 2 ROWS pieces of this wavefront's gate rows (16 query rows of a batch row, 1 KB each) go into the tile buffers
 	// that the last two tiles leave free -- the places of tiles n_t and n_t + 1, requested where those tiles would be -- and are
 	// read in the epilogue.  (Loaded there, they exposed a memory latency per workgroup: 36 of 448 us at 768 x 4 x 768 x 32, 9 of 81 at 384.)
-	auto load_gate = [&](int part, int buf_off) {
+	auto load_gate = [&](int part, int buf_off, int i) {
 		if constexpr(!GATE) return;
+		const args_t a = args();
 #pragma unroll
-		for(int i = 0; i < ROWS; i++) {
-			const int     k = part * ROWS + i, r = k >> 1;
-			const int64_t br = b0 + r < b_end ? b0 + r : b_end - 1, row = (int64_t)qtile * (NW * 32) + wave * 32 + 16 * (k & 1) + (lane >> 2);
-			const u32x4   g_rsrc = raw_rsrc(static_cast<const uint16_t*>(p.gate) + br * p.gate_stride[0] + h * p.gate_stride[1], (uint32_t)(((L - 1) * p.gate_stride[2] + D) * 2));
-			lds_dma_b128(g_rsrc, lds_addr_of(smem) + buf_off + (wave * ROWS + i) * 1024, (lane & 3) * 8 < D && row < L ? (int)(row * p.gate_stride[2] * 2) + (lane & 3) * 16 : 0x7FFF0000);
+		for(int j = 0; j < ROWS; j++) {
+			const int     k = part * ROWS + j, r = k >> 1;
+			const int64_t br = b0 + r < b_end ? b0 + r : b_end - 1, row = row00 + i * (NW * 32) + 16 * (k & 1) + (lane >> 2);
+			const u32x4   g_rsrc = raw_rsrc(static_cast<const uint16_t*>(a->gate) + br * a->gate_stride[0] + h * a->gate_stride[1], (uint32_t)(((L - 1) * a->gate_stride[2] + D) * 2));
+			lds_dma_b128(g_rsrc, lds_addr_of(smem) + buf_off + (wave * ROWS + j) * 1024, (lane & 3) * 8 < D && row < L ? (int)(row * a->gate_stride[2] * 2) + (lane & 3) * 16 : 0x7FFF0000);
 		}
 	};
-	auto load_tile_or_gate = [&](int t, int buf_off) {
+	auto load_tile_or_gate = [&](int t, int buf_off, int i) {
 		if(t < n_t) load_tile(t, buf_off);
-		else load_gate(t - n_t, buf_off);
+		else load_gate(t - n_t, buf_off, i);
 	};
 	// bias fragment of key tile t: 4 KB of this (head, query block)'s slab of the workspace -> this wavefront's slot
+	// (i: query tile of the workgroup, here and below; its blocks are NW slabs further on)
 	const int     n_qblocks = (int)((L + 31) / 32);
-	const int64_t qb        = (int64_t)qtile * NW + wave;
+	const int64_t qb        = (int64_t)qtile0 * NW + wave;
 	const int64_t qbc       = qb < n_qblocks ? qb : n_qblocks - 1;  // (blocks past the end only hold rows >= L)
-	const u32x4   ws_rsrc   = raw_rsrc(SLOT ? static_cast<const unsigned char*>(p.workspace) + ((h * n_qblocks + qbc) * n_t_all) * 4096 : nullptr, SLOT ? (uint32_t)(n_t_all * 4096) : 0u);
-	const int      ws_voff  = lane * 16;
+	const u32x4   ws_rsrc   = raw_rsrc(SLOT ? static_cast<const unsigned char*>(p.workspace) + ((h * n_qblocks + qbc) * n_t_all) * 4096 : nullptr,
+									   SLOT ? (uint32_t)((n_qblocks - qbc) * n_t_all) * 4096u : 0u);
+	const int      ws_voff  = lane * 16, ws_step = NW * n_t_all * 4096;
 	const uint32_t lds_slot = lds_addr_of(smem) + SLOT_BASE + wave * 4096;
-	auto load_bias_piece = [&](int t, auto pc_c) {
-		constexpr int PC = decltype(pc_c)::value;
-		if(!SLOT || t >= n_t) return;
-		lds_dma_b128(ws_rsrc, lds_slot + PC * 1024, ws_voff + (t * 4096 + PC * 1024));
+	auto load_bias = [&](int t, int i) {
+		if(!SLOT) return;
+		const int off = i * ws_step + t * 4096;
+#pragma unroll
+		for(int pc = 0; pc < 4; pc++) lds_dma_b128(ws_rsrc, lds_slot + pc * 1024, ws_voff + (off + pc * 1024));
 	};
-	auto load_bias = [&](int t) { load_bias_piece(t, ic<0>{}), load_bias_piece(t, ic<1>{}), load_bias_piece(t, ic<2>{}), load_bias_piece(t, ic<3>{}); };
 	// direct mode: this lane's four 8-byte pieces of a tile's bias, bias[h][q][32 t + 8 ld + 4 half .. + 3] (bf16), through a
 	// range-checked buffer over the head's slab; pieces whose keys lie at or beyond L are sent out of range and read as zero
+	// (workgroups of this mode take one query tile)
 	[[maybe_unused]] u32x2 braw[4] = {u32x2{0u, 0u}, u32x2{0u, 0u}, u32x2{0u, 0u}, u32x2{0u, 0u}};
-	const int64_t qrow_b = qrow < L ? qrow : L - 1;
+	const int64_t qrow_b = row00 + n < L ? row00 + n : L - 1;
 	const __amdgpu_buffer_rsrc_t bd_rsrc = __builtin_amdgcn_make_buffer_rsrc(
 		DIRECT ? const_cast<uint16_t*>(static_cast<const uint16_t*>(p.bias)) + h * p.bias_stride[0] : nullptr, 0, DIRECT ? (int)(((L - 1) * p.bias_stride[1] + L) * 2) : 0, 0x00020000);
 	const int bd_voff = (int)((qrow_b * p.bias_stride[1] + 4 * half) * 2);
 	// staged mode: lane i of load j fetches 16 bytes of row 16 j + i / 4 of the tile; the chunk it fetches is the one that
 	// belongs at its place under the swizzle (chunk c of row r sits at position c ^ ((r >> 2) & 3): the fragment reads of 32
-	// rows then spread over the banks).  Rows past L fetch row L - 1; chunks whose keys lie at or beyond L are sent out of
-	// range (nothing is fetched: the slot keeps finite data, and those keys carry the out-of-range mask value).
+	// rows then spread over the banks).  Rows past L and chunks whose keys lie at or beyond L are out of the buffer's range or
+	// hold other biases (their results are not stored, those keys carry the out-of-range mask value).
 	const u32x4 st_rsrc = raw_rsrc(STAGED ? static_cast<const uint16_t*>(p.bias) + h * p.bias_stride[0] : nullptr, STAGED ? (uint32_t)(((L - 1) * p.bias_stride[1] + L) * 2) : 0u);
 	int st_voff[2] = {0, 0};
 	int st_key[2]  = {0, 0};  // first key (within a tile) of the chunk this lane fetches
+	const int st_step = STAGED ? (int)(NW * 32 * p.bias_stride[1] * 2) : 0;
 	if constexpr(STAGED) {
 #pragma unroll
 		for(int j = 0; j < 2; j++) {
 			const int     r   = 16 * j + (lane >> 2), c = (lane & 3) ^ ((r >> 2) & 3);
-			const int64_t row = (int64_t)qtile * (NW * 32) + wave * 32 + r;
-			st_voff[j] = (int)((row < L ? row : L - 1) * p.bias_stride[1] * 2) + c * 16;
+			const int64_t row = row00 + r;
+			st_voff[j] = n_q > 1 || row < L ? (int)(row * p.bias_stride[1] * 2) + c * 16 : (int)((L - 1) * p.bias_stride[1] * 2) + c * 16;
 			st_key[j]  = c * 8;
 		}
 	}
-	auto load_bias_staged = [&](int t) {
-		if(!STAGED || t >= n_t) return;
+	auto load_bias_staged = [&](int t, int i, int parity) {
+		if(!STAGED) return;
 #pragma unroll
-		for(int j = 0; j < 2; j++) lds_dma_b128(st_rsrc, lds_slot + (t & 1) * 2048 + j * 1024, t * KT_R + st_key[j] < L ? st_voff[j] + t * (KT_R * 2) : 0x40000000);
+		for(int j = 0; j < 2; j++) lds_dma_b128(st_rsrc, lds_slot + (parity & 1) * 2048 + j * 1024, t * KT_R + st_key[j] < L ? st_voff[j] + (i * st_step + t * (KT_R * 2)) : 0x40000000);
 	};
 	auto load_bias_direct = [&](int t) {
-		if(!DIRECT || t >= n_t) return;
+		if(!DIRECT) return;
 #pragma unroll
 		for(int ld = 0; ld < 4; ld++) {
 			const bool in = t * KT_R + 8 * ld + 4 * half < L;
 			braw[ld] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(bd_rsrc, in ? bd_voff + ld * 16 : 0x40000000, t * (KT_R * 2), 0));
+		}
+	};
+	// q rows, gate rows and output rows of this wavefront's 32 rows of query tile i: per batch row a buffer that starts at the first of them and
+	// ends with row L - 1 (rows past it read zero and are not stored).  The addresses move along in scalar registers; lane offsets are
+	// made anew where they are used, from a lane number that the compiler cannot keep (it would hold a dozen registers through the walk).
+	auto lane_now = []() -> int {
+		int l;
+		asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+		return l;
+	};
+	const int      n_rows = (int)(b_end - b0 < ROWS ? b_end - b0 : ROWS);   // batch rows of this group
+	auto rows_left = [&](int i) -> int {   // (at most 32)
+		const int64_t left = L - row00 - i * (NW * 32);
+		return left < 0 ? 0 : left < 32 ? (int)left : 32;
+	};
+	auto buffer_of = [&](const void* base, int64_t row_stride, int rows, int el) -> __amdgpu_buffer_rsrc_t {   // (31 row strides fit 31 bits: mfma_rows_eligible)
+		return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, rows > 0 ? ((rows - 1) * (int)row_stride + D) * el : 0, 0x00020000);
+	};
+	u32x4 qraw[ROWS][2];
+	const uint16_t* q_row = nullptr;
+	int64_t         q_sb = 0;
+	int             q_sr = 0;   // (strides of batch rows and of query rows)
+	auto request_q = [&](auto r_c, int i) {   // (batch rows in their order)
+		constexpr int r  = decltype(r_c)::value;
+		if constexpr(r < ROWS) {
+			if constexpr(r == 0) {
+				const args_t a = args();
+				q_sb = a->q_stride[0], q_sr = (int)a->q_stride[2];
+				q_row = static_cast<const uint16_t*>(a->q) + b0 * q_sb + h * a->q_stride[1] + (row00 + i * (NW * 32)) * q_sr;
+			} else q_row += r < n_rows ? q_sb : 0;   // (rows past the last repeat it)
+			const __amdgpu_buffer_rsrc_t rsrc = buffer_of(q_row, q_sr, rows_left(i), 2);
+			const int l = lane_now(), d0 = 8 * (l >> 5), voff = ((l & 31) * q_sr + d0) * 2;
+#pragma unroll
+			for(int c = 0; c < 2; c++) qraw[r][c] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, 16 * c + d0 < D ? voff + 32 * c : 0x7FFF0000, 0, 0));
 		}
 	};
 
@@ -274,21 +327,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 	// memory latency, not a chain of them: the first K and V tiles, the first bias fragment (straight into LDS)
 	// and the raw q rows ----
 	load_tile(0, 0);
-	load_bias(0);
+	load_bias(0, 0);
 	load_bias_direct(0);
-	load_bias_staged(0);
-	u32x4 qraw[ROWS][2];
-#pragma unroll
-	for(int r = 0; r < ROWS; r++) {
-		const int64_t   br = b0 + r < b_end ? b0 + r : b_end - 1;
-		const uint16_t* qp = static_cast<const uint16_t*>(p.q) + br * p.q_stride[0] + h * p.q_stride[1] + qrow * p.q_stride[2];
-#pragma unroll
-		for(int c = 0; c < 2; c++) {
-			const int d0 = 16 * c + 8 * half;
-			qraw[r][c]   = u32x4{0u, 0u, 0u, 0u};
-			if(row_ok && d0 < D) qraw[r][c] = *reinterpret_cast<const u32x4*>(qp + d0);
-		}
-	}
+	load_bias_staged(0, 0, 0);
+	request_q(ic<0>{}, 0), request_q(ic<1>{}, 0), request_q(ic<2>{}, 0), request_q(ic<3>{}, 0);
 
 	// ---- key-mask table: entry = additive mask value of (tile, batch row, key) as bf16 bits; wavefront w fills row w ----
 	const int n_keys_tab = (n_t_all + 1) * KT_R;
@@ -375,20 +417,24 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 	// softmax_scale * log2 e in fp32 and rounded once to bf16 (the reference rounds the scaled q too,
 	// src/csrc/dot_product_attention.cpp:95-98).
 	bf16x8 qf[ROWS][2];
+	auto convert_q = [&](auto r_c) {
+		constexpr int r = decltype(r_c)::value;
+		if constexpr(r < ROWS) {
+			const float qmul = args()->softmax_scale * LOG2E;
 #pragma unroll
-	for(int r = 0; r < ROWS; r++) {
-		const float qmul = p.softmax_scale * LOG2E;
+			for(int c = 0; c < 2; c++) {
+				u32x4 sc4;
 #pragma unroll
-		for(int c = 0; c < 2; c++) {
-			u32x4 sc4;
-#pragma unroll
-			for(int j = 0; j < 4; j++) {
-				const uint32_t w = qraw[r][c][j];
-				sc4[j] = pack_bf16x2(bf16_bits_to_f32(w & 0xffffu) * qmul, bf16_bits_to_f32(w >> 16) * qmul);
+				for(int j = 0; j < 4; j++) {
+					const uint32_t w = qraw[r][c][j];
+					sc4[j] = pack_bf16x2(bf16_bits_to_f32(w & 0xffffu) * qmul, bf16_bits_to_f32(w >> 16) * qmul);
+				}
+				asm volatile("" : "+v"(sc4));   // (here, not where it is used: the wait for the loads would then take in younger tile loads)
+				qf[r][c] = __builtin_bit_cast(bf16x8, sc4);
 			}
-			qf[r][c] = __builtin_bit_cast(bf16x8, sc4);
 		}
-	}
+	};
+	convert_q(ic<0>{}), convert_q(ic<1>{}), convert_q(ic<2>{}), convert_q(ic<3>{});
 	asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wavefront's pieces of the first tile and its bias fragment have landed
 	__syncthreads();                                    // the mask table and the first tile are complete
 	// keys behind the last live key of every row carry weight 0 and are not walked; a row without live keys needs them all
@@ -409,11 +455,15 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 		t_force_max    = ft > t_force_max ? ft : t_force_max;
 	}
 	n_t = (l_eff + KT_R - 1) / KT_R;
+	if(n_q > 1 && n_t < 2) n_t = 2;   // (several query tiles: the walk of one requests two tiles of the next; keys behind the last live one weigh 0)
 
 	// a batch row without live keys gets q = 0
+	auto drop_q = [&]() {
 #pragma unroll
-	for(int r = 0; r < ROWS; r++)
-		if(dropped[r]) qf[r][0] = qf[r][1] = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
+		for(int r = 0; r < ROWS; r++)
+			if(dropped[r]) qf[r][0] = qf[r][1] = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
+	};
+	drop_q();
 	// ---- online-softmax state: one query row per lane and batch row (the two half-waves hold disjoint keys) ----
 	float  m_ref[ROWS];   // reference maximum, log2 units, exactly m_hi + m_lo of two bf16 values
 	float  lsum[ROWS];    // the row sum (complete: the same value in both half-waves)
@@ -484,11 +534,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 	// the next tile's bias fragment -> registers: from the slot, or (direct mode) from the raw bf16 pieces loaded a tile ago:
 	// clamped from below like the workspace's values (packed unsigned minimum: -2^16 and everything beyond it, -inf and
 	// -NaN patterns included), widened to fp32 and scaled by log2 e
-	auto next_bias_fragment = [&](int t_next) {  // t_next: the tile the fragment belongs to (staged mode: which half of the slot holds it)
+	auto next_bias_fragment = [&](int parity) {  // (staged mode: which half of the slot holds it)
 		// (The old fragment is named once more behind its last reader: the registers it occupied then are the only free block of
 		// 16 when the new one is defined, so the fragment keeps its place from tile to tile.  Without this the compiler lets
 		// that reader's result overwrite the old fragment, puts the new one elsewhere and copies 16 registers per tile.)
-		asm volatile("" ::"v"(bias_frag));
+		if constexpr(HAS_BIAS) asm volatile("" ::"v"(bias_frag));
 		if constexpr(SLOT) {
 #pragma unroll
 			for(int ld = 0; ld < 4; ld++) {
@@ -500,7 +550,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 			if constexpr(STAGED) {  // this lane's four 8-byte pieces, keys 8 ld + 4 half .. + 3 of row n: chunk ld at its swizzled place
 #pragma unroll
 				for(int ld = 0; ld < 4; ld++)
-					braw[ld] = *reinterpret_cast<const u32x2*>(smem + SLOT_BASE + wave * 4096 + (t_next & 1) * 2048 + n * 64 + ((ld ^ ((n >> 2) & 3)) << 4) + half * 8);
+					braw[ld] = *reinterpret_cast<const u32x2*>(smem + SLOT_BASE + wave * 4096 + (parity & 1) * 2048 + n * 64 + ((ld ^ ((n >> 2) & 3)) << 4) + half * 8);
 			}
 #pragma unroll
 			for(int ld = 0; ld < 4; ld++)
@@ -528,11 +578,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 	// first K.Q^T instruction of the next step).
 	// FIRST: a leading tile, in which a row that meets its first live key (`force`, wave-uniform) fixes its softmax reference.  CAREFUL: the walk that tests every step's row
 	// sums, and whose batch rows may lack live keys (they then take no bias: a wave-uniform branch that the quick walk does not carry).
-	auto step = [&](auto r_c, auto first_c, auto careful_c, bool force, int k_addr2, int m_addr, int v_addr, auto&& hook) {
+	auto step = [&](auto r_c, auto first_c, auto careful_c, bool force, int k_addr2, int m_addr, int v_addr, auto&& behind_reference, auto&& hook) {
 		constexpr int  R = decltype(r_c)::value, RN = (R + 1) % ROWS, RP = (R + ROWS - 1) % ROWS;
 		constexpr bool FIRST = decltype(first_c)::value != 0, CAREFUL = decltype(careful_c)::value != 0;
 		if constexpr(FIRST && CAREFUL) rereference(r_c, sc, force);
 		else if constexpr(FIRST) first_reference(r_c, sc);
+		behind_reference();
 		maskA[0] = *reinterpret_cast<const uint16_t*>(smem + m_addr);
 		u32x4  pcur[2];
 		f32x16 sn;
@@ -630,79 +681,221 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 		pprev[1] = pcur[1];
 	};
 
-	// One tile: ROWS steps.  Tile t sits in buffer t % 3.  In front of the last-but-one step the loads issued one tile
+	// What remains of query tile i's batch row R when its last product is in: divide by the row sum, gate, store.  GATE_LDS: the gate rows wait
+	// in LDS.  BF16: the output is known to be bf16.  The stores go through a range-checked buffer and are always four to a lane (columns
+	// from D on lie out of its range): the wait in the tile that follows counts them.
+	uint32_t redo[ROWS];   // query tiles of batch row r whose sums do not stand: walked again carefully
+#pragma unroll
+	for(int r = 0; r < ROWS; r++) redo[r] = 0u;
+	u32x2           graw[4];   // gate values of a batch row, as request_gate leaves them
+	const uint16_t* gate_ptr = nullptr;
+	auto request_gate = [&](auto r_c, int i) {   // (batch rows in their order)
+		constexpr int R = decltype(r_c)::value;
+		if constexpr(GATE && R < ROWS) {
+			const args_t a = args();
+			if constexpr(R == 0) gate_ptr = static_cast<const uint16_t*>(a->gate) + b0 * a->gate_stride[0] + h * a->gate_stride[1] + (row00 + i * (NW * 32)) * a->gate_stride[2];
+			else gate_ptr += R < n_rows ? a->gate_stride[0] : 0;
+			const __amdgpu_buffer_rsrc_t rsrc = buffer_of(gate_ptr, a->gate_stride[2], rows_left(i), 2);
+			const int l = lane_now(), voff = ((l & 31) * (int)a->gate_stride[2] + 4 * (l >> 5)) * 2;
+#pragma unroll
+			for(int g4 = 0; g4 < 4; g4++) graw[g4] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rsrc, 8 * g4 < D ? voff + 16 * g4 : 0x7FFF0000, 0, 0));
+		}
+	};
+	unsigned char* out_row = nullptr;
+	int64_t        out_sb = 0;
+	int            out_sr = 0, out_el = 2;   // (bytes from batch row to batch row, elements from query row to query row, bytes per element)
+	auto finish_row = [&](auto r_c, auto careful_c, auto gate_lds_c, auto bf16_c, int i, [[maybe_unused]] int gate_buf0, [[maybe_unused]] int gate_buf1) {   // (batch rows in their order)
+		constexpr int  R = decltype(r_c)::value;
+		constexpr bool CAREFUL = decltype(careful_c)::value != 0, GATE_LDS = decltype(gate_lds_c)::value != 0, BF16 = decltype(bf16_c)::value != 0;
+		if constexpr(R < ROWS) {
+			const int rows = rows_left(i);
+			bool      keep_row = R < n_rows;   // (wave-uniform)
+			if constexpr(!CAREFUL) {
+				// Sums that end below the careful walk's limit have stayed below it throughout: the results are the careful walk's.  Beyond it
+				// they stand all the same if they stay below 2^100 and the results are finite.
+				if(__ballot(!(lsum[R] < PSUM_LIMIT))) {   // rare
+					const int n_ = lane_now() & 31;
+					float     t = lsum[R] * 0x1p28f;   // (infinite from 2^100 on)
+#pragma unroll
+					for(int k = 0; k < 16; k++) t = fmaf(oacc[R][k], 0.f, t);
+					if(__ballot(n_ < rows && !(t < __builtin_inff()))) {
+						redo[R] |= 1u << i;
+						keep_row = false;
+						if(lane_now() == 0) atomicOr(&s_again, 1u << i);
+					}
+				}
+			} else {
+				keep_row = keep_row && ((redo[R] >> i) & 1u) != 0;
+			}
+			if constexpr(R == 0) {
+				const args_t a = args();
+				if(!BF16) out_el = a->out_dtype == AF3_BF16 ? 2 : 4;
+				const int es = BF16 ? 2 : out_el;
+				out_sb = a->out_stride[0] * es, out_sr = (int)a->out_stride[2];
+				out_row = static_cast<unsigned char*>(a->out) + (b0 * a->out_stride[0] + h * a->out_stride[1] + (row00 + i * (NW * 32)) * out_sr) * es;
+			} else out_row += out_sb;
+			const int es = BF16 ? 2 : out_el;
+			const __amdgpu_buffer_rsrc_t rsrc = buffer_of(out_row, out_sr, keep_row ? rows : 0, es);
+			const int l = lane_now(), half_ = l >> 5, n_ = l & 31, voff = (n_ * out_sr + 4 * half_) * es;
+			// (a Newton step behind the reciprocal: half an ulp, as the division)
+			const float r0 = __builtin_amdgcn_rcpf(lsum[R]), inv = __builtin_fmaf(r0, __builtin_fmaf(-lsum[R], r0, 1.f), r0);
+#pragma unroll
+			for(int k = 0; k < 16; k++) oacc[R][k] *= inv;
+			if constexpr(GATE) {
+				const int gk = 2 * R + (n_ >> 4);   // this query row's piece of the gate
+				const unsigned char* const gate_row = smem + (gk < ROWS ? gate_buf0 : gate_buf1) + (wave * ROWS + (gk < ROWS ? gk : gk - ROWS)) * 1024 + (n_ & 15) * 64 + half_ * 8;
+#pragma unroll
+				for(int g4 = 0; g4 < 4; g4++) {
+					u32x2 gw = graw[g4];
+					if constexpr(GATE_LDS) gw = *reinterpret_cast<const u32x2*>(gate_row + g4 * 16);
+					oacc[R][4 * g4] *= sigmoidf_fast(bf16_bits_to_f32(gw[0] & 0xffffu)), oacc[R][4 * g4 + 1] *= sigmoidf_fast(bf16_bits_to_f32(gw[0] >> 16));
+					oacc[R][4 * g4 + 2] *= sigmoidf_fast(bf16_bits_to_f32(gw[1] & 0xffffu)), oacc[R][4 * g4 + 3] *= sigmoidf_fast(bf16_bits_to_f32(gw[1] >> 16));
+				}
+			}
+			if(BF16 || es == 2) {   // (between query tiles no branch: the compiler's count of what is in flight would lose the stores)
+#pragma unroll
+				for(int g4 = 0; g4 < 4; g4++)
+					__builtin_amdgcn_raw_buffer_store_b64(u32x2{pack_bf16x2(oacc[R][4 * g4], oacc[R][4 * g4 + 1]), pack_bf16x2(oacc[R][4 * g4 + 2], oacc[R][4 * g4 + 3])}, rsrc,
+														  8 * g4 < D ? voff + 16 * g4 : 0x7FFF0000, 0, 0);
+			} else {
+#pragma unroll
+				for(int g4 = 0; g4 < 4; g4++)
+					__builtin_amdgcn_raw_buffer_store_b128(
+						u32x4{__float_as_uint(oacc[R][4 * g4]), __float_as_uint(oacc[R][4 * g4 + 1]), __float_as_uint(oacc[R][4 * g4 + 2]), __float_as_uint(oacc[R][4 * g4 + 3])}, rsrc,
+						8 * g4 < D ? voff + 32 * g4 : 0x7FFF0000, 0, 0);
+			}
+			lsum[R] = 0.f;
+#pragma unroll
+			for(int k = 0; k < 16; k++) oacc[R][k] = 0.f;
+		}
+	};
+
+	// One tile: ROWS steps.  The seq-th tile of the workgroup (tile t of query tile i) sits in buffer seq % 3.  In front of the last-but-one step the loads issued one tile
 	// earlier (tile t + 1 and its bias fragment: the youngest loads this wavefront has in flight) are awaited and a barrier
 	// publishes tile t + 1 -- that step fetches K fragments from it -- and tells that every wavefront is done with tile
 	// t - 1, whose buffer tile t + 2 then overwrites.  That step's first matrix instruction is the last reader of bias
 	// fragment t: behind it the fragment registers take fragment t + 1, and the slot (once those reads have returned: the
 	// last step's first matrix instruction waits for them) or the raw-piece registers are refilled with fragment t + 2.
-	auto tile = [&](auto first_c, auto careful_c, int t, int buf, int bufn, int bufnn) {
+	//
+	// Several query tiles of one head and the same batch rows: K, V and the masks stay, so the ring of tiles runs on -- behind the last
+	// tile come the first two again -- and so do the four chains.  The last tile's steps (LAST) request the next query tile's q rows
+	// as their predecessors' last readers pass, each three steps ahead of its first use; the next query tile's first tile (FIRST_NEXT) finishes and
+	// stores a batch row's results between the step's new reference and its exponentials.  A workgroup of one query tile spends 26 k clocks of its 79 k
+	// (L = 768) in front of its walk and behind it; from query tile to query tile it is 6 k.
+	// (INNER: a MIDDLE tile with two more of its query tile behind it; it asks nothing about what is to be requested.)
+	enum { MIDDLE = 0, FIRST = 1, LAST = 2, FIRST_NEXT = 3, CAREFUL_MIDDLE = 4, CAREFUL_FIRST = 5, INNER = -1 };
+	// more: this wavefront walks another query tile behind this one; more_wg: the workgroup does
+	auto tile = [&](auto kind_c, int t, int i, int seq, bool more, bool more_wg, int buf, int bufn, int bufnn) {
+		constexpr int  KIND = decltype(kind_c)::value;
+		constexpr auto first_c = ic<(KIND == FIRST || KIND == FIRST_NEXT || KIND == CAREFUL_FIRST) ? 1 : 0>{};
+		constexpr auto careful_c = ic<(KIND >= CAREFUL_MIDDLE) ? 1 : 0>{};
+		asm volatile("" : "+s"(t));   // (offsets of known tiles would be kept in registers, or spilled, through the walk)
 		const int m0 = mask_rd + t * (ROWS * 64);
+		// what is requested in this tile: the tile after the next
+		int tn = t + 2, tb = t + 2, ib = i;
+		if constexpr(KIND != INNER) {
+			if(tn >= n_t && more_wg) tn -= n_t;
+			if(tb >= n_t && more) tb -= n_t, ib = i + 1;
+		}
 		auto one = [&](auto r_c) {
 			constexpr int R = decltype(r_c)::value;
 			if constexpr(R < ROWS) {
 				constexpr int R1 = R + 1, R2 = R + 2;                        // the next step and the one after it ...
 				const int     k2 = (R2 >= ROWS ? bufn : buf) + (R2 % ROWS) * (2 * TILE_R);   // ... may belong to the next tile
-				const int     m1 = m0 + R1 * 64;                             // (row ROWS of tile t is row 0 of tile t + 1)
+				const int     m1 = KIND == LAST && R1 == ROWS ? mask_rd : m0 + R1 * 64;      // (row ROWS of tile t is row 0 of tile t + 1)
 				const int     vc = buf + R * (2 * TILE_R);
-				const bool    fr = decltype(first_c)::value != 0 && t == (int)((first_tiles >> (8 * (R < ROWS ? R : 0))) & 0xffu);
+				const bool    fr = KIND == CAREFUL_FIRST && t == (int)((first_tiles >> (8 * (R < ROWS ? R : 0))) & 0xffu);
+				if constexpr(KIND == LAST) {
+					request_q(r_c, i + 1);   // (row R: its last reader was the step before this one)
+					if constexpr(R1 == ROWS) {
+						convert_q(ic<0>{});
+						maskB[0][1] = 0u;
+						request_gate(ic<0>{}, i);
+					}
+				}
+				// (between the new reference's matrix instruction and the exponentials that wait for it)
+				auto finish = [&]() {
+					if constexpr(KIND == FIRST_NEXT) {
+						finish_row(r_c, ic<0>{}, ic<0>{}, ic<1>{}, i - 1, 0, 0);
+						request_gate(ic<R1>{}, i - 1);
+						if constexpr(R1 < ROWS) {
+							convert_q(ic<R1>{});
+							maskB[R1][1] = 0u;
+						}
+					}
+					if constexpr(R == ROWS - 2) {
+						// (with two rows the V^T fragments of tile t - 1 may still be on their way: they are consumed in this step; with more
+						// rows an earlier step of this tile has consumed them)
+						// (what was issued behind the awaited loads may stay in flight: the q rows of the steps so far, or the stores of finished rows)
+						constexpr int YOUNGER = KIND == LAST ? 2 * (ROWS - 1) : KIND == FIRST_NEXT ? (GATE ? 8 : 4) * (ROWS - 1) : 0;
+						if constexpr(ROWS == 2) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+						asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(YOUNGER) : "memory");
+					}
+				};
 				if constexpr(R == ROWS - 2) {
-					// (with two rows the V^T fragments of tile t - 1 may still be on their way: they are consumed in this step; with more
-					// rows an earlier step of this tile has consumed them)
-					if constexpr(ROWS == 2) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-					else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-					step(r_c, first_c, careful_c, fr, k2, m1, vc, [&](auto s_c) {
+					step(r_c, first_c, careful_c, fr, k2, m1, vc, finish, [&](auto s_c) {
 						constexpr int S = decltype(s_c)::value;
 						if constexpr(S == 1) {
-							load_tile_or_gate(t + 2, bufnn);
-							next_bias_fragment(t + 1);
-							load_bias_direct(t + 2);
-							load_bias_staged(t + 2);   // (into the half that held fragment t, read a tile ago)
+							if constexpr(KIND == INNER) load_tile(tn, bufnn);
+							else load_tile_or_gate(tn, bufnn, i);
+							next_bias_fragment(seq + 1);
+							if(KIND == INNER || tb < n_t) load_bias_direct(tb), load_bias_staged(tb, ib, seq);   // (into the half that held this tile's fragment, read a tile ago)
 						}
 					});
 				} else if constexpr(R == ROWS - 1) {
-					step(r_c, first_c, careful_c, fr, k2, m1, vc, [&](auto s_c) {
+					step(r_c, first_c, careful_c, fr, k2, m1, vc, finish, [&](auto s_c) {
 						constexpr int S = decltype(s_c)::value;
-						if constexpr(S == 1) load_bias(t + 2);   // (behind this step's first K.Q^T instruction, which has waited for the slot's reads)
+						if constexpr(S == 1)
+							if(KIND == INNER || tb < n_t) load_bias(tb, ib);   // (behind this step's first K.Q^T instruction, which has waited for the slot's reads)
 					});
 				} else {
-					step(r_c, first_c, careful_c, fr, k2, m1, vc, [](auto) {});
+					step(r_c, first_c, careful_c, fr, k2, m1, vc, finish, [](auto) {});
 				}
 			}
 		};
 		one(ic<0>{}), one(ic<1>{}), one(ic<2>{}), one(ic<3>{});
 	};
-	auto run = [&](auto careful_c) {
+	// the second tile and bias fragment, S^T of the first step, K fragments of the second (tile 0 and bias fragment 0 of query tile i are complete)
+	auto prologue = [&](auto careful_c, int i) {
 		constexpr bool CAREFUL = decltype(careful_c)::value != 0;
-		// ---- prologue: the second tile and bias fragment, S^T of the first step, K fragments of the second ----
-		// (tile 0 and bias fragment 0 were requested at the top of the kernel and are complete)
+#pragma unroll
+		for(int r = 0; r < ROWS; r++) {
+			m_ref[r] = 0.f;
+			lsum[r]  = 0.f;
+			maskB[r] = u32x2{half == 0 ? 0x3F80u : 0u, 0u};
+#pragma unroll
+			for(int k = 0; k < 16; k++) oacc[r][k] = 0.f;
+		}
+		rs_prev  = 0.f;
+		pprev[0] = pprev[1] = vprev[0] = vprev[1] = u32x4{0u, 0u, 0u, 0u};
 		next_bias_fragment(0);  // fragment 0 -> registers
 		asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-		load_tile_or_gate(1, BUF_R);
-		load_bias(1);
-		load_bias_direct(1);
-		load_bias_staged(1);
-		{
-			f32x16 s0;
+		load_tile_or_gate(1, BUF_R, i);
+		if(n_t > 1) load_bias(1, i), load_bias_direct(1), load_bias_staged(1, i, 1);
+		f32x16 s0;
 #pragma unroll
-			for(int i = 0; i < 16; i++) s0[i] = (HAS_BIAS && !(CAREFUL && dropped[0])) ? bias_frag[i] : 0.f;
+		for(int k = 0; k < 16; k++) s0[k] = (HAS_BIAS && !(CAREFUL && dropped[0])) ? bias_frag[k] : 0.f;
 #pragma unroll
-			for(int c = 0; c < 2; c++) s0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, read_kfrag(k_rd[c])), qf[0][c], s0, 0, 0, 0);
-			maskA[0] = *reinterpret_cast<const uint16_t*>(smem + mask_rd);
-			sc = mask_mfma(s0, maskB[0]);
-			kf[0] = read_kfrag(2 * TILE_R + k_rd[0]);
-			kf[1] = read_kfrag(2 * TILE_R + k_rd[1]);
-		}
-		int buf = 0, t = 0;
-		for(; t <= (CAREFUL ? t_force_max : 0); t++) {   // (more than one trip where some row's leading tiles hold dropped keys only)
-			const int bufn = buf == (NBUF_R - 1) * BUF_R ? 0 : buf + BUF_R, bufnn = bufn == (NBUF_R - 1) * BUF_R ? 0 : bufn + BUF_R;
-			tile(ic<1>{}, careful_c, t, buf, bufn, bufnn);
-			buf = bufn;
-		}
-		for(; t < n_t; t++) {
-			const int bufn = buf == (NBUF_R - 1) * BUF_R ? 0 : buf + BUF_R, bufnn = bufn == (NBUF_R - 1) * BUF_R ? 0 : bufn + BUF_R;
-			tile(ic<0>{}, careful_c, t, buf, bufn, bufnn);
-			buf = bufn;
+		for(int c = 0; c < 2; c++) s0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, read_kfrag(k_rd[c])), qf[0][c], s0, 0, 0, 0);
+		maskA[0] = *reinterpret_cast<const uint16_t*>(smem + mask_rd);
+		sc = mask_mfma(s0, maskB[0]);
+		kf[0] = read_kfrag(2 * TILE_R + k_rd[0]);
+		kf[1] = read_kfrag(2 * TILE_R + k_rd[1]);
+	};
+	auto last_product = [&]() {   // the last step's P.V product (the last batch row)
+		lsum[ROWS - 1] += rs_prev;
+		oacc[ROWS - 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vprev[0]), __builtin_bit_cast(bf16x8, pprev[0]), oacc[ROWS - 1], 0, 0, 0);
+		oacc[ROWS - 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vprev[1]), __builtin_bit_cast(bf16x8, pprev[1]), oacc[ROWS - 1], 0, 0, 0);
+	};
+	auto next_buf = [](int buf) { return buf == (NBUF_R - 1) * BUF_R ? 0 : buf + BUF_R; };
+	// a wavefront none of whose query rows exist (L % 128 != 0, the last query tile) fetches its batch row's tiles, keeps the barriers' count --
+	// one per tile -- and leaves the vector and matrix pipes to others
+	auto load_only = [&](int buf) {   // (tiles 0 and 1 are requested)
+		int bufnn = next_buf(next_buf(buf));
+		for(int t = 0; t < n_t; t++) {
+			asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+			if(t + 2 < n_t) load_tile(t + 2, bufnn);
+			bufnn = next_buf(bufnn);
 		}
 	};
 	// The key axis is walked without a look at the row sums on the way (a test per step made the wavefront wait for the matrix pipe
@@ -710,102 +903,107 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 	// that end below the careful walk's limit have stayed below it throughout: the results are the careful walk's.  Beyond it they
 	// stand all the same if the sums stay below 2^100 and the results are finite (probabilities and sums are floating-point: a
 	// reference left behind costs them no digits).  Otherwise the whole workgroup -- its wavefronts fetch tiles for one another --
-	// walks once more, carefully, and a workgroup with a batch row without a live key, or without one in its first tile, does so at once.
+	// walks that query tile once more, carefully, and a workgroup with a batch row without a live key, or without one in its first tile, walks all of them so.
 	bool careful = t_force_max > 0;
 #pragma unroll
 	for(int r = 0; r < ROWS; r++) careful = careful || dropped[r];   // (the same in every wavefront of the workgroup)
-	const bool no_rows = (int64_t)qtile * (NW * 32) + wave * 32 >= L;
-	auto walk = [&](auto careful_c) {
-		if(no_rows) {
-			// ---- no query row of this wavefront exists (L % 128 != 0, the last query tile): it fetches its batch row's tiles, keeps the
-			// barriers' count -- one per tile -- and leaves the vector and matrix pipes to others ----
-			load_tile(1, BUF_R);
-			int bufnn = 2 * BUF_R;
-			for(int t = 0; t < n_t; t++) {
-				asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-				load_tile(t + 2, bufnn);
-				bufnn = bufnn == (NBUF_R - 1) * BUF_R ? 0 : bufnn + BUF_R;
-			}
-		} else {
-#pragma unroll
-			for(int r = 0; r < ROWS; r++) {
-				m_ref[r] = 0.f;
-				lsum[r]  = 0.f;
-				maskB[r] = u32x2{half == 0 ? 0x3F80u : 0u, 0u};
-#pragma unroll
-				for(int i = 0; i < 16; i++) oacc[r][i] = 0.f;
-			}
-			rs_prev  = 0.f;
-			pprev[0] = pprev[1] = vprev[0] = vprev[1] = u32x4{0u, 0u, 0u, 0u};
-			run(careful_c);
-			lsum[ROWS - 1] += rs_prev;
-			// the last step's P.V product (batch row 3)
-			oacc[ROWS - 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vprev[0]), __builtin_bit_cast(bf16x8, pprev[0]), oacc[ROWS - 1], 0, 0, 0);
-			oacc[ROWS - 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vprev[1]), __builtin_bit_cast(bf16x8, pprev[1]), oacc[ROWS - 1], 0, 0, 0);
-		}
-		asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load may still be writing LDS when the workgroup's allocation is released
-	};
+	uint32_t again = 0xffffffffu >> (32 - n_q);
 	if(!careful) {
-		walk(ic<0>{});
-		bool over = false;
-#pragma unroll
-		for(int r = 0; r < ROWS; r++) over = over || !(lsum[r] < PSUM_LIMIT);
-		if(__ballot(row_ok && over)) {   // rare
-			bool bad = false;
-#pragma unroll
-			for(int r = 0; r < ROWS; r++) {
-				float t = lsum[r] * 0x1p28f;   // (infinite from 2^100 on)
-#pragma unroll
-				for(int i = 0; i < 16; i++) t = fmaf(oacc[r][i], 0.f, t);
-				bad = bad || !(t < __builtin_inff());
+		int buf = 0, seq = 0;
+		if(my_q > 0) {
+			prologue(ic<0>{}, 0);
+			bool more = my_q > 1, more_wg = n_q > 1;
+			tile(ic<FIRST>{}, 0, 0, 0, more, more_wg, 0, BUF_R, 2 * BUF_R);
+			buf = BUF_R, seq = 1;
+			int i = 0;
+			for(;;) {
+				const int t_end = more ? n_t - 1 : n_t;
+				int       t = 1;
+				for(; t < n_t - 2; t++) {
+					const int bufn = next_buf(buf), bufnn = next_buf(bufn);
+					tile(ic<INNER>{}, t, i, seq, more, more_wg, buf, bufn, bufnn);
+					buf = bufn, seq++;
+				}
+				for(; t < t_end; t++) {
+					const int bufn = next_buf(buf), bufnn = next_buf(bufn);
+					tile(ic<MIDDLE>{}, t, i, seq, more, more_wg, buf, bufn, bufnn);
+					buf = bufn, seq++;
+				}
+				if(!MULTI || !more) break;
+				{
+					const int bufn = next_buf(buf), bufnn = next_buf(bufn);
+					tile(ic<LAST>{}, n_t - 1, i, seq, true, true, buf, bufn, bufnn);
+					buf = bufn, seq++, i++;
+				}
+				more = i + 1 < my_q, more_wg = i + 1 < n_q;
+				{
+					const int bufn = next_buf(buf), bufnn = next_buf(bufn);
+					tile(ic<FIRST_NEXT>{}, 0, i, seq, more, more_wg, buf, bufn, bufnn);
+					buf = bufn, seq++;
+				}
 			}
-			if(__ballot(row_ok && bad) && lane == 0) s_again = 1;
+			last_product();
+			asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the gate rows)
+			const int gate0 = buf, gate1 = next_buf(buf);
+			auto finish_last = [&](auto r_c) {
+				if(!GATE || my_q == n_q) finish_row(r_c, ic<0>{}, ic<1>{}, ic<0>{}, i, gate0, gate1);
+				else request_gate(r_c, i), finish_row(r_c, ic<0>{}, ic<0>{}, ic<0>{}, i, 0, 0);   // (the workgroup walks on: its tile buffers are in use)
+			};
+			finish_last(ic<0>{}), finish_last(ic<1>{}), finish_last(ic<2>{}), finish_last(ic<3>{});
+		} else {
+			if(n_t > 1) load_tile(1, BUF_R);
 		}
-		__syncthreads();
-		if(__builtin_amdgcn_readfirstlane(s_again)) {   // rare
-			careful = true;
+		if(my_q < n_q) {
+			load_only(buf);
+			asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load may still be writing LDS when the workgroup's allocation is released
+		}
+		asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+		again = (uint32_t)__builtin_amdgcn_readfirstlane((int)*(volatile uint32_t*)&s_again);
+		if(again == 0u) return;
+	} else {
+#pragma unroll
+		for(int r = 0; r < ROWS; r++) redo[r] = again;
+	}
+	// ---- the careful walk of the query tiles in `again` (rare) ----
+	bool fresh = careful;   // the start's requests serve the first query tile
+	while(again) {
+		const int i = __builtin_ctz(again);
+		again &= again - 1;
+		if(!fresh || i > 0) {
+			__syncthreads();   // (every wavefront has left the tiles of the walk before)
 			load_tile(0, 0);
-			load_bias(0);
+			load_bias(0, i);
 			load_bias_direct(0);
-			load_bias_staged(0);
+			load_bias_staged(0, i, 0);
+			request_q(ic<0>{}, i), request_q(ic<1>{}, i), request_q(ic<2>{}, i), request_q(ic<3>{}, i);
+			convert_q(ic<0>{}), convert_q(ic<1>{}), convert_q(ic<2>{}), convert_q(ic<3>{});
+			drop_q();
 			asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 			__syncthreads();
 		}
-	}
-	if(careful) walk(ic<1>{});
-	if(no_rows) return;
-
-	// ---- epilogue: O^T register i is head column 8*(i/4) + 4*half + i%4; optional output gate (out *= sigmoid(gate), the
-	// reference's "weighted_avg *= sigmoid(gating_query(pair))", src/csrc/dot_product_attention.cpp:335-349) ----
-	const int gate_buf[2] = {(n_t % NBUF_R) * BUF_R, ((n_t + 1) % NBUF_R) * BUF_R};
-	if(row_ok) {
-#pragma unroll
-		for(int r = 0; r < ROWS; r++) {
-			if(b0 + r >= b_end) break;
-			[[maybe_unused]] const int gk = 2 * r + (n >> 4);   // this query row's piece of the gate
-			[[maybe_unused]] const unsigned char* const gate_row = smem + (gk < ROWS ? gate_buf[0] : gate_buf[1]) + (wave * ROWS + (gk < ROWS ? gk : gk - ROWS)) * 1024 + (n & 15) * 64;
-			const float   inv  = 1.f / lsum[r];
-			const int64_t ooff = (b0 + r) * p.out_stride[0] + h * p.out_stride[1] + qrow * p.out_stride[2];
-#pragma unroll
-			for(int g4 = 0; g4 < 4; g4++) {
-				const int d0 = 8 * g4 + 4 * half;
-				if(d0 >= D) continue;
-				float o0 = oacc[r][4 * g4] * inv, o1 = oacc[r][4 * g4 + 1] * inv, o2 = oacc[r][4 * g4 + 2] * inv, o3 = oacc[r][4 * g4 + 3] * inv;
-				if constexpr(GATE) {
-					const u32x2    gw = *reinterpret_cast<const u32x2*>(gate_row + d0 * 2);
-					const uint32_t g0 = gw[0], g1 = gw[1];
-					o0 *= sigmoidf_fast(bf16_bits_to_f32(g0 & 0xffffu)), o1 *= sigmoidf_fast(bf16_bits_to_f32(g0 >> 16));
-					o2 *= sigmoidf_fast(bf16_bits_to_f32(g1 & 0xffffu)), o3 *= sigmoidf_fast(bf16_bits_to_f32(g1 >> 16));
-				}
-				if(p.out_dtype == AF3_BF16) {
-					const u32x2 w = {pack_bf16x2(o0, o1), pack_bf16x2(o2, o3)};
-					*reinterpret_cast<u32x2*>(static_cast<uint16_t*>(p.out) + ooff + d0) = w;
-				} else {
-					const float4 w = {o0, o1, o2, o3};
-					*reinterpret_cast<float4*>(static_cast<float*>(p.out) + ooff + d0) = w;
-				}
-			}
+		fresh = false;
+		if(i >= my_q) {
+			if(n_t > 1) load_tile(1, BUF_R);
+			load_only(0);
+			asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+			continue;
 		}
+		prologue(ic<1>{}, i);
+		int buf = 0, t = 0;
+		for(; t <= t_force_max; t++) {   // (more than one trip where some row's leading tiles hold dropped keys only)
+			const int bufn = next_buf(buf), bufnn = next_buf(bufn);
+			tile(ic<CAREFUL_FIRST>{}, t, i, t, false, false, buf, bufn, bufnn);
+			buf = bufn;
+		}
+		for(; t < n_t; t++) {
+			const int bufn = next_buf(buf), bufnn = next_buf(bufn);
+			tile(ic<CAREFUL_MIDDLE>{}, t, i, t, false, false, buf, bufn, bufnn);
+			buf = bufn;
+		}
+		last_product();
+		asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load may still be writing LDS when the workgroup's allocation is released
+		const int gate0 = buf, gate1 = next_buf(buf);
+		finish_row(ic<0>{}, ic<1>{}, ic<1>{}, ic<0>{}, i, gate0, gate1), finish_row(ic<1>{}, ic<1>{}, ic<1>{}, ic<0>{}, i, gate0, gate1), finish_row(ic<2>{}, ic<1>{}, ic<1>{}, ic<0>{}, i, gate0, gate1), finish_row(ic<3>{}, ic<1>{}, ic<1>{}, ic<0>{}, i, gate0, gate1);
 	}
 }
 
@@ -849,11 +1047,37 @@ int rows_bias_mode(const af3_dpa_params& p) {
 	return ws_ok ? 1 : -1;
 }
 
+// How many query tiles a workgroup walks.  Its start and its end (masks, first tiles, q, the stores' way out) are paid once, but workgroups of several
+// query tiles come in fewer rounds of the 64 an XCD holds (two per compute unit), and query tiles that are walked one behind the other read K and V
+// from the L2 at different times, where neighbours read them together: a divisor of the number of query tiles up to 4, one that leaves whole rounds
+// where there is one, else the smallest; what does not make whole rounds ends in a round of single query tiles.  Five and
+// eleven query tiles go as 2 2 1 and 3 3 3 2; seven gained nothing.  us, one query tile each / so, one card, L x 4 x L x 32: 300 44.5 / 41.2, 384 61.0 / 59.5,
+// 400 97.8 / 89.6, 512 127.5 / 122.6, 600 204.5 / 200.5, 640 237.5 / 230.0, 768 393.8 / 377.3, 1024 874 / 841, 1200 1437 / 1397, 1300 1847 / 1813,
+// 1491 2643 / 2564; 2048 x 4 x 256 x 32 165.9 / 162.1, 512 x 4 x 768 x 24 242.6 / 234.3; larger chunks of more query tiles: 1491 in chunks of 12 3521, of 6 2802, of 3 2704.
+void plan_chunks(int n_qtiles, int64_t per_xcd, int& chunk, int& parts, int64_t& chunked) {
+	constexpr int64_t SLOTS = 64;
+	if(per_xcd * n_qtiles <= SLOTS) return;   // (one round as it is)
+	auto whole_rounds = [&](int c) { return per_xcd * ((n_qtiles + c - 1) / c) % SLOTS == 0; };
+	int  c = n_qtiles == 5 ? 2 : n_qtiles == 11 ? 3 : 1;
+	for(int i = 4; i >= 2; i--)
+		if(n_qtiles % i == 0 && (c == 1 || whole_rounds(i) || !whole_rounds(c))) c = i;
+	if(c == 1) return;
+	chunk = c, parts = (n_qtiles + c - 1) / c, chunked = per_xcd;
+	if(!whole_rounds(c)) {
+		const int64_t tail = (SLOTS + n_qtiles - 1) / n_qtiles;
+		chunked = per_xcd > tail ? per_xcd - tail : 0;
+	}
+}
+
 template <int ROWS, int BMODE>
 int launch_rows(const af3_dpa_params& p, int64_t b_first, int64_t b_count, hipStream_t s) {
 	const int     n_qtiles = (int)((p.L + 127) / 128);
 	const int64_t n_groups = ((b_count + ROWS - 1) / ROWS) * p.H;
-	const int64_t blocks   = ((n_groups + 7) / 8) * 8 * n_qtiles;
+	const int64_t per_xcd  = (n_groups + 7) / 8;
+	int           chunk = 1, parts = n_qtiles;
+	int64_t       chunked = 0;
+	if(several_query_tiles(ROWS, BMODE, p.gate != nullptr) && p.out_dtype == AF3_BF16) plan_chunks(n_qtiles, per_xcd, chunk, parts, chunked);
+	const int64_t blocks   = (chunked * parts + (per_xcd - chunked) * n_qtiles) * 8;
 	if(blocks <= 0 || blocks > 0x7fffffffLL) return AF3_ERR_BAD_SHAPE;
 	const size_t n_t_all = (size_t)((p.L + KT_R - 1) / KT_R);
 	const size_t smem    = (size_t)NBUF_R * ROWS * 2 * TILE_R + (BMODE == 1 || BMODE == 3 ? 4 * 4096 : 0) + (n_t_all + 1) * ROWS * 32 * 2;
@@ -861,7 +1085,7 @@ int launch_rows(const af3_dpa_params& p, int64_t b_first, int64_t b_count, hipSt
 	if(smem > 63 * 1024) {   // (the kernel's static words take 1 KB of the 64 that need no asking: smem's alignment)
 		if(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) return AF3_ERR_LAUNCH;
 	}
-	hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), smem, s, p, n_qtiles, n_groups, b_first, b_count);
+	hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), smem, s, p, n_qtiles, n_groups, b_first, b_count, chunk, parts, (int)chunked);
 	return launch_status();
 }
 
@@ -876,6 +1100,8 @@ int launch_rows_n(int rows, const af3_dpa_params& p, int64_t b_first, int64_t b_
 // head_dim <= 32, at least two batch rows, a length whose mask table fits beside the tile buffers, 16-byte aligned gate rows.
 bool mfma_rows_eligible(const af3_dpa_params& p) {
 	if(p.D > 32 || p.B < 2 || p.L > MAX_L_ROWS) return false;
+	constexpr int64_t MAX_ROW_STRIDE = 1 << 24;   // (elements: 32 rows of q, gate or out are addressed with 32-bit byte offsets)
+	if(p.q_stride[2] >= MAX_ROW_STRIDE || p.out_stride[2] >= MAX_ROW_STRIDE || (p.gate && p.gate_stride[2] >= MAX_ROW_STRIDE)) return false;
 	if(p.gate && ((reinterpret_cast<uintptr_t>(p.gate) & 15) || p.gate_stride[0] % 8 || p.gate_stride[1] % 8 || p.gate_stride[2] % 8)) return false;
 	return true;
 }

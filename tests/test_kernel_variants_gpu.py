@@ -503,6 +503,40 @@ def test_shared_bias_quick_and_careful_walks(af3, oracle, B, H, L, D, kind):
     assert (np.abs(out - want) / scale).max() <= 2e-2
 
 
+@pytest.mark.parametrize("B,H,L,D", [(404, 4, 300, 32), (261, 4, 264, 24), (130, 8, 512, 32), (96, 8, 640, 16), (500, 4, 200, 8), (128, 2, 1281, 32)])   # two to four of 3, 3, 4, 5, 2 and 11 query tiles one behind the other; last ones in which one to three wavefronts have rows
+@pytest.mark.parametrize("kind", ["random", "no bias", "first tile", "none", "120", "120 and none"])
+@pytest.mark.parametrize("gated", [False, True])
+def test_shared_bias_query_tiles_in_one_workgroup(af3, B, H, L, D, kind, gated):
+    """Workgroups that walk several query tiles: every row of every tile, keys that end in the first tile, workgroups that walk carefully from the
+    start, single query tiles whose sums send only these through the careful walk at the end."""
+    from af3_kernels_amd import _lib, ops
+    g = torch.Generator(device="cuda").manual_seed(L + D)
+    q, k, v, gate = (torch.randn(B, H, L, D, generator=g, device="cuda").to(torch.bfloat16) for _ in range(4))
+    bias = torch.randn(H, L, L, generator=g, device="cuda").to(torch.bfloat16)
+    keep = torch.rand(B, L, generator=g, device="cuda") < 0.8
+    keep[:, 0] = keep[:, L - 1] = True
+    if kind == "first tile":
+        keep[:, 20:] = False
+    if "none" in kind:
+        keep[B // 2] = False
+    if "120" in kind:
+        bias[:, [3, L // 2, L - 2], L - 1] = 120.0   # (rows of the first, a middle and the last query tile)
+    print("case", B, H, L, D, kind, gated, flush=True)
+    out = ops._dpa_forward_impl(q, k, v, ops._lift_mask(keep, L), None if kind == "no bias" else bias, _lib.AF3_BF16, False, gate=gate if gated else None).float()
+    torch.cuda.synchronize()
+    assert torch.isfinite(out).all()
+    for b in range(0, B, 32):   # (float32 on the GPU, some batch rows at a time)
+        qs, ks, vs = (t[b:b + 32].float().contiguous() for t in (q, k, v))
+        s = torch.matmul(qs * D ** -0.5, ks.transpose(-1, -2).contiguous())
+        if kind != "no bias":
+            s += bias.float()
+        w = torch.softmax(s.masked_fill(~keep[b:b + 32, None, None, :], -1e9), -1)
+        want = torch.matmul(w, vs)
+        if gated:
+            want *= torch.sigmoid(gate[b:b + 32].float())
+        assert (out[b:b + 32] - want).abs().max().item() <= 2e-2   # (bf16 q, k, v and probabilities; |v| < 6)
+
+
 @pytest.mark.parametrize("B,H,L,D", [(3, 2, 1, 32), (2, 1, 3, 16), (4, 2, 4, 32), (3, 2, 37, 32), (2, 2, 255, 24), (3, 1, 257, 32), (2, 1, 2047, 32), (2, 1, 2049, 32), (3, 1, 2306, 16),
                                      (4, 1, 2013, 32), (3, 1, 1984, 32)])   # (the last two: around the 64 KB of LDS that a launch gets without asking)
 @pytest.mark.parametrize("kind", ["random", "last", "head", "middle", "none", "bytes", "no mask"])
