@@ -62,7 +62,7 @@ __device__ __forceinline__ float max3(float a, float b, float c) {   // (written
 // KS: 1, or the number of parts that the tiles of a block of query rows are dealt to, each with wavefronts and buffers of its own
 // (for launches of few workgroups); their sums are merged through LDS at the end.
 template <int DP, bool COMP, bool ONES, int BMODE, int KS>
-__global__ void __launch_bounds__(KS * NW8 * 64) __attribute__((amdgpu_waves_per_eu(DP == 32 ? 4 : KS == 1 ? 3 : 2))) dpa_mfma_fp8_kernel(af3_dpa_params p, int n_qtiles, int n_units, int per_xcd) {
+__global__ void __launch_bounds__(KS * NW8 * 64) __attribute__((amdgpu_waves_per_eu(DP == 32 ? 4 : KS == 1 ? 3 : 2))) dpa_mfma_fp8_kernel(af3_dpa_params p, int n_qtiles, int n_units, int per_xcd, bool even) {
 	constexpr int NDB      = DP / 32;       // 32-row blocks of O^T
 	constexpr int K_TILE1  = KT8 * DP;      // bytes of one K tile
 	constexpr int K_TILE   = K_TILE1 * (COMP ? 2 : 1);  // hi tile followed by the residual tile
@@ -511,7 +511,9 @@ __global__ void __launch_bounds__(KS * NW8 * 64) __attribute__((amdgpu_waves_per
 	// Tile `it` is in buffer it % 3.  Order of this wavefront's loads: tile it + 1 (behind the barrier of iteration it - 1), its
 	// first half of bias (in the second stage of it - 1), its second half (in the first stage of it), tile it + 2, ...
 	int cur = buf0;
+	even_progress progress(nlive, even);
 	for(int it = 0; it < nlive; it++) {
+		progress.at(it);
 		const int  kt = entry & ~TILE_FULL, kt1 = entry1 & ~TILE_FULL;
 		const int  nxt = cur == buf0 + 2 * TILE ? buf0 : cur + TILE, nxt2 = nxt == buf0 + 2 * TILE ? buf0 : nxt + TILE;
 		const bool has1 = it + 1 < nlive, has2 = it + 2 < nlive;
@@ -613,9 +615,11 @@ int launch8_parts(const af3_dpa_params& p, hipStream_t s) {
 	const int64_t blocks   = per_xcd > 0 ? side_by : (n_groups + 7) / 8 * 8 * n_qtiles;
 	if(blocks <= 0 || blocks > 0x7fffffffLL) return AF3_ERR_BAD_SHAPE;
 	const size_t smem = (size_t)KS * (3 * (COMP ? 3 : 2) * KT8 * DP + (BMODE >= 2 ? NW8 * 2 * BIAS_HALF8 : 0)) + (size_t)n_ktiles * KT8 * 2 + (size_t)((n_ktiles + 15) & ~15);
+	const int64_t by_lds = 160 * 1024 / (int64_t)smem, by_regs = (DP == 32 ? 4 : KS == 1 ? 3 : 2) / KS;   // workgroups a compute unit holds
+	const int64_t per_cu = by_lds < 1 ? 1 : by_lds < by_regs ? by_lds : by_regs;
 	auto         kern = dpa_mfma_fp8_kernel<DP, COMP, ONES, BMODE, KS>;
 	if(smem > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) return AF3_ERR_LAUNCH;
-	hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(KS * NW8 * 64), smem, s, p, n_qtiles, (int)(per_xcd > 0 ? n_blocks : n_groups), (int)per_xcd);
+	hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(KS * NW8 * 64), smem, s, p, n_qtiles, (int)(per_xcd > 0 ? n_blocks : n_groups), (int)per_xcd, even_progress_wanted(n_groups * n_qtiles, 256 * per_cu));
 	return launch_status();
 }
 template <int DP, bool COMP, bool ONES, int BMODE>

@@ -101,7 +101,7 @@ __global__ void __launch_bounds__(256) bias_rows_prepass_kernel(const void* __re
 constexpr bool several_query_tiles(int rows, int bmode, bool gate) { return bmode != 2 && !(gate && rows == 4); }
 template <int ROWS, int BMODE, bool GATE>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) dpa_rows_bf16_kernel(af3_dpa_params p, int n_qtiles, int64_t n_groups, int64_t b_first, int64_t b_count, int q_chunk,
-																										   int n_chunks, int n_chunked) {
+																										   int n_chunks, int n_chunked, bool even) {
 	static_assert(ROWS >= 2 && ROWS <= 4, "two to four row chains per wavefront");
 	constexpr int  NW       = 4;
 	constexpr bool HAS_BIAS = BMODE != 0, SLOT = BMODE == 1, DIRECT = BMODE == 2, STAGED = BMODE == 3;
@@ -916,11 +916,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 			tile(ic<FIRST>{}, 0, 0, 0, more, more_wg, 0, BUF_R, 2 * BUF_R);
 			buf = BUF_R, seq = 1;
 			int i = 0;
+			even_progress progress(n_q * n_t, even);
 			for(;;) {
 				const int t_end = more ? n_t - 1 : n_t;
 				int       t = 1;
 				for(; t < n_t - 2; t++) {
 					const int bufn = next_buf(buf), bufnn = next_buf(bufn);
+					progress.at(seq);
 					tile(ic<INNER>{}, t, i, seq, more, more_wg, buf, bufn, bufnn);
 					buf = bufn, seq++;
 				}
@@ -1078,6 +1080,9 @@ int launch_rows(const af3_dpa_params& p, int64_t b_first, int64_t b_count, hipSt
 	int64_t       chunked = 0;
 	if(several_query_tiles(ROWS, BMODE, p.gate != nullptr) && p.out_dtype == AF3_BF16) plan_chunks(n_qtiles, per_xcd, chunk, parts, chunked);
 	const int64_t blocks   = (chunked * parts + (per_xcd - chunked) * n_qtiles) * 8;
+	// (by age / evenly, us: 384 x 4 x 384 x 32 62.1 / 60.5, 512 131.7 / 129.0, 768 389.8 / 383.7, 1491 2612 / 2598, 64 x 4 x 768 x 32 41.2 / 39.7, 5 x 16 x 2000 x 24
+	// 116.1 / 112.8, 400 90.2 / 91.4; many rounds of single query tiles: the grid block of 512 tokens 246 / 252, 832 511.5 / 514.9)
+	const bool even = chunked > 0 || (blocks <= 3 * 512 && even_progress_wanted(blocks, 512));
 	if(blocks <= 0 || blocks > 0x7fffffffLL) return AF3_ERR_BAD_SHAPE;
 	const size_t n_t_all = (size_t)((p.L + KT_R - 1) / KT_R);
 	const size_t smem    = (size_t)NBUF_R * ROWS * 2 * TILE_R + (BMODE == 1 || BMODE == 3 ? 4 * 4096 : 0) + (n_t_all + 1) * ROWS * 32 * 2;
@@ -1085,7 +1090,7 @@ int launch_rows(const af3_dpa_params& p, int64_t b_first, int64_t b_count, hipSt
 	if(smem > 63 * 1024) {   // (the kernel's static words take 1 KB of the 64 that need no asking: smem's alignment)
 		if(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) return AF3_ERR_LAUNCH;
 	}
-	hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), smem, s, p, n_qtiles, n_groups, b_first, b_count, chunk, parts, (int)chunked);
+	hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), smem, s, p, n_qtiles, n_groups, b_first, b_count, chunk, parts, (int)chunked, even);
 	return launch_status();
 }
 
