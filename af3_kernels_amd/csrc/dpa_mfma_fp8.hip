@@ -31,7 +31,7 @@
 //   * 39 KB of LDS and 128 registers: four workgroups of four wavefronts per compute unit.
 //   * Workgroups in an order that lets batch rows share the bias, tiles in two parts where workgroups are few: see launch8_parts, launch8.
 // us per call with its two quantising launches (6 to 13 us), 16 heads of 24, 16-deep products / these forms, workgroups by heads and one part / now:
-// 5x1536 89.0/71.3/68.4, 8x1536 133.6/104.9/101, 8x1301 (ragged rows) -/101.7/97, 8x1000 66.7/54.2/54, 5x300 37.9/20.3/17.5, 1x1536 42.1/34.2/27.6 (cards
+// 5x1536 89.0/71.3/64.5, 8x1536 133.6/104.9/98.8, 8x1301 (ragged rows) -/101.7/97, 8x1000 66.7/54.2/54, 5x300 37.9/20.3/17.5, 1x1536 42.1/34.2/27.6 (cards
 // differ: 5x1536 68 to 71).  Measured on the way: with the bias streamed once per batch row its loads were 13 us of 57 at 5x1536, the exponentials 4; four workgroups per compute unit instead of three changed nothing, nor did
 // pinning the matrix instructions between the exponentials: the vector port is busy three quarters of the time.
 #include "mfma_helpers.hpp"
@@ -52,6 +52,18 @@ __device__ __forceinline__ float max3(float a, float b, float c) {   // (written
 	float r;
 	asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
 	return r;
+}
+
+// the maximum of a lane's 16 logits and m, in two chains (one statement: the compiler puts a wait state behind each)
+__device__ __forceinline__ float max17(const f32x16& s, float m) {
+	float a, b;
+	asm("v_max3_f32 %0, %2, %3, %4\n\tv_max3_f32 %1, %5, %6, %7\n\t"
+		"v_max3_f32 %0, %0, %8, %9\n\tv_max3_f32 %1, %1, %10, %11\n\t"
+		"v_max3_f32 %0, %0, %12, %13\n\tv_max3_f32 %1, %1, %14, %15\n\t"
+		"v_max3_f32 %0, %0, %16, %17\n\tv_max3_f32 %0, %0, %1, %18"
+		: "=&v"(a), "=&v"(b)
+		: "v"(s[0]), "v"(s[1]), "v"(s[2]), "v"(s[3]), "v"(s[4]), "v"(s[5]), "v"(s[6]), "v"(s[7]), "v"(s[8]), "v"(s[9]), "v"(s[10]), "v"(s[11]), "v"(s[12]), "v"(s[13]), "v"(s[14]), "v"(s[15]), "v"(m));
+	return a;
 }
 
 // DP: head_dim padded to 32 or 64 (bytes per K row in LDS, rows of the V^T tile).
@@ -278,13 +290,14 @@ __global__ void __launch_bounds__(KS * NW8 * 64) __attribute__((amdgpu_waves_per
 	if(all_dropped) todo[0] = __ballot(lane < n_ktiles), todo[1] = __ballot(64 + lane < n_ktiles);
 	const int n_todo = __builtin_popcountll(todo[0]) + __builtin_popcountll(todo[1]);
 	const int nlive  = (n_todo - part + KS - 1) / KS, n_most = (n_todo + KS - 1) / KS;   // tiles of this part and of the first; they differ by one at most
-	int       entry_last = 0;
+	int       entry_last = 0, base = 0;
+	// (both words chosen between in every step, and maxima in statements of their own: 3x1000 29.0 us, 1x1301 28.5, 8x1536 100.1; so 28.1, 27.6, 98.8)
 	auto pop = [&]() -> int {   // the next tile's number and flag; behind the last one: that one again
-		const int i = todo[0] == 0 ? 1 : 0;
-		if(todo[i] != 0) {
-			const int t = __builtin_ctzll(todo[i]);
-			entry_last  = (64 * i + t) | ((some[i] >> t) & 1 ? 0 : TILE_FULL);
-			todo[i] &= todo[i] - 1;
+		if(todo[0] == 0) todo[0] = todo[1], some[0] = some[1], todo[1] = 0, base = 64;   // (once, or behind the last tile)
+		if(todo[0] != 0) {
+			const int t = __builtin_ctzll(todo[0]);
+			entry_last  = (base + t) | ((some[0] >> t) & 1 ? 0 : TILE_FULL);
+			todo[0] &= todo[0] - 1;
 		}
 		return entry_last;
 	};
@@ -414,11 +427,7 @@ __global__ void __launch_bounds__(KS * NW8 * 64) __attribute__((amdgpu_waves_per
 		if(!full_n) maskA[0] = *reinterpret_cast<const uint16_t*>(smem + mask_rd + kt_n * (KT8 * 2) + SUBN * 64);
 		// online softmax with the true running maximum (in accumulator units)
 		// (two chains of three-operand maxima)
-		float mx0 = max3(sc[0], sc[1], sc[2]), mx1 = max3(sc[3], sc[4], sc[5]);
-		mx0 = max3(mx0, sc[6], sc[7]), mx1 = max3(mx1, sc[8], sc[9]);
-		mx0 = max3(mx0, sc[10], sc[11]), mx1 = max3(mx1, sc[12], sc[13]);
-		mx0 = max3(mx0, sc[14], sc[15]);
-		mx0 = max3(mx0, mx1, m_run);
+		const float mx0 = max17(sc, m_run);
 		const auto  sw    = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx0), __float_as_uint(mx0), false, false);
 		const float m_new = max3(mx0, __uint_as_float(sw[0]), __uint_as_float(sw[1]));
 		if(__ballot(m_new > m_run)) {   // (the first time from -inf: the factor is 0, and nothing has been accumulated)
@@ -427,7 +436,8 @@ __global__ void __launch_bounds__(KS * NW8 * 64) __attribute__((amdgpu_waves_per
 #pragma unroll
 			for(int db = 0; db < NDB; db++)
 #pragma unroll
-				for(int i = 0; i < 16; i++) oacc[db][i] *= a;
+				for(int i = 0; i < 16; i++)
+					if(!(ONES && db == NDB - 1 && i > 12)) oacc[db][i] *= a;   // (those hold rows of zeros)
 			m_run = m_new;
 			mc    = m_new * c_exp - P_SHIFT;
 		}
