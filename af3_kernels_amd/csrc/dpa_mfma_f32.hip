@@ -68,7 +68,7 @@ __device__ __forceinline__ void split3(float x0, float x1, uint32_t& hi, uint32_
 // launches with too few blocks to fill the chip: wavefront ks takes tiles ks, ks + KS, ... of the walk, a step of the loop
 // moves KS tiles, and the partial (O, m, l) are merged through LDS at the end.
 template <int DP, int NW, int KS>
-__global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DP == 64 || KS > 1 ? 2 : NW == 4 ? 3 : 4))) dpa_mfma_f32_kernel(af3_dpa_params p, int n_qtiles, int64_t n_groups, bool even) {
+__global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DP == 64 || KS > 1 ? 2 : NW == 4 ? 3 : 4))) dpa_mfma_f32_kernel(af3_dpa_params p, int n_qtiles, int64_t n_groups, int even) {
 	constexpr int NC   = DP / 16;             // contraction chunks of K.Q^T
 	constexpr int NDB  = DP / 32;             // 32-row blocks of O^T
 	constexpr int TERM = F32_KT * DP * 2;     // bytes of one term of a tile
@@ -561,7 +561,7 @@ int launch(const af3_dpa_params& p, hipStream_t s) {
 	const int64_t per_cu = KS > 1 ? 1 : DP == 64 ? 2 : 4;   // workgroups a compute unit holds, by their registers
 	auto         kern = dpa_mfma_f32_kernel<DP, NW, KS>;
 	if(smem > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) return AF3_ERR_LAUNCH;
-	hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(NW * 64), smem, s, p, n_qtiles, groups, even_progress_wanted(groups * n_qtiles, 256 * per_cu));
+	hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(NW * 64), smem, s, p, n_qtiles, groups, progress_mode(groups * n_qtiles, 256 * per_cu));
 	return launch_status();
 }
 

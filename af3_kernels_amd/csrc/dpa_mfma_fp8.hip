@@ -74,7 +74,7 @@ __device__ __forceinline__ float max17(const f32x16& s, float m) {
 // KS: 1, or the number of parts that the tiles of a block of query rows are dealt to, each with wavefronts and buffers of its own
 // (for launches of few workgroups); their sums are merged through LDS at the end.
 template <int DP, bool COMP, bool ONES, int BMODE, int KS>
-__global__ void __launch_bounds__(KS * NW8 * 64) __attribute__((amdgpu_waves_per_eu(DP == 32 ? 4 : KS == 1 ? 3 : 2))) dpa_mfma_fp8_kernel(af3_dpa_params p, int n_qtiles, int n_units, int per_xcd, bool even) {
+__global__ void __launch_bounds__(KS * NW8 * 64) __attribute__((amdgpu_waves_per_eu(DP == 32 ? 4 : KS == 1 ? 3 : 2))) dpa_mfma_fp8_kernel(af3_dpa_params p, int n_qtiles, int n_units, int per_xcd, int even) {
 	constexpr int NDB      = DP / 32;       // 32-row blocks of O^T
 	constexpr int K_TILE1  = KT8 * DP;      // bytes of one K tile
 	constexpr int K_TILE   = K_TILE1 * (COMP ? 2 : 1);  // hi tile followed by the residual tile
@@ -629,7 +629,7 @@ int launch8_parts(const af3_dpa_params& p, hipStream_t s) {
 	const int64_t per_cu = by_lds < 1 ? 1 : by_lds < by_regs ? by_lds : by_regs;
 	auto         kern = dpa_mfma_fp8_kernel<DP, COMP, ONES, BMODE, KS>;
 	if(smem > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) return AF3_ERR_LAUNCH;
-	hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(KS * NW8 * 64), smem, s, p, n_qtiles, (int)(per_xcd > 0 ? n_blocks : n_groups), (int)per_xcd, even_progress_wanted(n_groups * n_qtiles, 256 * per_cu));
+	hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(KS * NW8 * 64), smem, s, p, n_qtiles, (int)(per_xcd > 0 ? n_blocks : n_groups), (int)per_xcd, progress_mode(n_groups * n_qtiles, 256 * per_cu));
 	return launch_status();
 }
 template <int DP, bool COMP, bool ONES, int BMODE>

@@ -101,7 +101,7 @@ __global__ void __launch_bounds__(256) bias_rows_prepass_kernel(const void* __re
 constexpr bool several_query_tiles(int rows, int bmode, bool gate) { return bmode != 2 && !(gate && rows == 4); }
 template <int ROWS, int BMODE, bool GATE>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) dpa_rows_bf16_kernel(af3_dpa_params p, int n_qtiles, int64_t n_groups, int64_t b_first, int64_t b_count, int q_chunk,
-																										   int n_chunks, int n_chunked, bool even) {
+																										   int n_chunks, int n_chunked, int even) {
 	static_assert(ROWS >= 2 && ROWS <= 4, "two to four row chains per wavefront");
 	constexpr int  NW       = 4;
 	constexpr bool HAS_BIAS = BMODE != 0, SLOT = BMODE == 1, DIRECT = BMODE == 2, STAGED = BMODE == 3;
@@ -1082,8 +1082,9 @@ int launch_rows(const af3_dpa_params& p, int64_t b_first, int64_t b_count, hipSt
 	if(several_query_tiles(ROWS, BMODE, p.gate != nullptr) && p.out_dtype == AF3_BF16) plan_chunks(n_qtiles, per_xcd, chunk, parts, chunked);
 	const int64_t blocks   = (chunked * parts + (per_xcd - chunked) * n_qtiles) * 8;
 	// (by age / evenly, us: 384 x 4 x 384 x 32 62.1 / 60.5, 512 131.7 / 129.0, 768 389.8 / 383.7, 1491 2612 / 2598, 64 x 4 x 768 x 32 41.2 / 39.7, 5 x 16 x 2000 x 24
-	// 116.1 / 112.8, 400 90.2 / 91.4; many rounds of single query tiles: the grid block of 512 tokens 246 / 252, 832 511.5 / 514.9)
-	const bool even = chunked > 0 || (blocks <= 3 * 512 && even_progress_wanted(blocks, 512));
+	// 116.1 / 112.8, 400 90.2 / 91.4; many rounds of single query tiles: the grid block of 512 tokens 246 / 252, 832 511.5 / 514.9;
+	// few rounds with a short last one, by age / last round first: 80 x 4 x 768 x 32 44.6 / 43.3, 150 x 4 x 384 x 32 27.3 / 25.7)
+	const int even = chunked > 0 ? EVENLY : blocks <= 3 * 512 ? progress_mode(blocks, 512) : BY_AGE;
 	if(blocks <= 0 || blocks > 0x7fffffffLL) return AF3_ERR_BAD_SHAPE;
 	const size_t n_t_all = (size_t)((p.L + KT_R - 1) / KT_R);
 	const size_t smem    = (size_t)NBUF_R * ROWS * 2 * TILE_R + (BMODE == 1 || BMODE == 3 ? 4 * 4096 : 0) + (n_t_all + 1) * ROWS * 32 * 2;

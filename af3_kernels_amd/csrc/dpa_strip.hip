@@ -430,7 +430,7 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 			// (tile t + 2) in slot c, V (t + 1) in slot 1, K and the biases' last dwords (t + 2) at the end.  The waits count the loads younger than what is read next.
 			int half = 0;
 			int i = 0;
-			even_progress progress(my_n, true);   // (the wavefronts meet only at the end.  16 heads of 24, by age / evenly: 768 7.95 / 7.85 us, 1280 14.38 / 14.21; of 48, 1536 20.28 / 20.02)
+			even_progress progress(my_n, EVENLY);   // (the wavefronts meet only at the end.  16 heads of 24, by age / evenly: 768 7.95 / 7.85 us, 1280 14.38 / 14.21; of 48, 1536 20.28 / 20.02)
 			auto tile = [&]() __attribute__((always_inline)) {
 				progress.at(i);
 				const int other = NB * 1024 - half;

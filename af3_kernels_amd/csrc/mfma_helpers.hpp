@@ -25,11 +25,11 @@ using ic = std::integral_constant<int, V>;
 
 // Wavefronts that share a SIMD are served oldest first: of four equal workgroups of a compute unit that start together the first is done after little more
 // than half the time (32, 41, 49 and 57 us in the fp8 kernel at 5 x 16 x 1536 x 24) and the last one walks its end alone, which keeps no pipe busy.  A
-// wavefront that lowers its priority with every quarter of its walk lets those behind it catch up; they end together.
+// wavefront that lowers its priority with every quarter of its walk lets those behind it catch up; they end together ...
 struct even_progress {
 	int quarter, next, level;
-	__device__ __forceinline__ even_progress(int steps, bool wanted) : quarter((steps + 3) >> 2), next(wanted ? quarter : 0x7fffffff), level(3) {
-		if(wanted) __builtin_amdgcn_s_setprio(3);
+	__device__ __forceinline__ even_progress(int steps, int from) : quarter((steps + 3) >> 2), next(from < 0 ? quarter : 0x7fffffff), level(3) {
+		if(from < 0 || (int)blockIdx.x >= from) __builtin_amdgcn_s_setprio(3);
 	}
 	__device__ __forceinline__ void at(int step) {   // (wave-uniform)
 		if(step >= next) {
@@ -40,13 +40,17 @@ struct even_progress {
 		}
 	}
 };
-// ... where the last of the launch's rounds is full enough: workgroups that end together leave a short last round nothing to overlap with, those that end
-// one after the other let it start early.  Served by age / evenly, us, by rounds of the fp32 kernel (B x 4 x 768 x 32): 0.94 85.7 / 82.4, 1.03 106.0 / 112.2,
-// 1.13 107.1 / 111.8, 1.22 108.8 / 112.0, 1.31 123.2 / 121.3, 1.41 125.6 / 123.9, 1.69 149.0 / 145.3, 1.88 166.3 / 160.9, 2.02 184.2 / 192.5, 2.34 207.3 / 206.8,
-// 3.0 258.0 / 251.4; of the fp8 kernel (B x 16 x 1536 x 24): 0.94 68.6 / 64.4, 1.13 82.8 / 87.1, 1.31 94.2 / 93.0, 1.5 98.8 / 97.4, 2.25 142.2 / 146.9.
-inline bool even_progress_wanted(int64_t workgroups, int64_t slots) {
+// ... in launches of whole rounds of workgroups, or with a last one that is more than half full.  Workgroups that end together leave a short last round nothing to
+// overlap with: there the earlier rounds go by age, so that places come free one after the other, and the workgroups of the last round, the last to
+// start, go before all others on their SIMD.  By rounds (1024 workgroups each), us, of the fp32 kernel (B x 4 x 768 x 32) by age / evenly: 0.94 85.7 / 82.4,
+// 1.03 106.0 / 112.2, 1.69 149.0 / 145.3, 1.88 166.3 / 160.9, 3.0 258.0 / 251.4; by age / last round first: 1.03 105.3 / 97.8, 1.13 105.8 / 99.3;
+// evenly / last round first: 1.31 120.0 / 119.7, 1.41 123.1 / 122.8, 1.5 128.0 / 127.1, 1.69 149.3 / 149.3, 1.78 155.0 / 163.8, 1.88 159.6 / 171.7,
+// 2.34 205.6 / 202.2, 2.58 221.0 / 225.5.  Of the fp8 kernel (B x 16 x 1536 x 24) by age / evenly: 0.94 68.6 / 64.4; by age / last round first: 1.13 81.6 / 76.1,
+// 2.25 139.4 / 137.3; evenly / last round first: 1.31 92.0 / 90.5, 1.5 96.5 / 95.7, 1.88 116.7 / 123.3, 2.44 152.3 / 148.1.
+constexpr int EVENLY = -1, BY_AGE = 0x7fffffff;
+inline int progress_mode(int64_t workgroups, int64_t slots) {   // EVENLY, or the first workgroup of the last round
 	const int64_t last = workgroups % slots;
-	return last == 0 || last * 7 > slots * 2;
+	return last == 0 || last * 2 > slots ? EVENLY : (int)(workgroups - last);
 }
 
 // ---- LDS layout -----------------------------------------------------------------------------
