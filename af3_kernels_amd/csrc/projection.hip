@@ -13,8 +13,8 @@
 // rows spread over the banks.  out^T = W . x^T on v_mfma_f32_32x32x16_bf16: a lane holds four times four consecutive columns
 // of one token, the accumulators start from the row, and the result leaves through a patch of LDS per wavefront as whole
 // 16-byte stores.
-// us per call, this kernel / hipBLASLt (device time, graph replays), K = 768, N = 3072: M = 64 4.6/5.6, 256 4.9/6.6, 768 8.2/10.0,
-// 1024 9.0/11.0, 1536 11.7/12.3, 2048 13.5/15.0, 3840 25.9/22.7; K = 384, N = 1536: 64 3.4/4.9, 1024 4.4/6.8, 2048 6.8/9.2,
+// us per call, this kernel / hipBLASLt (device time, graph replays), K = 768, N = 3072: M = 64 4.6/5.6, 256 4.9/6.6, 768 7.9/10.0,
+// 1024 8.6/11.0, 1536 11.7/12.3, 2048 13.5/15.0, 3840 25.9/22.7; K = 384, N = 1536: 64 3.4/4.9, 1024 4.4/6.8, 2048 6.5/9.2,
 // 7680 17.9/22.7.  The library keeps what is larger than that (af3_project_suits).
 #include "mfma_helpers.hpp"
 
@@ -176,11 +176,13 @@ extern "C" int af3_project(const void* x, const void* w, const void* row, void* 
 	// The smallest tile whose workgroups fit the 256 compute units in one round: what a call takes is the time of one workgroup
 	// (fixed part 2.3 us; per slab of 64 channels 0.20, 0.24, 0.33, 0.40, 0.50 us for these five) until there are two rounds.
 	if(form == 0) form = fits(64, 64) ? 11 : fits(128, 64) ? 21 : fits(64, 192) ? 13 : fits(128, 128) ? 22 : 23;
+	// Three slabs in the ring everywhere.  A fourth asks for more at the start than arrives before it is needed: 64 x 192 columns, four / three, us: 1024 x 3072 x 768
+	// 8.96 / 8.61, 2048 x 1536 x 384 6.72 / 6.48, 300 x 1536 x 384 5.24 / 5.02; 128 x 128 columns, 512 x 3072 x 768 8.64 / 8.47.  Two stand still: 11.4 us for the first.
 	switch(form) {
 	case 11: return launch<1, 1, 3>(xp, wp, rp, op, (int)M, (int)N, (int)K, s);
 	case 21: return launch<2, 1, 3>(xp, wp, rp, op, (int)M, (int)N, (int)K, s);
-	case 13: return launch<1, 3, 4>(xp, wp, rp, op, (int)M, (int)N, (int)K, s);
-	case 22: return launch<2, 2, 4>(xp, wp, rp, op, (int)M, (int)N, (int)K, s);
+	case 13: return launch<1, 3, 3>(xp, wp, rp, op, (int)M, (int)N, (int)K, s);
+	case 22: return launch<2, 2, 3>(xp, wp, rp, op, (int)M, (int)N, (int)K, s);
 	case 23: return launch<2, 3, 3>(xp, wp, rp, op, (int)M, (int)N, (int)K, s);
 	}
 	return AF3_ERR_BAD_ARGUMENT;
