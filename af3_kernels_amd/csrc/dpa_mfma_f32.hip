@@ -13,7 +13,7 @@
 // times 10 1.6e-7..2.3e-7 / 1.9e-7..3.8e-7, biases that grow by 40 along the row 2.1e-7..5.4e-7 / 3.0e-7..5.2e-7 (fewer, deeper
 // instructions round the accumulator less often).  Rows whose biases carry an offset of some hundreds or thousands: 0.14 to 1.41
 // times the fp32 instructions', by where the offset lies between two powers of two in either domain.
-// Measured (64 x 4 x 768 x 32): 234 us with the fp32 instructions (53 % of their peak), 131 to 139 us by card in this form.
+// Measured (64 x 4 x 768 x 32): 234 us with the fp32 instructions (53 % of their peak), 131 to 138 us by card in this form.
 //
 // Same transposed formulation as the bf16 kernel: S^T[key][q] = K.Q^T, so that in the 32x32
 // accumulator layout a lane (q = lane%32, half = lane/32) holds 16 keys of ONE query row

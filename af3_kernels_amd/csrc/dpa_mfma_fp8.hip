@@ -31,8 +31,8 @@
 //   * 39 KB of LDS and 128 registers: four workgroups of four wavefronts per compute unit.
 //   * Workgroups in an order that lets batch rows share the bias, tiles in two parts where workgroups are few: see launch8_parts, launch8.
 // us per call with its two quantising launches (6 to 13 us), 16 heads of 24, 16-deep products / these forms, workgroups by heads and one part / now:
-// 5x1536 89.0/71.3/64.5, 8x1536 133.6/104.9/98.8, 8x1301 (ragged rows) -/101.7/97, 8x1000 66.7/54.2/54, 5x300 37.9/20.3/17.5, 1x1536 42.1/34.2/27.6 (cards
-// differ: 5x1536 68 to 71).  Measured on the way: with the bias streamed once per batch row its loads were 13 us of 57 at 5x1536, the exponentials 4; four workgroups per compute unit instead of three changed nothing, nor did
+// 5x1536 89.0/71.3/63.6, 8x1536 133.6/104.9/97.0, 8x1301 (ragged rows) -/101.7/93.2, 8x1000 66.7/54.2/49.7, 5x300 37.9/20.3/17.1, 1x1536 42.1/34.2/26.3 (cards
+// differ: 5x1536 63 to 66).  Measured on the way: with the bias streamed once per batch row its loads were 13 us of 57 at 5x1536, the exponentials 4; four workgroups per compute unit instead of three changed nothing, nor did
 // pinning the matrix instructions between the exponentials: the vector port is busy three quarters of the time.
 #include "mfma_helpers.hpp"
 

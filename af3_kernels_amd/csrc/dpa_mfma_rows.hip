@@ -1029,7 +1029,7 @@ bool staged_bias_ok(const af3_dpa_params& p) {
 // Staging the bf16 bias costs each step 8 vector instructions (widening it) that the fp32 workspace does not -- about 5 % of
 // the kernel's time -- the workspace a prepass over the whole bias (about 3 us + 0.46 us per MB read and written) and twice
 // the bytes per tile.  Staged / workspace, us, prepass included: 32 x 16 x 1536 x 24 245 / 299, 64 x 4 x 768 x 32 50 / 55,
-// 128 x 4 x 768 x 32 90 / 91, 192 x 4 x 768 x 32 117 / 118, 384 x 4 x 384 x 32 60 / 62, 768 x 4 x 768 x 32 425 / 416.
+// 200 119 / 124, 256 132 / 131, 288 177 / 182, 512 263 / 257, 768 390 / 379, 384 x 4 x 384 x 32 60.2 / 60.3, 560 102 / 104, 640 102 / 101, 1024 160 / 156.
 // The prepass is worth its time from about 224 + 2.4e8 / (H L^2) batch rows on (the second term: its fixed cost against the
 // time of one batch row).
 constexpr int64_t STAGED_MAX_B_SMALL = 128;  // below this the kernel is taken for launches the one-row kernel would otherwise serve

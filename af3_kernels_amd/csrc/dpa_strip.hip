@@ -430,9 +430,13 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 			// (tile t + 2) in slot c, V (t + 1) in slot 1, K and the biases' last dwords (t + 2) at the end.  The waits count the loads younger than what is read next.
 			int half = 0;
 			int i = 0;
-			even_progress progress(my_n, EVENLY);   // (the wavefronts meet only at the end.  16 heads of 24, by age / evenly: 768 7.95 / 7.85 us, 1280 14.38 / 14.21; of 48, 1536 20.28 / 20.02)
+			// (The wavefronts meet only at the end.  16 heads of 24, by age / evenly: 700 7.80 / 7.71 us, 1001 11.71 / 11.38, 1280 14.50 / 14.27; of 48, 1536 21.60 / 21.47;
+			// but with one to three tiles to a wavefront 346 5.00 / 5.10, 560 6.47 / 6.56, 256 of 48 4.83 / 4.88.  Strips of one block have no more, and head_dim 25 to 32 comes
+			// as triangles of few tokens: there not even the question is asked.)
+			constexpr bool EVEN = NB > 1 && KIND != 1;
+			even_progress progress(my_n, EVEN && my_n > 2 ? EVENLY : BY_AGE);
 			auto tile = [&]() __attribute__((always_inline)) {
-				progress.at(i);
+				if constexpr(EVEN) progress.at(i);
 				const int other = NB * 1024 - half;
 				constexpr int K_SLOT = NB > 2 ? NB - 2 : NB - 1;
 				v_rsrc[2] = i + 1 < my_n ? v_bytes : 0u;

@@ -26,10 +26,10 @@ using ic = std::integral_constant<int, V>;
 // Wavefronts that share a SIMD are served oldest first: of four equal workgroups of a compute unit that start together the first is done after little more
 // than half the time (32, 41, 49 and 57 us in the fp8 kernel at 5 x 16 x 1536 x 24) and the last one walks its end alone, which keeps no pipe busy.  A
 // wavefront that lowers its priority with every quarter of its walk lets those behind it catch up; they end together ...
-struct even_progress {
+struct even_progress {   // from: EVENLY, BY_AGE or the first workgroup that goes before all others (below)
 	int quarter, next, level;
 	__device__ __forceinline__ even_progress(int steps, int from) : quarter((steps + 3) >> 2), next(from < 0 ? quarter : 0x7fffffff), level(3) {
-		if(from < 0 || (int)blockIdx.x >= from) __builtin_amdgcn_s_setprio(3);
+		if(from < 0 || (from != 0x7fffffff && (int)blockIdx.x >= from)) __builtin_amdgcn_s_setprio(3);
 	}
 	__device__ __forceinline__ void at(int step) {   // (wave-uniform)
 		if(step >= next) {
