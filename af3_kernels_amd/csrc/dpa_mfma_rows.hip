@@ -95,17 +95,20 @@ __global__ void __launch_bounds__(256) bias_rows_prepass_kernel(const void* __re
 // 2's cache-line requests, whose lanes each fetch from a row of their own).
 // The launch covers batch rows [b_first, b_first + b_count) in groups of ROWS.
 // GATE: out *= sigmoid(gate) in the epilogue.
-// Per XCD the first n_chunked (group, head) pairs are cut into n_chunks workgroups of q_chunk query tiles, the others into workgroups of one.
-// Whether workgroups may walk several query tiles.  Four batch rows and their gates do not fit the registers between two query tiles (14 spilled ones: the
+// MULTI: workgroups may walk several query tiles; per XCD the first n_chunked (group, head) pairs are cut into n_chunks workgroups of q_chunk query tiles, the
+// others into workgroups of one.  Launches of single query tiles take the form without: with the code of the longer walk in it (10 KB more, scalar and,
+// with four rows, 7 vector registers spilled) they took, us, that code in / out: 512 x 4 x 128 x 32 25.2 / 23.9, 1024 38.4 / 37.0, 1536 50.2 / 47.4, 1000 x 4 x 64 x 32
+// 26.4 / 24.9, 512 x 8 x 256 x 32 on packed rows 110.1 / 94.5.
+// Whether there is such a form.  Four batch rows and their gates do not fit the registers between two query tiles (14 spilled ones: the
 // grid block of 768 tokens 637 -> 655 us; with one query tile to a workgroup 633), the in-place form has not been given it.
 constexpr bool several_query_tiles(int rows, int bmode, bool gate) { return bmode != 2 && !(gate && rows == 4); }
-template <int ROWS, int BMODE, bool GATE>
+template <int ROWS, int BMODE, bool GATE, bool MULTI>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) dpa_rows_bf16_kernel(af3_dpa_params p, int n_qtiles, int64_t n_groups, int64_t b_first, int64_t b_count, int q_chunk,
 																										   int n_chunks, int n_chunked, int even) {
 	static_assert(ROWS >= 2 && ROWS <= 4, "two to four row chains per wavefront");
+	static_assert(!MULTI || several_query_tiles(ROWS, BMODE, GATE), "no such form");
 	constexpr int  NW       = 4;
 	constexpr bool HAS_BIAS = BMODE != 0, SLOT = BMODE == 1, DIRECT = BMODE == 2, STAGED = BMODE == 3;
-	constexpr bool MULTI    = several_query_tiles(ROWS, BMODE, GATE);
 	constexpr int  BUF_R    = ROWS * 2 * TILE_R;                    // one buffer: [row][K tile | V tile]
 	constexpr int  SLOT_BASE = NBUF_R * BUF_R;                      // per-wavefront bias slots (4 KB each)
 	constexpr int  MASK_BASE = SLOT_BASE + (SLOT || STAGED ? NW * 4096 : 0);
@@ -130,13 +133,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 	asm volatile("" ::"s"(p.q_stride[0]), "s"(p.q_stride[1]), "s"(p.q_stride[2]), "s"(p.k_stride[0]), "s"(p.k_stride[1]), "s"(p.k_stride[2]), "s"(p.v_stride[0]), "s"(p.v_stride[1]),
 				 "s"(p.v_stride[2]));
 	// (32-bit divisions: a 64-bit one is 150 instructions, i.e. 700 clocks of a start that waits for them)
-	const uint32_t slot = blockIdx.x >> 3, chunked = (uint32_t)n_chunked * (uint32_t)n_chunks;
-	const bool     single = slot >= chunked;
+	const uint32_t slot = blockIdx.x >> 3, chunked = MULTI ? (uint32_t)n_chunked * (uint32_t)n_chunks : 0u;
+	const bool     single = !MULTI || slot >= chunked;
 	const uint32_t s_rel = single ? slot - chunked : slot, parts = single ? (uint32_t)n_qtiles : (uint32_t)n_chunks, q_div = s_rel / parts;
-	const uint32_t group = (q_div + (single ? (uint32_t)n_chunked : 0u)) * 8 + (blockIdx.x & 7);
+	const uint32_t group = (q_div + (MULTI && single ? (uint32_t)n_chunked : 0u)) * 8 + (blockIdx.x & 7);
 	if(group >= (uint32_t)n_groups) return;
 	const int chunk = single ? 1 : q_chunk, qtile0 = (int)(s_rel - q_div * parts) * chunk;
-	const int n_q   = qtile0 + chunk <= n_qtiles ? chunk : n_qtiles - qtile0;   // query tiles of this workgroup
+	const int n_q   = !MULTI ? 1 : qtile0 + chunk <= n_qtiles ? chunk : n_qtiles - qtile0;   // query tiles of this workgroup
 	const int64_t g = group / (uint32_t)p.H, h = group - (uint32_t)g * (uint32_t)p.H;
 	const int64_t b0 = b_first + g * ROWS, b_end = b_first + b_count;   // (rows past b_end repeat the last one and are not stored)
 
@@ -1088,7 +1091,13 @@ int launch_rows(const af3_dpa_params& p, int64_t b_first, int64_t b_count, hipSt
 	if(blocks <= 0 || blocks > 0x7fffffffLL) return AF3_ERR_BAD_SHAPE;
 	const size_t n_t_all = (size_t)((p.L + KT_R - 1) / KT_R);
 	const size_t smem    = (size_t)NBUF_R * ROWS * 2 * TILE_R + (BMODE == 1 || BMODE == 3 ? 4 * 4096 : 0) + (n_t_all + 1) * ROWS * 32 * 2;
-	auto         kern    = p.gate ? dpa_rows_bf16_kernel<ROWS, BMODE, true> : dpa_rows_bf16_kernel<ROWS, BMODE, false>;
+	auto         kern    = p.gate ? dpa_rows_bf16_kernel<ROWS, BMODE, true, false> : dpa_rows_bf16_kernel<ROWS, BMODE, false, false>;
+	if(chunked > 0) {
+		if constexpr(several_query_tiles(ROWS, BMODE, true))
+			if(p.gate) kern = dpa_rows_bf16_kernel<ROWS, BMODE, true, true>;
+		if constexpr(several_query_tiles(ROWS, BMODE, false))
+			if(!p.gate) kern = dpa_rows_bf16_kernel<ROWS, BMODE, false, true>;
+	}
 	if(smem > 63 * 1024) {   // (the kernel's static words take 1 KB of the 64 that need no asking: smem's alignment)
 		if(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) return AF3_ERR_LAUNCH;
 	}

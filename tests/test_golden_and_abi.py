@@ -5,6 +5,7 @@ import ctypes
 import glob
 import os
 import re
+import subprocess
 
 import numpy as np
 import pytest
@@ -573,3 +574,32 @@ def test_hand_written_barriers_wait_for_lds_reads():
             if n:
                 bare[name] = n
     assert bare == {"dpa_mfma_rows.hip": 2, "projection.hip": 2}
+
+
+def _kernel_registers(tmp_path):
+    """name -> (spilled vector registers, vector registers) of every kernel in the built library, from its code objects' metadata."""
+    from af3_kernels_amd import build as hip_build
+    readelf = os.path.join(os.path.dirname(os.path.dirname(os.path.realpath(hip_build.HIPCC))), "llvm", "bin", "llvm-readelf")
+    if not os.path.exists(readelf):
+        pytest.skip("no llvm-readelf")
+    data = open(hip_build.LIB, "rb").read()
+    found = {}
+    for m in re.finditer(b"\x7fELF", data):
+        if m.start() == 0:
+            continue   # the host library itself
+        path = tmp_path / "code"
+        path.write_bytes(data[m.start():])
+        notes = subprocess.run([readelf, "--notes", str(path)], capture_output=True, text=True).stdout
+        for kernel in notes.split("- .agpr_count")[1:]:
+            field = lambda key: re.search(rf"\.{key}: +(\S+)", kernel).group(1)
+            found[field("symbol")] = int(field("vgpr_spill_count")), int(field("vgpr_count"))
+    return found
+
+
+def test_forms_for_single_query_tiles_spill_no_vector_registers(tmp_path):
+    """The shared-bias kernel's forms for workgroups of one query tile carry nothing of the longer walks: with it in them some spilled, and
+    launches of short rows took up to 14 % longer."""
+    kernels = {n: r for n, r in _kernel_registers(tmp_path).items() if "dpa_rows_bf16_kernelILi" in n}
+    single = {n: r for n, r in kernels.items() if re.search(r"ILi\dELi\dELb[01]ELb0EE", n)}
+    assert len(single) == 24 and len(kernels) == 24 + 15   # rows x bias modes x gate; without mode 2 and without four rows and a gate
+    assert {n: r for n, r in single.items() if r[0]} == {}
