@@ -65,8 +65,8 @@ struct strip_lds {
 };
 
 // KIND: 0 = head_dim up to 24 (row sums in V's column 24), 1 = 32, 2 = 40 and 48 (two contraction steps).  Grid: x = head (with a multiple of 8 heads the strips of one head share an XCD and
-// its L2 copy of K and V), y = strip, z = batch row.
-template <int NB, int KIND, bool ANY, int NW>
+// its L2 copy of K and V), y = strip, z = batch row.  EVEN: wavefronts that are behind on their walk go first (goes_evenly).
+template <int NB, int KIND, bool ANY, int NW, bool EVEN>
 __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) dpa_strip_bf16_kernel(strip_args p) {
 	using lds = strip_lds<NB, KIND, ANY, NW>;
 	static_assert(NB <= 4, "the walk has four slots a tile");
@@ -430,10 +430,6 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 			// (tile t + 2) in slot c, V (t + 1) in slot 1, K and the biases' last dwords (t + 2) at the end.  The waits count the loads younger than what is read next.
 			int half = 0;
 			int i = 0;
-			// (The wavefronts meet only at the end.  16 heads of 24, by age / evenly: 700 7.80 / 7.71 us, 1001 11.71 / 11.38, 1280 14.50 / 14.27; of 48, 1536 21.60 / 21.47;
-			// but with one to three tiles to a wavefront 346 5.00 / 5.10, 560 6.47 / 6.56, 256 of 48 4.83 / 4.88.  Strips of one block have no more, and head_dim 25 to 32 comes
-			// as triangles of few tokens: there not even the question is asked.)
-			constexpr bool EVEN = NB > 1 && KIND != 1;
 			even_progress progress(my_n, EVEN && my_n > 2 ? EVENLY : BY_AGE);
 			auto tile = [&]() __attribute__((always_inline)) {
 				if constexpr(EVEN) progress.at(i);
@@ -613,12 +609,23 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 
 }  // namespace
 
+// A strip's wavefronts meet only at its end; served by age, those that share a SIMD end one after the other.  The even walk pays from 2.5 tiles to a wavefront
+// on where one strip fills a compute unit, from more than two where two strips do; with fewer, its code costs more than it brings (the kernel's time is its
+// instructions), and the forms for those have none of it.  16 heads, us, without / with: one row of head_dim 24 560 5.92 / 5.98, 640 5.93 / 6.00,
+// 672 6.52 / 6.45, 704 6.56 / 6.48, 768 6.63 / 6.52, 1001 9.92 / 9.66, 1280 14.66 / 14.30; of 48 300 5.65 / 5.69, 640 7.41 / 7.51, 768 8.25 / 8.18; two strips to a
+// compute unit: 3 rows x 264 x 48 6.98 / 6.82, 4 x 264 x 24 6.54 / 6.41, 5 x 271 x 48 8.94 / 8.61, 4 x 320 x 48 8.59 / 8.44.  Strips of one block have no more
+// than two tiles, and head_dim 25 to 32 comes as triangles of few tokens.
+constexpr bool may_go_evenly(int nb, int kind) { return nb > 1 && kind != 1; }
+static bool goes_evenly(int64_t L, int nw) { return (L + KT_S - 1) / KT_S > (nw == 4 ? 8 : 20); }
+
 template <int NB, int KIND, bool ANY, int NW>
 static int launch_strip_n(const af3_dpa_params& p, hipStream_t s) {
 	using lds = strip_lds<NB, KIND, ANY, NW>;
 	constexpr int R    = lds::R;
 	const int     smem = lds::bytes((int)p.L);
-	auto          kern = dpa_strip_bf16_kernel<NB, KIND, ANY, NW>;
+	auto          kern = dpa_strip_bf16_kernel<NB, KIND, ANY, NW, false>;
+	if constexpr(may_go_evenly(NB, KIND))
+		if(goes_evenly(p.L, NW)) kern = dpa_strip_bf16_kernel<NB, KIND, ANY, NW, true>;
 	if(smem > 64 * 1024) {   // beyond the default limit: raise it for this kernel (the call costs the host 0.7 us)
 		if(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem) != hipSuccess) return AF3_ERR_LAUNCH;
 	}

@@ -603,3 +603,41 @@ def test_forms_for_single_query_tiles_spill_no_vector_registers(tmp_path):
     single = {n: r for n, r in kernels.items() if re.search(r"ILi\dELi\dELb[01]ELb0EE", n)}
     assert len(single) == 24 and len(kernels) == 24 + 15   # rows x bias modes x gate; without mode 2 and without four rows and a gate
     assert {n: r for n, r in single.items() if r[0]} == {}
+
+
+def _kernel_sizes(tmp_path):
+    """name -> bytes of code of every kernel in the built library."""
+    from af3_kernels_amd import build as hip_build
+    readelf = os.path.join(os.path.dirname(os.path.dirname(os.path.realpath(hip_build.HIPCC))), "llvm", "bin", "llvm-readelf")
+    if not os.path.exists(readelf):
+        pytest.skip("no llvm-readelf")
+    data = open(hip_build.LIB, "rb").read()
+    found = {}
+    for m in re.finditer(b"\x7fELF", data):
+        if m.start() == 0:
+            continue   # the host library itself
+        path = tmp_path / "code"
+        path.write_bytes(data[m.start():])
+        for line in subprocess.run([readelf, "-sW", str(path)], capture_output=True, text=True).stdout.splitlines():
+            f = line.split()
+            if len(f) >= 8 and f[3] == "FUNC":
+                found[f[7]] = int(f[2], 0)
+    return found
+
+
+def test_strips_of_short_walks_carry_no_priorities(tmp_path):
+    """The strip kernel's forms for walks of few tiles to a wavefront hold none of the code that lets wavefronts behind on theirs go first:
+    their time is their instructions.  (Strips of two blocks of rows and more, head_dim up to 24 and from 33 on, have both forms; the others one.)"""
+    sizes = {}
+    for name, size in _kernel_sizes(tmp_path).items():
+        m = re.search(r"dpa_strip_bf16_kernelILi(\d)ELi(\d)ELb([01])ELi(\d)ELb([01])EE", name)
+        assert m or "dpa_strip_bf16_kernel" not in name, name
+        if m:
+            nb, kind, odd, nw, even = map(int, m.groups())
+            sizes[nb, kind, odd, nw, even] = size
+    forms = [f[:4] for f in sizes if f[4] == 0]
+    assert len(forms) == 3 * 6 * 2 + 3
+    for f in forms:
+        without, with_it = sizes[f + (0,)], sizes.get(f + (1,))
+        assert (with_it is not None) == (f[0] > 1 and f[1] != 1)
+        assert with_it is None or with_it >= without + 400

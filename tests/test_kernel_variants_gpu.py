@@ -787,3 +787,23 @@ def test_strips(af3, oracle, B, H, L, D, kind):
     want = oracle.dpa_formula(f32np(q), f32np(k), f32np(v), keep.numpy(), f32np(bias)) if kind != "v inf" else oracle.dpa_formula(f32np(q), f32np(k), f32np(torch.nn.functional.pad(v, (0, 1))), keep.numpy(), f32np(bias))[..., : D - 1]
     # (a bias of -120 or 100 leaves its logit steps of 2^-17 or finer; 2e-2 is bf16's budget)
     assert np.abs(out - want).max() <= 2e-2
+
+
+@pytest.mark.parametrize("B,H,L,D", [(1, 16, 640, 24), (1, 16, 641, 24), (1, 16, 672, 48), (1, 16, 641, 40), (1, 16, 255, 24), (3, 16, 257, 24), (3, 16, 289, 48)])   # 20 and 21 tiles for eight wavefronts, 8 to 10 for four
+@pytest.mark.parametrize("kind", ["random", "three tiles", "one"])
+def test_strips_on_both_sides_of_the_even_walk(af3, oracle, B, H, L, D, kind):
+    """The forms whose wavefronts go by age and those in which the ones behind go first, with few live tiles too."""
+    g = torch.Generator().manual_seed(L + D)
+    q, k, v = (torch.randn(B, H, L, D, generator=g).to(torch.bfloat16) for _ in range(3))
+    bias = torch.randn(H, L, L, generator=g).to(torch.bfloat16)
+    keep = torch.rand(B, L, generator=g) < 0.8
+    keep[:, 0] = True
+    if kind != "random":
+        keep[:, 96 if kind == "three tiles" else 1:] = False
+    prev = af3.set_rows_kernel("never")
+    try:
+        print("case", B, H, L, D, kind, flush=True)
+        out = f32np(af3.dot_product_attention_cpp(q.cuda(), k.cuda(), v.cuda(), keep.cuda(), bias.cuda()))
+    finally:
+        af3.set_rows_kernel(prev)
+    assert np.abs(out - oracle.dpa_formula(f32np(q), f32np(k), f32np(v), keep.numpy(), f32np(bias))).max() <= 2e-2   # (bf16's budget)
