@@ -99,6 +99,17 @@ extern "C" int64_t af3_dpa_workspace_used(const af3_dpa_params* params) {
 // ... and which must know, before it lays out q, whether the kernel that will serve this call takes its logits in units of log2 e.
 extern "C" int af3_dpa_log2_domain(const af3_dpa_params* params) { return validate(params) == AF3_OK && select_kernel(*params) == 1 && mfma_bf16_log2_domain(*params) ? 1 : 0; }
 
+// For tests: how the shared-bias kernel would lay this call out (mfma_rows_plan); no pointer is followed.
+extern "C" int af3_dpa_rows_plan(const af3_dpa_params* params, int64_t (*plan)[5]) {
+	const int rc = validate(params);
+	if(rc != AF3_OK) return rc;
+	int64_t   found[3][5];
+	const int n = select_kernel(*params) == 1 ? mfma_bf16_rows_plan(*params, found) : 0;
+	for(int i = 0; i < n; i++)
+		for(int j = 0; j < 5; j++) plan[i][j] = found[i][j];
+	return n;
+}
+
 extern "C" int af3_dpa_select_kernel(const af3_dpa_params* params) {
 	const int rc = validate(params);
 	if(rc != AF3_OK) return rc;

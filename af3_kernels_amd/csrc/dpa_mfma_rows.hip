@@ -1052,21 +1052,54 @@ int rows_bias_mode(const af3_dpa_params& p) {
 	return ws_ok ? 1 : -1;
 }
 
+// Lines of 128 bytes that a key's K and V rows lie in, as a sum over `count` of its heads and neighbours: one to a key where rows follow one another or K and V of a
+// head share a line, two where they are views of [.., heads, 32] or of a packed projection, more where rows straddle lines.
+struct kv_lines {
+	int64_t sum = 0, count = 0;
+	bool    apart = true;   // K's lines hold nothing of V
+};
+kv_lines lines_of_a_key(const af3_dpa_params& p) {
+	if(p.k_stride[2] == p.D && p.v_stride[2] == p.D) return {1, 1, false};
+	kv_lines n;
+	for(int64_t h = 0; h < p.H && h < 8; h++)
+		for(int64_t key = 0; key < p.L && key < 4; key++) {
+			const uint64_t k = reinterpret_cast<uintptr_t>(p.k) + (h * p.k_stride[1] + key * p.k_stride[2]) * 2, v = reinterpret_cast<uintptr_t>(p.v) + (h * p.v_stride[1] + key * p.v_stride[2]) * 2;
+			const uint64_t k0 = k / 128, k1 = (k + p.D * 2 - 1) / 128, v0 = v / 128, v1 = (v + p.D * 2 - 1) / 128;
+			const bool     meet = k0 <= v1 && v0 <= k1;
+			n.sum += meet ? (k1 > v1 ? k1 : v1) - (k0 < v0 ? k0 : v0) + 1 : k1 - k0 + v1 - v0 + 2;
+			n.apart = n.apart && !meet;
+			n.count++;
+		}
+	return n;
+}
+
 // How many query tiles a workgroup walks.  Its start and its end (masks, first tiles, q, the stores' way out) are paid once, but workgroups of several
 // query tiles come in fewer rounds of the 64 an XCD holds (two per compute unit), and query tiles that are walked one behind the other read K and V
 // from the L2 at different times, where neighbours read them together: a divisor of the number of query tiles up to 4, one that leaves whole rounds (or nearly: 349 x 4 x 349 x 32
 // 55.6 one each, 51.0 in 0.92 of a round of three, 56.4 ending in single ones)
 // where there is one, else the smallest; what does not make whole rounds ends in a round of single query tiles.  Five and
-// eleven query tiles go as 2 2 1 and 3 3 3 2; seven gained nothing.  us, one query tile each / so, one card, L x 4 x L x 32: 300 44.5 / 41.2, 384 61.0 / 59.5,
+// eleven query tiles go as 2 2 1 and 3 3 3 2.  us, one query tile each / so, one card, L x 4 x L x 32: 300 44.5 / 41.2, 384 61.0 / 59.5,
 // 400 97.8 / 89.6, 512 127.5 / 122.6, 600 204.5 / 200.5, 640 237.5 / 230.0, 768 393.8 / 377.3, 1024 874 / 841, 1200 1437 / 1397, 1300 1847 / 1813,
 // 1491 2643 / 2564; 2048 x 4 x 256 x 32 165.9 / 162.1, 512 x 4 x 768 x 24 242.6 / 234.3; larger chunks of more query tiles: 1491 in chunks of 12 3521, of 6 2802, of 3 2704.
-void plan_chunks(int n_qtiles, int64_t per_xcd, int& chunk, int& parts, int64_t& chunked) {
+// Seven and thirteen tiles stay single: one each / in twos / threes / fours 832 507 / 535 / 521 / 565, 896 608 / 618 / 621 / 637, 300 x 4 x 1600 x 32 637 / 655 / 660 / 726.
+// Every tile that a workgroup walks behind the first fetches K and V once more, in whole lines.  Where a line holds rows of other heads too, that costs more than it saves
+// unless so many workgroups still walk a head side by side that its lines are fetched no oftener than those of dense rows are when one workgroup walks all its tiles.
+// us, one tile each / in chunks: [.., 4 heads, 32] 384 67.1 / 83.6 (all three in one workgroup), 512 142.5 / 135.5 (two of four), 768 445.0 / 431.0 (three of six),
+// packed 512 157.8 / 144.8, 1000 994 / 1016 (four of eight) / 956 (two), 640 273 / 280 (2 2 1); 8 heads 512 x 256 90.8 / 116.7 (both); head_dim 24, packed 300 x 16 x 384
+// 239.6 / 371.2, 512 x 4 x 512 149.9 / 158.9 (two of four); k | v of a head in whole lines 384 64.6 / 62.2, 1000 x 4 x 150 63.9 / 53.4, across lines 96 x 16 x 768 x 24
+// 232 / 226 (two of six), 128 x 16 x 512 x 24 141 / 147 (two of four).  From 9 heads on K and V apart gain by no chunk: 128 x 16 x 512 x 32 packed 137.9 / 149.2,
+// 64 x 32 x 512 145.6 / 173.6, 64 x 16 x 1024 x 24 256.5 / 272.3 (two of eight); with 8 256 x 512 138.9 / 142.4, 200 x 512 126.2 / 120.9, 128 x 1024 234.6 / 235.7.
+void plan_chunks(const af3_dpa_params& p, int n_qtiles, int64_t per_xcd, int& chunk, int& parts, int64_t& chunked) {
 	constexpr int64_t SLOTS = 64;
 	if(per_xcd * n_qtiles <= SLOTS) return;   // (one round as it is)
+	const kv_lines lines = lines_of_a_key(p);
+	if(lines.apart && p.H > 8) return;
+	const int most = lines.apart ? 3 : 4, room = lines.sum > lines.count && p.H > 8 ? 2 : 1;
 	auto whole_rounds = [&](int c) { const int64_t last = per_xcd * ((n_qtiles + c - 1) / c) % SLOTS; return last == 0 || last > SLOTS * 9 / 10; };
-	int  c = n_qtiles == 5 ? 2 : n_qtiles == 11 ? 3 : 1;
-	for(int i = 4; i >= 2; i--)
-		if(n_qtiles % i == 0 && (c == 1 || whole_rounds(i) || !whole_rounds(c))) c = i;
+	auto few_fetches  = [&](int c) { return c * lines.sum * room <= n_qtiles * lines.count; };
+	int  c = lines.apart ? 1 : n_qtiles == 5 && few_fetches(2) ? 2 : n_qtiles == 11 && few_fetches(3) ? 3 : 1;
+	for(int i = most; i >= 2; i--)
+		if(n_qtiles % i == 0 && few_fetches(i) && (c == 1 || whole_rounds(i) || !whole_rounds(c))) c = i;
 	if(c == 1) return;
 	chunk = c, parts = (n_qtiles + c - 1) / c, chunked = per_xcd;
 	if(!whole_rounds(c)) {
@@ -1075,24 +1108,32 @@ void plan_chunks(int n_qtiles, int64_t per_xcd, int& chunk, int& parts, int64_t&
 	}
 }
 
-template <int ROWS, int BMODE>
-int launch_rows(const af3_dpa_params& p, int64_t b_first, int64_t b_count, hipStream_t s) {
-	const int     n_qtiles = (int)((p.L + 127) / 128);
-	const int64_t n_groups = ((b_count + ROWS - 1) / ROWS) * p.H;
-	const int64_t per_xcd  = (n_groups + 7) / 8;
-	int           chunk = 1, parts = n_qtiles;
-	int64_t       chunked = 0;
-	if(several_query_tiles(ROWS, BMODE, p.gate != nullptr) && p.out_dtype == AF3_BF16) plan_chunks(n_qtiles, per_xcd, chunk, parts, chunked);
-	const int64_t blocks   = (chunked * parts + (per_xcd - chunked) * n_qtiles) * 8;
+// How a launch over b_count batch rows in groups of `rows` is laid out.
+struct rows_launch {
+	int     n_qtiles, chunk, parts, even;
+	int64_t n_groups, per_xcd, chunked, blocks;
+};
+rows_launch lay_out(const af3_dpa_params& p, int rows, int bmode, int64_t b_count) {
+	rows_launch l{};
+	l.n_qtiles = (int)((p.L + 127) / 128), l.n_groups = ((b_count + rows - 1) / rows) * p.H, l.per_xcd = (l.n_groups + 7) / 8;
+	l.chunk = 1, l.parts = l.n_qtiles;
+	if(several_query_tiles(rows, bmode, p.gate != nullptr) && p.out_dtype == AF3_BF16) plan_chunks(p, l.n_qtiles, l.per_xcd, l.chunk, l.parts, l.chunked);
+	l.blocks = (l.chunked * l.parts + (l.per_xcd - l.chunked) * l.n_qtiles) * 8;
 	// (by age / evenly, us: 384 x 4 x 384 x 32 62.1 / 60.5, 512 131.7 / 129.0, 768 389.8 / 383.7, 1491 2612 / 2598, 64 x 4 x 768 x 32 41.2 / 39.7, 5 x 16 x 2000 x 24
 	// 116.1 / 112.8, 400 90.2 / 91.4; many rounds of single query tiles: the grid block of 512 tokens 246 / 252, 832 511.5 / 514.9;
 	// few rounds with a short last one, by age / last round first: 80 x 4 x 768 x 32 44.6 / 43.3, 150 x 4 x 384 x 32 27.3 / 25.7)
-	const int even = chunked > 0 ? EVENLY : blocks <= 3 * 512 ? progress_mode(blocks, 512) : BY_AGE;
-	if(blocks <= 0 || blocks > 0x7fffffffLL) return AF3_ERR_BAD_SHAPE;
+	l.even = l.chunked > 0 ? EVENLY : l.blocks <= 3 * 512 ? progress_mode(l.blocks, 512) : BY_AGE;
+	return l;
+}
+
+template <int ROWS, int BMODE>
+int launch_rows(const af3_dpa_params& p, int64_t b_first, int64_t b_count, hipStream_t s) {
+	const rows_launch l = lay_out(p, ROWS, BMODE, b_count);
+	if(l.blocks <= 0 || l.blocks > 0x7fffffffLL) return AF3_ERR_BAD_SHAPE;
 	const size_t n_t_all = (size_t)((p.L + KT_R - 1) / KT_R);
 	const size_t smem    = (size_t)NBUF_R * ROWS * 2 * TILE_R + (BMODE == 1 || BMODE == 3 ? 4 * 4096 : 0) + (n_t_all + 1) * ROWS * 32 * 2;
 	auto         kern    = p.gate ? dpa_rows_bf16_kernel<ROWS, BMODE, true, false> : dpa_rows_bf16_kernel<ROWS, BMODE, false, false>;
-	if(chunked > 0) {
+	if(l.chunked > 0) {
 		if constexpr(several_query_tiles(ROWS, BMODE, true))
 			if(p.gate) kern = dpa_rows_bf16_kernel<ROWS, BMODE, true, true>;
 		if constexpr(several_query_tiles(ROWS, BMODE, false))
@@ -1101,7 +1142,7 @@ int launch_rows(const af3_dpa_params& p, int64_t b_first, int64_t b_count, hipSt
 	if(smem > 63 * 1024) {   // (the kernel's static words take 1 KB of the 64 that need no asking: smem's alignment)
 		if(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) return AF3_ERR_LAUNCH;
 	}
-	hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), smem, s, p, n_qtiles, n_groups, b_first, b_count, chunk, parts, (int)chunked, even);
+	hipLaunchKernelGGL(kern, dim3((unsigned)l.blocks), dim3(256), smem, s, p, l.n_qtiles, l.n_groups, b_first, b_count, l.chunk, l.parts, (int)l.chunked, l.even);
 	return launch_status();
 }
 
@@ -1144,32 +1185,15 @@ bool mfma_rows_suits_a_small_batch(const af3_dpa_params& p) {
 	return wgs >= 64 || p.L < 1024;
 }
 
-int launch_dpa_mfma_rows(const af3_dpa_params& p, hipStream_t s) {
-	const int mode = rows_bias_mode(p);
-	if(mode < 0) return AF3_ERR_BAD_ARGUMENT;
-	if(mode == 1) {
-		const bool     bf32      = p.bias_dtype == AF3_F32;
-		const int      n_qblocks = (int)((p.L + 31) / 32), n_t_all = (int)((p.L + KT_R - 1) / KT_R);
-		const int64_t  total     = p.H * n_qblocks * (int64_t)n_t_all * 256;
-		if(total / 256 >= ((int64_t)1 << 31)) return AF3_ERR_BAD_SHAPE;  // (the prepass counts its units in 32 bits)
-		const unsigned g         = (unsigned)((total + 255) / 256 > 65536 ? 65536 : (total + 255) / 256);
-		if(bf32)
-			hipLaunchKernelGGL(bias_rows_prepass_kernel<true>, dim3(g), dim3(256), 0, s, p.bias, static_cast<f32x4*>(p.workspace), p.H, p.L, p.bias_stride[0], p.bias_stride[1],
-							   n_qblocks, n_t_all);
-		else
-			hipLaunchKernelGGL(bias_rows_prepass_kernel<false>, dim3(g), dim3(256), 0, s, p.bias, static_cast<f32x4*>(p.workspace), p.H, p.L, p.bias_stride[0], p.bias_stride[1],
-							   n_qblocks, n_t_all);
-		const int rc = launch_status();
-		if(rc != AF3_OK) return rc;
-	}
-	// The batch is cut into groups of `rows` batch rows per wavefront, the remainder into groups of two or three (a
-	// remainder of one borrows from the last full group); every group of one launch has the same number of rows.  Four
-	// rows share a bias tile best, but what counts is how evenly the workgroups fill the GPU's 512 slots (two per
-	// compute unit): the launch time is about (rounds of 512 workgroups) x (rows per group) x (cost per row, which grows
-	// as fewer rows share a tile: measured 1 : 1.075 : 1.09 for 4 : 3 : 2 rows), and the cheapest plan is taken.  For a
-	// small batch the cheapest plan is often ONE launch whose last group is short (its missing rows repeat the last batch
-	// row and are not stored): launches run one after the other, so 3 + 2 rows in two launches of half-empty rounds take
-	// the time of five rows, the same five rows as 3 + (2 and a repeated one) in one launch the time of three.
+// The batch is cut into groups of `rows` batch rows per wavefront, the remainder into groups of two or three (a
+// remainder of one borrows from the last full group); every group of one launch has the same number of rows.  Four
+// rows share a bias tile best, but what counts is how evenly the workgroups fill the GPU's 512 slots (two per
+// compute unit): the launch time is about (rounds of 512 workgroups) x (rows per group) x (cost per row, which grows
+// as fewer rows share a tile: measured 1 : 1.075 : 1.09 for 4 : 3 : 2 rows), and the cheapest plan is taken.  For a
+// small batch the cheapest plan is often ONE launch whose last group is short (its missing rows repeat the last batch
+// row and are not stored): launches run one after the other, so 3 + 2 rows in two launches of half-empty rounds take
+// the time of five rows, the same five rows as 3 + (2 and a repeated one) in one launch the time of three.
+static bool cut_batch(const af3_dpa_params& p, int64_t (&count)[3], int (&rows_of)[3]) {
 	const int64_t B = p.B, per_row_wgs = p.H * ((p.L + 127) / 128);
 	auto plan = [&](int rows, int64_t (&count)[3], int (&rows_of)[3]) -> double {
 		static const double cost_per_row[5] = {0, 0, 1.09, 1.075, 1.0};
@@ -1193,8 +1217,7 @@ int launch_dpa_mfma_rows(const af3_dpa_params& p, hipStream_t s) {
 		}
 		return t;
 	};
-	int64_t count[3] = {0, 0, 0};
-	int     rows_of[3] = {0, 0, 0};
+	for(int i = 0; i < 3; i++) count[i] = 0, rows_of[i] = 0;
 	double  best = 1e30;
 	for(int rows = 4; rows >= 2; rows--) {
 		int64_t c[3];
@@ -1215,7 +1238,30 @@ int launch_dpa_mfma_rows(const af3_dpa_params& p, hipStream_t s) {
 			}
 		}
 	}
-	if(best >= 1e30) return AF3_ERR_BAD_SHAPE;  // (B == 1 is not eligible)
+	return best < 1e30;
+}
+
+int launch_dpa_mfma_rows(const af3_dpa_params& p, hipStream_t s) {
+	const int mode = rows_bias_mode(p);
+	if(mode < 0) return AF3_ERR_BAD_ARGUMENT;
+	if(mode == 1) {
+		const bool     bf32      = p.bias_dtype == AF3_F32;
+		const int      n_qblocks = (int)((p.L + 31) / 32), n_t_all = (int)((p.L + KT_R - 1) / KT_R);
+		const int64_t  total     = p.H * n_qblocks * (int64_t)n_t_all * 256;
+		if(total / 256 >= ((int64_t)1 << 31)) return AF3_ERR_BAD_SHAPE;  // (the prepass counts its units in 32 bits)
+		const unsigned g         = (unsigned)((total + 255) / 256 > 65536 ? 65536 : (total + 255) / 256);
+		if(bf32)
+			hipLaunchKernelGGL(bias_rows_prepass_kernel<true>, dim3(g), dim3(256), 0, s, p.bias, static_cast<f32x4*>(p.workspace), p.H, p.L, p.bias_stride[0], p.bias_stride[1],
+							   n_qblocks, n_t_all);
+		else
+			hipLaunchKernelGGL(bias_rows_prepass_kernel<false>, dim3(g), dim3(256), 0, s, p.bias, static_cast<f32x4*>(p.workspace), p.H, p.L, p.bias_stride[0], p.bias_stride[1],
+							   n_qblocks, n_t_all);
+		const int rc = launch_status();
+		if(rc != AF3_OK) return rc;
+	}
+	int64_t count[3];
+	int     rows_of[3];
+	if(!cut_batch(p, count, rows_of)) return AF3_ERR_BAD_SHAPE;  // (B == 1 is not eligible)
 	int64_t done = 0;
 	for(int i = 0; i < 3; i++) {
 		if(count[i] == 0) continue;
@@ -1224,6 +1270,21 @@ int launch_dpa_mfma_rows(const af3_dpa_params& p, hipStream_t s) {
 		done += count[i];
 	}
 	return AF3_OK;
+}
+
+int mfma_rows_plan(const af3_dpa_params& p, int64_t (&plan)[3][5]) {
+	int64_t count[3];
+	int     rows_of[3], n = 0;
+	const int mode = rows_bias_mode(p);
+	if(mode < 0 || !cut_batch(p, count, rows_of)) return 0;
+	for(int i = 0; i < 3; i++) {
+		if(count[i] == 0) continue;
+		const rows_launch l = lay_out(p, rows_of[i], mode, count[i]);
+		const int64_t     what[5] = {rows_of[i], mode, count[i], l.chunked > 0 ? l.chunk : 1, l.chunked * 8 < l.n_groups ? l.chunked * 8 : l.n_groups};
+		for(int j = 0; j < 5; j++) plan[n][j] = what[j];
+		n++;
+	}
+	return n;
 }
 
 }  // namespace af3
