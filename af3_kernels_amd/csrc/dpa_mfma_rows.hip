@@ -742,30 +742,32 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 			const int l = lane_now(), half_ = l >> 5, n_ = l & 31, voff = (n_ * out_sr + 4 * half_) * es;
 			// (a Newton step behind the reciprocal: half an ulp, as the division)
 			const float r0 = __builtin_amdgcn_rcpf(lsum[R]), inv = __builtin_fmaf(r0, __builtin_fmaf(-lsum[R], r0, 1.f), r0);
-#pragma unroll
-			for(int k = 0; k < 16; k++) oacc[R][k] *= inv;
-			if constexpr(GATE) {
+			if constexpr(GATE && GATE_LDS) {
 				const int gk = 2 * R + (n_ >> 4);   // this query row's piece of the gate
 				const unsigned char* const gate_row = smem + (gk < ROWS ? gate_buf0 : gate_buf1) + (wave * ROWS + (gk < ROWS ? gk : gk - ROWS)) * 1024 + (n_ & 15) * 64 + half_ * 8;
 #pragma unroll
-				for(int g4 = 0; g4 < 4; g4++) {
-					u32x2 gw = graw[g4];
-					if constexpr(GATE_LDS) gw = *reinterpret_cast<const u32x2*>(gate_row + g4 * 16);
-					oacc[R][4 * g4] *= sigmoidf_fast(bf16_bits_to_f32(gw[0] & 0xffffu)), oacc[R][4 * g4 + 1] *= sigmoidf_fast(bf16_bits_to_f32(gw[0] >> 16));
-					oacc[R][4 * g4 + 2] *= sigmoidf_fast(bf16_bits_to_f32(gw[1] & 0xffffu)), oacc[R][4 * g4 + 3] *= sigmoidf_fast(bf16_bits_to_f32(gw[1] >> 16));
-				}
+				for(int g4 = 0; g4 < 4; g4++) graw[g4] = *reinterpret_cast<const u32x2*>(gate_row + g4 * 16);
 			}
-			if(BF16 || es == 2) {   // (between query tiles no branch: the compiler's count of what is in flight would lose the stores)
+			auto columns = [&](int g4) {
+				float o[4];
 #pragma unroll
-				for(int g4 = 0; g4 < 4; g4++)
-					__builtin_amdgcn_raw_buffer_store_b64(u32x2{pack_bf16x2(oacc[R][4 * g4], oacc[R][4 * g4 + 1]), pack_bf16x2(oacc[R][4 * g4 + 2], oacc[R][4 * g4 + 3])}, rsrc,
-														  8 * g4 < D ? voff + 16 * g4 : 0x7FFF0000, 0, 0);
-			} else {
-#pragma unroll
-				for(int g4 = 0; g4 < 4; g4++)
-					__builtin_amdgcn_raw_buffer_store_b128(
-						u32x4{__float_as_uint(oacc[R][4 * g4]), __float_as_uint(oacc[R][4 * g4 + 1]), __float_as_uint(oacc[R][4 * g4 + 2]), __float_as_uint(oacc[R][4 * g4 + 3])}, rsrc,
-						8 * g4 < D ? voff + 32 * g4 : 0x7FFF0000, 0, 0);
+				for(int e = 0; e < 4; e++) o[e] = oacc[R][4 * g4 + e] * inv;
+				if constexpr(GATE) {
+					const u32x2 gw = graw[g4];
+					o[0] *= sigmoidf_fast(bf16_bits_to_f32(gw[0] & 0xffffu)), o[1] *= sigmoidf_fast(bf16_bits_to_f32(gw[0] >> 16));
+					o[2] *= sigmoidf_fast(bf16_bits_to_f32(gw[1] & 0xffffu)), o[3] *= sigmoidf_fast(bf16_bits_to_f32(gw[1] >> 16));
+				}
+				if(BF16 || es == 2)
+					__builtin_amdgcn_raw_buffer_store_b64(u32x2{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])}, rsrc, 8 * g4 < D ? voff + 16 * g4 : 0x7FFF0000, 0, 0);
+				else __builtin_amdgcn_raw_buffer_store_b128(u32x4{__float_as_uint(o[0]), __float_as_uint(o[1]), __float_as_uint(o[2]), __float_as_uint(o[3])}, rsrc, voff + 32 * g4, 0, 0);
+			};
+			// (head_dim 8 to 24 leave blocks of columns out; with all four gated and stored 2000 x 8 x 64 x 8 with a gate took 81.9 us, 300 x 8 x 300 x 8 80.4, so 69.5 and
+			// 72.8; between query tiles no branch: the compiler's count of what is in flight would lose the stores)
+			columns(0);
+			if(BF16 || D > 8) columns(1);
+			if(BF16 || D > 16) {
+				columns(2);
+				if(BF16 || D > 24) columns(3);
 			}
 			lsum[R] = 0.f;
 #pragma unroll

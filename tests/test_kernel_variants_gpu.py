@@ -807,3 +807,31 @@ def test_strips_on_both_sides_of_the_even_walk(af3, oracle, B, H, L, D, kind):
     finally:
         af3.set_rows_kernel(prev)
     assert np.abs(out - oracle.dpa_formula(f32np(q), f32np(k), f32np(v), keep.numpy(), f32np(bias))).max() <= 2e-2   # (bf16's budget)
+
+
+@pytest.mark.parametrize("B,H,L", [(5, 2, 72), (3, 2, 133), (404, 4, 300), (130, 8, 512)])   # single query tiles; several to a workgroup
+@pytest.mark.parametrize("D", [8, 16, 24, 32])
+@pytest.mark.parametrize("gated", [False, True])
+@pytest.mark.parametrize("out_type", [torch.bfloat16, torch.float32])
+def test_shared_bias_stores_head_dim_columns(af3, B, H, L, D, gated, out_type):
+    """Every column of every row, and nothing beside them: rows of the result that lie apart keep what stands between them."""
+    from af3_kernels_amd import _lib, ops
+    g = torch.Generator(device="cuda").manual_seed(L + D)
+    q, k, v, gate = (torch.randn(B, H, L, D, generator=g, device="cuda").to(torch.bfloat16) for _ in range(4))
+    bias = torch.randn(H, L, (L + 7) // 8 * 8, generator=g, device="cuda").to(torch.bfloat16)[..., :L]
+    room = torch.full((B, L + 1, H, D + 8), 7.0, dtype=out_type, device="cuda")
+    prev = af3.set_rows_kernel("always")
+    try:
+        print("case", B, H, L, D, gated, out_type, flush=True)
+        ops._dpa_forward_impl(q, k, v, None, bias, _lib.AF3_BF16, False, gate=gate if gated else None, out=room[:, :L, :, :D].transpose(1, 2))
+        torch.cuda.synchronize()
+    finally:
+        af3.set_rows_kernel(prev)
+    assert (room[:, L] == 7).all() and (room[..., D:] == 7).all()
+    out = room[:, :L, :, :D].transpose(1, 2)
+    for b in range(0, B, 32):   # (float32 on the GPU, some batch rows at a time)
+        qs, ks, vs = (t[b:b + 32].float().contiguous() for t in (q, k, v))
+        want = torch.matmul(torch.softmax(torch.matmul(qs * D ** -0.5, ks.transpose(-1, -2).contiguous()) + bias.float(), -1), vs)
+        if gated:
+            want *= torch.sigmoid(gate[b:b + 32].float())
+        assert (out[b:b + 32].float() - want).abs().max().item() <= 2e-2   # (bf16 q, k, v and probabilities; |v| < 6)
