@@ -100,13 +100,13 @@ extern "C" int64_t af3_dpa_workspace_used(const af3_dpa_params* params) {
 extern "C" int af3_dpa_log2_domain(const af3_dpa_params* params) { return validate(params) == AF3_OK && select_kernel(*params) == 1 && mfma_bf16_log2_domain(*params) ? 1 : 0; }
 
 // For tests: how the shared-bias kernel would lay this call out (mfma_rows_plan); no pointer is followed.
-extern "C" int af3_dpa_rows_plan(const af3_dpa_params* params, int64_t (*plan)[5]) {
+extern "C" int af3_dpa_rows_plan(const af3_dpa_params* params, int64_t (*plan)[6]) {
 	const int rc = validate(params);
 	if(rc != AF3_OK) return rc;
-	int64_t   found[3][5];
+	int64_t   found[3][6];
 	const int n = select_kernel(*params) == 1 ? mfma_bf16_rows_plan(*params, found) : 0;
 	for(int i = 0; i < n; i++)
-		for(int j = 0; j < 5; j++) plan[i][j] = found[i][j];
+		for(int j = 0; j < 6; j++) plan[i][j] = found[i][j];
 	return n;
 }
 

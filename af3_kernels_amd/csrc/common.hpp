@@ -77,8 +77,9 @@ bool mfma_rows_can_serve(const af3_dpa_params& p);   // eligible, and its bias c
 int64_t mfma_rows_workspace_bytes(const af3_dpa_params& p);
 bool mfma_rows_suits_a_small_batch(const af3_dpa_params& p);  // fewer than 128 batch rows and a bias that this kernel stages in place
 int launch_dpa_mfma_rows(const af3_dpa_params& p, hipStream_t s);
-// its launches: batch rows per wavefront, bias mode, batch rows, query tiles per workgroup, (group, head) pairs walked in such workgroups; their number, 0: none
-int mfma_rows_plan(const af3_dpa_params& p, int64_t (&plan)[3][5]);
+// its launches: batch rows per wavefront, bias mode, batch rows, query tiles per workgroup, (group, head) pairs walked in such workgroups, priorities (progress_mode); their
+// number, 0: none
+int mfma_rows_plan(const af3_dpa_params& p, int64_t (&plan)[3][6]);
 // dpa_strip.hip: the bf16 kernel for a bias that is read in place once per batch row; the caller has checked mfma_bf16_eligible
 bool mfma_strip_wanted(const af3_dpa_params& p);
 int launch_dpa_strip(const af3_dpa_params& p, hipStream_t s);
@@ -86,7 +87,7 @@ bool mfma_bf16_eligible(const af3_dpa_params& p);
 int64_t mfma_bf16_workspace_bytes(const af3_dpa_params& p);
 int64_t mfma_bf16_workspace_used(const af3_dpa_params& p);
 bool mfma_bf16_log2_domain(const af3_dpa_params& p);   // the call's kernel scales q by log2 e
-int mfma_bf16_rows_plan(const af3_dpa_params& p, int64_t (&plan)[3][5]);   // as mfma_rows_plan; 0: another kernel's call
+int mfma_bf16_rows_plan(const af3_dpa_params& p, int64_t (&plan)[3][6]);   // as mfma_rows_plan; 0: another kernel's call
 bool mfma_fp8_eligible(const af3_dpa_params& p);
 int launch_dpa_mfma_f32(const af3_dpa_params& p, hipStream_t s);
 bool mfma_f32_eligible(const af3_dpa_params& p);

@@ -1531,7 +1531,7 @@ static int launch_nw(const af3_dpa_params& p, hipStream_t s) {
 static bool uses_workspace(const af3_dpa_params& p) {   // (the one-row kernel)
 	return p.bias && p.workspace && p.B >= 2 && !one_row_in_place(p) && p.workspace_bytes >= ws_bytes_needed(p) && (reinterpret_cast<uintptr_t>(p.workspace) & 15) == 0;
 }
-int mfma_bf16_rows_plan(const af3_dpa_params& p, int64_t (&plan)[3][5]) { return rows_kernel_wanted(p) && mfma_rows_can_serve(p) ? mfma_rows_plan(p, plan) : 0; }
+int mfma_bf16_rows_plan(const af3_dpa_params& p, int64_t (&plan)[3][6]) { return rows_kernel_wanted(p) && mfma_rows_can_serve(p) ? mfma_rows_plan(p, plan) : 0; }
 
 bool mfma_bf16_log2_domain(const af3_dpa_params& p) { return (rows_kernel_wanted(p) && mfma_rows_can_serve(p)) || uses_workspace(p) || !p.bias; }
 

@@ -1121,9 +1121,13 @@ rows_launch lay_out(const af3_dpa_params& p, int rows, int bmode, int64_t b_coun
 	l.chunk = 1, l.parts = l.n_qtiles;
 	if(several_query_tiles(rows, bmode, p.gate != nullptr) && p.out_dtype == AF3_BF16) plan_chunks(p, l.n_qtiles, l.per_xcd, l.chunk, l.parts, l.chunked);
 	l.blocks = (l.chunked * l.parts + (l.per_xcd - l.chunked) * l.n_qtiles) * 8;
-	// (by age / evenly, us: 384 x 4 x 384 x 32 62.1 / 60.5, 512 131.7 / 129.0, 768 389.8 / 383.7, 1491 2612 / 2598, 64 x 4 x 768 x 32 41.2 / 39.7, 5 x 16 x 2000 x 24
-	// 116.1 / 112.8, 400 90.2 / 91.4; many rounds of single query tiles: the grid block of 512 tokens 246 / 252, 832 511.5 / 514.9;
-	// few rounds with a short last one, by age / last round first: 80 x 4 x 768 x 32 44.6 / 43.3, 150 x 4 x 384 x 32 27.3 / 25.7)
+	// Workgroups of several query tiles go evenly whatever the last round holds: it consists of single tiles or is nearly whole.  us, by age / evenly / by the rule for
+	// single ones, L x 4 x L x 32: 300 40.3 / 40.0 / 40.5, 384 60.3 / 59.2 / 58.8, 400 86.8 / 87.4 / 87.7, 440 103.6 / 105.0 / 104.3, 500 121.5 / 119.1 / 118.8,
+	// 600 210.4 / 209.7 / 208.6, 660 286.5 / 279.9 / 286.3, 768 388.2 / 376.8 / 380.2, 960 735 / 725 / 724, 1216 1433 / 1419 / 1436, 1300 1864 / 1831 / 1834, 1491 2576 / 2586 / 2583;
+	// 5 x 16 x 2000 x 24 83.1 / 78.4 / 79.0, 12 x 16 x 1536 97.3 / 98.6 / 96.0, 16 x 16 x 1536 134.9 / 130.7 / 131.6.  Single tiles, by age / evenly: less than a round 64 x 4 x 384 x 32
+	// 15.9 / 14.9, 150 x 4 x 384 x 32 27.4 / 26.4, 24 x 4 x 768 25.0 / 23.5, 80 x 4 x 768 45.1 / 44.3, of it half or less 16 x 4 x 384 11.1 / 11.3; many rounds: the grid block
+	// of 512 tokens 246 / 252, 832 511.5 / 514.9; few with a short last one, by age / evenly / the last one first: 32 x 4 x 1300 84.8 / 88.1 / 83.9, 104 x 4 x 640 packed
+	// 51.0 / 52.3 / 50.3, 520 x 4 x 128 20.0 / 20.0 / 19.9.
 	l.even = l.chunked > 0 ? EVENLY : l.blocks <= 3 * 512 ? progress_mode(l.blocks, 512) : BY_AGE;
 	return l;
 }
@@ -1274,7 +1278,7 @@ int launch_dpa_mfma_rows(const af3_dpa_params& p, hipStream_t s) {
 	return AF3_OK;
 }
 
-int mfma_rows_plan(const af3_dpa_params& p, int64_t (&plan)[3][5]) {
+int mfma_rows_plan(const af3_dpa_params& p, int64_t (&plan)[3][6]) {
 	int64_t count[3];
 	int     rows_of[3], n = 0;
 	const int mode = rows_bias_mode(p);
@@ -1282,8 +1286,8 @@ int mfma_rows_plan(const af3_dpa_params& p, int64_t (&plan)[3][5]) {
 	for(int i = 0; i < 3; i++) {
 		if(count[i] == 0) continue;
 		const rows_launch l = lay_out(p, rows_of[i], mode, count[i]);
-		const int64_t     what[5] = {rows_of[i], mode, count[i], l.chunked > 0 ? l.chunk : 1, l.chunked * 8 < l.n_groups ? l.chunked * 8 : l.n_groups};
-		for(int j = 0; j < 5; j++) plan[n][j] = what[j];
+		const int64_t     what[6] = {rows_of[i], mode, count[i], l.chunked > 0 ? l.chunk : 1, l.chunked * 8 < l.n_groups ? l.chunked * 8 : l.n_groups, l.even};
+		for(int j = 0; j < 6; j++) plan[n][j] = what[j];
 		n++;
 	}
 	return n;

@@ -48,7 +48,10 @@ struct even_progress {   // from: EVENLY, BY_AGE or the first workgroup that goe
 // 2.34 205.6 / 202.2, 2.58 221.0 / 225.5.  Of the fp8 kernel (B x 16 x 1536 x 24) by age / evenly: 0.94 68.6 / 64.4; by age / last round first: 1.13 81.6 / 76.1,
 // 2.25 139.4 / 137.3; evenly / last round first: 1.31 92.0 / 90.5, 1.5 96.5 / 95.7, 1.88 116.7 / 123.3, 2.44 152.3 / 148.1.
 constexpr int EVENLY = -1, BY_AGE = 0x7fffffff;
-inline int progress_mode(int64_t workgroups, int64_t slots) {   // EVENLY, or the first workgroup of the last round
+// (A launch of at most half a round has no earlier round: its wavefronts keep the priority that every other kernel's have.  The padding of a grid lies at its end, so
+// that the last round begins where its real workgroups do, or a few behind.)
+inline int progress_mode(int64_t workgroups, int64_t slots) {   // EVENLY, BY_AGE or the first workgroup of the last round
+	if(workgroups * 2 <= slots) return BY_AGE;
 	const int64_t last = workgroups % slots;
 	return last == 0 || last * 2 > slots ? EVENLY : (int)(workgroups - last);
 }

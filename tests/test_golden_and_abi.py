@@ -643,8 +643,8 @@ def test_strips_of_short_walks_carry_no_priorities(tmp_path):
         assert with_it is None or with_it >= without + 400
 
 
-def _rows_plan(B, H, L, D, layout="dense", gate=False, bias=True, out=1):
-    """The shared-bias kernel's launches of a call: (batch rows per wavefront, bias mode, batch rows, query tiles per workgroup, pairs walked so).
+def _rows_plan(B, H, L, D, layout="dense", gate=False, bias=True, out=1, always=False):
+    """The shared-bias kernel's launches of a call: (batch rows per wavefront, bias mode, batch rows, query tiles per workgroup, pairs walked so, priorities).
     layout: "dense" [B, H, L, D]; "heads last" [B, L, H, D]; "packed" [B, L, (k | v | q | gate), H, D]; "per head" [B, L, H, (k | v | q | gate), D]."""
     from af3_kernels_amd import _lib
     strides, apart = {"dense": ((H * L * D, L * D, D), 1 << 30), "heads last": ((L * H * D, D, H * D), 1 << 30),
@@ -653,10 +653,10 @@ def _rows_plan(B, H, L, D, layout="dense", gate=False, bias=True, out=1):
     base = 1 << 40   # (addresses that nothing follows)
     p = _lib.DpaParams(B=B, H=H, L=L, D=D, k=base, v=base + apart, q=base + 2 * apart, gate=base + 3 * apart if gate else None, out=base << 1,
                        q_stride=i64x3(*strides), k_stride=i64x3(*strides), v_stride=i64x3(*strides), gate_stride=i64x3(*strides), out_stride=i64x3(H * L * D, L * D, D),
-                       io_dtype=1, mma_dtype=1, out_dtype=out, softmax_scale=1.0, reserved=4, workspace=base << 2, workspace_bytes=1 << 40)
+                       io_dtype=1, mma_dtype=1, out_dtype=out, softmax_scale=1.0, reserved=4 | always, workspace=base << 2, workspace_bytes=1 << 40)
     if bias:
         p.bias, p.bias_stride, p.bias_dtype = base << 3, (ctypes.c_int64 * 2)(L * L, L), 1
-    plan = (ctypes.c_int64 * 5 * 3)()
+    plan = (ctypes.c_int64 * 6 * 3)()
     n = _lib.load().af3_dpa_rows_plan(ctypes.byref(p), plan)
     assert n >= 0
     return [tuple(launch) for launch in plan[:n]]
@@ -678,6 +678,20 @@ def test_shared_bias_chunks_where_lines_hold_other_heads():
     for H in (2, 4, 8, 12, 16):
         for L in range(129, 1600, 61):
             for D in (8, 16, 24, 32):
-                for _, _, _, c, _ in _rows_plan(3000 // H, H, L, D, layout="heads last"):
+                for _, _, _, c, _, _ in _rows_plan(3000 // H, H, L, D, layout="heads last"):
                     tiles = (L + 127) // 128
                     assert c == 1 or (H <= 8 and c < 4 and 2 * c <= tiles and tiles % c == 0)
+
+
+def test_small_launches_raise_no_priority():
+    """Wavefronts of a launch that fills at most half of a round have nobody to go before but other streams' kernels; the other rules of priorities:
+    evenly in nearly whole rounds and in workgroups of several query tiles, by age in many rounds of single ones, the last one of few rounds first
+    where it is short."""
+    EVENLY, BY_AGE = -1, 0x7fffffff
+    priorities = lambda *a, **k: [(launch[3], launch[5]) for launch in _rows_plan(*a, **k)]
+    assert priorities(16, 4, 384, 32, always=True) == [(1, BY_AGE)]          # 96 workgroups of 512
+    assert priorities(16, 4, 900, 32, always=True) == [(1, BY_AGE)]          # 256
+    assert priorities(64, 4, 384, 32) == [(1, EVENLY)]                       # 384
+    assert priorities(90, 4, 768, 32) == [(2, EVENLY)]
+    assert priorities(512, 4, 512, 32, gate=True) == [(1, BY_AGE)]           # four rounds
+    assert priorities(520, 4, 128, 32) == [(1, 512)]                         # 696
