@@ -15,7 +15,7 @@
 // MFMAs.
 //
 // Work split.  Workgroup = NW wavefronts = NW blocks of 32 query rows of one (group of 4 batch rows, head).  K and V
-// tiles (32 keys x 4 batch rows) are staged in LDS by loads that write LDS directly, four buffers deep, and shared
+// tiles (32 keys x 4 batch rows) are staged in LDS by loads that write LDS directly, three buffers deep, and shared
 // by the NW wavefronts; one workgroup barrier per tile, i.e. per four blocks of logits of every wavefront.  A workgroup may
 // walk several query tiles of its group and head one behind the other without coming to rest (plan_chunks).
 #include "mfma_helpers.hpp"
@@ -98,7 +98,8 @@ __global__ void __launch_bounds__(256) bias_rows_prepass_kernel(const void* __re
 // MULTI: workgroups may walk several query tiles; per XCD the first n_chunked (group, head) pairs are cut into n_chunks workgroups of q_chunk query tiles, the
 // others into workgroups of one.  Launches of single query tiles take the form without: with the code of the longer walk in it (10 KB more, scalar and,
 // with four rows, 7 vector registers spilled) they took, us, that code in / out: 512 x 4 x 128 x 32 25.2 / 23.9, 1024 38.4 / 37.0, 1536 50.2 / 47.4, 1000 x 4 x 64 x 32
-// 26.4 / 24.9, 512 x 8 x 256 x 32 on packed rows 110.1 / 94.5.
+// 26.4 / 24.9, 512 x 8 x 256 x 32 on packed rows 110.1 / 94.5.  With four rows and a bias staged in place the longer walk spills 7 vector registers, stored once per
+// workgroup and read back in the careful walk alone; every form of it holds 12 to 113 scalar registers in vector lanes.
 // Whether there is such a form.  Four batch rows and their gates do not fit the registers between two query tiles (14 spilled ones: the
 // grid block of 768 tokens 637 -> 655 us; with one query tile to a workgroup 633), the in-place form has not been given it.
 constexpr bool several_query_tiles(int rows, int bmode, bool gate) { return bmode != 2 && !(gate && rows == 4); }
@@ -784,9 +785,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 	//
 	// Several query tiles of one head and the same batch rows: K, V and the masks stay, so the ring of tiles runs on -- behind the last
 	// tile come the first two again -- and so do the four chains.  The last tile's steps (LAST) request the next query tile's q rows
-	// as their predecessors' last readers pass, each three steps ahead of its first use; the next query tile's first tile (FIRST_NEXT) finishes and
+	// as their predecessors' last readers pass, row r in step r and row 0 ROWS - 1 steps ahead of its first use; the next query tile's first tile (FIRST_NEXT) finishes and
 	// stores a batch row's results between the step's new reference and its exponentials.  A workgroup of one query tile spends 26 k clocks of its 79 k
 	// (L = 768) in front of its walk and behind it; from query tile to query tile it is 6 k.
+	// The hand-written waits in front of the barriers let what was issued behind the awaited loads stay in flight.  The compiler's own, for q rows and gates, do not count the
+	// loads that write LDS and so take in the next tile's, which are a step old by then.  With everything requested and awaited in front of those loads (they a step later, q
+	// rows converted and the gates of two rows requested in LAST) no wait did, in the same time: us, so / here: 384 x 4 x 384 x 32 58.3 / 58.1, with a gate 63.3 / 63.7,
+	// 768 374.1 / 373.9, 1491 2564 / 2558, 300 x 16 x 384 x 24 172.6 / 167.9, and 4 registers more spilled.
 	// (INNER: a MIDDLE tile with two more of its query tile behind it; it asks nothing about what is to be requested.)
 	enum { MIDDLE = 0, FIRST = 1, LAST = 2, FIRST_NEXT = 3, CAREFUL_MIDDLE = 4, CAREFUL_FIRST = 5, INNER = -1 };
 	// more: this wavefront walks another query tile behind this one; more_wg: the workgroup does

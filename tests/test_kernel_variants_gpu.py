@@ -503,7 +503,7 @@ def test_shared_bias_quick_and_careful_walks(af3, oracle, B, H, L, D, kind):
     assert (np.abs(out - want) / scale).max() <= 2e-2
 
 
-@pytest.mark.parametrize("B,H,L,D", [(404, 4, 300, 32), (261, 4, 264, 24), (130, 8, 512, 32), (96, 8, 640, 16), (500, 4, 200, 8), (128, 2, 1281, 32)])   # two to four of 3, 3, 4, 5, 2 and 11 query tiles one behind the other; last ones in which one to three wavefronts have rows
+@pytest.mark.parametrize("B,H,L,D", [(404, 4, 300, 32), (261, 4, 264, 24), (130, 8, 512, 32), (96, 8, 640, 16), (500, 4, 200, 8), (128, 2, 1281, 32)])   # 3 of 3, 3 of 3, 2 of 4, 2 of 5, 2 of 2 and 3 of 11 query tiles one behind the other (with a gate the second, fourth and fifth: single ones); last ones in which one to three wavefronts have rows
 @pytest.mark.parametrize("kind", ["random", "no bias", "first tile", "none", "120", "120 and none"])
 @pytest.mark.parametrize("gated", [False, True])
 def test_shared_bias_query_tiles_in_one_workgroup(af3, B, H, L, D, kind, gated):
@@ -835,3 +835,99 @@ def test_shared_bias_stores_head_dim_columns(af3, B, H, L, D, gated, out_type):
         if gated:
             want *= torch.sigmoid(gate[b:b + 32].float())
         assert (out[b:b + 32].float() - want).abs().max().item() <= 2e-2   # (bf16 q, k, v and probabilities; |v| < 6)
+
+
+def _rows_plan(q, k, v, out, bias, gate):
+    """The shared-bias kernel's launches of a call: (batch rows per wavefront, bias mode, query tiles per workgroup)."""
+    import ctypes
+    from af3_kernels_amd import _lib, ops
+    p = ops._fill_params(q, k, v, None, bias, out, _lib.AF3_BF16, False, gate=gate)
+    p.workspace, p.workspace_bytes = 1 << 40, 1 << 40   # (nothing follows the address)
+    plan = (ctypes.c_int64 * 6 * 3)()
+    n = _lib.load().af3_dpa_rows_plan(ctypes.byref(p), plan)
+    return [(launch[0], launch[1], launch[3]) for launch in plan[:n]]
+
+
+@pytest.mark.parametrize("B,H,L,D,gated,want", [
+    (460, 4, 460, 32, False, (4, 1, 4)),                                       # four tiles to a workgroup
+    (400, 4, 400, 32, False, (2, 3, 2)), (400, 4, 400, 32, True, (2, 3, 2)),   # two batch rows per wavefront
+    (404, 4, 300, 32, False, (2, 1, 3)), (404, 4, 300, 32, True, (2, 1, 3)),
+    (384, 4, 384, 32, False, (3, 3, 3)), (384, 4, 384, 32, True, (3, 3, 3)),
+    (768, 2, 768, 32, True, (3, 1, 2)),
+    (640, 2, 768, 32, False, (4, 1, 2)),                                       # four and the workspace
+    (128, 16, 512, 32, False, (4, 3, 2)),                                      # four and a bias staged in place
+])
+@pytest.mark.parametrize("layout", ["dense", "per head"])   # [B, H, L, D] each; k, v, q and gate side by side for each token and head, the result [B, L, H, D]
+@pytest.mark.parametrize("kind", ["random", "no bias", "first tile", "none", "120", "k inf"])
+def test_shared_bias_forms_of_the_longer_walk(af3, B, H, L, D, gated, want, layout, kind):
+    """Every number of batch rows per wavefront, place of the bias and number of query tiles one behind the other that a call can meet: keys that end
+    in the first tile, a batch row without a live key (walks carefully from the start), query tiles walked again, an infinity in K."""
+    from af3_kernels_amd import _lib, ops
+    g = torch.Generator(device="cuda").manual_seed(L + D)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda", dtype=torch.bfloat16)
+    if layout == "dense":
+        k, v, q, gate = (r(B, H, L, D) for _ in range(4))
+        out = torch.empty_like(q)
+    else:
+        k, v, q, gate = r(B, L, H, 4, D).permute(3, 0, 2, 1, 4).unbind(0)
+        out = torch.empty(B, L, H, D, device="cuda", dtype=torch.bfloat16).transpose(1, 2)
+    gate = gate if gated else None
+    bias = None if kind == "no bias" else r(H, L, L)
+    keep = torch.rand(B, L, generator=g, device="cuda") < 0.8
+    keep[:, 0] = keep[:, 70] = keep[:, L - 1] = True
+    if kind == "first tile":
+        keep[:, 20:] = False
+    elif kind == "none":
+        keep[B // 2] = False
+    elif kind == "120":
+        bias[:, [3, L // 2, L - 2], L - 1] = 120.0   # (rows of the first, a middle and the last query tile)
+    elif kind == "k inf":
+        k[B // 2, 1, 70, 1] = float("inf")
+    plan = _rows_plan(q, k, v, out, bias, gate)
+    assert plan[0][::2] == want[::2] and plan[0][1] == (0 if bias is None else want[1])
+    print("case", B, H, L, D, gated, layout, kind, flush=True)
+    ops._dpa_forward_impl(q, k, v, ops._lift_mask(keep, L), bias, _lib.AF3_BF16, False, gate=gate, out=out)
+    torch.cuda.synchronize()
+    for b in range(0, B, 32):   # (float32 on the GPU, some batch rows at a time)
+        qs, ks, vs = (t[b:b + 32].float().contiguous() for t in (q, k, v))
+        s = torch.matmul(qs * D ** -0.5, ks.transpose(-1, -2).contiguous())
+        if bias is not None:
+            s += bias.float()
+        ref = torch.matmul(torch.softmax(s.masked_fill(~keep[b:b + 32, None, None, :], -1e9), -1), vs)
+        if gated:
+            ref *= torch.sigmoid(gate[b:b + 32].float())
+        got, nan = out[b:b + 32].float(), ref.isnan()
+        if kind == "k inf" and b <= B // 2 < b + 32:   # (this kernel's NaN rows take the query row 16 further on or back with them, never another head or batch row)
+            block = slice(B // 2 - b, B // 2 - b + 1), slice(1, 2)
+            assert nan[block].any() and (got[block].isnan() >= nan[block]).all()
+            nan[block] |= got[block].isnan()
+        assert torch.equal(got.isnan(), nan)
+        assert (got - ref).masked_fill(nan, 0.0).abs().max().item() <= 2e-2   # (bf16 q, k, v and probabilities; |v| < 6)
+
+
+@pytest.mark.parametrize("row,taken", [((1 << 24) - 8, True), (1 << 24, False)])
+@pytest.mark.parametrize("which", ["q", "out"])
+def test_shared_bias_row_strides(af3, which, row, taken):
+    """Rows of q or of the result that lie up to 2^24 elements apart are addressed by the shared-bias kernel; calls with rows further apart go to the
+    one-row kernel."""
+    from af3_kernels_amd import _lib, ops
+    B, H, L, D = 2, 1, 133, 32
+    g = torch.Generator(device="cuda").manual_seed(row)
+    q, k, v = (torch.randn(B, H, L, D, generator=g, device="cuda").to(torch.bfloat16) for _ in range(3))
+    bias = torch.randn(H, L, 136, generator=g, device="cuda").to(torch.bfloat16)[..., :L]
+    wide = torch.empty((L - 1) * row + B * D, device="cuda", dtype=torch.bfloat16).as_strided((B, H, L, D), (D, D, row, 1))
+    out = torch.empty_like(q)
+    if which == "q":
+        qs, outs = wide.copy_(q), out
+    else:
+        qs, outs = q, wide
+    prev = af3.set_rows_kernel("always")
+    try:
+        assert bool(_rows_plan(qs, k, v, outs, bias, None)) == taken
+        print("case", which, row, flush=True)
+        ops._dpa_forward_impl(qs, k, v, None, bias, _lib.AF3_BF16, False, out=outs)
+        torch.cuda.synchronize()
+    finally:
+        af3.set_rows_kernel(prev)
+    want = torch.matmul(torch.softmax(torch.matmul(q.float() * D ** -0.5, k.float().transpose(-1, -2).contiguous()) + bias.float(), -1), v.float())
+    assert (outs.float() - want).abs().max().item() <= 2e-2   # (bf16 q, k, v and probabilities; |v| < 6)
