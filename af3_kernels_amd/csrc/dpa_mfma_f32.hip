@@ -431,10 +431,11 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DP
 		__syncthreads();
 		kt = ktn;
 	};
-	even_progress progress(n_steps, even);
+	// (forms whose workgroups stand alone on a compute unit lose by the code: 2 x 4 x 128 x 32 6.33 / 6.41 us without / with it, 5 x 4 x 333 19.8 / 20.1, 32 x 4 x 300 22.5 / 22.7)
+	even_progress progress(n_steps, KS == 1 ? even : BY_AGE);
 	step(ic<1>{}, 0);
 	for(int j = 1; j < n_steps; j++) {
-		progress.at(j);
+		if constexpr(KS == 1) progress.at(j);
 		step(ic<0>{}, j);
 	}
 	// Row numbers from here on come from the lane's number once more, out of the compiler's sight where the loop above has no
@@ -558,7 +559,7 @@ int launch(const af3_dpa_params& p, hipStream_t s) {
 	const int64_t grid     = ((groups + 7) / 8) * 8 * n_qtiles;
 	if(grid > 0x7fffffff) return AF3_ERR_BAD_SHAPE;
 	const size_t smem = (size_t)4 * KS * 3 * F32_KT * DP * 2 + (size_t)n_tiles * 4 + (size_t)n_tiles * 2 + 16;
-	const int64_t per_cu = KS > 1 ? 1 : DP == 64 ? 2 : 4;   // workgroups a compute unit holds, by their registers
+	const int64_t per_cu = DP == 64 ? 2 : 4;   // workgroups a compute unit holds, by their registers (KS = 1)
 	auto         kern = dpa_mfma_f32_kernel<DP, NW, KS>;
 	if(smem > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) return AF3_ERR_LAUNCH;
 	hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(NW * 64), smem, s, p, n_qtiles, groups, progress_mode(groups * n_qtiles, 256 * per_cu));

@@ -605,42 +605,48 @@ def test_forms_for_single_query_tiles_spill_no_vector_registers(tmp_path):
     assert {n: r for n, r in single.items() if r[0]} == {}
 
 
-def _kernel_sizes(tmp_path):
-    """name -> bytes of code of every kernel in the built library."""
+def _kernels_with_priorities(tmp_path):
+    """Names of the built library's kernels, and those that contain s_setprio."""
     from af3_kernels_amd import build as hip_build
-    readelf = os.path.join(os.path.dirname(os.path.dirname(os.path.realpath(hip_build.HIPCC))), "llvm", "bin", "llvm-readelf")
-    if not os.path.exists(readelf):
-        pytest.skip("no llvm-readelf")
+    objdump = os.path.join(os.path.dirname(os.path.dirname(os.path.realpath(hip_build.HIPCC))), "llvm", "bin", "llvm-objdump")
+    if not os.path.exists(objdump):
+        pytest.skip("no llvm-objdump")
     data = open(hip_build.LIB, "rb").read()
-    found = {}
+    names, raising = set(), set()
     for m in re.finditer(b"\x7fELF", data):
         if m.start() == 0:
             continue   # the host library itself
         path = tmp_path / "code"
         path.write_bytes(data[m.start():])
-        for line in subprocess.run([readelf, "-sW", str(path)], capture_output=True, text=True).stdout.splitlines():
-            f = line.split()
-            if len(f) >= 8 and f[3] == "FUNC":
-                found[f[7]] = int(f[2], 0)
-    return found
+        name = None
+        for line in subprocess.run([objdump, "-d", "--no-show-raw-insn", str(path)], capture_output=True, text=True).stdout.splitlines():
+            if line.endswith(">:"):
+                name = line.split("<")[1][:-2]
+                names.add(name)
+            elif "s_setprio" in line:
+                raising.add(name)
+    return names, raising
 
 
-def test_strips_of_short_walks_carry_no_priorities(tmp_path):
-    """The strip kernel's forms for walks of few tiles to a wavefront hold none of the code that lets wavefronts behind on theirs go first:
-    their time is their instructions.  (Strips of two blocks of rows and more, head_dim up to 24 and from 33 on, have both forms; the others one.)"""
-    sizes = {}
-    for name, size in _kernel_sizes(tmp_path).items():
+def test_priorities_stand_where_they_act(tmp_path):
+    """Kernel forms whose wavefronts have nobody to go before hold none of the code for it: their time is their instructions.  Strips of two blocks of
+    rows and more, head_dim up to 24 and from 33 on, have a form with it for longer walks and one without; the fp32 kernel has it where several
+    workgroups stand on a compute unit."""
+    names, raising = _kernels_with_priorities(tmp_path)
+    strips = {}
+    for name in names:
         m = re.search(r"dpa_strip_bf16_kernelILi(\d)ELi(\d)ELb([01])ELi(\d)ELb([01])EE", name)
         assert m or "dpa_strip_bf16_kernel" not in name, name
         if m:
-            nb, kind, odd, nw, even = map(int, m.groups())
-            sizes[nb, kind, odd, nw, even] = size
-    forms = [f[:4] for f in sizes if f[4] == 0]
-    assert len(forms) == 3 * 6 * 2 + 3
-    for f in forms:
-        without, with_it = sizes[f + (0,)], sizes.get(f + (1,))
-        assert (with_it is not None) == (f[0] > 1 and f[1] != 1)
-        assert with_it is None or with_it >= without + 400
+            strips[tuple(map(int, m.groups()))] = name
+    without = [f for f in strips if f[4] == 0]
+    assert len(without) == 3 * 6 * 2 + 3
+    for f in without:
+        assert strips[f] not in raising
+        assert (f[:4] + (1,) in strips) == (f[0] > 1 and f[1] != 1)
+    assert all(strips[f] in raising for f in strips if f[4] == 1)
+    fp32 = {name: int(m.group(1)) for name in names if (m := re.search(r"dpa_mfma_f32_kernelILi\d+ELi\dELi(\d)EE", name))}
+    assert len(fp32) == 7 and {name for name, parts in fp32.items() if parts == 1} == raising & set(fp32)
 
 
 def _rows_plan(B, H, L, D, layout="dense", gate=False, bias=True, out=1, always=False):
