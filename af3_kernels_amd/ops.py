@@ -236,11 +236,12 @@ def _dpa_forward_impl(q, k, v, keep, bias, mma_dtype: int, force_generic: bool, 
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
         p.workspace, p.workspace_bytes = ws.data_ptr(), ws_bytes
     with _on_device(q.device):
-        if _timers.enabled:
+        timed = _timers.enabled and not torch.cuda.is_current_stream_capturing()   # (an event recorded into a graph has no time)
+        if timed:
             s, e = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
             s.record()
         _lib.check(lib.af3_dpa_forward(ctypes.byref(p), _stream_ptr(q.device)), "af3_dpa_forward")
-        if _timers.enabled:
+        if timed:
             e.record()
             B, H, L, D = q.shape
             _timers.record(s, e, 4.0 * B * H * L * L * D)

@@ -883,6 +883,28 @@ def test_timers_report_calls(af3, capsys):
     assert "calls=3" in capsys.readouterr().out
 
 
+def test_timers_leave_captured_calls_out(af3, capsys):
+    """A call recorded into a graph has no time of its own; the calls around it keep theirs."""
+    from af3_kernels_amd import ops
+    q, k, v, m, bias = dev(*rand_inputs(1, 2, 64, 32, torch.bfloat16, seed=1))
+    was = ops._timers.enabled
+    af3.reset_debug_timers()
+    try:
+        first = af3.dot_product_attention_cpp(q, k, v, m, bias)
+        graph = torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph):
+            out = af3.dot_product_attention_cpp(q, k, v, m, bias)
+        graph.replay()
+        last = af3.dot_product_attention_cpp(q, k, v, m, bias)
+        af3.print_debug_timers()
+    finally:
+        ops._timers.reset()
+        ops._timers.enabled = was
+    assert "calls=2" in capsys.readouterr().out
+    assert torch.equal(first, out) and torch.equal(first, last)
+
+
 # ---- fp8 (e4m3) matrix-core path ------------------------------------------------------------
 # No reference behaviour exists for fp8 (the reference's e4m3 converters are unimplemented asserts); the only pin is
 # the fp32 formula on the un-quantised inputs within 6e-2.
