@@ -1082,37 +1082,49 @@ kv_lines lines_of_a_key(const af3_dpa_params& p) {
 
 // How many query tiles a workgroup walks.  Its start and its end (masks, first tiles, q, the stores' way out) are paid once, but workgroups of several
 // query tiles come in fewer rounds of the 64 an XCD holds (two per compute unit), and query tiles that are walked one behind the other read K and V
-// from the L2 at different times, where neighbours read them together: a divisor of the number of query tiles up to 4, one that leaves whole rounds (or nearly: 349 x 4 x 349 x 32
-// 55.6 one each, 51.0 in 0.92 of a round of three, 56.4 ending in single ones)
-// where there is one, else the smallest; what does not make whole rounds ends in a round of single query tiles.  Five and
-// eleven query tiles go as 2 2 1 and 3 3 3 2.  us, one query tile each / so, one card, L x 4 x L x 32: 300 44.5 / 41.2, 384 61.0 / 59.5,
-// 400 97.8 / 89.6, 512 127.5 / 122.6, 600 204.5 / 200.5, 640 237.5 / 230.0, 768 393.8 / 377.3, 1024 874 / 841, 1200 1437 / 1397, 1300 1847 / 1813,
+// from the L2 at different times, where neighbours read them together.  So a divisor of the number of query tiles: the smallest of those that leave whole rounds or a last
+// one more than nine tenths full, else of two and three that leave one more than four fifths full; else, from two rounds of single tiles on (three tiles to a head 1.75; eight and
+// more 3, nine 5, where single ones would not make whole rounds), two (three of three and nine), and what would be the last round ends in single tiles.
+// Time of single tiles = 1, by rounds of them: two tiles to a head, in twos 1.5 1.02-1.03, 1.62 0.89-0.94, 1.75 0.91-0.95, 2 0.89-0.97, 2.9 0.97; ending in single ones 1.5
+// 1.04-1.07, 1.62 1.01-1.04, 2.6-2.9 0.92-0.99, 5-6.9 0.93-1.02; three, in threes 2.5-2.6 0.92-0.93, 2.7-3 0.92-0.97, 4.9 1.03, 5.5 0.95-0.98; ending in single ones 1.4-1.6
+// 1.03-1.18, 1.7 0.99-1.02, 1.8-2 0.94-0.99, 2.5-2.6 1.03-1.06, 4.9-6.8 0.94-1.00; four, in twos 1.6-1.75 0.94-1.00, 1.9-2 0.95-0.99, 2.6-3 1.0-1.07; ending in single ones
+// 1.5-1.75 1.00-1.06, 2.6-3 0.90-0.99, 5-7 0.95-1.01; in fours 2.6-3 1.04-1.13, 3.6 0.90-0.92 (in twos 0.94), 4 0.98 (0.96); six, in twos 1.7 0.92-1.00, 1.9 0.94-0.99, 5.6 0.92-0.95;
+// ending 1.4-1.7 1.02-1.13, 2.6-6.8 0.94-1.00; eight and ten alike, but ending 2.5-2.8 0.97-1.05 and whole rounds of single ones 5 1.05-1.08; nine, in threes 2.8-3 0.98-1.00, ending 1.7-3.1 1.03-1.13, 3.5-4.5 0.98-1.04, 5-20 0.94-1.00.
+// Five go as 2 2 1, in one round (0.95-0.97) or, where the bias is not staged in place and single tiles would not make whole rounds, from three on, ending in single tiles
+// (3.75 0.95, 4.7 0.95-0.98, 5.5-6.8 0.95-0.99; whole rounds of single ones 3 1.01-1.05, 5 1.02-1.03; staged 0.99-1.05; 2 2 1 throughout 1.01-1.07).  Seven, eleven and thirteen stay single: 832 507 us, in twos / threes / fours 535 / 521 / 565, 896 608 / 618 / 621 / 637, 300 x 4 x 1600 x 32 637 / 655 / 660 / 726; eleven
+// as 3 3 3 2 0.99-1.10.  us, one query tile each / so, one card, L x 4 x L x 32: 300 41.8 / 40.9, 384 62.4 / 57.7, 512 131.6 / 122.2, 768 393.8 / 377.3, 1024 874 / 841,
 // 1491 2643 / 2564; 2048 x 4 x 256 x 32 165.9 / 162.1, 512 x 4 x 768 x 24 242.6 / 234.3; larger chunks of more query tiles: 1491 in chunks of 12 3521, of 6 2802, of 3 2704.
-// Seven and thirteen tiles stay single: one each / in twos / threes / fours 832 507 / 535 / 521 / 565, 896 608 / 618 / 621 / 637, 300 x 4 x 1600 x 32 637 / 655 / 660 / 726.
 // Every tile that a workgroup walks behind the first fetches K and V once more, in whole lines.  Where a line holds rows of other heads too, that costs more than it saves
 // unless so many workgroups still walk a head side by side that its lines are fetched no oftener than those of dense rows are when one workgroup walks all its tiles.
 // us, one tile each / in chunks: [.., 4 heads, 32] 384 67.1 / 83.6 (all three in one workgroup), 512 142.5 / 135.5 (two of four), 768 445.0 / 431.0 (three of six),
-// packed 512 157.8 / 144.8, 1000 994 / 1016 (four of eight) / 956 (two), 640 273 / 280 (2 2 1); 8 heads 512 x 256 90.8 / 116.7 (both); head_dim 24, packed 300 x 16 x 384
-// 239.6 / 371.2, 512 x 4 x 512 149.9 / 158.9 (two of four); k | v of a head in whole lines 384 64.6 / 62.2, 1000 x 4 x 150 63.9 / 53.4, across lines 96 x 16 x 768 x 24
-// 232 / 226 (two of six), 128 x 16 x 512 x 24 141 / 147 (two of four).  From 9 heads on K and V apart gain by no chunk: 128 x 16 x 512 x 32 packed 137.9 / 149.2,
-// 64 x 32 x 512 145.6 / 173.6, 64 x 16 x 1024 x 24 256.5 / 272.3 (two of eight); with 8 256 x 512 138.9 / 142.4, 200 x 512 126.2 / 120.9, 128 x 1024 234.6 / 235.7.
-void plan_chunks(const af3_dpa_params& p, int n_qtiles, int64_t per_xcd, int& chunk, int& parts, int64_t& chunked) {
+// packed 512 157.8 / 144.8, 1000 994 / 1016 (four of eight) / 956 (two), 640 273 / 280 (2 2 1); 8 heads 512 x 256 90.8 / 116.7 (both); k | v of a head in whole lines 384
+// 64.6 / 62.2, 1000 x 4 x 150 63.9 / 53.4, across lines 300 x 4 x 500 x 24 98.9 / 94.0 (two of four).  Rows apart from V's that lie across lines gain by no chunk (head_dim 24, packed
+// 512 x 4 x 512 149.9 / 158.9 in twos, 904 x 8 x 904 1335 / 1507), nor from 9 heads on does anything but whole lines (packed 300 x 16 x 384 x 24 239.6 / 371.2, 128 x 16 x 512 x 32
+// 137.9 / 149.2, 64 x 32 x 512 145.6 / 173.6, k | v across lines 128 x 16 x 512 x 24 141 / 147, 256 x 16 x 1232 x 24 1494 / 1582; with 8, packed 256 x 512 x 32 138.9 / 142.4, 200 x 512
+// 126.2 / 120.9, 128 x 1024 234.6 / 235.7), nor 2 2 1 (128 x 8 x 531 x 24 99.0 / 102.9); ending in single tiles they gain from three rounds on.
+void plan_chunks(const af3_dpa_params& p, int bmode, int n_qtiles, int64_t per_xcd, int& chunk, int& parts, int64_t& chunked) {
 	constexpr int64_t SLOTS = 64;
-	if(per_xcd * n_qtiles <= SLOTS) return;   // (one round as it is)
+	const int64_t tiles = per_xcd * n_qtiles;
+	if(tiles <= SLOTS) return;   // (one round as it is)
 	const kv_lines lines = lines_of_a_key(p);
-	if(lines.apart && p.H > 8) return;
-	const int most = lines.apart ? 3 : 4, room = lines.sum > lines.count && p.H > 8 ? 2 : 1;
-	auto whole_rounds = [&](int c) { const int64_t last = per_xcd * ((n_qtiles + c - 1) / c) % SLOTS; return last == 0 || last > SLOTS * 9 / 10; };
-	auto few_fetches  = [&](int c) { return c * lines.sum * room <= n_qtiles * lines.count; };
-	int  c = lines.apart ? 1 : n_qtiles == 5 && few_fetches(2) ? 2 : n_qtiles == 11 && few_fetches(3) ? 3 : 1;
-	for(int i = most; i >= 2; i--)
-		if(n_qtiles % i == 0 && few_fetches(i) && (c == 1 || whole_rounds(i) || !whole_rounds(c))) c = i;
+	const bool     five  = n_qtiles == 5;
+	if(lines.sum > lines.count && (five || p.H > 8 || (lines.apart && lines.sum > 2 * lines.count))) return;
+	auto few_fetches = [&](int c) { return c * lines.sum <= n_qtiles * lines.count; };
+	auto fullness    = [&](int c) {   // of the last round: 2, 1 or 0
+		const int64_t last = per_xcd * ((n_qtiles + c - 1) / c) % SLOTS;
+		return last == 0 || last > SLOTS * 9 / 10 ? 2 : last > SLOTS * 4 / 5 && c < 4 ? 1 : 0;
+	};
+	int c = five ? 2 : 1;
+	for(int i = lines.apart ? 3 : 4; i >= 2; i--)
+		if(n_qtiles % i == 0 && few_fetches(i) && (c == 1 || fullness(i) >= fullness(c))) c = i;
 	if(c == 1) return;
-	chunk = c, parts = (n_qtiles + c - 1) / c, chunked = per_xcd;
-	if(!whole_rounds(c)) {
-		const int64_t tail = (SLOTS + n_qtiles - 1) / n_qtiles;
-		chunked = per_xcd > tail ? per_xcd - tail : 0;
-	}
+	const bool whole  = fullness(c) > 0 && (!five || per_xcd * 3 <= SLOTS);
+	const bool partial = tiles % SLOTS > 0 && tiles % SLOTS <= SLOTS * 9 / 10;   // the last round of single ones
+	const bool enough  = five ? bmode != 3 && partial && tiles >= SLOTS * 3 : n_qtiles == 3 ? tiles * 4 >= SLOTS * 7 : c == 3 ? partial && tiles >= SLOTS * 5 :
+						 n_qtiles >= 8 ? partial && tiles >= SLOTS * 3 : tiles >= SLOTS * (lines.apart ? 3 : 2);
+	if(!whole && !enough) return;
+	chunk = c, parts = (n_qtiles + c - 1) / c;
+	chunked = whole ? per_xcd : per_xcd - (SLOTS + n_qtiles - 1) / n_qtiles;
 }
 
 // How a launch over b_count batch rows in groups of `rows` is laid out.
@@ -1124,7 +1136,7 @@ rows_launch lay_out(const af3_dpa_params& p, int rows, int bmode, int64_t b_coun
 	rows_launch l{};
 	l.n_qtiles = (int)((p.L + 127) / 128), l.n_groups = ((b_count + rows - 1) / rows) * p.H, l.per_xcd = (l.n_groups + 7) / 8;
 	l.chunk = 1, l.parts = l.n_qtiles;
-	if(several_query_tiles(rows, bmode, p.gate != nullptr) && p.out_dtype == AF3_BF16) plan_chunks(p, l.n_qtiles, l.per_xcd, l.chunk, l.parts, l.chunked);
+	if(several_query_tiles(rows, bmode, p.gate != nullptr) && p.out_dtype == AF3_BF16) plan_chunks(p, bmode, l.n_qtiles, l.per_xcd, l.chunk, l.parts, l.chunked);
 	l.blocks = (l.chunked * l.parts + (l.per_xcd - l.chunked) * l.n_qtiles) * 8;
 	// Workgroups of several query tiles go evenly whatever the last round holds: it consists of single tiles or is nearly whole.  us, by age / evenly / by the rule for
 	// single ones, L x 4 x L x 32: 300 40.3 / 40.0 / 40.5, 384 60.3 / 59.2 / 58.8, 400 86.8 / 87.4 / 87.7, 440 103.6 / 105.0 / 104.3, 500 121.5 / 119.1 / 118.8,

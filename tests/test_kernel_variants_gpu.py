@@ -503,7 +503,7 @@ def test_shared_bias_quick_and_careful_walks(af3, oracle, B, H, L, D, kind):
     assert (np.abs(out - want) / scale).max() <= 2e-2
 
 
-@pytest.mark.parametrize("B,H,L,D", [(404, 4, 300, 32), (261, 4, 264, 24), (130, 8, 512, 32), (96, 8, 640, 16), (500, 4, 200, 8), (128, 2, 1281, 32)])   # 3 of 3, 3 of 3, 2 of 4, 2 of 5, 2 of 2 and 3 of 11 query tiles one behind the other (with a gate the second, fourth and fifth: single ones); last ones in which one to three wavefronts have rows
+@pytest.mark.parametrize("B,H,L,D", [(404, 4, 300, 32), (261, 4, 264, 24), (130, 8, 512, 32), (96, 8, 640, 16), (500, 4, 200, 8), (128, 2, 1281, 32)])   # 3 of 3, 2 of 4 and 2 of 2 query tiles one behind the other (the last with a gate, the second, fourth and sixth: single ones); last ones in which one to three wavefronts have rows
 @pytest.mark.parametrize("kind", ["random", "no bias", "first tile", "none", "120", "120 and none"])
 @pytest.mark.parametrize("gated", [False, True])
 def test_shared_bias_query_tiles_in_one_workgroup(af3, B, H, L, D, kind, gated):
@@ -849,13 +849,12 @@ def _rows_plan(q, k, v, out, bias, gate):
 
 
 @pytest.mark.parametrize("B,H,L,D,gated,want", [
-    (460, 4, 460, 32, False, (4, 1, 4)),                                       # four tiles to a workgroup
-    (400, 4, 400, 32, False, (2, 3, 2)), (400, 4, 400, 32, True, (2, 3, 2)),   # two batch rows per wavefront
-    (404, 4, 300, 32, False, (2, 1, 3)), (404, 4, 300, 32, True, (2, 1, 3)),
+    (460, 4, 460, 32, False, (4, 1, 4)), (404, 4, 300, 32, False, (2, 1, 3)), (404, 4, 300, 32, True, (2, 1, 3)),   # two to four batch rows per wavefront, as many tiles
+    (400, 4, 400, 32, False, (2, 3, 2)), (400, 4, 400, 32, True, (2, 3, 2)),
     (384, 4, 384, 32, False, (3, 3, 3)), (384, 4, 384, 32, True, (3, 3, 3)),
-    (768, 2, 768, 32, True, (3, 1, 2)),
-    (640, 2, 768, 32, False, (4, 1, 2)),                                       # four and the workspace
-    (128, 16, 512, 32, False, (4, 3, 2)),                                      # four and a bias staged in place
+    (768, 2, 768, 32, False, (3, 1, 2)), (768, 2, 768, 32, True, (3, 1, 2)),
+    (461, 4, 300, 32, False, (4, 1, 3)), (640, 2, 768, 32, False, (4, 1, 2)),
+    (128, 16, 512, 32, False, (4, 3, 2)), (128, 8, 768, 32, False, (4, 3, 3)), (160, 4, 640, 32, False, (4, 3, 2)),
 ])
 @pytest.mark.parametrize("layout", ["dense", "per head"])   # [B, H, L, D] each; k, v, q and gate side by side for each token and head, the result [B, L, H, D]
 @pytest.mark.parametrize("kind", ["random", "no bias", "first tile", "none", "120", "k inf"])
