@@ -609,14 +609,18 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 
 }  // namespace
 
-// A strip's wavefronts meet only at its end; served by age, those that share a SIMD end one after the other.  The even walk pays from 2.5 tiles to a wavefront
-// on where one strip fills a compute unit, from more than two where two strips do; with fewer, its code costs more than it brings (the kernel's time is its
-// instructions), and the forms for those have none of it.  16 heads, us, without / with: one row of head_dim 24 560 5.92 / 5.98, 640 5.93 / 6.00,
-// 672 6.52 / 6.45, 704 6.56 / 6.48, 768 6.63 / 6.52, 1001 9.92 / 9.66, 1280 14.66 / 14.30; of 48 300 5.65 / 5.69, 640 7.41 / 7.51, 768 8.25 / 8.18; two strips to a
-// compute unit: 3 rows x 264 x 48 6.98 / 6.82, 4 x 264 x 24 6.54 / 6.41, 5 x 271 x 48 8.94 / 8.61, 4 x 320 x 48 8.59 / 8.44.  Strips of one block have no more
-// than two tiles, and head_dim 25 to 32 comes as triangles of few tokens.
+// A strip's wavefronts meet only at its end; served by age, those that share a SIMD end one after the other.  With few tiles to a wavefront the code of the even walk costs
+// more than it brings (the kernel's time is its instructions), and the forms for those have none of it.  Where one strip of eight wavefronts fills a compute unit, the older
+// wavefront of a SIMD takes the tile more where there is one: with one to four of the eight wavefronts so, going by age is what ends them together.  Even / by age, 8 heads of 24,
+// tiles: 18 to 20 1.00-1.01, 21 to 24 0.99-1.00, 25 to 28 1.02, 29 to 32 0.99-1.00, 33 to 36 1.03, 37 to 44 0.98-0.99; of 48 the same; 16 heads of 24 (odd rows) 18 to 20 1.01, 21 to
+// 24 0.97-0.98, 25 to 28 0.99-1.00, 29 to 32 0.96-0.97; from there on two strips of four wavefronts share a compute unit: more than two tiles to a wavefront are enough, 3 rows x
+// 264 x 48 6.98 us by age, 6.82 even, 4 x 264 x 24 6.54 / 6.41, 5 x 271 x 48 8.94 / 8.61, 4 x 320 x 48 8.59 / 8.44, 2 x 8 x 1105 x 24 13.2 / 12.7, one row of 16 x 1105 16.6 / 16.7.  Strips of one
+// block have no more than two tiles, and head_dim 25 to 32 comes as triangles of few tokens.
 constexpr bool may_go_evenly(int nb, int kind) { return nb > 1 && kind != 1; }
-static bool goes_evenly(int64_t L, int nw) { return (L + KT_S - 1) / KT_S > (nw == 4 ? 8 : 20); }
+static bool goes_evenly(int64_t L, int nw) {
+	const int64_t tiles = (L + KT_S - 1) / KT_S;
+	return nw == 4 ? tiles > 8 : tiles > 36 || (tiles > 20 && (tiles - 1) % 8 >= 4);
+}
 
 template <int NB, int KIND, bool ANY, int NW>
 static int launch_strip_n(const af3_dpa_params& p, hipStream_t s) {

@@ -789,7 +789,8 @@ def test_strips(af3, oracle, B, H, L, D, kind):
     assert np.abs(out - want).max() <= 2e-2
 
 
-@pytest.mark.parametrize("B,H,L,D", [(1, 16, 640, 24), (1, 16, 641, 24), (1, 16, 672, 48), (1, 16, 641, 40), (1, 16, 255, 24), (3, 16, 257, 24), (3, 16, 289, 48)])   # 20 and 21 tiles for eight wavefronts, 8 to 10 for four
+@pytest.mark.parametrize("B,H,L,D", [(1, 16, 640, 24), (1, 16, 641, 24), (1, 16, 672, 48), (1, 16, 641, 40), (1, 8, 800, 24), (1, 8, 897, 48), (1, 8, 1185, 24),
+                                     (1, 16, 255, 24), (3, 16, 257, 24), (3, 16, 289, 48)])   # 20, 21, 25, 29 and 38 tiles for eight wavefronts, 8 to 10 for four
 @pytest.mark.parametrize("kind", ["random", "three tiles", "one"])
 def test_strips_on_both_sides_of_the_even_walk(af3, oracle, B, H, L, D, kind):
     """The forms whose wavefronts go by age and those in which the ones behind go first, with few live tiles too."""
