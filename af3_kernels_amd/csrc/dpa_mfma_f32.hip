@@ -67,7 +67,7 @@ __device__ __forceinline__ void split3(float x0, float x1, uint32_t& hi, uint32_
 // DP: head_dim padded to 32 or 64.  NW: wavefronts per workgroup.  KS: wavefronts that share a block of 32 query rows, for
 // launches with too few blocks to fill the chip: wavefront ks takes tiles ks, ks + KS, ... of the walk, a step of the loop
 // moves KS tiles, and the partial (O, m, l) are merged through LDS at the end.
-template <int DP, int NW, int KS>
+template <int DP, int NW, int KS, bool EVEN>
 __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DP == 64 || KS > 1 ? 2 : NW == 4 ? 3 : 4))) dpa_mfma_f32_kernel(af3_dpa_params p, int n_qtiles, int64_t n_groups, int even) {
 	constexpr int NC   = DP / 16;             // contraction chunks of K.Q^T
 	constexpr int NDB  = DP / 32;             // 32-row blocks of O^T
@@ -431,11 +431,10 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DP
 		__syncthreads();
 		kt = ktn;
 	};
-	// (forms whose workgroups stand alone on a compute unit lose by the code: 2 x 4 x 128 x 32 6.33 / 6.41 us without / with it, 5 x 4 x 333 19.8 / 20.1, 32 x 4 x 300 22.5 / 22.7)
-	even_progress progress(n_steps, KS == 1 ? even : BY_AGE);
+	even_progress progress(n_steps, EVEN ? even : BY_AGE);
 	step(ic<1>{}, 0);
 	for(int j = 1; j < n_steps; j++) {
-		if constexpr(KS == 1) progress.at(j);
+		if constexpr(EVEN) progress.at(j);
 		step(ic<0>{}, j);
 	}
 	// Row numbers from here on come from the lane's number once more, out of the compiler's sight where the loop above has no
@@ -560,9 +559,15 @@ int launch(const af3_dpa_params& p, hipStream_t s) {
 	if(grid > 0x7fffffff) return AF3_ERR_BAD_SHAPE;
 	const size_t smem = (size_t)4 * KS * 3 * F32_KT * DP * 2 + (size_t)n_tiles * 4 + (size_t)n_tiles * 2 + 16;
 	const int64_t per_cu = DP == 64 ? 2 : 4;   // workgroups a compute unit holds, by their registers (KS = 1)
-	auto         kern = dpa_mfma_f32_kernel<DP, NW, KS>;
+	// Wavefronts that are behind on their walk go first (EVEN) where several workgroups stand on a compute unit and walk four tiles and more.  Elsewhere the code costs more than
+	// it brings, us without / with it: one workgroup to a compute unit 2 x 4 x 128 x 32 6.33 / 6.41, 5 x 4 x 333 19.8 / 20.1, 32 x 4 x 300 22.5 / 22.7; few tiles
+	// 100 x 8 x 22 x 48 13.9 / 14.2, 1 x 4 x 51 x 64 8.14 / 8.31, 100 x 4 x 74 x 8 9.49 / 9.64.
+	const int    even = KS == 1 && n_tiles >= 4 ? progress_mode(groups * n_qtiles, 256 * per_cu) : BY_AGE;
+	auto         kern = dpa_mfma_f32_kernel<DP, NW, KS, false>;
+	if constexpr(KS == 1)
+		if(even != BY_AGE) kern = dpa_mfma_f32_kernel<DP, NW, KS, true>;
 	if(smem > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) return AF3_ERR_LAUNCH;
-	hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(NW * 64), smem, s, p, n_qtiles, groups, progress_mode(groups * n_qtiles, 256 * per_cu));
+	hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(NW * 64), smem, s, p, n_qtiles, groups, even);
 	return launch_status();
 }
 

@@ -630,7 +630,7 @@ def _kernels_with_priorities(tmp_path):
 
 def test_priorities_stand_where_they_act(tmp_path):
     """Kernel forms whose wavefronts have nobody to go before hold none of the code for it: their time is their instructions.  Strips of two blocks of
-    rows and more, head_dim up to 24 and from 33 on, have a form with it for longer walks and one without; the fp32 kernel has it where several
+    rows and more, head_dim up to 24 and from 33 on, have a form with it for longer walks and one without; so has the fp32 kernel where several
     workgroups stand on a compute unit."""
     names, raising = _kernels_with_priorities(tmp_path)
     strips = {}
@@ -645,8 +645,9 @@ def test_priorities_stand_where_they_act(tmp_path):
         assert strips[f] not in raising
         assert (f[:4] + (1,) in strips) == (f[0] > 1 and f[1] != 1)
     assert all(strips[f] in raising for f in strips if f[4] == 1)
-    fp32 = {name: int(m.group(1)) for name in names if (m := re.search(r"dpa_mfma_f32_kernelILi\d+ELi\dELi(\d)EE", name))}
-    assert len(fp32) == 7 and {name for name, parts in fp32.items() if parts == 1} == raising & set(fp32)
+    fp32 = {name: m.groups() for name in names if (m := re.search(r"dpa_mfma_f32_kernelILi\d+ELi\dELi(\d)ELb([01])EE", name))}
+    assert len(fp32) == 7 + 2 and all(parts == "1" or even == "0" for parts, even in fp32.values())
+    assert {name for name, (_, even) in fp32.items() if even == "1"} == raising & set(fp32)
 
 
 def _rows_plan(B, H, L, D, layout="dense", gate=False, bias=True, out=1, always=False):
